@@ -279,6 +279,20 @@ int fused_psi_fxy(qp_field2d *q, qp_field2d *psi, qp_field2d *fxy);
 int fused_pass(const PassFields &f, double dex, bool qp, int l, double tol, int seed = 0,
                qp_field2d *ehist = nullptr, const int *seed_hist = nullptr,
                qp_field2d *ehist2 = nullptr);
+// The same solves with the y transforms and the modes in one kernel
+// (qp_spectral.hip), on the grids fused_fields accepts: a corrector pass from
+// the deposited cu, dcu, amu to psit and bxyz in real space (fft_r2k_batch,
+// fused_pass and fft_k2r_batch), and the start of a slice from its charges to
+// fxy, psi, psit and bxyz (both transforms of the charges' fields, elf,
+// fused_psi_fxy and the predictor)
+struct FrontFields {
+    qp_field2d *qb, *qe, *psi, *fxy;
+    qp_field2d *ehist, *ehist2;   // the corrector seed's history (or null), as fused_pass
+};
+bool fused_fields(const qp_ctx *c);
+int fused_solve_pass(const PassFields &f, double dex, int l, double tol);
+int fused_solve_front(const PassFields &f, const FrontFields &fr, double dex, int seed,
+                      const int *seed_hist);
 // Anderson mixing (depth 1) of the corrector iterate after pass l (f.gprev,
 // f.fprev set; the pass was run by fused_pass with them): unless pass l has
 // converged, epw <- g_l - gamma (g_l - g_{l-1}) and B_perp reassembled; mix =

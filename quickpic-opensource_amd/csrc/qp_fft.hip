@@ -22,66 +22,9 @@
 // the other powers formed by complex products).  A batch holds up to 8 components of
 // any fields (grid.y); an LDS-tiled transpose sits between the x and the y
 // pass.
-#include "qp_common.h"
+#include "qp_fft.h"
 
 namespace qp {
-
-template <typename R>
-__device__ __forceinline__ cplx<R> cmul(cplx<R> a, cplx<R> b)
-{
-    return {a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x};
-}
-template <typename R>
-__device__ __forceinline__ cplx<R> cadd(cplx<R> a, cplx<R> b) { return {a.x + b.x, a.y + b.y}; }
-template <typename R>
-__device__ __forceinline__ cplx<R> csub(cplx<R> a, cplx<R> b) { return {a.x - b.x, a.y - b.y}; }
-// -i z
-template <typename R>
-__device__ __forceinline__ cplx<R> cmi(cplx<R> a) { return {a.y, -a.x}; }
-
-// forward DFT of 4 points in place (natural order)
-template <typename R>
-__device__ __forceinline__ void dft4(cplx<R> &a0, cplx<R> &a1, cplx<R> &a2, cplx<R> &a3)
-{
-    cplx<R> t0 = cadd(a0, a2), t1 = csub(a0, a2), t2 = cadd(a1, a3), t3 = cmi(csub(a1, a3));
-    a0 = cadd(t0, t2);
-    a1 = cadd(t1, t3);
-    a2 = csub(t0, t2);
-    a3 = csub(t1, t3);
-}
-
-// forward DFT of 8 points in place (natural order): decimation in frequency,
-// X[2m] = DFT4(v[n] + v[n+4]), X[2m+1] = DFT4((v[n] - v[n+4]) w^n), w = e^{-i pi/4}
-template <typename R>
-__device__ __forceinline__ void dft8(cplx<R> *v)
-{
-    const R h = (R)0.70710678118654752440;
-    cplx<R> a0 = cadd(v[0], v[4]), a1 = cadd(v[1], v[5]), a2 = cadd(v[2], v[6]),
-            a3 = cadd(v[3], v[7]);
-    cplx<R> c0 = csub(v[0], v[4]), c1 = csub(v[1], v[5]), c2 = csub(v[2], v[6]),
-            c3 = csub(v[3], v[7]);
-    c1 = {(c1.x + c1.y) * h, (c1.y - c1.x) * h};     // * e^{-i pi/4}
-    c2 = cmi(c2);                                      // * e^{-i pi/2}
-    c3 = {(c3.y - c3.x) * h, -(c3.x + c3.y) * h};    // * e^{-3i pi/4}
-    dft4(a0, a1, a2, a3);
-    dft4(c0, c1, c2, c3);
-    v[0] = a0; v[2] = a1; v[4] = a2; v[6] = a3;
-    v[1] = c0; v[3] = c1; v[5] = c2; v[7] = c3;
-}
-
-// LDS index of FFT point i: one pad point after every 2^PS points
-template <int PS> __device__ __forceinline__ int padk(int i) { return i + (i >> PS); }
-
-template <int L, int PS = 3> struct FftShape {
-    static constexpr int M = 1 << L;                // complex points
-    static constexpr int N = M / 2;                 // transform length n
-    static constexpr int TF = M / 8;                // threads per transform
-    static constexpr int BS = TF > 256 ? TF : 256;  // threads per block
-    static constexpr int FB = BS / TF;              // transforms per block
-    static constexpr int NR8 = L / 3;               // radix-8 passes
-    static constexpr int REM = L % 3;               // closing radix-2 (1) / radix-4 (2)
-    static constexpr int LDSM = M + (M >> PS) + 1;  // padded LDS points per transform
-};
 
 template <typename R> struct CompSet {
     const R *src[8];
@@ -112,7 +55,7 @@ k_fft_rows(CompSet<R> cs, int nrows, int ld_src, int ld_dst, int types, R scale,
         return;
     }
     if (blockIdx.x == 0 && blockIdx.y == 0) run_res_job(rj);
-    constexpr int M = S::M, n = S::N, TF = S::TF;
+    constexpr int n = S::N, TF = S::TF;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     const int comp = blockIdx.y;
     const int type = (types >> comp) & 1;   // 0 sine, 1 cosine
@@ -122,11 +65,10 @@ k_fft_rows(CompSet<R> cs, int nrows, int ld_src, int ld_dst, int types, R scale,
     const bool live = ra < nrows, hb = ra + 1 < nrows;
     cplx<R> *buf = reinterpret_cast<cplx<R> *>(smem_raw) + f * S::LDSM;
 
-    // first pass: radix 8 on the extension, straight from memory.  The 16
-    // data loads are issued first and unconditionally (a missing second row
-    // re-reads the first, a block past the last row reads row 0; the values
-    // are then discarded), so one memory latency covers them and the twiddle
-    // loads issued after them.
+    // The extension straight from memory: the 16 data loads are issued first
+    // and unconditionally (a missing second row re-reads the first, a block
+    // past the last row reads row 0; the values are then discarded), so one
+    // memory latency covers them and the twiddle loads issued after them.
     R la[8], lb[8];
     {
         const R *base = cs.src[comp];
@@ -135,8 +77,7 @@ k_fft_rows(CompSet<R> cs, int nrows, int ld_src, int ld_dst, int types, R scale,
         const R *sb = (COL != 1 && live && hb) ? sa + ld_src : sa;
 #pragma unroll
         for (int r = 0; r < 8; ++r) {
-            const int idx = t + r * TF;
-            const int e = idx <= n ? idx : M - idx;
+            const int e = ext_pos<L>(t + r * TF);
             if (COL == 1) {
                 // the pair of columns ra, ra+1 of row e (ra even, ld_src even)
                 const cplx<R> p2 = *reinterpret_cast<const cplx<R> *>(sa + (size_t)e * ld_src);
@@ -148,143 +89,34 @@ k_fft_rows(CompSet<R> cs, int nrows, int ld_src, int ld_dst, int types, R scale,
             }
         }
     }
-
-    // twiddles of every pass after the first: pass p (Ns = 8^p) needs
-    // W^(r e), e = (t mod Ns) M / (8 Ns), r = 1..7: W^e, W^2e and W^4e come
-    // from the table, the other four are their products; the closing radix-4
-    // pass needs W^j, W^2j (table) and W^3j, the closing radix-2 pass W^j
-    constexpr int NTW8 = S::NR8 > 1 ? 3 * (S::NR8 - 1) : 1;
-    cplx<R> tw8[NTW8];
+    Twiddles<R, L> tw;
+    tw.load(W, t);
+    cplx<R> v[8], z[4], zn;
 #pragma unroll
-    for (int p = 1; p < S::NR8; ++p) {
-        const int Ns = 1 << (3 * p);
-        const int e = (t & (Ns - 1)) * (M / (8 * Ns));
-        tw8[3 * (p - 1)] = W[e];
-        tw8[3 * (p - 1) + 1] = W[2 * e];
-        tw8[3 * (p - 1) + 2] = W[4 * e];
-    }
-    constexpr int NTWR = S::REM == 2 ? 4 : (S::REM == 1 ? 4 : 1);
-    cplx<R> twr[NTWR];
-    if (S::REM == 2) {
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            twr[2 * s] = W[t + s * TF];
-            twr[2 * s + 1] = W[2 * (t + s * TF)];
-        }
-    } else if (S::REM == 1) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) twr[s] = W[t + s * TF];
-    }
-
-    cplx<R> v[8];
-#pragma unroll
-    for (int r = 0; r < 8; ++r) {
-        const int idx = t + r * TF;
-        const int e = idx <= n ? idx : M - idx;
-        R va = live ? la[r] : R(0);
-        R vb = (live && hb) ? lb[r] : R(0);
-        if (type == 0) {
-            const bool edge = e == 0 || e == n;
-            const R sg = idx > n ? R(-1) : R(1);
-            va = edge ? R(0) : sg * va;
-            vb = edge ? R(0) : sg * vb;
-        }
-        v[r] = {va, vb};
-    }
-    dft8(v);
+    for (int r = 0; r < 8; ++r)
+        v[r] = ext_value<R, L>(type, t + r * TF, live ? la[r] : R(0), (live && hb) ? lb[r] : R(0));
+    fft_core<R, L, PS>(v, buf, t, tw, z, zn);
+    if (!live) return;
 
     const R half = scale * R(0.5);
     R *da = cs.dst[comp] + (COL == 2 ? (size_t)ra : (size_t)ra * ld_dst);
     R *db = da + ld_dst;
     R *dg = (guard_row >= 0 && ra == 0) ? cs.dst[comp] + (size_t)guard_row * ld_dst : nullptr;
-    auto emit = [&](int k, cplx<R> z) {
-        if (!live || k > n) return;
-        R oa, ob;
-        if (type == 1) {
-            oa = z.x * half;
-            ob = z.y * half;
-        } else if (k == 0 || k == n) {
-            oa = R(0);
-            ob = R(0);
-        } else {
-            oa = -z.y * half;
-            ob = z.x * half;
-        }
+    auto emit = [&](int k, cplx<R> x) {
+        const cplx<R> o = row_values<R, L>(type, k, x, half);
         if (COL == 2) {
             R *d = da + (size_t)k * ld_dst;
-            if (hb) *reinterpret_cast<cplx<R> *>(d) = cplx<R>{oa, ob};
-            else d[0] = oa;
+            if (hb) *reinterpret_cast<cplx<R> *>(d) = o;
+            else d[0] = o.x;
         } else {
-            da[k] = oa;
-            if (hb) db[k] = ob;
-            if (dg) dg[k] = oa;
+            da[k] = o.x;
+            if (hb) db[k] = o.y;
+            if (dg) dg[k] = o.x;
         }
     };
-
-    if (S::NR8 == 1 && S::REM == 0) {   // M = 8 is below the supported sizes
 #pragma unroll
-        for (int r = 0; r < 8; ++r) emit(t + r * TF, v[r]);
-        return;
-    }
-    // first pass output (Ns = 1): index 8 t + r
-#pragma unroll
-    for (int r = 0; r < 8; ++r) buf[padk<PS>(8 * t + r)] = v[r];
-
-    // middle radix-8 passes
-#pragma unroll
-    for (int p = 1; p < S::NR8; ++p) {
-        const int Ns = 1 << (3 * p);
-        __syncthreads();
-        {
-            const cplx<R> w1 = tw8[3 * (p - 1)], w2 = tw8[3 * (p - 1) + 1],
-                          w4 = tw8[3 * (p - 1) + 2];
-            const cplx<R> w3 = cmul(w1, w2);
-            const cplx<R> w[8] = {w1, w1, w2, w3, w4, cmul(w1, w4), cmul(w2, w4), cmul(w3, w4)};
-#pragma unroll
-            for (int r = 0; r < 8; ++r) {
-                v[r] = buf[padk<PS>(t + r * TF)];
-                if (r) v[r] = cmul(v[r], w[r]);
-            }
-        }
-        dft8(v);
-        if (p == S::NR8 - 1 && S::REM == 0) {
-            // last pass (Ns = M/8): output index t + r M/8 goes to memory
-#pragma unroll
-            for (int r = 0; r < 8; ++r) emit(t + r * TF, v[r]);
-            return;
-        }
-        __syncthreads();
-        const int base = (t / Ns) * Ns * 8 + (t & (Ns - 1));
-#pragma unroll
-        for (int r = 0; r < 8; ++r) buf[padk<PS>(base + r * Ns)] = v[r];
-    }
-    __syncthreads();
-    if (S::REM == 2) {
-        // closing radix 4 (Ns = M/4): butterflies t and t + TF
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            const int j = t + s * TF;
-            const cplx<R> w1 = twr[2 * s], w2 = twr[2 * s + 1];
-            cplx<R> a0 = buf[padk<PS>(j)];
-            cplx<R> a1 = cmul(buf[padk<PS>(j + M / 4)], w1);
-            cplx<R> a2 = cmul(buf[padk<PS>(j + M / 2)], w2);
-            cplx<R> a3 = cmul(buf[padk<PS>(j + 3 * M / 4)], cmul(w1, w2));
-            dft4(a0, a1, a2, a3);
-            emit(j, a0);
-            emit(j + M / 4, a1);
-            emit(j + M / 2, a2);
-        }
-    } else {
-        // closing radix 2 (Ns = M/2): butterflies t + s TF
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const int j = t + s * TF;
-            cplx<R> a0 = buf[padk<PS>(j)];
-            cplx<R> a1 = cmul(buf[padk<PS>(j + M / 2)], twr[s]);
-            emit(j, cadd(a0, a1));
-            emit(j + M / 2, csub(a0, a1));
-        }
-    }
+    for (int i = 0; i < 4; ++i) emit(t + i * TF, z[i]);
+    if (t == 0) emit(n, zn);
 }
 
 // dst(c)[col][row] = src(c)[row][col] for row < rows, col < cols, by TS x TS
@@ -399,11 +231,6 @@ static int transpose(qp_ctx *c, const CompSet<R> &cs, int ncomp, int ld_src, int
     QP_LAUNCH_CHECK();
     return QP_OK;
 }
-
-// LDS padding of the transforms by default: one pad point per 16 points in
-// FP32 (a third fewer LDS bank conflicts than per 8 at 2048 points, measured
-// on MI355X), per 8 in FP64
-template <typename R> constexpr int pad_shift() { return sizeof(R) == 4 ? 4 : 3; }
 
 // the row transforms of the transpose path; QP_TUNE_FFT values 2-4 select
 // another LDS padding (one pad point per 8, 32 or 4 points)

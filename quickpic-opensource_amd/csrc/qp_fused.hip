@@ -3,7 +3,7 @@
 // mode by mode or node by node, with the same operations in the same order,
 // so its results are those of the separate calls; it only saves the launches
 // and the intermediate planes.
-#include "qp_common.h"
+#include "qp_pass.h"
 
 namespace qp {
 
@@ -85,46 +85,20 @@ k_pass(KGrid g, const R *__restrict__ ffg, const R *__restrict__ ffs, const R *_
             }
             ehist[o] = e1;
             ehist[cs + o] = e2;
-            if (seed == 2) {
-                e1 = R(2) * e1 - h1;
-                e2 = R(2) * e2 - h2;
-                epw[o] = e1;
-                epw[cs + o] = e2;
-            } else if (seed == 3) {
-                e1 = (R(3) * e1 - R(3) * h1) + g1;
-                e2 = (R(3) * e2 - R(3) * h2) + g2;
+            if (seed >= 2) {
+                e1 = seed_mode(seed, e1, h1, g1);
+                e2 = seed_mode(seed, e2, h2, g2);
                 epw[o] = e1;
                 epw[cs + o] = e2;
             }
         }
         if (QP) {
             const R old1 = e1, old2 = e2;
-            R n1 = R(0), n2 = R(0);
-            if (tab) {
-                R at2 = R(1) * fg / (R(1) + aa * fg);
-                R at1 = at2 * fs;
-                if (kx > 0 && ky > 0) {
-                    R d1 = -dcu[o] + dkx * amu[o] - dky * amu[2 * cs + o];
-                    R aat1 = d1 - dkx * c3 * idex;
-                    R d2 = -dcu[cs + o] - dkx * amu[2 * cs + o] + dky * amu[cs + o];
-                    R aat2 = d2 - dky * c3 * idex;
-                    dcu[o] = d1;
-                    dcu[cs + o] = d2;
-                    n1 = at1 * aat1 + aa * at2 * old1;
-                    n2 = at1 * aat2 + aa * at2 * old2;
-                } else if (kx > 0) {
-                    R d1 = -dcu[o] + dkx * amu[o];
-                    R d2 = -dcu[cs + o] - dkx * amu[2 * cs + o];
-                    dcu[o] = d1;
-                    dcu[cs + o] = d2;
-                    n2 = at1 * d2 + aa * at2 * old2;
-                } else if (ky > 0) {
-                    R d1 = -dcu[o] - dky * amu[2 * cs + o];
-                    R d2 = -dcu[cs + o] + dky * amu[cs + o];
-                    dcu[o] = d1;
-                    dcu[cs + o] = d2;
-                    n1 = at1 * d1 + aa * at2 * old1;
-                }
+            R n1, n2, d1 = dcu[o], d2 = dcu[cs + o];
+            if (corrector_mode(tab, kx, ky, fg, fs, dkx, dky, aa, idex, c3, amu[o], amu[cs + o],
+                               amu[2 * cs + o], old1, old2, d1, d2, n1, n2)) {
+                dcu[o] = d1;
+                dcu[cs + o] = d2;
             }
             epw[o] = n1;
             epw[cs + o] = n2;
@@ -143,18 +117,9 @@ k_pass(KGrid g, const R *__restrict__ ffg, const R *__restrict__ ffs, const R *_
             e1 = n1;
             e2 = n2;
         }
-        // psit: div (MPPDIVFD2) -> pot (MPPOTPD2) -> * (-dex)
-        R ps = R(0);
-        if (kx > 0 && kx < g.nx && ky > 0 && ky < g.ny) ps = fg * (-(dkx * c1 + dky * c2));
-        psit[o] = ps * (-dex);
-        // bf (MPPBBPOISD23, ci = 1): only its z component survives the assembly
-        R b3 = R(0);
-        if (tab) {
-            const R at1 = R(1) * fg * fs;
-            if (kx > 0 && ky > 0) b3 = (dkx * at1) * c2 - (dky * at1) * c1;
-            else if (kx > 0) b3 = dkx * at1 * c2;
-            else if (ky > 0) b3 = -(dky * at1) * c1;
-        }
+        const bool inner = kx > 0 && kx < g.nx && ky > 0 && ky < g.ny;
+        psit[o] = psit_mode(inner, fg, dkx, dky, c1, c2, dex);
+        const R b3 = bz_mode(tab, kx, ky, fg, fs, dkx, dky, c1, c2);
         bxyz[o] = e2 * (-dex) - epwb[cs + o];
         bxyz[cs + o] = e1 * dex + epwb[o];
         bxyz[2 * cs + o] = b3 * dex;

@@ -1,0 +1,69 @@
+// The slice loop's k-space arithmetic of one mode, shared by the kernels that
+// run it on its own (qp_fused.hip) and between transforms (qp_spectral.hip).
+#pragma once
+
+#include "qp_common.h"
+
+namespace qp {
+
+// One mode of PBPOISD22N_QP isign = 1 (bfqp): d1, d2 (dcu) and n1, n2 (the
+// new B_perp from the old one) of mode (kx, ky); modes off the tables (tab =
+// false) and (0, 0) keep dcu and get zero.  Returns whether dcu changed.
+template <typename R>
+__device__ __forceinline__ bool corrector_mode(bool tab, int kx, int ky, R fg, R fs, R dkx, R dky,
+                                               R aa, R idex, R c3, R a1, R a2, R a3, R old1,
+                                               R old2, R &d1, R &d2, R &n1, R &n2)
+{
+    n1 = n2 = R(0);
+    if (!tab || (kx == 0 && ky == 0)) return false;
+    const R at2 = R(1) * fg / (R(1) + aa * fg);
+    const R at1 = at2 * fs;
+    if (kx > 0 && ky > 0) {
+        d1 = -d1 + dkx * a1 - dky * a3;
+        const R aat1 = d1 - dkx * c3 * idex;
+        d2 = -d2 - dkx * a3 + dky * a2;
+        const R aat2 = d2 - dky * c3 * idex;
+        n1 = at1 * aat1 + aa * at2 * old1;
+        n2 = at1 * aat2 + aa * at2 * old2;
+    } else if (kx > 0) {
+        d1 = -d1 + dkx * a1;
+        d2 = -d2 - dkx * a3;
+        n2 = at1 * d2 + aa * at2 * old2;
+    } else {
+        d1 = -d1 - dky * a3;
+        d2 = -d2 + dky * a2;
+        n1 = at1 * d1 + aa * at2 * old1;
+    }
+    return true;
+}
+
+// div (MPPDIVFD2) -> pot (MPPOTPD2) -> * (-dex) of the current: psit
+template <typename R>
+__device__ __forceinline__ R psit_mode(bool inner, R fg, R dkx, R dky, R c1, R c2, R dex)
+{
+    const R ps = inner ? fg * (-(dkx * c1 + dky * c2)) : R(0);
+    return ps * (-dex);
+}
+
+// bf (MPPBBPOISD23, ci = 1): only its z component survives the B assembly
+template <typename R>
+__device__ __forceinline__ R bz_mode(bool tab, int kx, int ky, R fg, R fs, R dkx, R dky, R c1, R c2)
+{
+    if (!tab) return R(0);
+    const R at1 = R(1) * fg * fs;
+    if (kx > 0 && ky > 0) return (dkx * at1) * c2 - (dky * at1) * c1;
+    if (kx > 0) return dkx * at1 * c2;
+    if (ky > 0) return -(dky * at1) * c1;
+    return R(0);
+}
+
+// The seed by extrapolation in xi of one component: e = B(j-1) becomes 2 e - h
+// (seed 2) or 3 e - 3 h + g (seed 3), h = B(j-2), g = B(j-3)
+template <typename R> __device__ __forceinline__ R seed_mode(int seed, R e, R h, R g)
+{
+    if (seed == 2) return R(2) * e - h;
+    if (seed == 3) return (R(3) * e - R(3) * h) + g;
+    return e;
+}
+
+}  // namespace qp

@@ -226,24 +226,19 @@ int qp_sim_begin_step(qp_sim *s)
 //    runs at the end of this one, beside psit's;
 //  * -fxy + B, the predictor cu -= dxi dcu and the slice writes are one
 //    kernel each.
-// first part of a slice: beam and plasma charge, psi, E_perp, the psi
-// gather (:650-670), up to the corrector seed
-int qp_slice_prepare(qp_sim *s, int j)
+
+// beam charge (:650-655) and plasma charge (:657-661) of slice j
+static int slice_charges(qp_sim *s, int j)
 {
-    QP_REQUIRE(s, QP_ERR_ARG, "qp_slice_prepare: null sim");
     qp_ctx *c = s->ctx;
     QP_REQUIRE(j >= 1 && j <= c->nz, QP_ERR_ARG, "qp_slice_prepare: slice %d outside 1..%d", j,
                c->nz);
-    qp_field2d **F = s->f;
-    qp_field2d *qb = F[QP_F_QB], *qe = F[QP_F_QE], *psi = F[QP_F_PSI], *fxy = F[QP_F_FXY];
-    qp_field2d *epwb = F[QP_F_EPWB];
+    qp_field2d *qb = s->f[QP_F_QB], *qe = s->f[QP_F_QE];
     const int nsp = (int)s->sp.size();
     // the move check of an earlier slice, if it has arrived (captured
     // slices leave the error word on the device; qp_scan_run reads it)
     if (!s->graph)
         for (qp_species *sp : s->sp) RC(species_check_poll(sp, false));
-    // beam charge (:650-655) and plasma charge (:657-661); the two forward
-    // transforms are independent and run as one batch
     const int *jdev = s->graph ? s->ctl.as<int>() : nullptr;
     if (s->bm.empty()) RC(qp_field2d_as(qb, 0.0));
     for (size_t i = 0; i < s->bm.size(); ++i) {
@@ -253,10 +248,23 @@ int qp_slice_prepare(qp_sim *s, int j)
     if (nsp == 0) RC(qp_field2d_as(qe, 0.0));
     for (int i = 0; i < nsp; ++i) RC(species_qdp_fused(s->sp[i], qe, i == 0));
     QP_REQUIRE(qb->state == 0 && qe->state == 0, QP_ERR_STATE, "fftrk: data is in ks");
+    return QP_OK;
+}
+
+// first part of a slice: beam and plasma charge, psi, E_perp, the psi
+// gather (:650-670), up to the corrector seed
+int qp_slice_prepare(qp_sim *s, int j)
+{
+    QP_REQUIRE(s, QP_ERR_ARG, "qp_slice_prepare: null sim");
+    RC(slice_charges(s, j));
+    qp_field2d **F = s->f;
+    qp_field2d *qb = F[QP_F_QB], *qe = F[QP_F_QE], *psi = F[QP_F_PSI], *fxy = F[QP_F_FXY];
+    qp_field2d *epwb = F[QP_F_EPWB];
+    // the two forward transforms are independent and run as one batch
     {
         qp_field2d *fs[2] = {qb, qe};
         const int kinds[2] = {1, 1};
-        RC(fft_r2k_batch(c, fs, kinds, 2));
+        RC(fft_r2k_batch(s->ctx, fs, kinds, 2));
         qb->state = qe->state = 1;
     }
     // the beam's transverse field (:656), psi and E_perp (:662-666)
@@ -265,7 +273,7 @@ int qp_slice_prepare(qp_sim *s, int j)
     {
         qp_field2d *fs[2] = {fxy, psi};
         const int kinds[2] = {1, 1};
-        RC(fft_k2r_batch(c, fs, kinds, 2));
+        RC(fft_k2r_batch(s->ctx, fs, kinds, 2));
         fxy->state = psi->state = 0;
     }
     // the species' psi gather (:667-669) runs inside the first corrector pass
@@ -273,12 +281,13 @@ int qp_slice_prepare(qp_sim *s, int j)
     return QP_OK;
 }
 
-// the rest of the slice: corrector seed, predictor, passes, push, slice writes
-int qp_slice_finish(qp_sim *s, int j, int iter_max, double tol, int *iters_used, double *residual)
+// the rest of the slice: corrector seed, predictor, passes, push, slice
+// writes.  front: only the charges are there (slice_charges); the fields of
+// qp_slice_prepare are solved for together with the predictor's.
+static int slice_finish(qp_sim *s, int j, int iter_max, double tol, int *iters_used,
+                        double *residual, bool front)
 {
-    QP_REQUIRE(s, QP_ERR_ARG, "qp_slice_finish: null sim");
     qp_ctx *c = s->ctx;
-    QP_REQUIRE(s->prepared == j, QP_ERR_STATE, "qp_slice_finish: slice %d was not prepared", j);
     QP_REQUIRE(iter_max >= 1, QP_ERR_ARG, "qp_slice_finish: iter_max %d", iter_max);
     s->prepared = 0;
     const double dex = c->dex, dxi = c->dxi;
@@ -312,11 +321,18 @@ int qp_slice_finish(qp_sim *s, int j, int iter_max, double tol, int *iters_used,
         seed = s->hist_slices >= 3 ? 3 : (s->hist_slices >= 2 ? 2 : 1);
         ++s->hist_slices;
     }
-    RC(fused_pass(pf, dex, false, 0, 0.0, seed, s->epw_hist,
-                  graph && seed ? s->ctl.as<int>() + 1 : nullptr,
-                  quad ? s->epw_hist2 : nullptr));
-    RC(fft_k2r_batch(c, inv, inv_kinds, 2));
-    psit->state = bxyz->state = 0;
+    const int *seed_hist = graph && seed ? s->ctl.as<int>() + 1 : nullptr;
+    if (front) {
+        const FrontFields fr{F[QP_F_QB], F[QP_F_QE], psi, fxy, s->epw_hist,
+                             quad ? s->epw_hist2 : nullptr};
+        RC(fused_solve_front(pf, fr, dex, seed, seed_hist));
+    } else {
+        RC(fused_pass(pf, dex, false, 0, 0.0, seed, s->epw_hist, seed_hist,
+                      quad ? s->epw_hist2 : nullptr));
+        RC(fft_k2r_batch(c, inv, inv_kinds, 2));
+        psit->state = bxyz->state = 0;
+    }
+    const bool fused = fused_fields(c) && !mixing;
     // corrector passes (:676-710)
     int *flags = c->flags.as<int>();
     // launches of pass l carry tag tag0 + l, unique to this slice, so that
@@ -344,6 +360,11 @@ int qp_slice_finish(qp_sim *s, int j, int iter_max, double tol, int *iters_used,
     auto tail = [&](int l) -> int {
         c->prof_tag = tag0 + l;
         if (c->skip) c->skip = flags + (l - 1);
+        if (fused) {
+            RC(fused_solve_pass(pf, dex, l, tol));
+            c->prof_tag = 0;
+            return QP_OK;
+        }
         RC(fft_r2k_batch(c, fwd, fwd_kinds, 3));
         cu->state = dcu->state = amu->state = 1;
         RC(fused_pass(pc, dex, true, l, tol));
@@ -464,6 +485,13 @@ int qp_slice_finish(qp_sim *s, int j, int iter_max, double tol, int *iters_used,
     return QP_OK;
 }
 
+int qp_slice_finish(qp_sim *s, int j, int iter_max, double tol, int *iters_used, double *residual)
+{
+    QP_REQUIRE(s, QP_ERR_ARG, "qp_slice_finish: null sim");
+    QP_REQUIRE(s->prepared == j, QP_ERR_STATE, "qp_slice_finish: slice %d was not prepared", j);
+    return slice_finish(s, j, iter_max, tol, iters_used, residual, false);
+}
+
 int qp_slice_residuals(const qp_sim *s, double *res, int max, int *n)
 {
     QP_REQUIRE(s && res && n && max >= 0, QP_ERR_ARG, "qp_slice_residuals: bad argument");
@@ -478,8 +506,13 @@ int qp_slice_residuals(const qp_sim *s, double *res, int max, int *n)
 
 int qp_slice_run(qp_sim *s, int j, int iter_max, double tol, int *iters_used, double *residual)
 {
-    RC(qp_slice_prepare(s, j));
-    return qp_slice_finish(s, j, iter_max, tol, iters_used, residual);
+    QP_REQUIRE(s, QP_ERR_ARG, "qp_slice_run: null sim");
+    if (!fused_fields(s->ctx)) {
+        RC(qp_slice_prepare(s, j));
+        return qp_slice_finish(s, j, iter_max, tol, iters_used, residual);
+    }
+    RC(slice_charges(s, j));
+    return slice_finish(s, j, iter_max, tol, iters_used, residual, true);
 }
 
 int qp_sim_push_beams(qp_sim *s)
@@ -568,8 +601,7 @@ static int scan_capture(qp_scan *sc, int parity)
         if (e != hipSuccess) { rc = hip_fail(e, "hipStreamWaitEvent", __FILE__, __LINE__); break; }
         const int hist = s->hist_slices;   // the captured seed counts on the device
         s->graph = true;
-        rc = qp_slice_prepare(s, 1);
-        if (!rc) rc = qp_slice_finish(s, 1, sc->iter_max, sc->tol, nullptr, nullptr);
+        rc = qp_slice_run(s, 1, sc->iter_max, sc->tol, nullptr, nullptr);
         s->graph = false;
         s->prepared = 0;
         s->hist_slices = hist;

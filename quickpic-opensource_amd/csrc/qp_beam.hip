@@ -821,6 +821,19 @@ int beam_slice_assign(qp_beam *b, qp_field2d *q, int slice, const int *jdev)
 {
     return slice_copy(b, q, slice, 1, jdev);
 }
+// the same as a job for another kernel
+int beam_slice_plane(qp_beam *b, qp_field2d *q, int slice, const int *jdev, BeamPlane *bp)
+{
+    BCHECK(b);
+    QP_REQUIRE(q && q->dim >= 1, QP_ERR_ARG, "qdpcopy: bad field");
+    qp_ctx *c = b->ctx;
+    QP_REQUIRE(jdev || (slice >= 1 && slice <= c->nz + 1), QP_ERR_ARG, "qdpcopy: slice %d", slice);
+    *bp = BeamPlane{b->q3.as<long long>() + (jdev ? 0 : (size_t)(slice - 1) * c->rplane), q->rs.p,
+                    c->rplane, jdev, c->nz};
+    q->state = 0;
+    q->gcells = 1;
+    return QP_OK;
+}
 // the copies of the other beams (qdpcopy), with the slice index on the device
 int beam_slice_add_dev(qp_beam *b, qp_field2d *q, const int *jdev)
 {

@@ -298,14 +298,28 @@ int fused_solve_front(const PassFields &f, const FrontFields &fr, double dex, in
 // converged, epw <- g_l - gamma (g_l - g_{l-1}) and B_perp reassembled; mix =
 // 0 (first pass, last allowed pass) only keeps g_l for the next pass.
 int fused_mix(const PassFields &f, double dex, int l, double tol, bool mix);
-int fused_predict_cu(qp_field2d *cu, qp_field2d *dcu, double dxi);
-int fused_efield(qp_field2d *fxy, const qp_field2d *bxyz);
-// jdev (captured slices): plane lpos - 1 is read from device memory instead;
-// ctl (eager slices): the device slice words are set to lpos (the next
-// slice) and hist (the seed's recorded slices)
-int fused_slice_write(qp_field2d *fxy, const qp_field2d *psit, qp_field2d *bxyz, qp_field2d *psi,
-                      qp_field3d *bexyz, qp_field3d *bbxyz, int lpos, double dex, double dd,
-                      const int *jdev = nullptr, int *ctl = nullptr, int hist = 0);
+// The end of a slice: E_perp, the predictor current, the wake planes lpos and
+// the move checks' words (k_slice_end_fields).  jdev (captured slices): plane
+// lpos - 1 is read from device memory instead; ctl (eager slices): the device
+// slice words are set to lpos (the next slice) and hist (the seed's recorded
+// slices); spec: the k planes of psit and bxyz are written too
+struct EndFields {
+    qp_field2d *fxy, *psi;
+    qp_field3d *bexyz, *bbxyz;
+    int lpos;
+    const int *jdev;
+    int *ctl, hist;
+    bool spec;
+    int nerr, slice;
+    const int *err[4];
+    int *h_err[4];
+};
+int fused_slice_end(const PassFields &f, const EndFields &e);
+
+// -fxy + (B_y, -B_x) (simulation_class.f03:721-723): the E_perp that the push
+// gathers and the end of the slice stores
+template <typename R> __device__ __forceinline__ R efield_x(R fx, R by) { return fx * R(-1) + by; }
+template <typename R> __device__ __forceinline__ R efield_y(R fy, R bx) { return fy * R(-1) - bx; }
 
 // the value a new context gives tuning knob `knob` (qp_ctx_tune)
 int tune_default_of(int precision, int knob);
@@ -326,6 +340,31 @@ struct ProfScope {
         : c(cc), slot((cc->prof_on >> kind) & 1u ? prof_begin(cc, kind, bytes) : -1) {}
     ~ProfScope() { if (slot >= 0) prof_end(c, slot); }
 };
+
+// One xi plane of a beam's fixed-point charge and the plane it is converted
+// into (qdpcopy after asc(0)): n elements; jdev (captured slices): q3 is the
+// volume, and plane j, read from device memory, 1 <= j <= nz, is taken
+struct BeamPlane {
+    const long long *q3;
+    void *q2;
+    size_t n;
+    const int *jdev;
+    int nz;
+};
+// elements first, first + step, ... of the conversion
+template <typename R>
+__device__ __forceinline__ void beam_plane_convert(const BeamPlane &b, size_t first, size_t step)
+{
+    const long long *q3 = b.q3;
+    if (b.jdev) {
+        const int j = *b.jdev;
+        if (j < 1 || j > b.nz) return;   // the host checks it before a replay
+        q3 += (size_t)j * b.n;
+    }
+    R *q2 = static_cast<R *>(b.q2);
+    for (size_t i = first; i < b.n; i += step)
+        q2[i] = R(0) + (R)((double)q3[i] * (1.0 / BEAM_FIX));
+}
 
 // ---- species internals used by the slice driver (qp_particles.hip) ----
 int species_qdp_into(qp_species *sp, qp_field2d *q);

@@ -200,66 +200,108 @@ k_mix(KGrid g, R *epw, R *gprev, const R *__restrict__ epwb, R *bxyz, R dex,
     }
 }
 
-// after the loop (simulation_class.f03:725-726): dcu *= dxi; cu(1:2) -= dcu(1:2)
-template <typename R>
-__global__ void k_predict_cu(size_t n, size_t cs, R *cu, R *dcu, R dxi)
-{
-    for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < n;
-         e += (size_t)gridDim.x * blockDim.x) {
-        const R d1 = dcu[e] * dxi, d2 = dcu[cs + e] * dxi;
-        dcu[e] = d1;
-        dcu[cs + e] = d2;
-        cu[e] = cu[e] - d1;
-        cu[cs + e] = cu[cs + e] - d2;
-    }
-}
+// The end of a slice, element by element (simulation_class.f03:721-735):
+// real planes (the first nreal blocks)
+//   fxy = (-fxy + (B_y, -B_x)) dex, copied to bexyz(1:2); psit to bexyz(3);
+//   bxyz(1:2) *= dex; bxyz to bbxyz(1:3); and the psi *= dex^2 of :670 (psi has
+//   no reader after extpsi in the slice)
+// k planes (the other blocks)
+//   dcu *= dxi; cu(1:2) -= dcu(1:2), the next slice's predictor current; and,
+//   where the field solves do not write them (spec), psit and bxyz of the last
+//   pass, from the cu, epw and epwb that they are functions of
+// and block 0 posts the move check's words (k_post_err) of up to 4 species.
+// One launch: the slices of small grids are bound by their number.
+template <typename R> struct EndArgs {
+    size_t n, cs;                      // real planes
+    R *fxy, *bxyz, *psi, *be, *bb;
+    const R *psit;
+    size_t st;                         // component stride of be, bb
+    R dex, dd;
+    const int *jdev;
+    int nz, nreal;
+    int *ctl, jnext, hist;
+    KGrid g;                           // k planes
+    const R *ffg, *ffs, *epw, *epwb;
+    R *cu, *dcu, *kpsit, *kbxyz;
+    R dxi;
+    int spec, nerr, slice;
+    const int *err[4];
+    int *h_err[4];
+};
 
-// (simulation_class.f03:721-723) fxy = -fxy; fxy(1) += bxyz(2); fxy(2) -= bxyz(1)
 template <typename R>
-__global__ void k_efield(size_t n, size_t cs, R *fxy, const R *__restrict__ bxyz)
+__global__ void __launch_bounds__(256) k_slice_end_fields(EndArgs<R> a)
 {
-    for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < n;
-         e += (size_t)gridDim.x * blockDim.x) {
-        const R f1 = fxy[e] * R(-1), f2 = fxy[cs + e] * R(-1);
-        fxy[e] = f1 + bxyz[cs + e];
-        fxy[cs + e] = f2 - bxyz[e];
+    if ((int)blockIdx.x >= a.nreal) {
+        const size_t cs = a.g.cs;
+        const unsigned nk = gridDim.x - a.nreal, total = (unsigned)cs;
+        for (unsigned m = (blockIdx.x - a.nreal) * 256 + threadIdx.x; m < total; m += nk * 256) {
+            const R c1 = a.cu[m], c2 = a.cu[cs + m];
+            const R d1 = a.dcu[m] * a.dxi, d2 = a.dcu[cs + m] * a.dxi;
+            if (a.spec) {
+                const int kx = m / (unsigned)a.g.ldk, ky = m - kx * a.g.ldk;
+                if (ky <= a.g.ny) {
+                    const bool tab = kx < a.g.nx && ky < a.g.ny;
+                    const unsigned ti = tab ? (unsigned)kx * a.g.ny + ky : 0;
+                    const R fg = tab ? a.ffg[ti] : R(0), fs = tab ? a.ffs[ti] : R(0);
+                    const R e1 = a.epw[m], e2 = a.epw[cs + m];
+                    const R w1 = a.epwb[m], w2 = a.epwb[cs + m];
+                    const R dkx = dk<R>(a.g.nx, kx), dky = dk<R>(a.g.ny, ky);
+                    a.kpsit[m] = psit_mode(tab && kx > 0 && ky > 0, fg, dkx, dky, c1, c2, a.dex);
+                    a.kbxyz[m] = e2 * (-a.dex) - w2;
+                    a.kbxyz[cs + m] = e1 * a.dex + w1;
+                    a.kbxyz[2 * cs + m] =
+                        bz_mode(tab, kx, ky, fg, fs, dkx, dky, c1, c2) * a.dex;
+                }
+            }
+            a.dcu[m] = d1;
+            a.dcu[cs + m] = d2;
+            a.cu[m] = c1 - d1;
+            a.cu[cs + m] = c2 - d2;
+        }
+        return;
     }
-}
-
-// slice writes (simulation_class.f03:731-735): fxy *= dex, copied to
-// bexyz(1:2); psit to bexyz(3); bxyz(1:2) *= dex; bxyz to bbxyz(1:3); and
-// the psi *= dex^2 of :670 (psi has no reader after extpsi in the slice)
-template <typename R>
-__global__ void k_slice_write(size_t n, size_t cs, R *fxy, const R *__restrict__ psit, R *bxyz,
-                              R *psi, R *be1, R *be2, R *be3, R *bb1, R *bb2, R *bb3, R dex,
-                              R dd, const int *jdev, int nz, int *ctl, int jnext, int hist)
-{
-    // eager slices keep the device slice word of captured ones in step
-    if (ctl && blockIdx.x == 0 && threadIdx.x == 0) {
-        ctl[0] = jnext;
-        ctl[1] = hist;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        // eager slices keep the device slice word of captured ones in step
+        if (a.ctl) {
+            a.ctl[0] = a.jnext;
+            a.ctl[1] = a.hist;
+        }
+#pragma unroll   // constant indices: the arguments stay out of scratch memory
+        for (int i = 0; i < 4; ++i) {
+            if (i >= a.nerr) break;
+            const int e = *a.err[i];
+            a.h_err[i][0] = e;
+            if (e && a.h_err[i][1] == 0) a.h_err[i][1] = a.slice;
+        }
+        if (a.nerr) __threadfence_system();
     }
-    if (jdev) {   // plane lpos - 1 = j, read from device memory (captured slices)
-        const int j = *jdev;
-        if (j < 1 || j > nz) return;   // the host checks it before a replay
-        const size_t z = (size_t)j * n;
-        be1 += z; be2 += z; be3 += z; bb1 += z; bb2 += z; bb3 += z;
+    if (a.jdev) {   // plane lpos - 1 = j, read from device memory (captured slices)
+        const int j = *a.jdev;
+        if (j < 1 || j > a.nz) return;   // the host checks it before a replay
+        a.be += (size_t)j * a.n;
+        a.bb += (size_t)j * a.n;
     }
-    for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < n;
-         e += (size_t)gridDim.x * blockDim.x) {
-        psi[e] = psi[e] * dd;
-        const R f1 = fxy[e] * dex, f2 = fxy[cs + e] * dex;
-        const R b1 = bxyz[e] * dex, b2 = bxyz[cs + e] * dex;
-        fxy[e] = f1;
-        fxy[cs + e] = f2;
-        bxyz[e] = b1;
-        bxyz[cs + e] = b2;
-        be1[e] = f1;
-        be2[e] = f2;
-        be3[e] = psit[e];
-        bb1[e] = b1;
-        bb2[e] = b2;
-        bb3[e] = bxyz[2 * cs + e];
+    const size_t cs = a.cs, st = a.st;
+    const R dex = a.dex;
+    for (size_t e = blockIdx.x * (size_t)256 + threadIdx.x; e < a.n; e += (size_t)a.nreal * 256) {
+        // every load before the first store (the planes are disjoint, which the
+        // compiler cannot know)
+        const R x = a.bxyz[e], y = a.bxyz[cs + e], z = a.bxyz[2 * cs + e];
+        const R fx = a.fxy[e], fy = a.fxy[cs + e], p = a.psi[e], q = a.psit[e];
+        const R f1 = efield_x(fx, y) * dex, f2 = efield_y(fy, x) * dex;
+        const R b1 = x * dex, b2 = y * dex;
+        a.psi[e] = p * a.dd;
+        a.fxy[e] = f1;
+        a.fxy[cs + e] = f2;
+        a.bxyz[e] = b1;
+        a.bxyz[cs + e] = b2;
+        a.be[e] = f1;
+        a.be[st + e] = f2;
+        a.be[2 * st + e] = q;
+        a.bb[e] = b1;
+        a.bb[st + e] = b2;
+        a.bb[2 * st + e] = z;
     }
 }
 
@@ -360,74 +402,42 @@ int fused_mix(const PassFields &f, double dex, int l, double tol, bool mix)
                                        : mix_t<float>(f, dex, l, tol, mix);
 }
 
-template <typename R>
-static int predict_cu_t(qp_field2d *cu, qp_field2d *dcu, double dxi)
+template <typename R> static int slice_end_t(const PassFields &f, const EndFields &e)
 {
-    qp_ctx *c = cu->ctx;
-    const size_t n = c->kplane;
+    qp_ctx *c = f.cu->ctx;
+    EndArgs<R> a{};
+    a.n = a.cs = c->rplane;
+    a.st = (size_t)(c->nz + 1) * c->rplane;
+    const size_t z = e.jdev ? 0 : (size_t)(e.lpos - 1) * a.n;
+    a.fxy = e.fxy->rs.as<R>(); a.bxyz = f.bxyz->rs.as<R>(); a.psi = e.psi->rs.as<R>();
+    a.psit = f.psit->rs.as<R>();
+    a.be = e.bexyz->buf.as<R>() + z; a.bb = e.bbxyz->buf.as<R>() + z;
+    a.dex = (R)c->dex; a.dd = (R)(c->dex * c->dex);
+    a.jdev = e.jdev; a.nz = c->nz;
+    a.ctl = e.ctl; a.jnext = e.lpos; a.hist = e.hist;
+    a.g = kgrid(c);
+    a.ffg = c->ffg.as<R>(); a.ffs = c->ffs.as<R>();
+    a.epw = f.epw->ks.as<R>(); a.epwb = f.epwb->ks.as<R>();
+    a.cu = f.cu->ks.as<R>(); a.dcu = f.dcu->ks.as<R>();
+    a.kpsit = f.psit->ks.as<R>(); a.kbxyz = f.bxyz->ks.as<R>();
+    a.dxi = (R)c->dxi;
+    a.spec = e.spec ? 1 : 0;
+    a.nerr = e.nerr; a.slice = e.slice;
+    for (int i = 0; i < e.nerr; ++i) { a.err[i] = e.err[i]; a.h_err[i] = e.h_err[i]; }
+    a.nreal = (int)flat_grid(a.n).x;
+    const int nk = (int)flat_grid(c->kplane).x;
     {
-    ProfScope _ps(c, QP_PROF_ELEMENTWISE, 8.0 * n * sizeof(R));
-    hipLaunchKernelGGL(k_predict_cu<R>, flat_grid(n), dim3(256), 0, c->stream, n, n,
-                       cu->ks.as<R>(), dcu->ks.as<R>(), (R)dxi);
+    ProfScope _ps(c, QP_PROF_ELEMENTWISE, (18.0 * a.n + (a.spec ? 18.0 : 8.0) * c->kplane) * sizeof(R));
+    hipLaunchKernelGGL(k_slice_end_fields<R>, dim3(a.nreal + nk), dim3(256), 0, c->stream, a);
     }
     QP_LAUNCH_CHECK();
     return QP_OK;
 }
 
-int fused_predict_cu(qp_field2d *cu, qp_field2d *dcu, double dxi)
+int fused_slice_end(const PassFields &f, const EndFields &e)
 {
-    return cu->ctx->prec == QP_FP64 ? predict_cu_t<double>(cu, dcu, dxi)
-                                    : predict_cu_t<float>(cu, dcu, dxi);
-}
-
-template <typename R>
-static int efield_t(qp_field2d *fxy, const qp_field2d *bxyz)
-{
-    qp_ctx *c = fxy->ctx;
-    const size_t n = c->rplane;
-    {
-    ProfScope _ps(c, QP_PROF_ELEMENTWISE, 6.0 * n * sizeof(R));
-    hipLaunchKernelGGL(k_efield<R>, flat_grid(n), dim3(256), 0, c->stream, n, n,
-                       fxy->rs.as<R>(), bxyz->rs.as<R>());
-    }
-    QP_LAUNCH_CHECK();
-    return QP_OK;
-}
-
-int fused_efield(qp_field2d *fxy, const qp_field2d *bxyz)
-{
-    return fxy->ctx->prec == QP_FP64 ? efield_t<double>(fxy, bxyz) : efield_t<float>(fxy, bxyz);
-}
-
-template <typename R>
-static int slice_write_t(qp_field2d *fxy, const qp_field2d *psit, qp_field2d *bxyz,
-                         qp_field2d *psi, qp_field3d *bexyz, qp_field3d *bbxyz, int lpos,
-                         double dex, double dd, const int *jdev, int *ctl, int hist)
-{
-    qp_ctx *c = fxy->ctx;
-    const size_t n = c->rplane, st = (size_t)(c->nz + 1) * n;
-    const size_t z = jdev ? 0 : (size_t)(lpos - 1) * n;
-    R *be = bexyz->buf.as<R>() + z, *bb = bbxyz->buf.as<R>() + z;
-    {
-    ProfScope _ps(c, QP_PROF_ELEMENTWISE, 18.0 * n * sizeof(R));
-    hipLaunchKernelGGL(k_slice_write<R>, flat_grid(n), dim3(256), 0, c->stream, n, n,
-                       fxy->rs.as<R>(), psit->rs.as<R>(), bxyz->rs.as<R>(), psi->rs.as<R>(), be,
-                       be + st, be + 2 * st, bb, bb + st, bb + 2 * st, (R)dex, (R)dd, jdev,
-                       c->nz, ctl, lpos, hist);
-    }
-    QP_LAUNCH_CHECK();
-    return QP_OK;
-}
-
-int fused_slice_write(qp_field2d *fxy, const qp_field2d *psit, qp_field2d *bxyz, qp_field2d *psi,
-                      qp_field3d *bexyz, qp_field3d *bbxyz, int lpos, double dex, double dd,
-                      const int *jdev, int *ctl, int hist)
-{
-    return fxy->ctx->prec == QP_FP64
-               ? slice_write_t<double>(fxy, psit, bxyz, psi, bexyz, bbxyz, lpos, dex, dd, jdev,
-                                       ctl, hist)
-               : slice_write_t<float>(fxy, psit, bxyz, psi, bexyz, bbxyz, lpos, dex, dd, jdev,
-                                      ctl, hist);
+    QP_REQUIRE(e.nerr <= 4, QP_ERR_ARG, "fused_slice_end: %d move checks", e.nerr);
+    return f.cu->ctx->prec == QP_FP64 ? slice_end_t<double>(f, e) : slice_end_t<float>(f, e);
 }
 
 }  // namespace qp

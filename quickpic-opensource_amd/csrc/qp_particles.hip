@@ -28,6 +28,7 @@ struct qp_species {
     qp::DevBuf a[8], b[8];     // x, y, px, py, pz, p6, p7, q (current, alternate)
     qp::DevBuf key, slot;      // per particle: destination bin and rank (push), key and index (load)
     qp::DevBuf bins;           // per tile: counts, then starts, of the 9 x 256 destination bins
+    qp::DevBuf tot;            // particles bound for each tile and group of tiles (push)
     qp::DevBuf count, off;     // per cell (ncells + 1)
     qp::DevBuf off_new;        // the push's new cell offsets, swapped with off
     // every particle has charge q_value (a uniform plasma, or an upload that
@@ -282,10 +283,19 @@ __device__ __forceinline__ void emit_nodes(const R *nacc, const DepOut<R> &out, 
 
 // PPGPPOST2L (part2d_lib77.f:194-309): q(n,m) += qm (1-dx)(1-dy) etc.
 // UQ: every particle's charge is quni (not staged or read).
+// The workgroups past the tiles convert the slice's beam plane (bp), which the
+// deposit does not touch: a launch less.
+constexpr int BEAM_BLOCKS = 512;
 template <typename R, int RG, int CH, int WPE, bool UQ>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, 8)))
-k_deposit_q(TileGeom g, Soa<R> s, const int *__restrict__ off, DepOut<R> out, R *halo, R quni)
+k_deposit_q(TileGeom g, Soa<R> s, const int *__restrict__ off, DepOut<R> out, R *halo, R quni,
+            BeamPlane bp)
 {
+    if ((int)blockIdx.x >= g.mx1 * g.my1) {
+        beam_plane_convert<R>(bp, ((size_t)blockIdx.x - g.mx1 * g.my1) * 256 + threadIdx.x,
+                              (size_t)BEAM_BLOCKS * 256);
+        return;
+    }
     constexpr int T = TILE / RG, NP = Stage<CH>::N;
     extern __shared__ unsigned char smem_raw[];
     R *sx = reinterpret_cast<R *>(smem_raw), *sy = sx + NP, *sq = sy + NP, *nacc = sq + NP;
@@ -1016,15 +1026,21 @@ k_amjdp_w(TileGeom g, Soa<R> s, const int *__restrict__ off, const R *fxy, const
 // within its cell) and the scan of the new cell counts into off_new: it
 // repeats the push on the unchanged input, so bins and ranks are those of
 // MODE 1, and stores each particle at off_new[cell] + start + rank of the
-// alternate arrays o.  The two passes read the particle record twice and
+// alternate arrays o.  raw: fxy holds grad(psi) still, and the gathered E_perp
+// is formed from it and B_perp (efield_x, efield_y).  tot (MODE 1): the
+// particles bound for every tile, summed for k_bin_offsets (one atomic per
+// neighbour that gets any: one per wave and group of tiles took 80 us more at
+// 1024^2); MODE 2 clears them for the next push.  The two passes read the particle record twice and
 // write it once, where push and scatter read it twice and write it twice.
 constexpr int NBINS = 9 * TCELLS;
+constexpr int GROUP = 256;  // tiles per group of the offsets' two-level sum
 
 template <typename R, int MODE>
 __global__ void __launch_bounds__(256)
 k_push(TileGeom g, Soa<R> s, Soa<R> o, const int *__restrict__ off,
        const int *__restrict__ off_new, const R *fxy, const R *bxy, const R *psit, size_t cs,
-       R qbm, R dt, R dex, int *bin, int *rank, int *cnt, int *err, int64_t np, int uq)
+       R qbm, R dt, R dex, int *bin, int *rank, int *cnt, int *err, int64_t np, int uq, int raw,
+       int *tot)
 {
     __shared__ int hist[NBINS];
     __shared__ R fnode[6][289];   // the six fields at the tile's 17 x 17 nodes
@@ -1061,7 +1077,10 @@ k_push(TileGeom g, Soa<R> s, Soa<R> o, const int *__restrict__ off,
                 const int f = n / 289, m = n % 289;
                 const R *pl = f == 0 ? fxy : f == 1 ? fxy + cs : f == 2 ? psit
                             : f == 3 ? bxy : f == 4 ? bxy + cs : bxy + 2 * cs;
-                tv[k] = pl[(size_t)(ty0 * TILE + m / 17) * g.ldr + tx0 * TILE + m % 17];
+                const size_t o = (size_t)(ty0 * TILE + m / 17) * g.ldr + tx0 * TILE + m % 17;
+                tv[k] = pl[o];
+                if (raw && f < 2)
+                    tv[k] = f == 0 ? efield_x(tv[k], bxy[cs + o]) : efield_y(tv[k], bxy[o]);
             }
         }
 #pragma unroll
@@ -1262,9 +1281,32 @@ k_push(TileGeom g, Soa<R> s, Soa<R> o, const int *__restrict__ off,
             }
         }
     }
-    if (MODE == 2) return;
+    if (MODE == 2) {
+        if (tid == 0) tot[S] = 0;
+        return;
+    }
     __syncthreads();
-    for (int k = tid; k < NBINS; k += TCELLS) cnt[(size_t)S * NBINS + k] = hist[k];
+    __shared__ int s_tot[9];   // particles bound for each neighbour
+    if (MODE == 1 && tid < 9) s_tot[tid] = 0;
+    int h[9];
+#pragma unroll
+    for (int nb = 0; nb < 9; ++nb) {
+        h[nb] = hist[nb * TCELLS + tid];
+        cnt[(size_t)S * NBINS + nb * TCELLS + tid] = h[nb];
+    }
+    if (MODE != 1) return;
+    __syncthreads();
+#pragma unroll
+    for (int nb = 0; nb < 9; ++nb) {
+        if (!__any(h[nb])) continue;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) h[nb] += __shfl_xor(h[nb], o);
+        if (lane == 0) atomicAdd(&s_tot[nb], h[nb]);
+    }
+    __syncthreads();
+    if (tid < 9 && s_tot[tid])
+        atomicAdd(&tot[wrap1(ty0 + tid / 3 - 1, g.my1) * g.mx1 + wrap1(tx0 + tid % 3 - 1, g.mx1)],
+                  s_tot[tid]);
 }
 
 // Per destination cell d (in tile T, local cell cl): its particles come from
@@ -1289,6 +1331,80 @@ __global__ void k_bin_starts(TileGeom g, int *cnt, int *count)
         run += c;
     }
     count[d] = run;
+}
+
+// Totals of groups of GROUP tiles, for k_bin_offsets on large grids
+__global__ void __launch_bounds__(GROUP) k_group_totals(int ntiles, const int *tot, int *grp)
+{
+    __shared__ int s[GROUP / 64];
+    const int t = blockIdx.x * GROUP + threadIdx.x;
+    int v = t < ntiles ? tot[t] : 0;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int sum = 0;
+        for (int w = 0; w < GROUP / 64; ++w) sum += s[w];
+        grp[blockIdx.x] = sum;
+    }
+}
+
+// The same as k_bin_starts, and the new cell offsets in place of the counts: a
+// tile's first particle is the sum of the tiles before it, from the totals that
+// the counting push has added up (integer sums: any order), and its cells
+// follow by a prefix sum over the workgroup.  grp (above 8192 tiles): the
+// totals of the groups of tiles before; below, reading at most 32 KB of totals
+// per workgroup from L2 costs less than the launch that makes them.  One launch
+// for three of the counts' kernel and a library scan: 27 us at 1024^2 (4.6 of
+// them the scan's set-up) become 16, and 10 become 3.4 at 128^2.
+__global__ void __launch_bounds__(TCELLS)
+k_bin_offsets(TileGeom g, int *cnt, const int *__restrict__ tot, const int *__restrict__ grp,
+              int *off)
+{
+    __shared__ int s_sum[2][TCELLS / 64];
+    const int T = blockIdx.x, cl = threadIdx.x, lane = cl & 63, wave = cl >> 6;
+    const int ntiles = g.mx1 * g.my1;
+    const int tx = T % g.mx1, ty = T / g.mx1;
+    size_t k[9];
+    int c[9];
+#pragma unroll
+    for (int nb = 0; nb < 9; ++nb) {
+        const int sx = wrap1(tx - (nb % 3 - 1), g.mx1), sy = wrap1(ty - (nb / 3 - 1), g.my1);
+        k[nb] = (size_t)(sy * g.mx1 + sx) * NBINS + nb * TCELLS + cl;
+        c[nb] = cnt[k[nb]];
+    }
+    int base = 0;
+    int t0 = 0;
+    if (grp) {
+        t0 = T / GROUP * GROUP;
+        for (int i = cl; i < T / GROUP; i += TCELLS) base += grp[i];
+    }
+    for (int i = t0 + cl; i < T; i += TCELLS) base += tot[i];
+    int run = 0;
+#pragma unroll
+    for (int nb = 0; nb < 9; ++nb) {
+        cnt[k[nb]] = run;
+        run += c[nb];
+    }
+    int pre = run;   // inclusive prefix over the wave
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(pre, o);
+        if (lane >= o) pre += v;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) base += __shfl_xor(base, o);
+    if (lane == 63) {
+        s_sum[0][wave] = pre;
+        s_sum[1][wave] = base;
+    }
+    __syncthreads();
+    int first = 0;
+#pragma unroll
+    for (int w = 0; w < TCELLS / 64; ++w) first += s_sum[1][w] + (w < wave ? s_sum[0][w] : 0);
+    off[T * TCELLS + cl] = first + pre - run;
+    if (T == ntiles - 1 && cl == TCELLS - 1) off[ntiles * TCELLS] = first + pre;
 }
 
 // destination of particle i: off[cell] + start of its bin in the cell + rank
@@ -1391,13 +1507,13 @@ static TileGeom geom(qp_ctx *c) { return TileGeom{c->nx, c->ny, c->mx1, c->my1, 
 
 static dim3 pgrid(int64_t n) { return dim3((unsigned)((n + 255) / 256)); }
 
-// cell offsets from the per-cell counts, into off (or the buffer given)
-static int scan_counts(qp_species *sp, DevBuf *dst = nullptr)
+// cell offsets from the per-cell counts
+static int scan_counts(qp_species *sp)
 {
     qp_ctx *c = sp->ctx;
     size_t tb = sp->scan_bytes;
     QP_HIP(hipcub::DeviceScan::ExclusiveSum(sp->scan_tmp.p, tb, sp->count.as<int>(),
-                                            (dst ? dst : &sp->off)->as<int>(), c->ncells + 1,
+                                            sp->off.as<int>(), c->ncells + 1,
                                             c->stream));
     return QP_OK;
 }
@@ -1546,7 +1662,7 @@ static int allow_lds(K kernel, size_t bytes, qp_ctx *c)
 }
 
 template <typename R, int V>
-static int deposit_q_v(qp_species *sp, const DepOut<R> &out, R *halo)
+static int deposit_q_v(qp_species *sp, const DepOut<R> &out, R *halo, const BeamPlane *bp)
 {
     qp_ctx *c = sp->ctx;
     constexpr DepShape d = DepTab<R>::q[V];
@@ -1559,8 +1675,9 @@ static int deposit_q_v(qp_species *sp, const DepOut<R> &out, R *halo)
     // x, y (and q unless uniform) per particle, one plane
     const double words = sp->q_uniform ? 2.0 : 3.0;
     ProfScope _ps(c, QP_PROF_DEPOSIT_Q, (words * sp->np + (c->nx + 1.0) * (c->ny + 1.0)) * sizeof(R));
-    hipLaunchKernelGGL(kern, dim3(c->ntiles), dim3(256), lds, c->stream, geom(c),
-                       soa<R>(sp->a), sp->off.as<int>(), out, halo, (R)sp->q_value);
+    hipLaunchKernelGGL(kern, dim3(c->ntiles + (bp ? BEAM_BLOCKS : 0)), dim3(256), lds, c->stream,
+                       geom(c), soa<R>(sp->a), sp->off.as<int>(), out, halo, (R)sp->q_value,
+                       bp ? *bp : BeamPlane{});
     }
     QP_LAUNCH_CHECK();
     return QP_OK;
@@ -1568,15 +1685,16 @@ static int deposit_q_v(qp_species *sp, const DepOut<R> &out, R *halo)
 
 // halo: the tile-border buffer (null: the context's)
 template <typename R>
-static int deposit_q_out(qp_species *sp, const DepOut<R> &out, R *halo = nullptr)
+static int deposit_q_out(qp_species *sp, const DepOut<R> &out, R *halo = nullptr,
+                         const BeamPlane *bp = nullptr)
 {
     int rc;
     if (!halo) halo = sp->ctx->halo.as<R>();
     switch (sp->ctx->tune[QP_TUNE_DEPOSIT_Q]) {
-    case 1: rc = deposit_q_v<R, 1>(sp, out, halo); break;
-    case 2: rc = deposit_q_v<R, 2>(sp, out, halo); break;
-    case 3: rc = deposit_q_v<R, 3>(sp, out, halo); break;
-    default: rc = deposit_q_v<R, 0>(sp, out, halo); break;
+    case 1: rc = deposit_q_v<R, 1>(sp, out, halo, bp); break;
+    case 2: rc = deposit_q_v<R, 2>(sp, out, halo, bp); break;
+    case 3: rc = deposit_q_v<R, 3>(sp, out, halo, bp); break;
+    default: rc = deposit_q_v<R, 0>(sp, out, halo, bp); break;
     }
     if (rc) return rc;
     return deposit_border<R>(sp->ctx, out, 1, 1, halo);
@@ -1856,6 +1974,7 @@ static int alloc_particles(qp_species *sp, int64_t np)
     if (!rc) rc = sp->slot.alloc((size_t)np * 4);
     if (!rc) rc = sp->count.alloc((size_t)(c->ncells + 1) * 4);
     if (!rc) rc = sp->bins.alloc((size_t)c->ntiles * NBINS * 4);
+    if (!rc) rc = sp->tot.alloc((size_t)(c->ntiles + (c->ntiles + GROUP - 1) / GROUP) * 4);
     if (!rc) rc = sp->off.alloc((size_t)(c->ncells + 1) * 4);
     if (!rc) rc = sp->off_new.alloc((size_t)(c->ncells + 1) * 4);
     if (!rc) rc = sp->err.alloc(sizeof(int));
@@ -1974,7 +2093,7 @@ static int amjdp_t(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
 
 template <typename R>
 static int push_t(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
-                  const qp_field2d *psit, double dex, bool check)
+                  const qp_field2d *psit, double dex, bool check, bool raw = false)
 {
     qp_ctx *c = sp->ctx;
     const TileGeom g = geom(c);
@@ -1989,16 +2108,17 @@ static int push_t(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
     hipLaunchKernelGGL(kern, dim3(c->ntiles), dim3(TCELLS), 0, c->stream, g, a, b, off, off_new,
                        ef->rs.as<R>(), bf->rs.as<R>(), psit->rs.as<R>(), c->rplane,
                        (R)sp->qbm, (R)sp->dt, (R)dex, sp->key.as<int>(), sp->slot.as<int>(),
-                       sp->bins.as<int>(), sp->err.as<int>(), sp->np, 0);
-    }
-    QP_LAUNCH_CHECK();
-    {
-    ProfScope _ps(c, QP_PROF_SORT, 8.0 * (double)c->ntiles * NBINS);
-    hipLaunchKernelGGL(k_bin_starts, dim3(c->ncells / 256 + 1), dim3(256), 0, c->stream, g,
-                       sp->bins.as<int>(), sp->count.as<int>());
+                       sp->bins.as<int>(), sp->err.as<int>(), sp->np, 0, raw ? 1 : 0,
+                       sp->tot.as<int>());
     }
     QP_LAUNCH_CHECK();
     if (scatter) {
+        {
+        ProfScope _ps(c, QP_PROF_SORT, 8.0 * (double)c->ntiles * NBINS);
+        hipLaunchKernelGGL(k_bin_starts, dim3(c->ncells / 256 + 1), dim3(256), 0, c->stream, g,
+                           sp->bins.as<int>(), sp->count.as<int>());
+        }
+        QP_LAUNCH_CHECK();
         int rc = scan_counts(sp);
         if (rc) return rc;
         {
@@ -2009,8 +2129,18 @@ static int push_t(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
         }
         QP_LAUNCH_CHECK();
     } else {
-        int rc = scan_counts(sp, &sp->off_new);
-        if (rc) return rc;
+        int *tot = sp->tot.as<int>(), *grp = c->ntiles > 8192 ? tot + c->ntiles : nullptr;
+        if (grp) {
+            hipLaunchKernelGGL(k_group_totals, dim3((c->ntiles + GROUP - 1) / GROUP), dim3(GROUP),
+                               0, c->stream, c->ntiles, tot, grp);
+            QP_LAUNCH_CHECK();
+        }
+        {
+        ProfScope _ps(c, QP_PROF_SORT, 8.0 * (double)c->ntiles * NBINS);
+        hipLaunchKernelGGL(k_bin_offsets, dim3(c->ntiles), dim3(TCELLS), 0, c->stream, g,
+                           sp->bins.as<int>(), tot, grp, off_new);
+        }
+        QP_LAUNCH_CHECK();
         {
         // 8 arrays read, 8 written at their sorted places
         ProfScope _ps(c, QP_PROF_SORT, (sp->q_uniform ? 14.0 : 16.0) * sp->np * sizeof(R) + fields);
@@ -2018,7 +2148,8 @@ static int push_t(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
         hipLaunchKernelGGL(kern, dim3(c->ntiles), dim3(TCELLS), 0, c->stream, g, a, b,
                            off, off_new, ef->rs.as<R>(), bf->rs.as<R>(), psit->rs.as<R>(),
                            c->rplane, (R)sp->qbm, (R)sp->dt, (R)dex, nullptr, nullptr,
-                           sp->bins.as<int>(), sp->err.as<int>(), sp->np, sp->q_uniform ? 1 : 0);
+                           sp->bins.as<int>(), sp->err.as<int>(), sp->np, sp->q_uniform ? 1 : 0,
+                           raw ? 1 : 0, sp->tot.as<int>());
         }
         QP_LAUNCH_CHECK();
         std::swap(sp->off, sp->off_new);
@@ -2074,6 +2205,7 @@ int qp_species_destroy(qp_species *sp)
     sp->key.release(); sp->slot.release(); sp->count.release(); sp->off.release();
     sp->off_new.release();
     sp->bins.release();
+    sp->tot.release();
     sp->scan_tmp.release(); sp->err.release(); sp->radial.release();
     if (sp->h_err) (void)hipHostFree(sp->h_err);
     if (sp->err_ev) (void)hipEventDestroy(sp->err_ev);
@@ -2420,10 +2552,11 @@ int qp_species_tile_counts(const qp_species *sp, int32_t *kpic)
 
 // entry points used by the slice driver without the per-call error sync
 namespace qp {
+// ef holds grad(psi) still (see k_push)
 int species_push_nocheck(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
                          const qp_field2d *psit, double dex)
 {
-    return DISPATCH(sp->ctx, push_t, sp, ef, bf, psit, dex, false);
+    return DISPATCH(sp->ctx, push_t, sp, ef, bf, psit, dex, false, true);
 }
 int species_check(qp_species *sp) { return check_err(sp, "pmove"); }
 
@@ -2440,16 +2573,27 @@ void species_flip(qp_species *sp, bool offsets)
 
 // The slice loop does not wait for the move check of each push: the error
 // word is copied to pinned memory behind the push, and a later slice (or the
-// end of the step, which waits) reports it.
+// end of the step, which waits) reports it.  The words to copy are given to
+// the kernel that ends the slice (species_err_words, then species_check_mark
+// behind it); species_check_post copies them by a launch of its own.
+void species_err_words(qp_species *sp, const int **err, int **h_err)
+{
+    *err = sp->err.as<int>();
+    *h_err = sp->h_err;
+}
+int species_check_mark(qp_species *sp)
+{
+    QP_HIP(hipEventRecord(sp->err_ev, sp->ctx->stream));
+    sp->err_pending = true;
+    return QP_OK;
+}
 int species_check_post(qp_species *sp, int slice)
 {
     qp_ctx *c = sp->ctx;
     hipLaunchKernelGGL(k_post_err, dim3(1), dim3(64), 0, c->stream, sp->err.as<int>(), sp->h_err,
                        slice);
     QP_LAUNCH_CHECK();
-    QP_HIP(hipEventRecord(sp->err_ev, c->stream));
-    sp->err_pending = true;
-    return QP_OK;
+    return species_check_mark(sp);
 }
 
 // The move check of the slices posted so far, once their push has run
@@ -2478,9 +2622,10 @@ int species_check_poll(qp_species *sp, bool wait)
 
 // qdp_species2d with the slice's additions fused into the deposit
 // (species2d_class.f03:166-185): this%q = deposit; q = this%q + q;
-// q = qn + q.  first: q holds nothing yet (the slice loop zeroed it).
+// q = qn + q.  first: q holds nothing yet (the slice loop zeroed it).  bp: the
+// beam plane to convert beside it (or null).
 template <typename R>
-static int qdp_fused_t(qp_species *sp, qp_field2d *q, bool first)
+static int qdp_fused_t(qp_species *sp, qp_field2d *q, bool first, const BeamPlane *bp)
 {
     R *qp = q->rs.as<R>();
     DepOut<R> o{};
@@ -2489,16 +2634,16 @@ static int qdp_fused_t(qp_species *sp, qp_field2d *q, bool first)
     o.outer[0] = sp->qn->rs.as<R>();
     o.p2[0] = sp->q->rs.as<R>();
     o.scale = o.scale2 = R(1);
-    int rc = deposit_q_out<R>(sp, o);
+    int rc = deposit_q_out<R>(sp, o, nullptr, bp);
     sp->q->state = 0;
     sp->q->gcells = 1;
     q->state = 0;
     return rc;
 }
 
-int species_qdp_fused(qp_species *sp, qp_field2d *q, bool first)
+int species_qdp_fused(qp_species *sp, qp_field2d *q, bool first, const BeamPlane *bp)
 {
-    return DISPATCH(sp->ctx, qdp_fused_t, sp, q, first);
+    return DISPATCH(sp->ctx, qdp_fused_t, sp, q, first, bp);
 }
 
 // amjdp_species2d plus the slice loop's scaling (species2d_class.f03:187-218,

@@ -19,9 +19,12 @@ int species_check(qp_species *sp);
 const void *species_buffer_key(const qp_species *sp);
 void species_flip(qp_species *sp, bool offsets);
 int species_check_post(qp_species *sp, int slice);
+void species_err_words(qp_species *sp, const int **err, int **h_err);
+int species_check_mark(qp_species *sp);
 int species_check_poll(qp_species *sp, bool wait);
-int species_qdp_fused(qp_species *sp, qp_field2d *q, bool first);
+int species_qdp_fused(qp_species *sp, qp_field2d *q, bool first, const BeamPlane *bp);
 int beam_slice_assign(qp_beam *b, qp_field2d *q, int slice, const int *jdev = nullptr);
+int beam_slice_plane(qp_beam *b, qp_field2d *q, int slice, const int *jdev, BeamPlane *bp);
 int beam_slice_add_dev(qp_beam *b, qp_field2d *q, const int *jdev);
 int species_q3_initial(qp_species *sp, qp_field3d *q3);
 int species_amjdp_fused(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
@@ -224,8 +227,10 @@ int qp_sim_begin_step(qp_sim *s)
 //    the B assembly that follows it (:677-680) are one k-space kernel, so the
 //    inverse transform of bxyz that opens the next pass (or follows the loop)
 //    runs at the end of this one, beside psit's;
-//  * -fxy + B, the predictor cu -= dxi dcu and the slice writes are one
-//    kernel each.
+//  * -fxy + B is formed where the push gathers it and, with the predictor
+//    cu -= dxi dcu and the slice writes, stored at the end of the slice by one
+//    kernel; the first beam's charge plane is converted beside the first
+//    species' charge deposit.
 
 // beam charge (:650-655) and plasma charge (:657-661) of slice j
 static int slice_charges(qp_sim *s, int j)
@@ -240,13 +245,15 @@ static int slice_charges(qp_sim *s, int j)
     if (!s->graph)
         for (qp_species *sp : s->sp) RC(species_check_poll(sp, false));
     const int *jdev = s->graph ? s->ctl.as<int>() : nullptr;
+    BeamPlane bp{};
     if (s->bm.empty()) RC(qp_field2d_as(qb, 0.0));
-    for (size_t i = 0; i < s->bm.size(); ++i) {
-        if (i == 0) RC(beam_slice_assign(s->bm[0], qb, j + 1, jdev));
-        else RC(jdev ? beam_slice_add_dev(s->bm[i], qb, jdev) : qp_beam_qdpcopy(s->bm[i], qb, j + 1));
-    }
+    else if (nsp == 0) RC(beam_slice_assign(s->bm[0], qb, j + 1, jdev));
+    else RC(beam_slice_plane(s->bm[0], qb, j + 1, jdev, &bp));
     if (nsp == 0) RC(qp_field2d_as(qe, 0.0));
-    for (int i = 0; i < nsp; ++i) RC(species_qdp_fused(s->sp[i], qe, i == 0));
+    for (int i = 0; i < nsp; ++i)
+        RC(species_qdp_fused(s->sp[i], qe, i == 0, i == 0 && bp.q3 ? &bp : nullptr));
+    for (size_t i = 1; i < s->bm.size(); ++i)
+        RC(jdev ? beam_slice_add_dev(s->bm[i], qb, jdev) : qp_beam_qdpcopy(s->bm[i], qb, j + 1));
     QP_REQUIRE(qb->state == 0 && qe->state == 0, QP_ERR_STATE, "fftrk: data is in ks");
     return QP_OK;
 }
@@ -290,13 +297,12 @@ static int slice_finish(qp_sim *s, int j, int iter_max, double tol, int *iters_u
     qp_ctx *c = s->ctx;
     QP_REQUIRE(iter_max >= 1, QP_ERR_ARG, "qp_slice_finish: iter_max %d", iter_max);
     s->prepared = 0;
-    const double dex = c->dex, dxi = c->dxi;
+    const double dex = c->dex;
     qp_field2d **F = s->f;
     qp_field2d *psi = F[QP_F_PSI], *fxy = F[QP_F_FXY];
     qp_field2d *cu = F[QP_F_CU], *dcu = F[QP_F_DCU], *amu = F[QP_F_AMU], *bxyz = F[QP_F_BXYZ];
     qp_field2d *psit = F[QP_F_PSIT], *epw = F[QP_F_EPW], *epwb = F[QP_F_EPWB];
     const int nsp = (int)s->sp.size();
-    const double dd = dex * dex;   // psi *= dex^2 (:670) is applied with the slice writes
     // predictor fields from the carried current (:671-675) and the B assembly
     const PassFields pf{cu, dcu, amu, epw, epwb, psit, bxyz, nullptr, nullptr};
     qp_field2d *inv[2] = {psit, bxyz};
@@ -454,15 +460,24 @@ static int slice_finish(qp_sim *s, int j, int iter_max, double tol, int *iters_u
     // the current of the last pass, scaled by dex, into cu3d (:696-698):
     // its real-space planes are kept by the forward transform
     if (s->cu3d) RC(copy_planes(c, cu, s->cu3d, j + 1));
-    // final E_perp and predictor current (:721-726); B is already assembled
-    RC(fused_efield(fxy, bxyz));
-    RC(fused_predict_cu(cu, dcu, dxi));
-    // plasma push (:727-730)
+    // plasma push (:727-730); B is already assembled, and E_perp (:721-723) is
+    // formed where it is gathered
     for (qp_species *sp : s->sp) RC(species_push_nocheck(sp, fxy, bxyz, psit, dex));
-    // slice j+1 of the 3-D wake (:731-735)
-    RC(fused_slice_write(fxy, psit, bxyz, psi, s->bexyz, s->bbxyz, j + 1, dex, dd,
-                         graph ? s->ctl.as<int>() : nullptr, graph ? nullptr : s->ctl.as<int>(),
-                         s->hist_slices));
+    // E_perp, the predictor current (:724-726), slice j+1 of the 3-D wake
+    // (:731-735) and the move checks' words
+    EndFields e{fxy, psi, s->bexyz, s->bbxyz, j + 1};
+    e.jdev = graph ? s->ctl.as<int>() : nullptr;
+    e.ctl = graph ? nullptr : s->ctl.as<int>();
+    e.hist = s->hist_slices;
+    e.spec = fused;
+    e.slice = j;
+    if (!graph)
+        for (qp_species *sp : s->sp)
+            if (e.nerr < 4) {
+                species_err_words(sp, &e.err[e.nerr], &e.h_err[e.nerr]);
+                ++e.nerr;
+            }
+    RC(fused_slice_end(pf, e));
     if (graph) {
         hipLaunchKernelGGL(k_slice_end, dim3(1), dim3(64), 0, c->stream, s->ctl.as<int>(), flags,
                            iter_max, adaptive ? 1 : 0, seed ? 1 : 0, s->passes_dev.as<int>(),
@@ -474,7 +489,8 @@ static int slice_finish(qp_sim *s, int j, int iter_max, double tol, int *iters_u
     }
     // psi * dex^2 into psi3d (:670-671); the slice write applied the scaling
     if (s->psi3d) RC(copy_planes(c, psi, s->psi3d, j + 1));
-    for (qp_species *sp : s->sp) RC(species_check_post(sp, j));
+    for (size_t i = 0; i < s->sp.size(); ++i)
+        RC((int)i < e.nerr ? species_check_mark(s->sp[i]) : species_check_post(s->sp[i], j));
     // strict move check: wait for this slice's check before returning
     if (c->tune[QP_TUNE_STRICT])
         for (qp_species *sp : s->sp) RC(species_check_poll(sp, true));

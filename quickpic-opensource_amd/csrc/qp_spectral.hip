@@ -194,7 +194,7 @@ template <typename R> struct MidArgs {
     R *dst;                    // inverse components, cs apart, before the x pass
     const cplx<R> *W;
     const R *ffg, *ffs;
-    R *cu, *dcu, *amu, *epw, *epwb, *psit, *bxyz;    // k planes
+    R *cu, *dcu, *amu, *epw, *epwb;                   // k planes
     R *qb, *qe, *psi, *fxy, *ehist, *ehist2;         // k planes of the front
     R aa, idex, dex;
     double *partial;           // pass: per-block residual sums
@@ -206,7 +206,8 @@ template <typename R> struct MidArgs {
 // The arithmetic of mode (kx, ky): in[] are the forward components' values
 // (pass: cu 3, dcu 2, amu 3; front: qb, qe), out[] the inverse components'
 // (pass: psit, bxyz 3; front: fxy 2, psi, psit, bxyz 3).  The planes that keep
-// k values are written here, except those of in[] itself.
+// k values are written here, except those of in[] itself and, being functions
+// of what is kept, psit's and bxyz's (the end of the slice writes them).
 template <typename R, int N, bool FRONT, int NF, int NI>
 __device__ __forceinline__ void do_mode(const MidArgs<R> &a, int kx, int ky, int seed,
                                         const R (&in)[NF], R (&out)[NI], double &num, double &den)
@@ -284,10 +285,6 @@ __device__ __forceinline__ void do_mode(const MidArgs<R> &a, int kx, int ky, int
     out[P + 1] = e2 * (-a.dex) - b2;
     out[P + 2] = e1 * a.dex + b1;
     out[P + 3] = bz_mode(tab, kx, ky, fg, fs, dkx, dky, c1, c2) * a.dex;
-    at(a.psit, m) = out[P];
-    at(a.bxyz, m) = out[P + 1];
-    at(a.bxyz + cs, m) = out[P + 2];
-    at(a.bxyz + 2 * cs, m) = out[P + 3];
 }
 
 // y types (bit c: cosine) of the forward components, qb, qe sine or cu (S, C,
@@ -353,9 +350,6 @@ __device__ __forceinline__ void last_row_pass(const MidArgs<R> &a, double &num)
         at(a.epw + row, k) = at(a.epw + cs + row, k) = R(0);
         at(a.cu + cs + row, k) = at(a.cu + 2 * cs + row, k) = at(a.dcu + cs + row, k) = R(0);
         at(a.amu + row, k) = at(a.amu + cs + row, k) = R(0);
-        at(a.psit + row, k) = R(0);
-#pragma unroll
-        for (int c = 0; c < 3; ++c) at(a.bxyz + c * cs + row, k) = R(0);
 #pragma unroll
         for (int c = 0; c < 4; ++c) at(a.dst + c * cs + row, k) = R(0);
     }
@@ -669,7 +663,7 @@ static int mid_launch(qp_ctx *c, const MidArgs<R> &a)
     if (rc) return rc;
     {
     // two y transforms of each component and the planes of the modes
-    const double planes = FRONT ? 2 * 2 + 2 * 7 + 12 : 2 * 8 + 2 * 4 + 8;
+    const double planes = FRONT ? 2 * 2 + 2 * 7 + 8 : 2 * 8 + 2 * 4 + 4;
     ProfScope _ps(c, QP_PROF_KSPACE, planes * (c->nx + 1.0) * (c->ny + 1.0) * sizeof(R));
     hipLaunchKernelGGL(kern, dim3(c->nx / 2), dim3(bs), lds, c->stream, a);
     }
@@ -750,7 +744,6 @@ static int solve_t(const PassFields &f, const FrontFields *fr, double dex, int l
     a.ffg = c->ffg.as<R>(); a.ffs = c->ffs.as<R>();
     a.cu = f.cu->ks.as<R>(); a.dcu = f.dcu->ks.as<R>(); a.amu = f.amu->ks.as<R>();
     a.epw = f.epw->ks.as<R>(); a.epwb = f.epwb->ks.as<R>();
-    a.psit = f.psit->ks.as<R>(); a.bxyz = f.bxyz->ks.as<R>();
     a.aa = (R)(dex * dex); a.idex = (R)(1.0 / dex); a.dex = (R)dex;
     a.partial = c->red.as<double>();
     a.flags = c->flags.as<int>();

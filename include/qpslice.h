@@ -448,14 +448,15 @@ int qp_sim_renew(qp_sim *sim, double s);
 /* batched parameter scan (no counterpart in the reference, which runs one */
 /* simulation per MPI job)                                                 */
 /* ---------------------------------------------------------------------- */
-/* One HIP graph holding one xi slice of each of n simulations (their own
+/* HIP graphs holding one xi slice of each of n simulations (their own
  * contexts, so their own streams; any grids, species, beams and
  * precisions; all on one device).  The slice is qp_slice_run's with these
  * differences: the slice index is a device word of each simulation
  * (qp_sim_begin_step sets it to 1, each captured slice advances it), so the
- * one graph serves every slice; with tol > 0 all iter_max passes are
- * enqueued and the kernels of the passes after the converged one return at
- * once (the stopping test and the result are qp_slice_run's); the particle
+ * same graphs serve every slice; with tol > 0 a slice is cut into graphs
+ * between its passes, of which qp_scan_run launches as many as each
+ * simulation's residuals ask for (the kernels of a pass behind the converged
+ * one return at once; the stopping test and the result are qp_slice_run's); the particle
  * move check is read once per qp_scan_run; the mixed corrector and the 3-D
  * diagnostics (cbq, psi, current) are not available (QP_ERR_UNSUPPORTED).
  * Create after qp_sim_begin_step; the simulations must have profiling off. */

@@ -288,122 +288,206 @@ int qp_slice_prepare(qp_sim *s, int j)
     return QP_OK;
 }
 
-// the rest of the slice: corrector seed, predictor, passes, push, slice
-// writes.  front: only the charges are there (slice_charges); the fields of
-// qp_slice_prepare are solved for together with the predictor's.
-static int slice_finish(qp_sim *s, int j, int iter_max, double tol, int *iters_used,
-                        double *residual, bool front)
-{
-    qp_ctx *c = s->ctx;
-    QP_REQUIRE(iter_max >= 1, QP_ERR_ARG, "qp_slice_finish: iter_max %d", iter_max);
-    s->prepared = 0;
-    const double dex = c->dex;
-    qp_field2d **F = s->f;
-    qp_field2d *psi = F[QP_F_PSI], *fxy = F[QP_F_FXY];
-    qp_field2d *cu = F[QP_F_CU], *dcu = F[QP_F_DCU], *amu = F[QP_F_AMU], *bxyz = F[QP_F_BXYZ];
-    qp_field2d *psit = F[QP_F_PSIT], *epw = F[QP_F_EPW], *epwb = F[QP_F_EPWB];
-    const int nsp = (int)s->sp.size();
+}  // extern "C"
+
+namespace {
+
+// The parts of a slice after its charges, enqueued in order: begin (corrector
+// seed and predictor; with front also psi and E_perp, solved for together with
+// the predictor's fields), pass 1, 2, ... (head and tail), and end (push and
+// slice writes).  Inside captured slices (s->graph) the slice index and the
+// seed's count are read from device memory.
+struct SliceRun {
+    qp_sim *s;
+    int j, iter_max;
+    double tol;
+    qp_ctx *c;
+    bool adaptive, mixing, fused;
+    int seed = 0, tag0 = 0;
+    PassFields pf, pc;
+
+    SliceRun(qp_sim *sim, int jj, int imax, double t)
+        : s(sim), j(jj), iter_max(imax), tol(t), c(sim->ctx), adaptive(t > 0.0),
+          // the mixed corrector (QP_TUNE_MIX) applies only to runs to a
+          // tolerance outside captured slices
+          mixing(t > 0.0 && !sim->graph && sim->ctx->tune[QP_TUNE_MIX] == 1),
+          fused(fused_fields(sim->ctx) && !mixing),
+          pf{sim->f[QP_F_CU], sim->f[QP_F_DCU], sim->f[QP_F_AMU], sim->f[QP_F_EPW],
+             sim->f[QP_F_EPWB], sim->f[QP_F_PSIT], sim->f[QP_F_BXYZ], nullptr, nullptr},
+          pc(pf)
+    {
+        if (mixing) {
+            pc.gprev = s->gprev;
+            pc.fprev = s->fprev;
+        }
+    }
+
+    int *flags() const { return c->flags.as<int>(); }
+
     // predictor fields from the carried current (:671-675) and the B assembly
-    const PassFields pf{cu, dcu, amu, epw, epwb, psit, bxyz, nullptr, nullptr};
-    qp_field2d *inv[2] = {psit, bxyz};
-    const int inv_kinds[2] = {1, 2};
-    qp_field2d *fwd[3] = {cu, dcu, amu};
-    const int fwd_kinds[3] = {1, 1, 3};
-    const bool adaptive = tol > 0.0;
-    const bool graph = s->graph;
-    // the mixed corrector (QP_TUNE_MIX) applies only to runs to a tolerance
-    // outside captured slices
-    const bool mixing = adaptive && !graph && c->tune[QP_TUNE_MIX] == 1;
-    PassFields pc = pf;
-    if (mixing) {
-        pc.gprev = s->gprev;
-        pc.fprev = s->fprev;
+    int begin(bool front)
+    {
+        QP_REQUIRE(iter_max >= 1, QP_ERR_ARG, "qp_slice_finish: iter_max %d", iter_max);
+        s->prepared = 0;
+        // the extrapolated corrector seed is applied by the predictor's kernel:
+        // linear (QP_TUNE_SEED = 1) or quadratic (3) in xi
+        const bool quad = c->tune[QP_TUNE_SEED] == 3;
+        if (adaptive && (c->tune[QP_TUNE_SEED] == 1 || quad)) {
+            seed = s->hist_slices >= 3 ? 3 : (s->hist_slices >= 2 ? 2 : 1);
+            ++s->hist_slices;
+        }
+        const int *seed_hist = s->graph && seed ? s->ctl.as<int>() + 1 : nullptr;
+        qp_field2d *hist2 = quad ? s->epw_hist2 : nullptr;
+        if (front) {
+            const FrontFields fr{s->f[QP_F_QB], s->f[QP_F_QE], s->f[QP_F_PSI], s->f[QP_F_FXY],
+                                 s->epw_hist, hist2};
+            RC(fused_solve_front(pf, fr, c->dex, seed, seed_hist));
+        } else {
+            RC(fused_pass(pf, c->dex, false, 0, 0.0, seed, s->epw_hist, seed_hist, hist2));
+            RC(inverse());
+        }
+        // launches of pass l carry tag tag0 + l, unique to this slice, so that
+        // the timing of a speculative pass that returned at once is dropped
+        // without touching the earlier slices' pending timings
+        c->prof_epoch = (c->prof_epoch + 1) & 0xffffff;
+        tag0 = c->prof_epoch << 6;
+        return QP_OK;
     }
-    // the extrapolated corrector seed is applied by the predictor's kernel:
-    // linear (QP_TUNE_SEED = 1) or quadratic (3) in xi
-    int seed = 0;
-    const bool quad = c->tune[QP_TUNE_SEED] == 3;
-    if (adaptive && (c->tune[QP_TUNE_SEED] == 1 || quad)) {
-        seed = s->hist_slices >= 3 ? 3 : (s->hist_slices >= 2 ? 2 : 1);
-        ++s->hist_slices;
+
+    int inverse()
+    {
+        qp_field2d *inv[2] = {pf.psit, pf.bxyz};
+        const int kinds[2] = {1, 2};
+        RC(fft_k2r_batch(c, inv, kinds, 2));
+        pf.psit->state = pf.bxyz->state = 0;
+        return QP_OK;
     }
-    const int *seed_hist = graph && seed ? s->ctl.as<int>() + 1 : nullptr;
-    if (front) {
-        const FrontFields fr{F[QP_F_QB], F[QP_F_QE], psi, fxy, s->epw_hist,
-                             quad ? s->epw_hist2 : nullptr};
-        RC(fused_solve_front(pf, fr, dex, seed, seed_hist));
-    } else {
-        RC(fused_pass(pf, dex, false, 0, 0.0, seed, s->epw_hist, seed_hist,
-                      quad ? s->epw_hist2 : nullptr));
-        RC(fft_k2r_batch(c, inv, inv_kinds, 2));
-        psit->state = bxyz->state = 0;
-    }
-    const bool fused = fused_fields(c) && !mixing;
-    // corrector passes (:676-710)
-    int *flags = c->flags.as<int>();
-    // launches of pass l carry tag tag0 + l, unique to this slice, so that
-    // the timing of a speculative pass that returned at once is dropped
-    // without touching the earlier slices' pending timings
-    c->prof_epoch = (c->prof_epoch + 1) & 0xffffff;
-    const int tag0 = c->prof_epoch << 6;
-    // a pass is its deposits (head) and its field solve (tail)
-    auto head = [&](int l) -> int {
+
+    // corrector passes (:676-710): a pass is its deposits (head) and its field
+    // solve (tail); with c->skip set, its kernels return at once when flag word
+    // l - 1 says that an earlier pass has converged
+    int head(int l)
+    {
         c->prof_tag = tag0 + l;
-        if (c->skip) c->skip = flags + (l - 1);
+        if (c->skip) c->skip = flags() + (l - 1);
+        const int nsp = (int)s->sp.size();
         if (nsp == 0) {
-            RC(qp_field2d_as(cu, 0.0));
-            RC(qp_field2d_as(dcu, 0.0));
-            RC(qp_field2d_as(amu, 0.0));
+            RC(qp_field2d_as(pf.cu, 0.0));
+            RC(qp_field2d_as(pf.dcu, 0.0));
+            RC(qp_field2d_as(pf.amu, 0.0));
         }
         // the first pass applies the species' psi gather (extpsi, :667-669)
         // to each particle just before its deposit
         for (int i = 0; i < nsp; ++i)
-            RC(species_amjdp_fused(s->sp[i], fxy, bxyz, psit, cu, dcu, amu, dex, i == 0,
-                                   i == nsp - 1, l == 1 ? psi : nullptr));
+            RC(species_amjdp_fused(s->sp[i], s->f[QP_F_FXY], pf.bxyz, pf.psit, pf.cu, pf.dcu,
+                                   pf.amu, c->dex, i == 0, i == nsp - 1,
+                                   l == 1 ? s->f[QP_F_PSI] : nullptr));
         c->prof_tag = 0;
         return QP_OK;
-    };
-    auto tail = [&](int l) -> int {
+    }
+
+    int tail(int l)
+    {
         c->prof_tag = tag0 + l;
-        if (c->skip) c->skip = flags + (l - 1);
+        if (c->skip) c->skip = flags() + (l - 1);
         if (fused) {
-            RC(fused_solve_pass(pf, dex, l, tol));
-            c->prof_tag = 0;
-            return QP_OK;
+            RC(fused_solve_pass(pf, c->dex, l, tol));
+        } else {
+            qp_field2d *fwd[3] = {pf.cu, pf.dcu, pf.amu};
+            const int kinds[3] = {1, 1, 3};
+            RC(fft_r2k_batch(c, fwd, kinds, 3));
+            pf.cu->state = pf.dcu->state = pf.amu->state = 1;
+            RC(fused_pass(pc, c->dex, true, l, tol));
+            if (mixing) RC(fused_mix(pc, c->dex, l, tol, l >= 2 && l < iter_max));
+            RC(inverse());
         }
-        RC(fft_r2k_batch(c, fwd, fwd_kinds, 3));
-        cu->state = dcu->state = amu->state = 1;
-        RC(fused_pass(pc, dex, true, l, tol));
-        if (mixing) RC(fused_mix(pc, dex, l, tol, l >= 2 && l < iter_max));
-        RC(fft_k2r_batch(c, inv, inv_kinds, 2));
-        psit->state = bxyz->state = 0;
         c->prof_tag = 0;
         return QP_OK;
-    };
-    auto pass = [&](int l) -> int {
+    }
+
+    int pass(int l)
+    {
         RC(head(l));
         return tail(l);
-    };
+    }
+
+    // passes l0..l1 of a captured slice
+    int captured(int l0, int l1)
+    {
+        c->skip = adaptive ? flags() : nullptr;
+        int rc = QP_OK;
+        for (int l = l0; l <= l1 && !rc; ++l) rc = pass(l);
+        c->skip = nullptr;
+        return rc;
+    }
+
+    int end()
+    {
+        const bool graph = s->graph;
+        // plasma push (:727-730); B is already assembled, and E_perp (:721-723)
+        // is formed where it is gathered
+        for (qp_species *sp : s->sp)
+            RC(species_push_nocheck(sp, s->f[QP_F_FXY], pf.bxyz, pf.psit, c->dex));
+        // E_perp, the predictor current (:724-726), slice j+1 of the 3-D wake
+        // (:731-735) and the move checks' words
+        EndFields e{s->f[QP_F_FXY], s->f[QP_F_PSI], s->bexyz, s->bbxyz, j + 1};
+        e.jdev = graph ? s->ctl.as<int>() : nullptr;
+        e.ctl = graph ? nullptr : s->ctl.as<int>();
+        e.hist = s->hist_slices;
+        e.spec = fused;
+        e.slice = j;
+        if (!graph)
+            for (qp_species *sp : s->sp)
+                if (e.nerr < 4) {
+                    species_err_words(sp, &e.err[e.nerr], &e.h_err[e.nerr]);
+                    ++e.nerr;
+                }
+        RC(fused_slice_end(pf, e));
+        if (graph) {
+            hipLaunchKernelGGL(k_slice_end, dim3(1), dim3(64), 0, c->stream, s->ctl.as<int>(),
+                               flags(), iter_max, adaptive ? 1 : 0, seeding() ? 1 : 0,
+                               s->passes_dev.as<int>(), c->nz);
+            QP_LAUNCH_CHECK();
+            return QP_OK;
+        }
+        for (size_t i = 0; i < s->sp.size(); ++i)
+            RC((int)i < e.nerr ? species_check_mark(s->sp[i]) : species_check_post(s->sp[i], j));
+        return QP_OK;
+    }
+
+    bool seeding() const
+    {
+        return adaptive && (c->tune[QP_TUNE_SEED] == 1 || c->tune[QP_TUNE_SEED] == 3);
+    }
+};
+
+// what comes before SliceRun::begin, and begin
+int slice_begin(SliceRun &r)
+{
+    if (fused_fields(r.c)) {
+        RC(slice_charges(r.s, r.j));
+        return r.begin(true);
+    }
+    RC(qp_slice_prepare(r.s, r.j));
+    return r.begin(false);
+}
+
+// the passes and the end of a slice that has begun
+int slice_finish(SliceRun &r, int *iters_used, double *residual)
+{
+    qp_sim *s = r.s;
+    qp_ctx *c = r.c;
+    const double tol = r.tol;
+    const int j = r.j, iter_max = r.iter_max, nsp = (int)s->sp.size();
     int l = 0;
     double res = -1.0;
-    if (!adaptive) {
-        for (l = 1; l <= iter_max; ++l) RC(pass(l));
-        l = iter_max;
-    } else if (graph) {
-        // every pass is enqueued; once pass l converges (flag word l), the
-        // kernels of the later passes return at once and pass the flag on
-        QP_REQUIRE(iter_max < FLAG_WORDS, QP_ERR_ARG, "captured slice: iter_max %d >= %d",
-                   iter_max, FLAG_WORDS);
-        c->skip = flags;
-        int rc = QP_OK;
-        for (l = 1; l <= iter_max && !rc; ++l) rc = pass(l);
-        c->skip = nullptr;
-        RC(rc);
+    if (!r.adaptive) {
+        for (l = 1; l <= iter_max; ++l) RC(r.pass(l));
         l = iter_max;
     } else if (nsp == 0 || !c->tune[QP_TUNE_SPECULATE] || iter_max >= FLAG_WORDS) {
         // read each residual in turn
         for (l = 1;; ++l) {
-            RC(pass(l));
+            RC(r.pass(l));
             QP_HIP(hipStreamSynchronize(c->stream));
             res = c->h_res[l % RES_SLOTS];
             if (res < tol || l == iter_max) break;
@@ -423,15 +507,15 @@ static int slice_finish(qp_sim *s, int j, int iter_max, double tol, int *iters_u
             qp_ctx *c;
             ~SkipGuard() { c->skip = nullptr; }
         } guard{c};
-        c->skip = flags;
+        c->skip = r.flags();
         const int P = c->tune[QP_TUNE_SPECULATE] == 2
                           ? std::max(1, std::min(iter_max, s->pred_passes)) : 1;
-        for (int k = 1; k <= P; ++k) RC(pass(k));
+        for (int k = 1; k <= P; ++k) RC(r.pass(k));
         QP_HIP(hipEventRecord(c->pass_ev[P & 1], c->stream));
         int lo = 1;   // the first pass whose residual has not been read
         for (l = P;; ++l) {
             const bool more = l < iter_max;
-            if (more) RC(head(l + 1));
+            if (more) RC(r.head(l + 1));
             QP_HIP(hipEventSynchronize(c->pass_ev[l & 1]));
             // passes lo..l ran (those after a converged one returned at once
             // and left their residual slots alone): the first below tol
@@ -441,11 +525,11 @@ static int slice_finish(qp_sim *s, int j, int iter_max, double tol, int *iters_u
             if (conv || !more) {
                 const int last = conv ? conv : l;
                 res = c->h_res[last % RES_SLOTS];
-                for (int k = last + 1; k <= l + (more ? 1 : 0); ++k) prof_discard(c, tag0 + k);
+                for (int k = last + 1; k <= l + (more ? 1 : 0); ++k) prof_discard(c, r.tag0 + k);
                 l = last;
                 break;
             }
-            RC(tail(l + 1));
+            RC(r.tail(l + 1));
             QP_HIP(hipEventRecord(c->pass_ev[(l + 1) & 1], c->stream));
             lo = l + 1;
         }
@@ -459,53 +543,32 @@ static int slice_finish(qp_sim *s, int j, int iter_max, double tol, int *iters_u
         if (s->q3s[i]) RC(qp_species_cbq(s->sp[i], s->q3s[i], j + 1));
     // the current of the last pass, scaled by dex, into cu3d (:696-698):
     // its real-space planes are kept by the forward transform
-    if (s->cu3d) RC(copy_planes(c, cu, s->cu3d, j + 1));
-    // plasma push (:727-730); B is already assembled, and E_perp (:721-723) is
-    // formed where it is gathered
-    for (qp_species *sp : s->sp) RC(species_push_nocheck(sp, fxy, bxyz, psit, dex));
-    // E_perp, the predictor current (:724-726), slice j+1 of the 3-D wake
-    // (:731-735) and the move checks' words
-    EndFields e{fxy, psi, s->bexyz, s->bbxyz, j + 1};
-    e.jdev = graph ? s->ctl.as<int>() : nullptr;
-    e.ctl = graph ? nullptr : s->ctl.as<int>();
-    e.hist = s->hist_slices;
-    e.spec = fused;
-    e.slice = j;
-    if (!graph)
-        for (qp_species *sp : s->sp)
-            if (e.nerr < 4) {
-                species_err_words(sp, &e.err[e.nerr], &e.h_err[e.nerr]);
-                ++e.nerr;
-            }
-    RC(fused_slice_end(pf, e));
-    if (graph) {
-        hipLaunchKernelGGL(k_slice_end, dim3(1), dim3(64), 0, c->stream, s->ctl.as<int>(), flags,
-                           iter_max, adaptive ? 1 : 0, seed ? 1 : 0, s->passes_dev.as<int>(),
-                           c->nz);
-        QP_LAUNCH_CHECK();
-        if (iters_used) *iters_used = -1;
-        if (residual) *residual = -1.0;
-        return QP_OK;
-    }
+    if (s->cu3d) RC(copy_planes(c, r.pf.cu, s->cu3d, j + 1));
+    RC(r.end());
     // psi * dex^2 into psi3d (:670-671); the slice write applied the scaling
-    if (s->psi3d) RC(copy_planes(c, psi, s->psi3d, j + 1));
-    for (size_t i = 0; i < s->sp.size(); ++i)
-        RC((int)i < e.nerr ? species_check_mark(s->sp[i]) : species_check_post(s->sp[i], j));
+    if (s->psi3d) RC(copy_planes(c, s->f[QP_F_PSI], s->psi3d, j + 1));
     // strict move check: wait for this slice's check before returning
     if (c->tune[QP_TUNE_STRICT])
         for (qp_species *sp : s->sp) RC(species_check_poll(sp, true));
     s->last_passes = l;
-    s->last_adaptive = adaptive;
+    s->last_adaptive = r.adaptive;
     if (iters_used) *iters_used = l;
-    if (residual) *residual = adaptive ? res : -1.0;
+    if (residual) *residual = r.adaptive ? res : -1.0;
     return QP_OK;
 }
 
+}  // namespace
+
+extern "C" {
+
+// the rest of the slice: corrector seed, predictor, passes, push, slice writes
 int qp_slice_finish(qp_sim *s, int j, int iter_max, double tol, int *iters_used, double *residual)
 {
     QP_REQUIRE(s, QP_ERR_ARG, "qp_slice_finish: null sim");
     QP_REQUIRE(s->prepared == j, QP_ERR_STATE, "qp_slice_finish: slice %d was not prepared", j);
-    return slice_finish(s, j, iter_max, tol, iters_used, residual, false);
+    SliceRun r(s, j, iter_max, tol);
+    RC(r.begin(false));
+    return slice_finish(r, iters_used, residual);
 }
 
 int qp_slice_residuals(const qp_sim *s, double *res, int max, int *n)
@@ -523,12 +586,9 @@ int qp_slice_residuals(const qp_sim *s, double *res, int max, int *n)
 int qp_slice_run(qp_sim *s, int j, int iter_max, double tol, int *iters_used, double *residual)
 {
     QP_REQUIRE(s, QP_ERR_ARG, "qp_slice_run: null sim");
-    if (!fused_fields(s->ctx)) {
-        RC(qp_slice_prepare(s, j));
-        return qp_slice_finish(s, j, iter_max, tol, iters_used, residual);
-    }
-    RC(slice_charges(s, j));
-    return slice_finish(s, j, iter_max, tol, iters_used, residual, true);
+    SliceRun r(s, j, iter_max, tol);
+    RC(slice_begin(r));
+    return slice_finish(r, iters_used, residual);
 }
 
 int qp_sim_push_beams(qp_sim *s)
@@ -558,83 +618,169 @@ int qp_sim_end_step(qp_sim *s, double snew)
     return qp_sim_renew(s, snew);
 }
 
-// ---- batched scan: one HIP graph holding one xi slice of many instances ----
+// ---- batched scan: xi slices of many instances as HIP graphs ----
 
+// A slice of one instance, captured on the instance's own stream.  With a fixed
+// number of passes it is one graph.  To a tolerance it is cut: the start with
+// SCAN_FIRST passes, one graph per further pass, and the end; the host reads the
+// residuals (pinned memory) and enqueues no pass after the one that converges.
+//
 // The plasma push moves the particles between two sets of arrays and swaps
-// the host's pointers to them, which a graph cannot repeat: the scan holds
-// two graphs, one captured with each buffer parity, and launches the one
-// that matches where the particles are (the first species of the instances
-// tells), swapping the host pointers after each launch as the push would.
-struct qp_scan {
-    std::vector<qp_sim *> sims;
-    int iter_max = 0;
-    double tol = 0.0;
-    hipStream_t origin = nullptr;          // the stream the graphs are launched on
-    hipEvent_t fork = nullptr;
-    std::vector<hipEvent_t> join;
-    hipGraph_t graph[2] = {nullptr, nullptr};
-    hipGraphExec_t exec[2] = {nullptr, nullptr};
-    std::vector<const void *> key0;        // per instance: particle buffer of parity 0
-    std::vector<char> offsets;             // per instance: the push swaps cell offsets
+// the host's pointers to them, which a graph cannot repeat: each instance holds
+// its slice twice, captured with each buffer parity, and launches the one that
+// matches where the particles are, swapping the host pointers after each
+// slice as the push would.
+struct ScanPart {
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;   // made when it is first launched
 };
 
-static void scan_flip(qp_scan *sc)
+struct ScanSlice {
+    ScanPart start, end;             // fixed passes: the whole slice is start
+    std::vector<ScanPart> pass;      // passes SCAN_FIRST + 1 ...
+};
+
+struct ScanInstance {
+    qp_sim *s = nullptr;
+    ScanSlice slice[2];                // per buffer parity
+    const void *key0 = nullptr;        // the particle buffer of parity 0
+    bool offsets = false;              // the push swaps cell offsets
+    int pred = 0;                      // passes the last slice needed
+    // while a run is under way
+    int parity = 0, left = 0, done = 0;
+};
+
+struct qp_scan {
+    std::vector<ScanInstance> inst;
+    int iter_max = 0;
+    double tol = 0.0;
+};
+
+}  // extern "C"
+
+// The host polls for the slowest kernels in between: after this many looks
+// without news it asks the stream whether it still runs.
+static constexpr int SCAN_POLLS = 1 << 14;
+
+// Passes in the first graph.  24 slices of 12 instances on 256^2 and 512^2, 4.8
+// to 5.8 passes of at most 20: one graph holding a slice of all instances with
+// all 20 passes 87 ms (a pass after convergence still costs its launches), cut
+// with a wait for the slowest instance in each slice 80 ms and 33 ms for freeing
+// its graphs, the instances apart from each other 76 ms and 1 ms.
+static constexpr int SCAN_FIRST = 4;
+
+static void part_free(ScanPart &p)
 {
-    for (size_t i = 0; i < sc->sims.size(); ++i)
-        for (qp_species *sp : sc->sims[i]->sp) species_flip(sp, sc->offsets[i] != 0);
+    if (p.exec) (void)hipGraphExecDestroy(p.exec);
+    if (p.graph) (void)hipGraphDestroy(p.graph);
 }
+
+static int part_launch(ScanPart &p, hipStream_t st)
+{
+    if (!p.exec) QP_HIP(hipGraphInstantiate(&p.exec, p.graph, nullptr, nullptr, 0));
+    QP_HIP(hipGraphLaunch(p.exec, st));
+    return QP_OK;
+}
+
+template <typename F> static int part_capture(ScanPart &p, const qp_scan *sc, qp_sim *s, F part)
+{
+    QP_HIP(hipStreamBeginCapture(s->ctx->stream, hipStreamCaptureModeRelaxed));
+    const int hist = s->hist_slices;   // the captured seed counts on the device
+    s->graph = true;
+    SliceRun r(s, 1, sc->iter_max, sc->tol);
+    int rc = part(r);
+    s->graph = false;
+    s->prepared = 0;
+    s->hist_slices = hist;
+    hipError_t e = hipStreamEndCapture(s->ctx->stream, &p.graph);
+    if (!rc && e != hipSuccess) rc = hip_fail(e, "hipStreamEndCapture", __FILE__, __LINE__);
+    return rc;
+}
+
+static int slice_capture(ScanSlice &sl, const qp_scan *sc, qp_sim *s)
+{
+    const bool adaptive = sc->tol > 0.0;
+    const int first = adaptive ? std::min(SCAN_FIRST, sc->iter_max) : sc->iter_max;
+    RC(part_capture(sl.start, sc, s, [&](SliceRun &r) -> int {
+        RC(slice_begin(r));
+        RC(r.captured(1, first));
+        return adaptive ? QP_OK : r.end();
+    }));
+    if (!adaptive) return QP_OK;
+    sl.pass.resize(sc->iter_max - first);
+    for (int l = first + 1; l <= sc->iter_max; ++l)
+        RC(part_capture(sl.pass[l - first - 1], sc, s,
+                        [&](SliceRun &r) -> int { return r.captured(l, l); }));
+    return part_capture(sl.end, sc, s, [&](SliceRun &r) -> int { return r.end(); });
+}
+
+// enqueues the start of an instance's next slice and as many passes as its last
+// one needed.  None of its passes is in flight: the ones of the slice before
+// that ran have written their residuals.
+static int scan_start(qp_scan *sc, ScanInstance &in)
+{
+    ScanSlice &sl = in.slice[in.parity];
+    hipStream_t st = in.s->ctx->stream;
+    if (sc->tol <= 0.0) {
+        RC(part_launch(sl.start, st));
+    } else {
+        volatile double *h = in.s->ctx->h_res;
+        for (int l = 1; l <= sc->iter_max; ++l) h[l % RES_SLOTS] = -1.0;
+        RC(part_launch(sl.start, st));
+        const int first = sc->iter_max - (int)sl.pass.size();
+        for (in.done = first; in.done < in.pred; ++in.done)
+            RC(part_launch(sl.pass[in.done - first], st));
+    }
+    return QP_OK;
+}
+
+// the slice is enqueued to its end: the next one
+static int scan_next(qp_scan *sc, ScanInstance &in)
+{
+    for (qp_species *sp : in.s->sp) species_flip(sp, in.offsets);
+    in.parity ^= 1;
+    return --in.left ? scan_start(sc, in) : QP_OK;
+}
+
+// One look at an instance that runs to the tolerance: news is set when its
+// enqueued passes are through, after the next pass, or the end and the start of
+// the next slice, have been enqueued.
+static int scan_step(qp_scan *sc, ScanInstance &in, bool *news)
+{
+    const volatile double *h = in.s->ctx->h_res;
+    int conv = 0;
+    for (int l = 1; l <= in.done && !conv; ++l) {
+        const double r = h[l % RES_SLOTS];
+        if (r == -1.0) return QP_OK;
+        if (r >= 0.0 && r < sc->tol) conv = l;
+    }
+    *news = true;
+    ScanSlice &sl = in.slice[in.parity];
+    if (!conv && in.done < sc->iter_max) {
+        const int first = sc->iter_max - (int)sl.pass.size();
+        RC(part_launch(sl.pass[in.done - first], in.s->ctx->stream));
+        ++in.done;
+        return QP_OK;
+    }
+    in.pred = conv ? conv : in.done;
+    RC(part_launch(sl.end, in.s->ctx->stream));
+    return scan_next(sc, in);
+}
+
+extern "C" {
 
 int qp_scan_destroy(qp_scan *sc)
 {
     if (!sc) return QP_OK;
-    if (sc->origin) (void)hipStreamSynchronize(sc->origin);
-    for (int p = 0; p < 2; ++p) {
-        if (sc->exec[p]) (void)hipGraphExecDestroy(sc->exec[p]);
-        if (sc->graph[p]) (void)hipGraphDestroy(sc->graph[p]);
+    for (ScanInstance &in : sc->inst) {
+        if (in.s) (void)hipStreamSynchronize(in.s->ctx->stream);
+        for (ScanSlice &sl : in.slice) {
+            part_free(sl.start);
+            for (ScanPart &p : sl.pass) part_free(p);
+            part_free(sl.end);
+        }
     }
-    for (hipEvent_t e : sc->join)
-        if (e) (void)hipEventDestroy(e);
-    if (sc->fork) (void)hipEventDestroy(sc->fork);
-    if (sc->origin) (void)hipStreamDestroy(sc->origin);
     delete sc;
-    return QP_OK;
-}
-
-// The capture: the origin stream forks to every instance's own stream, each
-// instance enqueues one slice there (prepare + finish in graph mode, which
-// reads the slice index from its device word and ends with k_slice_end), and
-// the streams join back.  Instances are independent branches of the graph.
-static int scan_capture(qp_scan *sc, int parity)
-{
-    QP_HIP(hipStreamBeginCapture(sc->origin, hipStreamCaptureModeRelaxed));
-    int rc = QP_OK;
-    hipError_t e = hipEventRecord(sc->fork, sc->origin);
-    if (e != hipSuccess) rc = hip_fail(e, "hipEventRecord", __FILE__, __LINE__);
-    for (size_t i = 0; i < sc->sims.size() && !rc; ++i) {
-        qp_sim *s = sc->sims[i];
-        qp_ctx *c = s->ctx;
-        e = hipStreamWaitEvent(c->stream, sc->fork, 0);
-        if (e != hipSuccess) { rc = hip_fail(e, "hipStreamWaitEvent", __FILE__, __LINE__); break; }
-        const int hist = s->hist_slices;   // the captured seed counts on the device
-        s->graph = true;
-        rc = qp_slice_run(s, 1, sc->iter_max, sc->tol, nullptr, nullptr);
-        s->graph = false;
-        s->prepared = 0;
-        s->hist_slices = hist;
-        if (rc) break;
-        e = hipEventRecord(sc->join[i], c->stream);
-        if (e == hipSuccess) e = hipStreamWaitEvent(sc->origin, sc->join[i], 0);
-        if (e != hipSuccess) rc = hip_fail(e, "capture join", __FILE__, __LINE__);
-    }
-    hipGraph_t g = nullptr;
-    e = hipStreamEndCapture(sc->origin, &g);
-    if (!rc && e != hipSuccess) rc = hip_fail(e, "hipStreamEndCapture", __FILE__, __LINE__);
-    if (rc) {
-        if (g) (void)hipGraphDestroy(g);
-        return rc;
-    }
-    sc->graph[parity] = g;
-    QP_HIP(hipGraphInstantiate(&sc->exec[parity], g, nullptr, nullptr, 0));
     return QP_OK;
 }
 
@@ -661,31 +807,23 @@ int qp_scan_create(qp_sim *const *sims, int n, int iter_max, double tol, qp_scan
     }
     QP_HIP(hipSetDevice(sims[0]->ctx->device));
     qp_scan *sc = new qp_scan();
-    sc->sims.assign(sims, sims + n);
+    sc->inst.resize(n);
     sc->iter_max = iter_max;
     sc->tol = tol;
-    sc->join.assign(n, nullptr);
     int rc = QP_OK;
-    hipError_t e = hipStreamCreateWithFlags(&sc->origin, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&sc->fork, hipEventDisableTiming);
-    for (int i = 0; i < n && e == hipSuccess; ++i)
-        e = hipEventCreateWithFlags(&sc->join[i], hipEventDisableTiming);
-    if (e != hipSuccess) rc = hip_fail(e, "qp_scan_create", __FILE__, __LINE__);
-    // the instances' pending work (set-up, begin_step) is not part of the graph
     for (int i = 0; i < n && !rc; ++i) {
-        e = hipStreamSynchronize(sims[i]->ctx->stream);
+        ScanInstance &in = sc->inst[i];
+        in.s = sims[i];
+        if (!in.s->sp.empty()) in.key0 = species_buffer_key(in.s->sp[0]);
+        in.offsets = in.s->ctx->tune[QP_TUNE_PUSH] != 1;
+        // the instance's pending work (set-up, begin_step) is not part of the graphs
+        hipError_t e = hipStreamSynchronize(in.s->ctx->stream);
         if (e != hipSuccess) rc = hip_fail(e, "hipStreamSynchronize", __FILE__, __LINE__);
+        // each capture swaps the host pointers once (the push's host side), so
+        // after the two the host is back where it started
+        if (!rc) rc = slice_capture(in.slice[0], sc, in.s);
+        if (!rc) rc = slice_capture(in.slice[1], sc, in.s);
     }
-    sc->key0.assign(n, nullptr);
-    sc->offsets.assign(n, 0);
-    for (int i = 0; i < n; ++i) {
-        if (!sims[i]->sp.empty()) sc->key0[i] = species_buffer_key(sims[i]->sp[0]);
-        sc->offsets[i] = sims[i]->ctx->tune[QP_TUNE_PUSH] == 1 ? 0 : 1;
-    }
-    // each capture swaps the host pointers once (the push's host side), so
-    // after the two the host is back where it started
-    if (!rc) rc = scan_capture(sc, 0);
-    if (!rc) rc = scan_capture(sc, 1);
     if (rc) { qp_scan_destroy(sc); return rc; }
     *out = sc;
     return QP_OK;
@@ -693,22 +831,22 @@ int qp_scan_create(qp_sim *const *sims, int n, int iter_max, double tol, qp_scan
 
 int qp_scan_run(qp_scan *sc, int nslices)
 {
-    QP_REQUIRE(sc && sc->exec[0] && sc->exec[1] && nslices >= 0, QP_ERR_ARG,
-               "qp_scan_run: bad argument");
+    QP_REQUIRE(sc && !sc->inst.empty() && nslices >= 0, QP_ERR_ARG, "qp_scan_run: bad argument");
     // the buffer parity of every instance (they must agree: an instance
     // advanced by eager slices in between would not match the graphs)
     int parity = -1;
-    for (size_t i = 0; i < sc->sims.size(); ++i) {
-        if (!sc->key0[i]) continue;
-        const int p = species_buffer_key(sc->sims[i]->sp[0]) == sc->key0[i] ? 0 : 1;
+    for (size_t i = 0; i < sc->inst.size(); ++i) {
+        const ScanInstance &in = sc->inst[i];
+        if (!in.key0) continue;
+        const int p = species_buffer_key(in.s->sp[0]) == in.key0 ? 0 : 1;
         QP_REQUIRE(parity < 0 || p == parity, QP_ERR_STATE,
                    "qp_scan_run: instance %zu's particles are in the other buffer", i);
         parity = p;
     }
     if (parity < 0) parity = 0;
     // the slices left in each instance's step (its device slice word)
-    for (size_t i = 0; i < sc->sims.size(); ++i) {
-        qp_sim *s = sc->sims[i];
+    for (size_t i = 0; i < sc->inst.size(); ++i) {
+        qp_sim *s = sc->inst[i].s;
         int j = 0;
         QP_HIP(hipMemcpyAsync(&j, s->ctl.p, sizeof(int), hipMemcpyDeviceToHost, s->ctx->stream));
         QP_HIP(hipStreamSynchronize(s->ctx->stream));
@@ -716,24 +854,53 @@ int qp_scan_run(qp_scan *sc, int nslices)
                    "qp_scan_run: instance %zu is at slice %d; %d more exceed its %d slices", i, j,
                    nslices, s->ctx->nz);
     }
-    // the graph runs after what the instances' streams hold, and they wait
-    // for it in turn, so the library's eager calls before and after order
-    // with the captured slices
-    for (size_t i = 0; i < sc->sims.size(); ++i) {
-        QP_HIP(hipEventRecord(sc->join[i], sc->sims[i]->ctx->stream));
-        QP_HIP(hipStreamWaitEvent(sc->origin, sc->join[i], 0));
+    // the instances' streams are independent, and the library's eager calls
+    // before and after order with the slices on them
+    size_t busy = 0;
+    for (ScanInstance &in : sc->inst) {
+        in.parity = parity;
+        in.left = nslices;
+        if (nslices) {
+            RC(scan_start(sc, in));
+            ++busy;
+        }
     }
-    for (int k = 0; k < nslices; ++k) {
-        QP_HIP(hipGraphLaunch(sc->exec[parity], sc->origin));
-        scan_flip(sc);
-        parity ^= 1;
+    if (sc->tol <= 0.0) {
+        for (int k = 0; k < nslices; ++k)
+            for (ScanInstance &in : sc->inst) RC(scan_next(sc, in));
+        busy = 0;
     }
-    QP_HIP(hipEventRecord(sc->fork, sc->origin));
-    for (qp_sim *s : sc->sims) QP_HIP(hipStreamWaitEvent(s->ctx->stream, sc->fork, 0));
-    QP_HIP(hipStreamSynchronize(sc->origin));
+    for (int idle = 0; busy;) {
+        bool news = false;
+        for (ScanInstance &in : sc->inst) {
+            if (!in.left) continue;
+            RC(scan_step(sc, in, &news));
+            if (!in.left) --busy;
+        }
+        if (news) {
+            idle = 0;
+        } else if (++idle == SCAN_POLLS) {
+            // a stream that failed, or ended without its residual, ends the wait
+            idle = 0;
+            for (ScanInstance &in : sc->inst) {
+                if (!in.left) continue;
+                const hipError_t e = hipStreamQuery(in.s->ctx->stream);
+                if (e == hipErrorNotReady) {
+                    (void)hipGetLastError();
+                    continue;
+                }
+                QP_HIP(e);
+                bool now = false;
+                RC(scan_step(sc, in, &now));
+                QP_REQUIRE(now, QP_ERR_STATE, "qp_scan_run: a slice ended without a residual");
+                if (!in.left) --busy;
+            }
+        }
+    }
+    for (ScanInstance &in : sc->inst) QP_HIP(hipStreamSynchronize(in.s->ctx->stream));
     // the particle move checks of the replayed slices (PPPCHECK2L)
-    for (size_t i = 0; i < sc->sims.size(); ++i)
-        for (qp_species *sp : sc->sims[i]->sp) {
+    for (size_t i = 0; i < sc->inst.size(); ++i)
+        for (qp_species *sp : sc->inst[i].s->sp) {
             int rc = species_check(sp);
             if (rc) {
                 const std::string msg = qp_last_error();
@@ -746,9 +913,9 @@ int qp_scan_run(qp_scan *sc, int nslices)
 
 int qp_scan_passes(const qp_scan *sc, int instance, int *passes, int nslices)
 {
-    QP_REQUIRE(sc && passes && instance >= 0 && instance < (int)sc->sims.size() && nslices >= 0,
+    QP_REQUIRE(sc && passes && instance >= 0 && instance < (int)sc->inst.size() && nslices >= 0,
                QP_ERR_ARG, "qp_scan_passes: bad argument");
-    const qp_sim *s = sc->sims[instance];
+    const qp_sim *s = sc->inst[instance].s;
     QP_REQUIRE(nslices <= s->ctx->nz, QP_ERR_ARG, "qp_scan_passes: %d slices > nz", nslices);
     std::vector<int> h((size_t)s->ctx->nz + 2);
     QP_HIP(hipMemcpyAsync(h.data(), s->passes_dev.p, h.size() * sizeof(int), hipMemcpyDeviceToHost,

@@ -7,12 +7,13 @@ U[0.3, 1.5], per-instance beam seed).  The transverse grids are powers of
 two, as the reference's are (indx, indy are log2 sizes,
 simulation_class.f03:151-224), so a scan draws them from 2^indx choices.
 
-run_graph captures one slice of every instance into one HIP graph
-(qpslice.Scan, qp_scan_*: the instances are independent branches, each slice
-index a device word) and replays it once per slice, so the GPU works on all
-instances at once from a single launch per slice; the corrector runs either
-the reference's fixed number of passes or to a residual tolerance (the
-passes after convergence return at once inside the graph).  run_batched
+run_graph captures one slice of every instance into HIP graphs
+(qpslice.Scan, qp_scan_*: each instance on its own stream, each slice index a
+device word) and replays them for every slice, so the GPU works on all
+instances at once from a few launches per slice; the corrector runs either
+the reference's fixed number of passes (one graph per slice) or to a residual
+tolerance (graphs cut between the passes, launched until an instance's
+residual is below it).  run_batched
 enqueues slice j of every instance before slice j+1 of any, each on its
 instance's stream, with fixed passes.  run_sequential runs the instances one
 after the other.  All three give bitwise-equal fields per instance (every
@@ -190,7 +191,7 @@ def run_sequential(insts, nslices):
 
 
 def run_graph(insts, nslices, chunk=None):
-    """All instances from one captured slice graph, replayed nslices times
+    """All instances from their captured slices, replayed nslices times
     (in runs of `chunk` slices); returns the wall time of the replays.  Each
     instance's passes per slice go to x.passes."""
     for x in insts:

@@ -696,8 +696,8 @@ class Sim:
 
 
 class Scan:
-    """One HIP graph holding one xi slice of each simulation (qp_scan_*):
-    run(n) replays it n times, every simulation continuing from its own
+    """HIP graphs holding one xi slice of each simulation (qp_scan_*):
+    run(n) replays them for n slices, every simulation continuing from its own
     last slice.  Create it after each simulation's begin_step."""
 
     def __init__(self, sims, iter_max=2, tol=0.0):

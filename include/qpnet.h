@@ -38,8 +38,25 @@ int qp_net_conv3x3(void *stream, const uint16_t *x, const uint16_t *mask, int H,
 int qp_net_conv3x3_wgrad(void *stream, const uint16_t *x, int cs_in, int cin,
                          const uint16_t *dy, const uint16_t *yout, int cs_out, int cout, int H,
                          int W, int nchunk, float *part, float *dw, float *db);
+/* the same for n layers at once (dw, db of each): part is scratch of npart
+ * floats for all of them, 10 * nchunk * cout * cin floats a layer for the best
+ * speed; any size will do */
+typedef struct {
+    const uint16_t *x, *dy, *yout;
+    float *dw, *db;
+    int cs_x, cin, cs_y, cout, H, W;
+} qp_net_layer;
+int qp_net_wgrad_layers(void *stream, const qp_net_layer *layers, int n, int nchunk, float *part,
+                        size_t npart);
 /* wt[tap][cin][cout] = w[8 - tap][cout][cin] (kernel of the data gradient) */
 int qp_net_flip_weights(void *stream, const uint16_t *w, int cout, int cin, uint16_t *wt);
+/* the same for n layers at once */
+typedef struct {
+    const uint16_t *w;
+    uint16_t *wt;
+    int cout, cin;
+} qp_net_flip;
+int qp_net_flip_layers(void *stream, const qp_net_flip *layers, int n);
 /* 2x2 average pooling (H, W even) and its gradient (din = / += dout / 4) */
 int qp_net_pool2(void *stream, const uint16_t *in, int cs_in, uint16_t *out, int cs_out, int H,
                  int W, int C);
@@ -91,7 +108,52 @@ int qp_net_mse(void *stream, const float *o, const float *t, size_t n, float *gr
  * BF16 copy */
 int qp_net_adam(void *stream, float *wm, const float *g, float *m, float *v, size_t n, float lr,
                 float b1, float b2, float eps, int step, uint16_t *wb);
+/* the same for n vectors at once */
+typedef struct {
+    float *w;
+    const float *g;
+    float *m, *v;
+    uint16_t *wb;
+    size_t n;
+} qp_net_param;
+int qp_net_adam_params(void *stream, const qp_net_param *params, int n, float lr, float b1,
+                       float b2, float eps, int step);
 int qp_net_to_bf16(void *stream, const float *a, size_t n, uint16_t *b);
+
+/* The whole U-Net (qpnet.UNet): its device buffers and layers.  Level l is the
+ * grid coarsened 2^l times, l = 0..3; c[l] channels there (multiples of 16). */
+typedef struct {
+    const uint16_t *w; /* BF16 [9][cout][cin] */
+    const float *b;
+    uint16_t *wt; /* scratch of the flipped weights */
+    float *gw, *gb;
+    int cin, cout;
+} qp_net_conv;
+typedef struct {
+    uint16_t *x0;      /* input, 16 channels */
+    uint16_t *ea[3];   /* first convolution of encoder level l, c[l] */
+    uint16_t *cat[3];  /* decoder input, c[l + 1] from below and c[l] of the encoder */
+    uint16_t *pool[3]; /* pooled level l, c[l] */
+    uint16_t *ba, *bb; /* level 3, c[3] */
+    uint16_t *da[3], *db[3]; /* decoder level l, c[l] */
+} qp_net_maps;
+typedef struct {
+    qp_net_conv enc[8], dec[6]; /* encoder levels 0..3, decoder levels 2..0, two each */
+    qp_net_maps a, g;           /* activations and their gradients */
+    const float *in_scale, *hw, *hb; /* input scales; head [nout][c[0]], [nout] */
+    float *ghwb;                     /* head gradient, nout rows of c[0] + 1 */
+    float *out, *gout;               /* [nout][H W] */
+    double *mse_part;                /* nmse partial sums of the squared error */
+    float *part;                     /* npart >= nhead nout (c[0] + 1): scratch of the gradients */
+    size_t npart;
+    int c[4], nin, nout, H, W; /* H, W divisible by 8 */
+    int nmse, nhead, nchunk;   /* parts of the loss, head and weight sums */
+} qp_net_unet;
+/* out = the network's output for nin FP32 planes (plane apart, pitch ld) */
+int qp_net_unet_forward(void *stream, const qp_net_unet *u, const float *planes, size_t plane,
+                        int ld);
+/* after it: every gradient of the mean squared error against target */
+int qp_net_unet_backward(void *stream, const qp_net_unet *u, const float *target);
 
 /* HIP-graph capture of a fixed launch sequence (the network's forward pass
  * on fixed buffers): begin capturing the stream's work, end it into an

@@ -10,6 +10,9 @@
 //
 // MFMA v_mfma_f32_16x16x16bf16_1k, one wave: lane l holds A[l%16][4(l/16)+i],
 // B[4(l/16)+i][l%16] and D[4(l/16)+i][l%16], i = 0..3.
+#include <algorithm>
+#include <cmath>
+
 #include "qp_common.h"
 #include "../../include/qpnet.h"
 
@@ -28,9 +31,8 @@ __device__ __forceinline__ uint16_t f2bf(float f)
 __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
 // 4 consecutive BF16 channels as an MFMA operand (8-byte aligned)
-__device__ __forceinline__ v4s load4(const uint16_t *p)
+__device__ __forceinline__ v4s frag(uint2 u)
 {
-    const uint2 u = *reinterpret_cast<const uint2 *>(p);
     v4s r;
     r[0] = (short)(u.x & 0xffff);
     r[1] = (short)(u.x >> 16);
@@ -38,174 +40,474 @@ __device__ __forceinline__ v4s load4(const uint16_t *p)
     r[3] = (short)(u.y >> 16);
     return r;
 }
+__device__ __forceinline__ v4s load4(const uint16_t *p)
+{
+    return frag(*reinterpret_cast<const uint2 *>(p));
+}
 
 // ---------------------------------------------------------------------------
 // 3x3 convolution, 'same' zero padding:
 //   y[p][co] = bias[co] + sum_{tap, ci} x'[p + off(tap)][ci] w[tap][co][ci]
 // x' = x, or x * (mask > 0) when mask is given (the ReLU derivative of the
 // layer that produced x, for the data gradient).  out = relu?(y) as BF16,
-// added to out when accum.  A workgroup computes 64 pixels of one row; each
-// wave 16 pixels and all cout (up to 192 = 12 MFMA column tiles).
+// added to out when accum.
+//
+// A wave computes 16 pixels of one row and 16 output channels, as one chain of
+// 9 cin / 16 MFMAs (tap by tap, 16 input channels at a time).  What bounds it is
+// the latency of the operands, which come from the caches beyond L2 (other dies
+// wrote them; the seed network's layers hold 0.1 to 2 MB), so there is a wave
+// for every tile, 16 to 768 blocks a convolution of a training step at 128^2,
+// and two ways of not waiting for each step:
+//  k_conv3x3: up to CONV_CIN input channels.  A block's waves are TX x TY pixel
+//    groups, and the pixels around them (zero outside the plane, masked) and the
+//    weights go to LDS first, in loads of 16 bytes that are in flight together.
+//    A row of LDS is a pixel or a (tap, co), padded by 16 bytes: the 16 rows of
+//    an operand then lie in different banks.
+//  k_conv3x3_deep: more channels than LDS holds.  The chain is cut in groups of
+//    9 steps, whose loads are issued before the group in front is multiplied.
+// One wave with all output channels of its pixels, loading step by step, took
+// 33.7 us a convolution (27 of a training step); all by k_conv3x3_deep 11.8 us,
+// by k_conv3x3 8.5 us.
 // ---------------------------------------------------------------------------
-constexpr int MAXNT = 12;
+// D[pixel 4q+i][co]: pixels xp.. of row y
+__device__ __forceinline__ void conv_store(v4f acc, const float *bias, int co, int y, int xp, int W,
+                                           uint16_t *out, int cs_out, int relu, int accum)
+{
+    const float bv = bias ? bias[co] : 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (xp + i >= W) continue;
+        float v = acc[i] + bv;
+        if (relu) v = v > 0.f ? v : 0.f;
+        uint16_t *o = out + ((size_t)y * W + xp + i) * cs_out + co;
+        if (accum) v += bf2f(*o);
+        *o = f2bf(v);
+    }
+}
 
+constexpr int CONV_CIN = 192;   // (3 x 66 pixels and 9 x 16 weight rows) x 400 B: 137 KB of LDS
+
+// quotient of small numbers, 0 <= a < 2^20, 1 <= b: ib = 1 / b
+__device__ __forceinline__ int small_div(int a, float ib) { return (int)(((float)a + 0.5f) * ib); }
+
+__device__ __forceinline__ uint32_t positive2(uint32_t v, uint32_t k)
+{
+    const bool lo = bf2f((uint16_t)k) > 0.f, hi = bf2f((uint16_t)(k >> 16)) > 0.f;
+    return (lo ? v & 0xffffu : 0u) | (hi ? v & 0xffff0000u : 0u);
+}
+
+template <bool MASK>
 __global__ void __launch_bounds__(256)
-k_conv3x3(const uint16_t *__restrict__ x, const uint16_t *__restrict__ mask, int H, int W,
+k_conv3x3(const uint16_t *__restrict__ x, const uint16_t *__restrict__ mask, int H, int W, int nbx,
+          int tx, int cs_in, int Cin, const uint16_t *__restrict__ w,
+          const float *__restrict__ bias, uint16_t *out, int cs_out, int Cout, int relu, int accum)
+{
+    extern __shared__ uint4 lds4[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ty = 4 / tx, by = blockIdx.x / nbx, bx = blockIdx.x - by * nbx;
+    const int x0 = bx * 16 * tx, y0 = by * ty;        // the block's first pixel
+    const int rw = 16 * tx + 2, npx = rw * (ty + 2);  // the pixels around it
+    const int kc = Cin >> 3, ld = kc + 1;             // 16-byte words of a row, pitch
+    const float irw = 1.f / (float)rw;
+    // thread: word c of the rows r, r + rs, ...; a few threads are left over
+    const int rs = 256 / kc, r = small_div(tid, 1.f / (float)kc), c = tid - r * kc;
+    const int cot = blockIdx.y;
+    const uint16_t *wc = w + ((size_t)16 * cot * Cin + 8 * c);
+    // rows y0 - 1 ..: offsets from here are small; outside the plane the block's
+    // first pixel is read, and its value is dropped
+    const size_t orow = (size_t)y0 * W * cs_in + 8 * c;
+    const uint16_t *xc = x + orow, *kc0 = mask + (MASK ? orow : 0);
+    constexpr int UW = 8, UP = 10;
+    for (int w0 = r, p0 = r; r < rs && (w0 < 144 || p0 < npx); w0 += UW * rs, p0 += UP * rs) {
+        uint4 vw[UW], vp[UP], vk[MASK ? UP : 1];
+        uint32_t in = 0;   // bit u: inside the plane
+#pragma unroll
+        for (int u = 0; u < UW; ++u) {
+            const int row = min(w0 + u * rs, 143);
+            vw[u] = *reinterpret_cast<const uint4 *>(
+                wc + (uint32_t)(((row >> 4) * Cout + (row & 15)) * Cin));
+        }
+#pragma unroll
+        for (int u = 0; u < UP; ++u) {
+            const int row = min(p0 + u * rs, npx - 1);
+            const int ry = small_div(row, irw), rx = row - ry * rw;
+            const int yy = y0 + ry - 1, xx = x0 + rx - 1;
+            const bool ok = (unsigned)yy < (unsigned)H && (unsigned)xx < (unsigned)W;
+            const ptrdiff_t o = ok ? ((ry - 1) * W + xx) * cs_in : x0 * cs_in;
+            vp[u] = *reinterpret_cast<const uint4 *>(xc + o);
+            if (MASK) vk[u] = *reinterpret_cast<const uint4 *>(kc0 + o);
+            in |= (uint32_t)ok << u;
+        }
+#pragma unroll
+        for (int u = 0; u < UW; ++u)
+            if (w0 + u * rs < 144) lds4[(npx + w0 + u * rs) * ld + c] = vw[u];
+#pragma unroll
+        for (int u = 0; u < UP; ++u) {
+            uint4 q = vp[u];
+            if (MASK)
+                q = uint4{positive2(q.x, vk[u].x), positive2(q.y, vk[u].y),
+                          positive2(q.z, vk[u].z), positive2(q.w, vk[u].w)};
+            if (!((in >> u) & 1)) q = uint4{0, 0, 0, 0};
+            if (p0 + u * rs < npx) lds4[(p0 + u * rs) * ld + c] = q;
+        }
+    }
+    __syncthreads();
+    const int wy = wave / tx, y = y0 + wy, px0 = x0 + 16 * (wave - wy * tx);
+    if (y >= H || px0 >= W) return;
+    const int m = lane & 15, q = lane >> 4;           // A row (pixel) and k quad
+    const uint2 *l2 = reinterpret_cast<const uint2 *>(lds4);
+    const int KT = Cin >> 4, ld2 = 2 * ld;
+    const uint2 *pa = l2 + (wy * rw + 16 * (wave - wy * tx) + m) * ld2 + q;
+    const uint2 *pb = l2 + (npx + m) * ld2 + q;
+    int tap = 0, kk = 0;                              // of the next step to load
+    auto load = [&](uint2 *a, uint2 *b) {
+#pragma unroll
+        for (int i = 0; i < 9; ++i) {
+            const int dy = (tap * 11) >> 5;           // tap / 3
+            a[i] = pa[(dy * rw + tap - 3 * dy) * ld2 + 4 * kk];
+            b[i] = pb[16 * tap * ld2 + 4 * kk];
+            if (++kk == KT) { kk = 0; ++tap; }
+        }
+    };
+    v4f acc = {0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](const uint2 *a, const uint2 *b) {
+#pragma unroll
+        for (int i = 0; i < 9; ++i)
+            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(frag(a[i]), frag(b[i]), acc, 0, 0, 0);
+    };
+    uint2 a0[9], b0[9], a1[9], b1[9];
+    load(a0, b0);
+    for (int k = 0; k < KT; k += 2) {
+        if (k + 1 < KT) load(a1, b1);
+        multiply(a0, b0);
+        if (k + 1 >= KT) break;
+        if (k + 2 < KT) load(a0, b0);
+        multiply(a1, b1);
+    }
+    conv_store(acc, bias, 16 * cot + m, y, px0 + 4 * q, W, out, cs_out, relu, accum);
+}
+
+template <bool MASK> struct ConvFrag {
+    v4s a[9], b[9], k[MASK ? 9 : 1];
+    uint32_t in;   // bit i: step i's pixel is inside
+};
+
+template <bool MASK>
+__global__ void __launch_bounds__(256)
+k_conv3x3_deep(const uint16_t *__restrict__ x, const uint16_t *__restrict__ mask, int H, int W, int gw,
           int cs_in, int Cin, const uint16_t *__restrict__ w, const float *__restrict__ bias,
           uint16_t *out, int cs_out, int Cout, int relu, int accum)
 {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int y = blockIdx.y;
-    const int px0 = blockIdx.x * 64 + wave * 16;      // this wave's first pixel in the row
-    const int NT = Cout >> 4;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = blockIdx.x * 4 + wave;              // this wave's pixel group
+    if (g >= H * gw) return;
+    const int y = g / gw, px0 = (g - y * gw) * 16;
     const int m = lane & 15, q = lane >> 4;           // A row (pixel) and k quad
-    v4f acc[MAXNT];
+    const int co = 16 * blockIdx.y + m;
+    const int KT = Cin >> 4;
+    const uint16_t *wl = w + (size_t)co * Cin + 4 * q;
+    int tap = 0, c = 0;                               // of the next step to load
+    auto load = [&](ConvFrag<MASK> &f) {
+        f.in = 0;
 #pragma unroll
-    for (int t = 0; t < MAXNT; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
-    for (int tap = 0; tap < 9; ++tap) {
-        const int dy = tap / 3 - 1, dx = tap % 3 - 1;
-        const int yy = y + dy, xx = px0 + m + dx;
-        const bool in = yy >= 0 && yy < H && xx >= 0 && xx < W;
-        const size_t pix = in ? ((size_t)yy * W + xx) * cs_in : 0;
-        for (int c0 = 0; c0 < Cin; c0 += 16) {
-            v4s a = {0, 0, 0, 0};
-            if (in) {
-                a = load4(x + pix + c0 + 4 * q);
-                if (mask) {
-                    const v4s mk = load4(mask + pix + c0 + 4 * q);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        if (!(bf2f((uint16_t)mk[i]) > 0.f)) a[i] = 0;
-                }
-            }
-            const uint16_t *wt = w + ((size_t)tap * Cout + m) * Cin + c0 + 4 * q;
-#pragma unroll
-            for (int t = 0; t < MAXNT; ++t) {
-                if (t < NT) {
-                    const v4s b = load4(wt + (size_t)t * 16 * Cin);
-                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[t], 0, 0, 0);
-                }
-            }
+        for (int i = 0; i < 9; ++i) {
+            const int ty = (tap * 11) >> 5;           // tap / 3
+            const int yy = y + ty - 1, xx = px0 + m + (tap - 3 * ty) - 1;
+            const bool in = yy >= 0 && yy < H && xx >= 0 && xx < W;
+            // outside: any address of the plane, the value is dropped
+            const size_t o = (size_t)(in ? yy : 0) * W * cs_in + (in ? xx : 0) * cs_in + 16 * c + 4 * q;
+            f.in |= (uint32_t)in << i;
+            f.a[i] = load4(x + o);
+            if (MASK) f.k[i] = load4(mask + o);
+            f.b[i] = load4(wl + (size_t)tap * Cout * Cin + 16 * c);
+            if (++c == KT) { c = 0; ++tap; }
         }
-    }
-    // D[pixel 4q+i][cout 16t + m]
-#pragma unroll
-    for (int t = 0; t < MAXNT; ++t) {
-        if (t >= NT) continue;
-        const int co = 16 * t + m;
-        const float bv = bias ? bias[co] : 0.f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int xp = px0 + 4 * q + i;
-            if (xp >= W) continue;
-            float v = acc[t][i] + bv;
-            if (relu) v = v > 0.f ? v : 0.f;
-            uint16_t *o = out + ((size_t)y * W + xp) * cs_out + co;
-            if (accum) v += bf2f(*o);
-            *o = f2bf(v);
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Weight gradient of a 3x3 convolution:
-//   dw[tap][co][ci] = sum_p dy'[p][co] x[p + off(tap)][ci]
-// dy' = dy * (yout > 0) (ReLU derivative from the layer's own output).  The
-// reduction over pixels is the MFMA K dimension.  Workgroup (co tile, ci
-// tile, tap) x chunk: its 4 waves take 16-pixel groups of the chunk in turn;
-// the 4 wave sums are added in wave order and written to
-// part[chunk][tap][co][ci]; k_sum_chunks adds the chunks in order.
-// ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256)
-k_conv3x3_wgrad(const uint16_t *__restrict__ x, int cs_in, int Cin,
-                const uint16_t *__restrict__ dy, const uint16_t *__restrict__ yout, int cs_out,
-                int Cout, int H, int W, int nchunk, float *part)
-{
-    __shared__ float red[4][256];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int ntc = Cin >> 4;
-    const int cot = blockIdx.x / ntc, cit = blockIdx.x % ntc;
-    const int tap = blockIdx.y, chunk = blockIdx.z;
-    const int dyo = tap / 3 - 1, dxo = tap % 3 - 1;
-    const int npix = H * W;
-    const int per = (npix + nchunk - 1) / nchunk;
-    const int p0 = chunk * per, p1 = min(npix, p0 + per);
-    const int m = lane & 15, q = lane >> 4;
+    };
     v4f acc = {0.f, 0.f, 0.f, 0.f};
-    for (int g = p0 + wave * 16; g < p1; g += 64) {
-        // A[co = m][k = pixel g + 4q + i], B[k = pixel g + 4q + i][ci = m]
-        v4s a, b;
+    auto multiply = [&](const ConvFrag<MASK> &f) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int p = g + 4 * q + i;
-            short av = 0, bv = 0;
-            if (p < p1) {
-                const size_t po = (size_t)p * cs_out + cot * 16 + m;
-                const uint16_t d = dy[po];
-                if (bf2f(yout[po]) > 0.f) av = (short)d;
-                const int py = p / W, pxx = p - py * W;
-                const int sy = py + dyo, sx = pxx + dxo;
-                if (sy >= 0 && sy < H && sx >= 0 && sx < W)
-                    bv = (short)x[((size_t)sy * W + sx) * cs_in + cit * 16 + m];
+        for (int i = 0; i < 9; ++i) {
+            v4s a = f.a[i];
+            const bool in = (f.in >> i) & 1;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (!in) a[j] = 0;
+                if (MASK)
+                    if (!(bf2f((uint16_t)f.k[i][j]) > 0.f)) a[j] = 0;
             }
-            a[i] = av;
-            b[i] = bv;
+            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, f.b[i], acc, 0, 0, 0);
         }
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
+    };
+    ConvFrag<MASK> f0, f1;
+    if (KT > 0) load(f0);
+    for (int k = 0; k < KT; k += 2) {
+        if (k + 1 < KT) load(f1);
+        multiply(f0);
+        if (k + 1 >= KT) break;
+        if (k + 2 < KT) load(f0);
+        multiply(f1);
+    }
+    conv_store(acc, bias, co, y, px0 + 4 * q, W, out, cs_out, relu, accum);
+}
+
+// ---------------------------------------------------------------------------
+// Tables of a launch over several layers: block b belongs to the entry e with
+// first[e] <= b < first[e + 1].  A table is read in the kernel's argument
+// segment.
+// ---------------------------------------------------------------------------
+constexpr int MAXL = 16;   // convolutions of one launch
+constexpr int MAXE = 36;   // vectors of one launch
+
+__device__ __forceinline__ int table_entry(const int *first, int n)
+{
+    const int lane = threadIdx.x & 63;
+    const bool behind = lane < n && first[lane < n ? lane : 0] <= (int)blockIdx.x;
+    return (int)__popcll(__ballot(behind)) - 1;
+}
+
+// ---------------------------------------------------------------------------
+// Weight and bias gradients of 3x3 convolutions:
+//   dw[tap][co][ci] = sum_p dy'[p][co] x[p + off(tap)][ci]
+//   db[co]          = sum_p dy'[p][co]
+// dy' = dy * (yout > 0) (ReLU derivative from the layer's own output).  The
+// reduction over pixels is the MFMA K dimension (db: against ones).  The pixels
+// are cut in nchunk chunks, a chunk in four interleaved runs of 16-pixel
+// groups; a run is one MFMA chain, its chunk's four are added in order, and so
+// are the chunks.
+//
+// A wave takes a chunk for one (co tile, ci tile, row of taps): the three taps
+// of a row share dy' and six pixels of x, 14 loads a step of three MFMAs, and
+// its four runs are four independent steps, so 56 loads are in flight.  A block
+// has four waves.  Chunks of at most WG_WHOLE pixels: a block goes through all
+// chunks, 16 at a time, and adds them up in LDS.  Larger ones: four chunks a
+// block, and k_sum_parts adds the partial sums from memory.  All layers of a
+// network go in one launch: at 128^2 a block per (tile, tap, chunk), a serial
+// sum for db and two sums over the chunks, layer by layer, took 68 us a layer;
+// the 14 layers together take 47 us and the sum 4 us.
+// ---------------------------------------------------------------------------
+constexpr int WG_WHOLE = 64;   // one step of the four runs
+constexpr int WG_SLOTS = 16;
+
+struct WgradLayer {
+    const uint16_t *x, *dy, *yout;
+    float *dw, *db;        // db may be null
+    float *part, *partb;   // partial sums per chunk; null: the block adds up all chunks
+    int cs_in, cin, cs_out, cout, H, W;
+};
+struct WgradArgs {
+    WgradLayer l[MAXL];
+    int first[MAXL];
+    int n, nchunk;
+};
+
+struct WgradTile {
+    v4f w[3], b;   // taps (dyo, -1..1) and the bias: D[co 4q + i][ci m]
+};
+
+// NC chunks at once, each in its first 4 / NC runs (the others have no pixels: a
+// chunk of at most 16 pixels has one run).  A chunk's tile is r[4 / NC * chunk].
+template <int NC>
+__device__ __forceinline__ void wgrad_runs(const WgradLayer &L, int co, int ci, int dyo, bool bias,
+                                           const int *p0, const int *p1, int q, WgradTile *r)
+{
+    constexpr int NV = 4 / NC;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+#pragma unroll
+        for (int t = 0; t < 3; ++t) r[v].w[t] = v4f{0.f, 0.f, 0.f, 0.f};
+        r[v].b = v4f{0.f, 0.f, 0.f, 0.f};
+    }
+    const int H = L.H, W = L.W, npix = H * W;
+    const v4s one = {(short)0x3f80, (short)0x3f80, (short)0x3f80, (short)0x3f80};
+    for (int g = 0; g < (NC > 1 ? min(npix, 64) : p1[0] - p0[0]); g += 64) {
+        uint16_t d[4][4], yo[4][4], xv[4][6];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            // pixel p of the plane is p - g0 elements of cs on from the bases; a
+            // pixel's neighbour (dyo, dx) is dyo W + dx pixels on; past the plane's
+            // ends the last or first pixel stands in, and is dropped below
+            const int g0 = min(p0[v / NV] + g, npix - 1);
+            const uint16_t *dyp = L.dy + (size_t)g0 * L.cs_out, *yp = L.yout + (size_t)g0 * L.cs_out;
+            const uint16_t *xp = L.x + ((ptrdiff_t)g0 - W - 1) * L.cs_in;
+            const int dmax = min(npix - 1 - g0, 63);
+            const int xlo = max(0, W + 1 - g0), xhi = min(npix - 1 - g0, 64 + 2 * W) + W + 1;
+            const int p = 16 * (v % NV) + 4 * q;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t o = (uint32_t)__mul24(min(p + i, dmax), L.cs_out) + co;
+                d[v][i] = dyp[o];
+                yo[v][i] = yp[o];
+            }
+#pragma unroll
+            for (int j = 0; j < 6; ++j) {
+                const int k = p + (dyo + 1) * W + j;
+                xv[v][j] = xp[(uint32_t)__mul24(min(max(k, xlo), xhi), L.cs_in) + ci];
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int p = p0[v / NV] + g + 16 * (v % NV) + 4 * q;
+            int py = p / W, px = p - py * W;
+            v4s a, b[3];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const bool in = p + i < p1[v / NV];
+                a[i] = in && bf2f(yo[v][i]) > 0.f ? (short)d[v][i] : (short)0;
+                const bool row = in && (unsigned)(py + dyo) < (unsigned)H;
+                b[0][i] = row && px > 0 ? (short)xv[v][i] : (short)0;
+                b[1][i] = row ? (short)xv[v][i + 1] : (short)0;
+                b[2][i] = row && px + 1 < W ? (short)xv[v][i + 2] : (short)0;
+                if (++px == W) { px = 0; ++py; }
+            }
+#pragma unroll
+            for (int t = 0; t < 3; ++t)
+                r[v].w[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b[t], r[v].w[t], 0, 0, 0);
+            if (bias) r[v].b = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, one, r[v].b, 0, 0, 0);
+        }
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) red[wave][lane * 4 + i] = acc[i];
-    __syncthreads();
-    if (wave == 0) {
+    for (int v = 0; v < 4; ++v) {
+        if (v % NV == 0) continue;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float s = ((red[0][lane * 4 + i] + red[1][lane * 4 + i]) + red[2][lane * 4 + i])
-                            + red[3][lane * 4 + i];
-            const int co = cot * 16 + 4 * q + i, ci = cit * 16 + m;
-            part[(((size_t)chunk * 9 + tap) * Cout + co) * Cin + ci] = s;
+        for (int t = 0; t < 3; ++t) r[v - v % NV].w[t] += r[v].w[t];
+        r[v - v % NV].b += r[v].b;
+    }
+}
+
+// a block's chunks base .. base + ns, tiles to LDS, NC chunks of a wave at a time
+template <int NC>
+__device__ __forceinline__ void wgrad_slots(const WgradLayer &L, int co, int ci, int dyo, bool bias,
+                                            int base, int ns, int per, int wave, int lane,
+                                            v4f (*red)[3][64], float (*redb)[16])
+{
+    const int npix = L.H * L.W;
+    for (int k0 = wave; k0 < ns; k0 += 4 * NC) {
+        int p0[NC], p1[NC];
+#pragma unroll
+        for (int n = 0; n < NC; ++n) {
+            const int k = k0 + 4 * n;
+            p0[n] = k < ns ? min((base + k) * per, npix) : npix;
+            p1[n] = min(npix, p0[n] + per);
+        }
+        WgradTile r[4];
+        wgrad_runs<NC>(L, co, ci, dyo, bias, p0, p1, lane >> 4, r);
+#pragma unroll
+        for (int n = 0; n < NC; ++n) {
+            const int k = k0 + 4 * n;
+            if (k >= ns) break;
+            const WgradTile &s = r[n * (4 / NC)];
+#pragma unroll
+            for (int t = 0; t < 3; ++t) red[k][t][lane] = s.w[t];
+            if ((lane & 15) == 0) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) redb[k][4 * (lane >> 4) + i] = s.b[i];
+            }
         }
     }
 }
 
-// bias gradient: db[co] = sum_p dy'[p][co], per chunk (same chunks)
-__global__ void k_bias_grad(const uint16_t *__restrict__ dy, const uint16_t *__restrict__ yout,
-                            int cs_out, int Cout, int npix, int nchunk, float *part)
+__global__ void __launch_bounds__(256) k_wgrad(const WgradArgs A)
 {
-    const int co = threadIdx.x, chunk = blockIdx.x;
-    if (co >= Cout) return;
-    const int per = (npix + nchunk - 1) / nchunk;
-    const int p0 = chunk * per, p1 = min(npix, p0 + per);
-    float s = 0.f;
-    for (int p = p0; p < p1; ++p) {
-        const size_t o = (size_t)p * cs_out + co;
-        if (bf2f(yout[o]) > 0.f) s += bf2f(dy[o]);
+    __shared__ v4f red[WG_SLOTS][3][64];
+    __shared__ float redb[WG_SLOTS][16];
+    const int e = table_entry(A.first, A.n);
+    const WgradLayer L = A.l[e];
+    const int nchunk = A.nchunk;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int m = lane & 15, q = lane >> 4;
+    const int nb = L.part ? (nchunk + 3) / 4 : 1;
+    const int unit = ((int)blockIdx.x - A.first[e]) / nb;
+    const int cb = ((int)blockIdx.x - A.first[e]) - unit * nb;
+    const int ntc = L.cin >> 4;
+    const int ty = unit % 3, cit = (unit / 3) % ntc, cot = unit / 3 / ntc;
+    const bool bias = L.db && cit == 0 && ty == 1;
+    const int npix = L.H * L.W, per = (npix + nchunk - 1) / nchunk;
+    if (L.part) {
+        const int chunk = cb * 4 + wave;
+        if (chunk >= nchunk) return;
+        const int p0 = min(chunk * per, npix), p1 = min(npix, p0 + per);
+        WgradTile r[4];
+        wgrad_runs<1>(L, cot * 16 + m, cit * 16 + m, ty - 1, bias, &p0, &p1, q, r);
+        const WgradTile &s = r[0];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int co = cot * 16 + 4 * q + i;
+#pragma unroll
+            for (int t = 0; t < 3; ++t)
+                L.part[(((size_t)chunk * 9 + 3 * ty + t) * L.cout + co) * L.cin + cit * 16 + m] =
+                    s.w[t][i];
+            if (bias && m == 0) L.partb[(size_t)chunk * L.cout + co] = s.b[i];
+        }
+        return;
     }
-    part[(size_t)chunk * Cout + co] = s;
+    // thread t sums element t of the tiles, in the order of the chunks
+    float tot[3] = {0.f, 0.f, 0.f}, totb = 0.f;
+    const int tid = threadIdx.x;
+    for (int base = 0; base < nchunk; base += WG_SLOTS) {
+        const int ns = min(WG_SLOTS, nchunk - base);
+        const int co = cot * 16 + m, ci = cit * 16 + m;
+        if (per <= 16)
+            wgrad_slots<4>(L, co, ci, ty - 1, bias, base, ns, per, wave, lane, red, redb);
+        else if (per <= 32)
+            wgrad_slots<2>(L, co, ci, ty - 1, bias, base, ns, per, wave, lane, red, redb);
+        else
+            wgrad_slots<1>(L, co, ci, ty - 1, bias, base, ns, per, wave, lane, red, redb);
+        __syncthreads();
+        for (int k = 0; k < ns; ++k) {
+#pragma unroll
+            for (int t = 0; t < 3; ++t) tot[t] += reinterpret_cast<const float *>(red[k][t])[tid];
+            if (tid < 16) totb += redb[k][tid];
+        }
+        __syncthreads();
+    }
+    const int l = tid >> 2, co = cot * 16 + 4 * (l >> 4) + (tid & 3), ci = cit * 16 + (l & 15);
+#pragma unroll
+    for (int t = 0; t < 3; ++t)
+        L.dw[((size_t)(3 * ty + t) * L.cout + co) * L.cin + ci] = tot[t];
+    if (bias && tid < 16) L.db[cot * 16 + tid] = totb;
 }
 
 // out[i] = sum over chunks (in order) of part[chunk][i]
-__global__ void k_sum_chunks(const float *__restrict__ part, size_t n, int nchunk, float *out)
+struct SumArgs {
+    const float *part[MAXE];
+    float *out[MAXE];
+    int len[MAXE], first[MAXE];
+    int n, nchunk;
+};
+__global__ void __launch_bounds__(256) k_sum_parts(const SumArgs A)
 {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * blockDim.x) {
-        float s = 0.f;
-        for (int c = 0; c < nchunk; ++c) s += part[(size_t)c * n + i];
-        out[i] = s;
-    }
+    const int e = table_entry(A.first, A.n);
+    const int i = ((int)blockIdx.x - A.first[e]) * 256 + (int)threadIdx.x;
+    const int n = A.len[e];
+    if (i >= n) return;
+    const float *p = A.part[e] + i;
+    float s = 0.f;
+#pragma unroll 16
+    for (int c = 0; c < A.nchunk; ++c) s += p[(size_t)c * n];
+    A.out[e][i] = s;
 }
 
 // w'[tap][ci][co] = w[8 - tap][co][ci]: the data gradient is the forward
 // convolution of dy with the flipped, transposed kernel
-__global__ void k_flip_weights(const uint16_t *__restrict__ w, int Cout, int Cin, uint16_t *wt)
+struct FlipArgs {
+    const uint16_t *w[MAXL];
+    uint16_t *wt[MAXL];
+    int cout[MAXL], cin[MAXL], first[MAXL];
+    int n;
+};
+__global__ void __launch_bounds__(256) k_flip_weights(const FlipArgs A)
 {
-    const size_t n = (size_t)9 * Cout * Cin;
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * blockDim.x) {
-        const int tap = (int)(i / ((size_t)Cin * Cout));
-        const int r = (int)(i % ((size_t)Cin * Cout));
-        const int ci = r / Cout, co = r % Cout;
-        wt[i] = w[((size_t)(8 - tap) * Cout + co) * Cin + ci];
-    }
+    const int e = table_entry(A.first, A.n);
+    const int i = ((int)blockIdx.x - A.first[e]) * 256 + (int)threadIdx.x;
+    const int Cout = A.cout[e], Cin = A.cin[e];
+    if (i >= 9 * Cout * Cin) return;
+    const int tap = i / (Cin * Cout);
+    const int r = i - tap * Cin * Cout;
+    const int ci = r / Cout, co = r - ci * Cout;
+    A.wt[e][i] = A.w[e][((size_t)(8 - tap) * Cout + co) * Cin + ci];
 }
 
 // ---------------------------------------------------------------------------
@@ -387,29 +689,67 @@ __global__ void k_head(const uint16_t *__restrict__ h, int cs, int cin, const fl
 }
 
 // head backward: dh[p][k] = sum_c w[c][k] do[c][p] (BF16); per-chunk partial
-// weight / bias gradients part[chunk][c][k] and part[chunk][c][cin]
-__global__ void k_head_bwd(const uint16_t *__restrict__ h, int cs, int cin,
-                           const float *__restrict__ w, int cout, size_t npix,
-                           const float *__restrict__ dout, uint16_t *dh, int nchunk, float *part)
+// weight / bias gradients part[chunk][c][k] and part[chunk][c][cin], each one
+// thread's sum over the chunk's pixels in order.  The pixels go through LDS in
+// tiles, so that serial sum waits for LDS and not for memory (37 us from memory,
+// 10.6 us so, 64 chunks of 256 pixels).
+constexpr int HEAD_H = 16384, HEAD_D = 4096;   // tile elements of h and do in LDS
+__global__ void __launch_bounds__(256)
+k_head_bwd(const uint16_t *__restrict__ h, int cs, int cin, const float *__restrict__ w, int cout,
+           size_t npix, const float *__restrict__ dout, uint16_t *dh, int nchunk, int tile,
+           int vec, float *part)
 {
-    const int chunk = blockIdx.x;
+    __shared__ __attribute__((aligned(16))) uint16_t sh[HEAD_H];
+    __shared__ float sd[HEAD_D], sw[256];
+    const int chunk = blockIdx.x, t = threadIdx.x;
+    if (t < cout * cin) sw[t] = w[t];
     const size_t per = (npix + nchunk - 1) / nchunk;
-    const size_t p0 = chunk * per, p1 = min(npix, p0 + per);
-    // weight partials: thread t < cout*(cin+1) owns one (c, k) sum over the chunk
-    const int t = threadIdx.x;
-    if (t < cout * (cin + 1)) {
-        const int c = t / (cin + 1), k = t % (cin + 1);
-        float s = 0.f;
-        for (size_t p = p0; p < p1; ++p)
-            s += dout[c * npix + p] * (k < cin ? bf2f(h[p * cs + k]) : 1.f);
-        part[(size_t)chunk * cout * (cin + 1) + t] = s;
-    }
-    for (size_t p = p0 + threadIdx.x; p < p1; p += blockDim.x)
-        for (int k = 0; k < cin; ++k) {
-            float s = 0.f;
-            for (int c = 0; c < cout; ++c) s += w[c * cin + k] * dout[c * npix + p];
-            dh[p * cs + k] = f2bf(s);
+    const size_t p0 = min(npix, chunk * per), p1 = min(npix, p0 + per);
+    const int c = t / (cin + 1), k = t % (cin + 1);
+    float s = 0.f;
+    for (size_t base = p0; base < p1; base += tile) {
+        const int np = (int)min((size_t)tile, p1 - base);
+        if (vec) {
+            const int kc = cin >> 3;
+            uint4 *s4 = reinterpret_cast<uint4 *>(sh);
+            for (int i = t; i < np * kc; i += 256)
+                s4[i] = *reinterpret_cast<const uint4 *>(h + (base + i / kc) * cs + 8 * (i % kc));
+        } else {
+            for (int i = t; i < np * cin; i += 256) sh[i] = h[(base + i / cin) * cs + i % cin];
         }
+        for (int i = t; i < np * cout; i += 256) sd[i] = dout[(i / np) * npix + base + i % np];
+        __syncthreads();
+        // thread t < cout*(cin+1) owns one (c, k) sum
+        if (t < cout * (cin + 1)) {
+            const uint16_t *hp = sh + (k < cin ? k : 0);
+            const float *dp = sd + c * np;
+#pragma unroll 8
+            for (int p = 0; p < np; ++p) {
+                const float hv = bf2f(hp[p * cin]);
+                s += dp[p] * (k < cin ? hv : 1.f);
+            }
+        }
+        auto grad = [&](int p, int kk) -> uint32_t {
+            float v = 0.f;
+            for (int cc = 0; cc < cout; ++cc) v += sw[cc * cin + kk] * sd[cc * np + p];
+            return f2bf(v);
+        };
+        if (vec) {
+            const int kc = cin >> 3;
+            for (int i = t; i < np * kc; i += 256) {
+                const int p = i / kc, k0 = 8 * (i % kc);
+                uint32_t u[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) u[j] = grad(p, k0 + 2 * j) | grad(p, k0 + 2 * j + 1) << 16;
+                *reinterpret_cast<uint4 *>(dh + (base + p) * cs + k0) = uint4{u[0], u[1], u[2], u[3]};
+            }
+        } else {
+            for (int i = t; i < np * cin; i += 256)
+                dh[(base + i / cin) * cs + i % cin] = (uint16_t)grad(i / cin, i % cin);
+        }
+        __syncthreads();
+    }
+    if (t < cout * (cin + 1)) part[(size_t)chunk * cout * (cin + 1) + t] = s;
 }
 
 // mean squared error over n values and its gradient 2 (o - t) / n; the loss
@@ -434,21 +774,32 @@ __global__ void k_mse(const float *__restrict__ o, const float *__restrict__ t, 
     if (threadIdx.x == 0) partial[blockIdx.x] = s[0];
 }
 
-// Adam step on FP32 master weights, refreshing their BF16 copy (if any)
-__global__ void k_adam(float *wm, const float *__restrict__ g, float *mo, float *ve, size_t n,
-                       float lr, float b1, float b2, float eps, float c1, float c2, uint16_t *wb)
+// Adam step on FP32 master weights, refreshing their BF16 copies (if any): all
+// vectors of a network in one launch (30 launches of 2.2 us with the gaps
+// between them before, one of 5.5 us now)
+struct AdamArgs {
+    float *w[MAXE];
+    const float *g[MAXE];
+    float *m[MAXE], *v[MAXE];
+    uint16_t *wb[MAXE];
+    int len[MAXE], first[MAXE];
+    int n;
+    float lr, b1, b2, eps, c1, c2;
+};
+__global__ void __launch_bounds__(256) k_adam(const AdamArgs A)
 {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * blockDim.x) {
-        const float gi = g[i];
-        const float mi = b1 * mo[i] + (1.f - b1) * gi;
-        const float vi = b2 * ve[i] + (1.f - b2) * gi * gi;
-        mo[i] = mi;
-        ve[i] = vi;
-        const float wv = wm[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-        wm[i] = wv;
-        if (wb) wb[i] = f2bf(wv);
-    }
+    const int e = table_entry(A.first, A.n);
+    const int i = ((int)blockIdx.x - A.first[e]) * 256 + (int)threadIdx.x;
+    if (i >= A.len[e]) return;
+    const float b1 = A.b1, b2 = A.b2;
+    const float gi = A.g[e][i];
+    const float mi = b1 * A.m[e][i] + (1.f - b1) * gi;
+    const float vi = b2 * A.v[e][i] + (1.f - b2) * gi * gi;
+    A.m[e][i] = mi;
+    A.v[e][i] = vi;
+    const float wv = A.w[e][i] - A.lr * (mi / A.c1) / (sqrtf(vi / A.c2) + A.eps);
+    A.w[e][i] = wv;
+    if (A.wb[e]) A.wb[e][i] = f2bf(wv);
 }
 
 __global__ void k_to_bf16(const float *__restrict__ a, size_t n, uint16_t *b)
@@ -456,6 +807,24 @@ __global__ void k_to_bf16(const float *__restrict__ a, size_t n, uint16_t *b)
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
          i += (size_t)gridDim.x * blockDim.x)
         b[i] = f2bf(a[i]);
+}
+
+static void add_sum(SumArgs &a, const float *part, int len, float *out)
+{
+    const int e = a.n++;
+    a.part[e] = part;
+    a.out[e] = out;
+    a.len[e] = len;
+    a.first[e] = e ? a.first[e - 1] + (a.len[e - 1] + 255) / 256 : 0;
+}
+
+static int launch_sums(const SumArgs &a, hipStream_t st)
+{
+    if (!a.n) return QP_OK;
+    const int blocks = a.first[a.n - 1] + (a.len[a.n - 1] + 255) / 256;
+    hipLaunchKernelGGL(k_sum_parts, dim3(blocks), dim3(256), 0, st, a);
+    QP_LAUNCH_CHECK();
+    return QP_OK;
 }
 
 static dim3 g1(size_t n)
@@ -470,6 +839,11 @@ static dim3 g1(size_t n)
 using namespace qp;
 
 #define NET_CHECK(cond, ...) QP_REQUIRE(cond, QP_ERR_ARG, __VA_ARGS__)
+#define RC(expr)              \
+    do {                      \
+        const int rc_ = expr; \
+        if (rc_) return rc_;  \
+    } while (0)
 
 extern "C" {
 
@@ -479,36 +853,130 @@ int qp_net_conv3x3(void *stream_, const uint16_t *x, const uint16_t *mask, int H
 {
     hipStream_t st = (hipStream_t)stream_;
     NET_CHECK(x && w && out && H > 0 && W > 0, "qp_net_conv3x3: bad argument");
-    NET_CHECK(cin % 16 == 0 && cout % 16 == 0 && cout <= 16 * MAXNT && cin <= cs_in &&
+    NET_CHECK(cin % 16 == 0 && cout % 16 == 0 && cout <= 192 && cin <= cs_in &&
                   cout <= cs_out && cs_in % 4 == 0,
               "qp_net_conv3x3: channels cin %d cout %d (multiples of 16, cout <= 192)", cin, cout);
-    dim3 grid((W + 63) / 64, H);
-    hipLaunchKernelGGL(k_conv3x3, grid, dim3(256), 0, st, x, mask, H, W, cs_in, cin, w, bias,
-                       out, cs_out, cout, relu, accum);
+    if (cout <= 0) return QP_OK;
+    const int gw = (W + 15) / 16;
+    // 16-byte loads of the pixels and weights where they are aligned for it
+    const bool al = cs_in % 8 == 0 && !(((uintptr_t)x | (uintptr_t)mask | (uintptr_t)w) & 15);
+    if (cin > 0 && cin <= CONV_CIN && al) {
+        const int tx = gw >= 3 ? 4 : gw, ty = 4 / tx, nbx = (gw + tx - 1) / tx;
+        const size_t lds = (size_t)((16 * tx + 2) * (ty + 2) + 144) * (cin / 8 + 1) * 16;
+        const dim3 grid((unsigned)((size_t)((H + ty - 1) / ty) * nbx), cout / 16);
+        const void *k = mask ? (const void *)k_conv3x3<true> : (const void *)k_conv3x3<false>;
+        if (lds > 65536)
+            QP_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        if (mask)
+            hipLaunchKernelGGL(k_conv3x3<true>, grid, dim3(256), lds, st, x, mask, H, W, nbx, tx,
+                               cs_in, cin, w, bias, out, cs_out, cout, relu, accum);
+        else
+            hipLaunchKernelGGL(k_conv3x3<false>, grid, dim3(256), lds, st, x, mask, H, W, nbx, tx,
+                               cs_in, cin, w, bias, out, cs_out, cout, relu, accum);
+        QP_LAUNCH_CHECK();
+        return QP_OK;
+    }
+    const dim3 grid((unsigned)(((size_t)H * gw + 3) / 4), cout / 16);
+    if (mask)
+        hipLaunchKernelGGL(k_conv3x3_deep<true>, grid, dim3(256), 0, st, x, mask, H, W, gw, cs_in,
+                           cin, w, bias, out, cs_out, cout, relu, accum);
+    else
+        hipLaunchKernelGGL(k_conv3x3_deep<false>, grid, dim3(256), 0, st, x, mask, H, W, gw,
+                           cs_in, cin, w, bias, out, cs_out, cout, relu, accum);
     QP_LAUNCH_CHECK();
     return QP_OK;
+}
+
+}  // extern "C"
+
+// partb: the partial sums of the bias of a single layer, if not in part
+static int wgrad_layers(hipStream_t st, const qp_net_layer *layers, int n, int nchunk, float *part,
+                        size_t npart, float *partb)
+{
+    for (int i0 = 0; i0 < n; i0 += MAXL) {
+        WgradArgs a{};
+        SumArgs sums{}, sumb{};
+        a.n = std::min(MAXL, n - i0);
+        a.nchunk = sums.nchunk = sumb.nchunk = nchunk;
+        int blocks = 0;
+        size_t used = 0;
+        for (int e = 0; e < a.n; ++e) {
+            const qp_net_layer &l = layers[i0 + e];
+            const int units = (l.cout / 16) * (l.cin / 16) * 3;
+            const int per = (int)(((size_t)l.H * l.W + nchunk - 1) / nchunk);
+            const size_t nw = (size_t)9 * l.cout * l.cin, nb = l.db && !partb ? l.cout : 0;
+            // a layer whose partial sums find no room: its blocks take all chunks
+            const bool parts = per > WG_WHOLE && part && used + (nw + nb) * nchunk <= npart;
+            a.l[e] = WgradLayer{l.x, l.dy, l.yout, l.dw, l.db, nullptr, nullptr,
+                                l.cs_x, l.cin, l.cs_y, l.cout, l.H, l.W};
+            a.first[e] = blocks;
+            if (parts) {
+                a.l[e].part = part + used;
+                a.l[e].partb = partb ? partb : part + used + nw * nchunk;
+                used += (nw + nb) * nchunk;
+                if (l.db) add_sum(partb ? sumb : sums, a.l[e].partb, l.cout, l.db);
+                add_sum(sums, a.l[e].part, (int)nw, l.dw);
+            }
+            blocks += units * (parts ? (nchunk + 3) / 4 : 1);
+        }
+        hipLaunchKernelGGL(k_wgrad, dim3(blocks), dim3(256), 0, st, a);
+        QP_LAUNCH_CHECK();
+        RC(launch_sums(sumb, st));
+        RC(launch_sums(sums, st));
+    }
+    return QP_OK;
+}
+
+extern "C" {
+
+int qp_net_wgrad_layers(void *stream_, const qp_net_layer *layers, int n, int nchunk, float *part,
+                        size_t npart)
+{
+    NET_CHECK((layers || !n) && n >= 0 && nchunk > 0, "qp_net_wgrad_layers: bad argument");
+    for (int i = 0; i < n; ++i) {
+        const qp_net_layer &l = layers[i];
+        NET_CHECK(l.x && l.dy && l.yout && l.dw && l.H > 0 && l.W > 0 && l.cin > 0 && l.cout > 0 &&
+                      l.cin % 16 == 0 && l.cout % 16 == 0,
+                  "qp_net_wgrad_layers: layer %d", i);
+    }
+    return wgrad_layers((hipStream_t)stream_, layers, n, nchunk, part, npart, nullptr);
 }
 
 int qp_net_conv3x3_wgrad(void *stream_, const uint16_t *x, int cs_in, int cin,
                          const uint16_t *dy, const uint16_t *yout, int cs_out, int cout, int H,
                          int W, int nchunk, float *part, float *dw, float *db)
 {
-    hipStream_t st = (hipStream_t)stream_;
     NET_CHECK(x && dy && yout && part && dw && nchunk > 0, "qp_net_conv3x3_wgrad: bad argument");
     NET_CHECK(cin % 16 == 0 && cout % 16 == 0, "qp_net_conv3x3_wgrad: channels");
-    dim3 grid((cout / 16) * (cin / 16), 9, nchunk);
-    hipLaunchKernelGGL(k_conv3x3_wgrad, grid, dim3(256), 0, st, x, cs_in, cin, dy, yout, cs_out,
-                       cout, H, W, nchunk, part);
-    QP_LAUNCH_CHECK();
-    const size_t n = (size_t)9 * cout * cin;
-    hipLaunchKernelGGL(k_sum_chunks, g1(n), dim3(256), 0, st, part, n, nchunk, dw);
-    QP_LAUNCH_CHECK();
-    if (db) {
-        hipLaunchKernelGGL(k_bias_grad, dim3(nchunk), dim3(cout < 64 ? 64 : cout), 0, st, dy,
-                           yout, cs_out, cout, H * W, nchunk, part);
-        QP_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_sum_chunks, g1(cout), dim3(256), 0, st, part, (size_t)cout, nchunk,
-                           db);
+    const qp_net_layer l = {x, dy, yout, dw, db, cs_in, cin, cs_out, cout, H, W};
+    // the scratch holds the weights' partial sums; the bias's wait in dw, which is
+    // written behind them, if they fit there
+    const bool room = !db || nchunk <= 9 * cin;
+    return wgrad_layers((hipStream_t)stream_, &l, 1, nchunk, room ? part : nullptr,
+                        (size_t)nchunk * 9 * cout * cin, db ? dw : nullptr);
+}
+
+int qp_net_flip_layers(void *stream_, const qp_net_flip *layers, int n)
+{
+    hipStream_t st = (hipStream_t)stream_;
+    NET_CHECK((layers || !n) && n >= 0, "qp_net_flip_layers: bad argument");
+    for (int i = 0; i < n; ++i)
+        NET_CHECK(layers[i].w && layers[i].wt, "qp_net_flip_weights: null");
+    for (int i0 = 0; i0 < n; i0 += MAXL) {
+        FlipArgs a{};
+        a.n = std::min(MAXL, n - i0);
+        int blocks = 0;
+        for (int e = 0; e < a.n; ++e) {
+            const qp_net_flip &l = layers[i0 + e];
+            a.w[e] = l.w;
+            a.wt[e] = l.wt;
+            a.cout[e] = l.cout;
+            a.cin[e] = l.cin;
+            a.first[e] = blocks;
+            blocks += (9 * l.cout * l.cin + 255) / 256;
+        }
+        if (!blocks) continue;
+        hipLaunchKernelGGL(k_flip_weights, dim3(blocks), dim3(256), 0, st, a);
         QP_LAUNCH_CHECK();
     }
     return QP_OK;
@@ -516,12 +984,8 @@ int qp_net_conv3x3_wgrad(void *stream_, const uint16_t *x, int cs_in, int cin,
 
 int qp_net_flip_weights(void *stream_, const uint16_t *w, int cout, int cin, uint16_t *wt)
 {
-    hipStream_t st = (hipStream_t)stream_;
-    NET_CHECK(w && wt, "qp_net_flip_weights: null");
-    hipLaunchKernelGGL(k_flip_weights, g1((size_t)9 * cout * cin), dim3(256), 0, st, w, cout,
-                       cin, wt);
-    QP_LAUNCH_CHECK();
-    return QP_OK;
+    const qp_net_flip l = {w, wt, cout, cin};
+    return qp_net_flip_layers(stream_, &l, 1);
 }
 
 int qp_net_pool2(void *stream_, const uint16_t *in, int cs_in, uint16_t *out, int cs_out, int H,
@@ -674,13 +1138,16 @@ int qp_net_head_bwd(void *stream_, const uint16_t *h, int cs, int cin, const flo
 {
     hipStream_t st = (hipStream_t)stream_;
     NET_CHECK(cout * (cin + 1) <= 256, "qp_net_head_bwd: head too large");
+    // 16 bytes at a time where the pixels are aligned for it
+    const int vec = cin % 8 == 0 && cs % 8 == 0 && !(((uintptr_t)h | (uintptr_t)dh) & 15);
+    const int tile = std::min(256, std::min(HEAD_H / std::max(cin, 1), HEAD_D / std::max(cout, 1)));
     hipLaunchKernelGGL(k_head_bwd, dim3(nchunk), dim3(256), 0, st, h, cs, cin, w, cout, npix,
-                       dout, dh, nchunk, part);
+                       dout, dh, nchunk, tile, vec, part);
     QP_LAUNCH_CHECK();
-    const size_t n = (size_t)cout * (cin + 1);
-    hipLaunchKernelGGL(k_sum_chunks, g1(n), dim3(256), 0, st, part, n, nchunk, dwb);
-    QP_LAUNCH_CHECK();
-    return QP_OK;
+    SumArgs a{};
+    a.nchunk = nchunk;
+    add_sum(a, part, cout * (cin + 1), dwb);
+    return launch_sums(a, st);
 }
 
 int qp_net_mse(void *stream_, const float *o, const float *t, size_t n, float *grad,
@@ -692,15 +1159,52 @@ int qp_net_mse(void *stream_, const float *o, const float *t, size_t n, float *g
     return QP_OK;
 }
 
+int qp_net_adam_params(void *stream_, const qp_net_param *params, int n, float lr, float b1,
+                       float b2, float eps, int step)
+{
+    hipStream_t st = (hipStream_t)stream_;
+    NET_CHECK((params || !n) && n >= 0, "qp_net_adam_params: bad argument");
+    AdamArgs a{};
+    a.lr = lr;
+    a.b1 = b1;
+    a.b2 = b2;
+    a.eps = eps;
+    a.c1 = 1.f - powf(b1, (float)step);
+    a.c2 = 1.f - powf(b2, (float)step);
+    int blocks = 0;
+    auto flush = [&]() -> int {
+        if (blocks) {
+            hipLaunchKernelGGL(k_adam, dim3(blocks), dim3(256), 0, st, a);
+            QP_LAUNCH_CHECK();
+        }
+        a.n = blocks = 0;
+        return QP_OK;
+    };
+    for (int i = 0; i < n; ++i) {
+        const qp_net_param &p = params[i];
+        // a vector longer than an entry can hold goes in pieces
+        for (size_t o = 0; o < p.n; o += (size_t)1 << 28) {
+            const int len = (int)std::min(p.n - o, (size_t)1 << 28);
+            if (a.n == MAXE || blocks > (1 << 20)) RC(flush());
+            const int e = a.n++;
+            a.w[e] = p.w + o;
+            a.g[e] = p.g + o;
+            a.m[e] = p.m + o;
+            a.v[e] = p.v + o;
+            a.wb[e] = p.wb ? p.wb + o : nullptr;
+            a.len[e] = len;
+            a.first[e] = blocks;
+            blocks += (len + 255) / 256;
+        }
+    }
+    return flush();
+}
+
 int qp_net_adam(void *stream_, float *wm, const float *g, float *m, float *v, size_t n, float lr,
                 float b1, float b2, float eps, int step, uint16_t *wb)
 {
-    hipStream_t st = (hipStream_t)stream_;
-    const float c1 = 1.f - powf(b1, (float)step), c2 = 1.f - powf(b2, (float)step);
-    hipLaunchKernelGGL(k_adam, g1(n), dim3(256), 0, st, wm, g, m, v, n, lr, b1, b2, eps, c1, c2,
-                       wb);
-    QP_LAUNCH_CHECK();
-    return QP_OK;
+    const qp_net_param p = {wm, g, m, v, wb, n};
+    return qp_net_adam_params(stream_, &p, 1, lr, b1, b2, eps, step);
 }
 
 int qp_net_to_bf16(void *stream_, const float *a, size_t n, uint16_t *b)
@@ -709,6 +1213,94 @@ int qp_net_to_bf16(void *stream_, const float *a, size_t n, uint16_t *b)
     hipLaunchKernelGGL(k_to_bf16, g1(n), dim3(256), 0, st, a, n, b);
     QP_LAUNCH_CHECK();
     return QP_OK;
+}
+
+// The U-Net's passes: the launches in order, from one call (22 of a forward and
+// 25 of a backward pass took 10 us each from Python, more than most of their
+// kernels take).  Level l is the grid coarsened 2^l times; cat[l] holds what the
+// decoder convolves there: c[l + 1] channels from below and c[l] from the encoder.
+int qp_net_unet_forward(void *st, const qp_net_unet *u, const float *planes, size_t plane, int ld)
+{
+    NET_CHECK(u && planes, "qp_net_unet_forward: null");
+    const qp_net_conv *e = u->enc, *d = u->dec;
+    const qp_net_maps &a = u->a;
+    const int *c = u->c;
+    auto conv = [&](const uint16_t *x, int l, int cs, const qp_net_conv &v, uint16_t *out,
+                    int cs_out) {
+        return qp_net_conv3x3(st, x, nullptr, u->H >> l, u->W >> l, cs, v.cin, v.w, v.b, out, cs_out,
+                              v.cout, 1, 0);
+    };
+    RC(qp_net_pack_input(st, planes, u->nin, plane, ld, u->in_scale, u->H, u->W, a.x0, 16));
+    const uint16_t *in = a.x0;
+    int cs = 16;
+    for (int l = 0; l < 3; ++l) {
+        RC(conv(in, l, cs, e[2 * l], a.ea[l], c[l]));
+        RC(conv(a.ea[l], l, c[l], e[2 * l + 1], a.cat[l] + c[l + 1], c[l + 1] + c[l]));
+        RC(qp_net_pool2(st, a.cat[l] + c[l + 1], c[l + 1] + c[l], a.pool[l], c[l], u->H >> l,
+                        u->W >> l, c[l]));
+        in = a.pool[l];
+        cs = c[l];
+    }
+    RC(conv(in, 3, cs, e[6], a.ba, c[3]));
+    RC(conv(a.ba, 3, c[3], e[7], a.bb, c[3]));
+    in = a.bb;
+    for (int l = 2; l >= 0; --l) {
+        const qp_net_conv *v = d + 2 * (2 - l);
+        RC(qp_net_up2(st, in, c[l + 1], a.cat[l], c[l + 1] + c[l], u->H >> (l + 1),
+                      u->W >> (l + 1), c[l + 1]));
+        RC(conv(a.cat[l], l, c[l + 1] + c[l], v[0], a.da[l], c[l]));
+        RC(conv(a.da[l], l, c[l], v[1], a.db[l], c[l]));
+        in = a.db[l];
+    }
+    return qp_net_head(st, a.db[0], c[0], c[0], u->hw, u->hb, u->nout, (size_t)u->H * u->W, u->out);
+}
+
+int qp_net_unet_backward(void *st, const qp_net_unet *u, const float *target)
+{
+    NET_CHECK(u && target, "qp_net_unet_backward: null");
+    const qp_net_conv *e = u->enc, *d = u->dec;
+    const qp_net_maps &a = u->a, &g = u->g;
+    const int *c = u->c;
+    const size_t npix = (size_t)u->H * u->W;
+    RC(qp_net_mse(st, u->out, target, u->nout * npix, u->gout, u->mse_part, u->nmse));
+    RC(qp_net_head_bwd(st, a.db[0], c[0], c[0], u->hw, u->nout, npix, u->gout, g.db[0], u->nhead,
+                       u->part, u->ghwb));
+    qp_net_flip fl[14];
+    for (int i = 0; i < 14; ++i) {
+        const qp_net_conv &v = i < 8 ? e[i] : d[i - 8];
+        fl[i] = qp_net_flip{v.w, v.wt, v.cout, v.cin};
+    }
+    RC(qp_net_flip_layers(st, fl + 1, 13));   // the input's gradient is not wanted
+    // A convolution's data gradient into gx (if given) from gy, the gradient of its
+    // ReLU output y.  Its weight gradient waits for nothing but gy, and all gy are
+    // still as their layers left them at the end: one launch for all.
+    qp_net_layer wg[14];
+    int nwg = 0;
+    auto conv = [&](const uint16_t *x, int l, int cs, const qp_net_conv &v, const uint16_t *y,
+                    const uint16_t *gy, int cs_y, uint16_t *gx) -> int {
+        wg[nwg++] = qp_net_layer{x, gy, y, v.gw, v.gb, cs, v.cin, cs_y, v.cout, u->H >> l, u->W >> l};
+        if (!gx) return QP_OK;
+        return qp_net_conv3x3(st, gy, y, u->H >> l, u->W >> l, cs_y, v.cout, v.wt, nullptr, gx, cs,
+                              v.cin, 0, 0);
+    };
+    for (int l = 0; l < 3; ++l) {
+        const qp_net_conv *v = d + 2 * (2 - l);
+        RC(conv(a.da[l], l, c[l], v[1], a.db[l], g.db[l], c[l], g.da[l]));
+        RC(conv(a.cat[l], l, c[l + 1] + c[l], v[0], a.da[l], g.da[l], c[l], g.cat[l]));
+        RC(qp_net_up2_bwd(st, g.cat[l], c[l + 1] + c[l], l < 2 ? g.db[l + 1] : g.bb, c[l + 1],
+                          u->H >> (l + 1), u->W >> (l + 1), c[l + 1]));
+    }
+    RC(conv(a.ba, 3, c[3], e[7], a.bb, g.bb, c[3], g.ba));
+    RC(conv(a.pool[2], 3, c[2], e[6], a.ba, g.ba, c[3], g.pool[2]));
+    for (int l = 2; l >= 0; --l) {
+        // the encoder's part of cat[l]: its gradient is the skip's and the pool's
+        const int off = c[l + 1], cs = c[l + 1] + c[l];
+        RC(qp_net_pool2_bwd(st, g.pool[l], c[l], g.cat[l] + off, cs, u->H >> l, u->W >> l, c[l], 1));
+        RC(conv(a.ea[l], l, c[l], e[2 * l + 1], a.cat[l] + off, g.cat[l] + off, cs, g.ea[l]));
+        RC(conv(l ? a.pool[l - 1] : a.x0, l, l ? c[l - 1] : 16, e[2 * l], a.ea[l], g.ea[l], c[l],
+                l ? g.pool[l - 1] : nullptr));
+    }
+    return qp_net_wgrad_layers(st, wg, nwg, u->nchunk, u->part, u->npart);
 }
 
 }  // extern "C"

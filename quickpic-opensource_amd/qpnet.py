@@ -44,6 +44,9 @@ def _lib():
             "qp_net_head_bwd": [vp, u16p, i, i, fp, i, sz, fp, u16p, i, fp, fp],
             "qp_net_mse": [vp, fp, fp, sz, fp, dp, i],
             "qp_net_adam": [vp, fp, fp, fp, fp, sz, f, f, f, f, i, u16p],
+            "qp_net_unet_forward": [vp, vp, fp, sz, i],
+            "qp_net_unet_backward": [vp, vp, fp],
+            "qp_net_adam_params": [vp, vp, i, f, f, f, f, i],
             "qp_net_to_bf16": [vp, fp, sz, u16p],
             "qp_net_block_mean": [vp, i, C.POINTER(C.c_void_p), C.POINTER(C.c_int), i, i, i, i,
                                   fp],
@@ -60,6 +63,29 @@ def _lib():
             fn.restype = C.c_int
         _NET = L
     return _NET
+
+
+class _Conv(C.Structure):
+    _fields_ = [(k, C.c_void_p) for k in ("w", "b", "wt", "gw", "gb")] + \
+        [("cin", C.c_int), ("cout", C.c_int)]
+
+
+class _Unet(C.Structure):
+    """qp_net_unet; a and g: x0, ea[3], cat[3], pool[3], ba, bb, da[3], db[3]."""
+    _fields_ = [("conv", _Conv * 14), ("a", C.c_void_p * 18), ("g", C.c_void_p * 18)] + \
+        [(k, C.c_void_p) for k in ("in_scale", "hw", "hb", "ghwb", "out", "gout", "mse_part",
+                                   "part")] + \
+        [("npart", C.c_size_t), ("c", C.c_int * 4)] + \
+        [(k, C.c_int) for k in ("nin", "nout", "H", "W", "nmse", "nhead", "nchunk")]
+
+
+# the network's maps in the order of qp_net_maps
+MAPS = ("x0", "e1a", "e2a", "e3a", "cat1", "cat2", "cat3", "p1", "p2", "p3", "ba", "bb",
+        "d1a", "d2a", "d3a", "d1b", "d2b", "d3b")
+
+
+class _Param(C.Structure):
+    _fields_ = [(k, C.c_void_p) for k in ("w", "g", "m", "v", "wb")] + [("n", C.c_size_t)]
 
 
 def _call(fn, *args):
@@ -211,49 +237,37 @@ class UNet:
         self.g = {k: torch.zeros_like(v) for k, v in s.items()}
         self.out = torch.zeros((NOUT, H * W), device=self.dev)
         self.gout = torch.zeros_like(self.out)
-        npmax = H * W * 192
-        self.part = torch.zeros(max(32 * 9 * 192 * 128, 64 * NOUT * (c1 + 1)), device=self.dev)
+        # partial sums of the gradients: the layers of the two finer levels, and
+        # of the coarser ones where they have as many pixels
+        cut = [sum(10 * v.cin * v.cout for v in cv) for cv in self._levels()]
+        npart = 32 * sum(n for i, n in enumerate(cut) if i < 2 or H * W >> 2 * i > 2048)
+        self.part = torch.zeros(max(npart, 64 * NOUT * (c1 + 1)), device=self.dev)
         self.mse_part = torch.zeros(256, dtype=torch.float64, device=self.dev)
         self._shape = (H, W)
-        del npmax
+
+    def _levels(self):
+        """The convolutions on the grid coarsened 1, 2, 4 and 8 times."""
+        e, d = self.enc, self.dec
+        return [e[0:2] + d[4:6], e[2:4] + d[2:4], e[4:6] + d[0:2], e[6:8]]
+
+    def _table(self):
+        """The network's buffers for qp_net_unet_forward and _backward."""
+        p = torch.Tensor.data_ptr
+        t = _Unet((_Conv * 14)(*[(p(v.w16), p(v.b), p(v.wt16), p(v.gw), p(v.gb), v.cin, v.cout)
+                                 for v in self.enc + self.dec]),
+                  (C.c_void_p * 18)(*[p(self.a[k]) for k in MAPS]),
+                  (C.c_void_p * 18)(*[p(self.g[k]) for k in MAPS]),
+                  *[p(x) for x in (self.in_scale, self.hw, self.hb, self.ghwb, self.out, self.gout,
+                                   self.mse_part, self.part)],
+                  self.part.numel(), CH, NIN, NOUT, *self._shape, self.mse_part.numel(), 64, 32)
+        return t
 
     # -- forward --------------------------------------------------------------
     def forward(self, planes, plane, ld, H, W):
         """planes: FP32 device tensor holding NIN planes (plane elements apart,
         row pitch ld); returns the FP32 output [NOUT][H*W] (in output units)."""
         self._alloc(H, W)
-        a = self.a
-        c1, c2, c3, c4 = CH
-        _call(_lib().qp_net_pack_input, stream(), ptr(planes), NIN, plane, ld, ptr(self.in_scale),
-              H, W, ptr(a["x0"]), 16)
-        e, d = self.enc, self.dec
-        conv3x3(a["x0"], H, W, 16, 16, e[0].w16, e[0].b, a["e1a"], c1, c1)
-        conv3x3(a["e1a"], H, W, c1, c1, e[1].w16, e[1].b, a["cat1"], c2 + c1, c1, out_off=c2)
-        _call(_lib().qp_net_pool2, stream(), ptr(a["cat1"], c2), c2 + c1, ptr(a["p1"]), c1, H, W, c1)
-        H2, W2 = H // 2, W // 2
-        conv3x3(a["p1"], H2, W2, c1, c1, e[2].w16, e[2].b, a["e2a"], c2, c2)
-        conv3x3(a["e2a"], H2, W2, c2, c2, e[3].w16, e[3].b, a["cat2"], c3 + c2, c2, out_off=c3)
-        _call(_lib().qp_net_pool2, stream(), ptr(a["cat2"], c3), c3 + c2, ptr(a["p2"]), c2, H2, W2,
-              c2)
-        H4, W4 = H // 4, W // 4
-        conv3x3(a["p2"], H4, W4, c2, c2, e[4].w16, e[4].b, a["e3a"], c3, c3)
-        conv3x3(a["e3a"], H4, W4, c3, c3, e[5].w16, e[5].b, a["cat3"], c4 + c3, c3, out_off=c4)
-        _call(_lib().qp_net_pool2, stream(), ptr(a["cat3"], c4), c4 + c3, ptr(a["p3"]), c3, H4, W4,
-              c3)
-        H8, W8 = H // 8, W // 8
-        conv3x3(a["p3"], H8, W8, c3, c3, e[6].w16, e[6].b, a["ba"], c4, c4)
-        conv3x3(a["ba"], H8, W8, c4, c4, e[7].w16, e[7].b, a["bb"], c4, c4)
-        _call(_lib().qp_net_up2, stream(), ptr(a["bb"]), c4, ptr(a["cat3"]), c4 + c3, H8, W8, c4)
-        conv3x3(a["cat3"], H4, W4, c4 + c3, c4 + c3, d[0].w16, d[0].b, a["d3a"], c3, c3)
-        conv3x3(a["d3a"], H4, W4, c3, c3, d[1].w16, d[1].b, a["d3b"], c3, c3)
-        _call(_lib().qp_net_up2, stream(), ptr(a["d3b"]), c3, ptr(a["cat2"]), c3 + c2, H4, W4, c3)
-        conv3x3(a["cat2"], H2, W2, c3 + c2, c3 + c2, d[2].w16, d[2].b, a["d2a"], c2, c2)
-        conv3x3(a["d2a"], H2, W2, c2, c2, d[3].w16, d[3].b, a["d2b"], c2, c2)
-        _call(_lib().qp_net_up2, stream(), ptr(a["d2b"]), c2, ptr(a["cat1"]), c2 + c1, H2, W2, c2)
-        conv3x3(a["cat1"], H, W, c2 + c1, c2 + c1, d[4].w16, d[4].b, a["d1a"], c1, c1)
-        conv3x3(a["d1a"], H, W, c1, c1, d[5].w16, d[5].b, a["d1b"], c1, c1)
-        _call(_lib().qp_net_head, stream(), ptr(a["d1b"]), c1, c1, ptr(self.hw), ptr(self.hb), NOUT,
-              H * W, ptr(self.out))
+        _call(_lib().qp_net_unet_forward, stream(), C.byref(self._table()), ptr(planes), plane, ld)
         return self.out
 
     def forward_graph(self, planes, plane, ld, H, W):
@@ -293,81 +307,27 @@ class UNet:
             self._graph = None
 
     # -- backward -------------------------------------------------------------
-    def _conv_bwd(self, cv, x, cs_in, H, W, y, gy, cs_out, gx, x_off=0, y_off=0, gx_off=0,
-                  accum=False):
-        """Gradients of one conv: weights and bias into cv.gw/gb, data into gx
-        (if given), from gy (the gradient of its ReLU output y)."""
-        conv3x3_wgrad(x, cs_in, cv.cin, gy, y, cs_out, cv.cout, H, W, self.part, cv.gw, cv.gb,
-                      x_off=x_off, y_off=y_off)
-        if gx is not None:
-            flip_weights(cv.w16, cv.cout, cv.cin, cv.wt16)
-            conv3x3(gy, H, W, cs_out, cv.cout, cv.wt16, None, gx, cs_in, cv.cin, relu=False,
-                    accum=accum, mask=y, x_off=y_off, out_off=gx_off)
-
     def backward(self, target):
         """MSE against target [NOUT][H*W] (output units); fills every
         gradient; returns the loss."""
-        H, W = self._shape
-        a, g = self.a, self.g
-        c1, c2, c3, c4 = CH
-        n = NOUT * H * W
-        _call(_lib().qp_net_mse, stream(), ptr(self.out), ptr(target), n, ptr(self.gout),
-              ptr(self.mse_part), 256)
-        _call(_lib().qp_net_head_bwd, stream(), ptr(a["d1b"]), c1, c1, ptr(self.hw), NOUT, H * W,
-              ptr(self.gout), ptr(g["d1b"]), 64, ptr(self.part), ptr(self.ghwb))
-        e, d = self.enc, self.dec
-        H2, W2, H4, W4, H8, W8 = H // 2, W // 2, H // 4, W // 4, H // 8, W // 8
-        # decoder level 1
-        self._conv_bwd(d[5], a["d1a"], c1, H, W, a["d1b"], g["d1b"], c1, g["d1a"])
-        self._conv_bwd(d[4], a["cat1"], c2 + c1, H, W, a["d1a"], g["d1a"], c1, g["cat1"])
-        _call(_lib().qp_net_up2_bwd, stream(), ptr(g["cat1"]), c2 + c1, ptr(g["d2b"]), c2, H2, W2,
-              c2)
-        # decoder level 2
-        self._conv_bwd(d[3], a["d2a"], c2, H2, W2, a["d2b"], g["d2b"], c2, g["d2a"])
-        self._conv_bwd(d[2], a["cat2"], c3 + c2, H2, W2, a["d2a"], g["d2a"], c2, g["cat2"])
-        _call(_lib().qp_net_up2_bwd, stream(), ptr(g["cat2"]), c3 + c2, ptr(g["d3b"]), c3, H4, W4,
-              c3)
-        # decoder level 3
-        self._conv_bwd(d[1], a["d3a"], c3, H4, W4, a["d3b"], g["d3b"], c3, g["d3a"])
-        self._conv_bwd(d[0], a["cat3"], c4 + c3, H4, W4, a["d3a"], g["d3a"], c3, g["cat3"])
-        _call(_lib().qp_net_up2_bwd, stream(), ptr(g["cat3"]), c4 + c3, ptr(g["bb"]), c4, H8, W8,
-              c4)
-        # bottleneck
-        self._conv_bwd(e[7], a["ba"], c4, H8, W8, a["bb"], g["bb"], c4, g["ba"])
-        self._conv_bwd(e[6], a["p3"], c3, H8, W8, a["ba"], g["ba"], c4, g["p3"])
-        # encoder level 3: e3 = cat3[c4:], its gradient = skip part + pooled path
-        _call(_lib().qp_net_pool2_bwd, stream(), ptr(g["p3"]), c3, ptr(g["cat3"], c4), c4 + c3,
-              H4, W4, c3, 1)
-        self._conv_bwd(e[5], a["e3a"], c3, H4, W4, a["cat3"], g["cat3"], c4 + c3, g["e3a"],
-                       y_off=c4)
-        self._conv_bwd(e[4], a["p2"], c2, H4, W4, a["e3a"], g["e3a"], c3, g["p2"])
-        _call(_lib().qp_net_pool2_bwd, stream(), ptr(g["p2"]), c2, ptr(g["cat2"], c3), c3 + c2,
-              H2, W2, c2, 1)
-        self._conv_bwd(e[3], a["e2a"], c2, H2, W2, a["cat2"], g["cat2"], c3 + c2, g["e2a"],
-                       y_off=c3)
-        self._conv_bwd(e[2], a["p1"], c1, H2, W2, a["e2a"], g["e2a"], c2, g["p1"])
-        _call(_lib().qp_net_pool2_bwd, stream(), ptr(g["p1"]), c1, ptr(g["cat1"], c2), c2 + c1, H,
-              W, c1, 1)
-        self._conv_bwd(e[1], a["e1a"], c1, H, W, a["cat1"], g["cat1"], c2 + c1, g["e1a"],
-                       y_off=c2)
-        self._conv_bwd(e[0], a["x0"], 16, H, W, a["e1a"], g["e1a"], c1, None)
+        n = self.out.numel()
+        _call(_lib().qp_net_unet_backward, stream(), C.byref(self._table()), ptr(target))
         return float(self.mse_part.sum().item()) / n
 
     def adam(self, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8):
         self.step += 1
-        L = _lib()
-        for cv in self.enc + self.dec:
-            for w, gw, m, v, w16 in cv.params():
-                _call(L.qp_net_adam, stream(), ptr(w), ptr(gw), ptr(m), ptr(v), w.numel(), lr, b1,
-                      b2, eps, self.step, ptr(w16))
+        ps = [_Param(w.data_ptr(), gw.data_ptr(), m.data_ptr(), v.data_ptr(),
+                     w16.data_ptr() if w16 is not None else None, w.numel())
+              for cv in self.enc + self.dec for w, gw, m, v, w16 in cv.params()]
+        # the head's gradients: per output a row of its weights' and its bias's
         c1 = CH[0]
-        g = self.ghwb.view(NOUT, c1 + 1)
-        gw = g[:, :c1].contiguous()
-        gb = g[:, c1].contiguous()
-        for w, gg, m, v in ((self.hw, gw, self.hm[0], self.hv[0]),
-                            (self.hb, gb, self.hm[1], self.hv[1])):
-            _call(L.qp_net_adam, stream(), ptr(w), ptr(gg), ptr(m), ptr(v), w.numel(), lr, b1, b2,
-                  eps, self.step, None)
+        for o in range(NOUT):
+            for n, at, off, t in ((c1, o * c1, 0, (self.hw, self.hm[0], self.hv[0])),
+                                  (1, o, c1, (self.hb, self.hm[1], self.hv[1]))):
+                w, m, v = (x.data_ptr() + 4 * at for x in t)
+                ps.append(_Param(w, self.ghwb.data_ptr() + 4 * (o * (c1 + 1) + off), m, v, None, n))
+        _call(_lib().qp_net_adam_params, stream(), (_Param * len(ps))(*ps), len(ps), lr, b1, b2,
+              eps, self.step)
 
     # -- persistence ------------------------------------------------------------
     def state(self):

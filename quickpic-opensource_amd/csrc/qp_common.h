@@ -26,6 +26,8 @@ namespace qp {
 constexpr int TILE = 16;                 // cells per tile edge (part2d_class.f03:99)
 constexpr int TCELLS = TILE * TILE;      // cells per tile = threads per particle block
 constexpr int HALO = 4 * TILE;           // border nodes of a 17x17 tile block
+// border nodes of a band of rb of a tile's rows, 17 x (rb + 1) nodes
+__host__ __device__ constexpr int band_halo(int rb) { return 2 * (TILE + rb); }
 constexpr double TWOPI_REF = 6.28318530717959;  // the reference's 2*pi literal
 constexpr double BEAM_FIX = 17592186044416.0;   // 2^44: beam charge fixed point
 constexpr int MAX_BATCH = 8;            // components in one batched transform
@@ -122,6 +124,7 @@ struct qp_ctx {
     qp::DevBuf halo;              // deposit tile borders, 8 comps
     qp::DevBuf red;               // reduction partials (double)
     size_t max_lds;               // LDS bytes one workgroup may use
+    int cus;                      // compute units
     // kernel-class timing (qp_ctx_profile)
     unsigned prof_on;     // bit k: launches of class k are timed
     int prof_every;       // time one launch in prof_every of a class (0, 1: all)
@@ -364,6 +367,17 @@ __device__ __forceinline__ void beam_plane_convert(const BeamPlane &b, size_t fi
     R *q2 = static_cast<R *>(b.q2);
     for (size_t i = first; i < b.n; i += step)
         q2[i] = R(0) + (R)((double)q3[i] * (1.0 / BEAM_FIX));
+}
+
+// Bands of rows that the current deposit cuts a tile in.  A grid of fewer tiles
+// than compute units leaves units idle, and a tile's few waves wait for their
+// loads and divisions in turn; up to four bands of at least four rows (64 cells
+// at 4 lanes) still fill a block of 256.  With more blocks than units the extra
+// border nodes cost more than the overlap gives.  FP64, 4 particles a cell:
+// 64 x 32 13.4 us in one band, 10.5 in four; 128^2 15.6 and 11.0.
+inline int deposit_bands(const qp_ctx *c)
+{
+    return c->ntiles * 4 <= c->cus ? 4 : c->ntiles * 2 <= c->cus ? 2 : 1;
 }
 
 // ---- species internals used by the slice driver (qp_particles.hip) ----

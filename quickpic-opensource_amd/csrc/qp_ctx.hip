@@ -273,13 +273,16 @@ int qp_ctx_create(int indx, int indy, int indz, const double box[6], int precisi
     int lds = 0;
     hipError_t e = hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device);
     c->max_lds = (e == hipSuccess && lds > 0) ? (size_t)lds : 65536;
+    if (hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
+        c->cus = 0;
     e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
     if (e != hipSuccess) { delete c; return hip_fail(e, "hipStreamCreate", __FILE__, __LINE__); }
     int rc = precision == QP_FP64 ? make_tables<double>(c) : make_tables<float>(c);
     size_t pl = c->rplane > c->kplane ? c->rplane : c->kplane;
     if (!rc) rc = c->scr_r.alloc(MAX_BATCH * pl * c->esize);
     if (!rc) rc = c->scr_k.alloc(MAX_BATCH * pl * c->esize);
-    if (!rc) rc = c->halo.alloc((size_t)8 * c->ntiles * HALO * c->esize);
+    const int nb = deposit_bands(c);
+    if (!rc) rc = c->halo.alloc((size_t)8 * c->ntiles * nb * band_halo(TILE / nb) * c->esize);
     if (!rc) rc = c->red.alloc(sizeof(double) * 8192);
     if (!rc) rc = c->flags.alloc(sizeof(int) * 64);
     if (rc) { qp_ctx_destroy(c); return rc; }

@@ -120,12 +120,13 @@ __device__ __forceinline__ R gather(const Corners<R> &f, R amx, R amy, R dxp, R 
     return d + dyp * (dxp * f.f11 + a);
 }
 
-__device__ __forceinline__ int halo_index(int i, int j)
+// (a block of RB rows of cells: 17 x (RB + 1) nodes)
+template <int RB = TILE> __device__ __forceinline__ int halo_index(int i, int j)
 {
     if (j == 0) return i;
-    if (j == TILE) return 17 + i;
+    if (j == RB) return 17 + i;
     if (i == 0) return 34 + (j - 1);
-    return 49 + (j - 1);
+    return 33 + RB + (j - 1);
 }
 
 // Where a deposit's node sums go.  For component c and node value v:
@@ -165,40 +166,43 @@ template <typename R> static DepOut<R> dep_plain(R *const *planes, int n)
 // with fold, row ny is added into row 0 and cleared (PPNACGUARD2L nvp = 1).
 // One thread per border node and component (one thread taking every
 // component of a node measured 1.5x slower: too few waves per CU).
-template <typename R>
+template <typename R, int RB>
 __global__ void k_deposit_border(TileGeom g, const R *__restrict__ halo, size_t halo_cs,
                                  DepOut<R> out, int fold, const int *skip)
 {
     if (skip && *skip) return;
     const int comp = blockIdx.y;
-    const int rows_n = (g.my1 + 1) * (g.nx + 1);
-    const int cols_n = (g.mx1 + 1) * g.my1 * (TILE - 1);
+    constexpr int B = TILE / RB;   // blocks of a tile, and their nodes in the buffer
+    const int myb = g.my1 * B;
+    const int rows_n = (myb + 1) * (g.nx + 1);
+    const int cols_n = (g.mx1 + 1) * myb * (RB - 1);
     int id = blockIdx.x * blockDim.x + threadIdx.x;
     int X, Y;
     if (id < rows_n) {
-        Y = (id / (g.nx + 1)) * TILE;
+        Y = (id / (g.nx + 1)) * RB;
         X = id % (g.nx + 1);
     } else if (id < rows_n + cols_n) {
         int k = id - rows_n;
-        int per_col = g.my1 * (TILE - 1);
+        int per_col = myb * (RB - 1);
         X = (k / per_col) * TILE;
         int r = k % per_col;
-        Y = (r / (TILE - 1)) * TILE + 1 + r % (TILE - 1);
+        Y = (r / (RB - 1)) * RB + 1 + r % (RB - 1);
     } else {
         return;
     }
     const R *h = halo + comp * halo_cs;
     auto node_sum = [&](int XX, int YY) -> R {
         R s = R(0);
-        for (int tyc = (YY >> 4) - 1; tyc <= (YY >> 4); ++tyc) {
-            if (tyc < 0 || tyc >= g.my1) continue;
-            int ly = YY - TILE * tyc;
-            if (ly < 0 || ly > TILE) continue;
+        for (int tyc = YY / RB - 1; tyc <= YY / RB; ++tyc) {
+            if (tyc < 0 || tyc >= myb) continue;
+            int ly = YY - RB * tyc;
+            if (ly < 0 || ly > RB) continue;
             for (int txc = (XX >> 4) - 1; txc <= (XX >> 4); ++txc) {
                 if (txc < 0 || txc >= g.mx1) continue;
                 int lx = XX - TILE * txc;
                 if (lx < 0 || lx > TILE) continue;
-                s += h[(size_t)(tyc * g.mx1 + txc) * HALO + halo_index(lx, ly)];
+                s += h[(size_t)(((tyc / B) * g.mx1 + txc) * B + tyc % B) * band_halo(RB) +
+                       halo_index<RB>(lx, ly)];
             }
         }
         return s;
@@ -257,18 +261,19 @@ __device__ __forceinline__ void stage_in(const R *const (&src)[NA], R *const (&d
 }
 
 // Interior nodes of the tile's 17x17 block to the output plane, border nodes
-// to the halo buffer (summed over tiles by k_deposit_border).
-template <typename R>
+// to the halo buffer (summed over tiles by k_deposit_border).  With bands, of
+// band `band`, RB rows of cells.
+template <typename R, int RB = TILE>
 __device__ __forceinline__ void emit_nodes(const R *nacc, const DepOut<R> &out, int c, int ldr,
-                                           R *halo, int tile, int tx, int ty)
+                                           R *halo, int tile, int tx, int ty, int band = 0)
 {
-    for (int n = threadIdx.x; n < 17 * 17; n += TCELLS) {
+    for (int n = threadIdx.x; n < 17 * (RB + 1); n += TCELLS) {
         const int i = n % 17, j = n / 17;
         const R v = nacc[n];
-        if (i >= 1 && i < TILE && j >= 1 && j < TILE)
-            dep_store(out, c, (size_t)(ty * TILE + j) * ldr + tx * TILE + i, v);
+        if (i >= 1 && i < TILE && j >= 1 && j < RB)
+            dep_store(out, c, (size_t)(ty * TILE + band * RB + j) * ldr + tx * TILE + i, v);
         else
-            halo[(size_t)tile * HALO + halo_index(i, j)] = v;
+            halo[(size_t)(tile * (TILE / RB) + band) * band_halo(RB) + halo_index<RB>(i, j)] = v;
     }
 }
 
@@ -563,7 +568,8 @@ __device__ __forceinline__ R amjdp_one(const Fields6<R> &F, R fx, R fy, R x, R y
 // in dense tiles (where the lanes of the cells a chunk does not hold wait),
 // and a sparse tile takes fewer, larger groups.  (Compiling each T as its
 // own path was measured slower: 443-444 against 454.6 slices/s at THR = 4.)
-template <typename R, int RG, int CH, int WPE, bool PSI, bool UQ, int THR = 4>
+// B: a tile is cut in B bands of rows, one block each (deposit_bands).
+template <typename R, int RG, int CH, int WPE, bool PSI, bool UQ, int THR = 4, int B = 1>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, 8)))
 k_amjdp(TileGeom g, Soa<R> s, const int *__restrict__ off, const R *fxy, const R *bxy,
         const R *psit, size_t cs, DepOut<R> out, R *halo, size_t halo_cs, R qbm, R dt, R dex,
@@ -575,10 +581,11 @@ k_amjdp(TileGeom g, Soa<R> s, const int *__restrict__ off, const R *fxy, const R
     extern __shared__ unsigned char smem_raw[];
     R *sx = reinterpret_cast<R *>(smem_raw), *sy = sx + NP, *spx = sy + NP, *spy = spx + NP;
     R *sp6 = spy + NP, *sp7 = sp6 + NP, *sq = sp7 + NP, *nacc = sq + NP;   // nacc: 8 x 289
-    const int tid = threadIdx.x, tile = blockIdx.x;
+    constexpr int RB = TILE / B;   // rows of a band
+    const int tid = threadIdx.x, tile = (int)blockIdx.x / B, row0 = (int)blockIdx.x % B * RB;
     const int tx = tile % g.mx1, ty = tile / g.mx1, kb = tile * TCELLS;
     for (int n = tid; n < 8 * 289; n += TCELLS) nacc[n] = R(0);
-    int T = RG > 0 ? TILE / (RG > 0 ? RG : 1) : 1;
+    int T = RG > 0 ? TILE / (RG > 0 ? RG : 1) : B;
     if (RG == 0) {
         const int ntile = off[kb + TCELLS] - off[kb];
         while (T < TILE && 4 * ntile > THR * CH * T) T *= 2;
@@ -586,7 +593,7 @@ k_amjdp(TileGeom g, Soa<R> s, const int *__restrict__ off, const R *fxy, const R
     const int rg = TILE / T;   // rows per group
     const int cl = tid / T, sub = tid % T;
     const R qtmh = R(0.5) * qbm * dt, dti = R(1) / dt, idex = R(1) / dex;
-    for (int row = 0; row < TILE; row += rg) {
+    for (int row = row0; row < row0 + RB; row += rg) {
         const int lrow = row + cl / TILE, lcol = cl % TILE;
         const int key = kb + lrow * TILE + lcol;
         const int i0 = off[key], i1 = off[key + 1];
@@ -641,7 +648,7 @@ k_amjdp(TileGeom g, Soa<R> s, const int *__restrict__ off, const R *fxy, const R
         for (int k = 0; k < 4; ++k) {
             __syncthreads();
             if (sub == 0) {
-                const int node = (lrow + (k >> 1)) * 17 + lcol + (k & 1);
+                const int node = (lrow - row0 + (k >> 1)) * 17 + lcol + (k & 1);
 #pragma unroll
                 for (int c = 0; c < 8; ++c) nacc[c * 289 + node] += acc[c][k];
             }
@@ -650,7 +657,8 @@ k_amjdp(TileGeom g, Soa<R> s, const int *__restrict__ off, const R *fxy, const R
     __syncthreads();
 #pragma unroll
     for (int c = 0; c < 8; ++c)
-        emit_nodes(nacc + c * 289, out, c, g.ldr, halo + c * halo_cs, tile, tx, ty);
+        emit_nodes<R, RB>(nacc + c * 289, out, c, g.ldr, halo + c * halo_cs, tile, tx, ty,
+                          row0 / RB);
 }
 
 // The same deposit with the next chunk's particles loaded into registers
@@ -1608,16 +1616,19 @@ static int rebin_unsorted(qp_species *sp, const std::vector<int> *hkeys = nullpt
 
 template <typename R>
 static int deposit_border(qp_ctx *c, const DepOut<R> &out, int ncomp, int fold,
-                          R *halo = nullptr)
+                          const R *halo = nullptr, int bands = 1)
 {
     QP_REQUIRE(ncomp >= 1 && ncomp <= 8, QP_ERR_ARG, "deposit border: %d components", ncomp);
     TileGeom g = geom(c);
-    int n = (c->my1 + 1) * (c->nx + 1) + (c->mx1 + 1) * c->my1 * (TILE - 1);
+    const int rb = TILE / bands, myb = c->my1 * bands;
+    int n = (myb + 1) * (c->nx + 1) + (c->mx1 + 1) * myb * (rb - 1);
     {
     ProfScope _ps(c, QP_PROF_BORDER, 2.0 * ncomp * (double)n * sizeof(R));
-    hipLaunchKernelGGL(k_deposit_border<R>, dim3((n + 255) / 256, ncomp), dim3(256), 0, c->stream,
-                       g, halo ? halo : c->halo.as<R>(), (size_t)c->ntiles * HALO, out, fold,
-                       c->skip);
+    auto kern = bands == 4 ? k_deposit_border<R, TILE / 4>
+              : bands == 2 ? k_deposit_border<R, TILE / 2> : k_deposit_border<R, TILE>;
+    hipLaunchKernelGGL(kern, dim3((n + 255) / 256, ncomp), dim3(256), 0, c->stream,
+                       g, halo ? halo : c->halo.as<R>(),
+                       (size_t)c->ntiles * bands * band_halo(rb), out, fold, c->skip);
     }
     QP_LAUNCH_CHECK();
     return QP_OK;
@@ -2016,14 +2027,14 @@ static int extpsi_t(qp_species *sp, const qp_field2d *psi, double dex)
     return QP_OK;
 }
 
-template <typename R, int V>
+template <typename R, int V, int B = 1>
 static int amjdp_v(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
                    const qp_field2d *psit, double dex, const DepOut<R> &out,
                    const qp_field2d *psi)
 {
     qp_ctx *c = sp->ctx;
     const size_t pl = c->rplane;
-    const size_t hcs = (size_t)c->ntiles * HALO;
+    const size_t hcs = (size_t)c->ntiles * B * band_halo(TILE / B);
     constexpr DepShape d = DepTab<R>::j[V];
     size_t lds;
     void (*kern)(TileGeom, Soa<R>, const int *, const R *, const R *, const R *, size_t,
@@ -2041,11 +2052,11 @@ static int amjdp_v(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
     } else {
         lds = (7 * (size_t)Stage<d.ch>::N + 8 * 289) * sizeof(R);
         if (sp->q_uniform)
-            kern = psi ? k_amjdp<R, d.rg, d.ch, d.wpe, true, true, d.thr>
-                       : k_amjdp<R, d.rg, d.ch, d.wpe, false, true, d.thr>;
+            kern = psi ? k_amjdp<R, d.rg, d.ch, d.wpe, true, true, d.thr, B>
+                       : k_amjdp<R, d.rg, d.ch, d.wpe, false, true, d.thr, B>;
         else
-            kern = psi ? k_amjdp<R, d.rg, d.ch, d.wpe, true, false, d.thr>
-                       : k_amjdp<R, d.rg, d.ch, d.wpe, false, false, d.thr>;
+            kern = psi ? k_amjdp<R, d.rg, d.ch, d.wpe, true, false, d.thr, B>
+                       : k_amjdp<R, d.rg, d.ch, d.wpe, false, false, d.thr, B>;
     }
     int rc = allow_lds(kern, lds, c);
     if (rc) return rc;
@@ -2055,7 +2066,7 @@ static int amjdp_v(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
     const double words = (psi ? 9.0 : 8.0) - (sp->q_uniform && d.wave == 0 ? 1.0 : 0.0);
     const double planes = psi ? 15.0 : 14.0;
     ProfScope _ps(c, QP_PROF_AMJDP, (words * sp->np + planes * (c->nx + 1.0) * (c->ny + 1.0)) * sizeof(R));
-    hipLaunchKernelGGL(kern, dim3(c->ntiles), dim3(256), lds, c->stream, geom(c),
+    hipLaunchKernelGGL(kern, dim3(c->ntiles * B), dim3(256), lds, c->stream, geom(c),
                        soa<R>(sp->a), sp->off.as<int>(), ef->rs.as<R>(), bf->rs.as<R>(),
                        psit->rs.as<R>(), pl, out, c->halo.as<R>(), hcs, (R)sp->qbm, (R)sp->dt,
                        (R)dex, c->skip, psi ? psi->rs.as<R>() : nullptr, (R)sp->q_value);
@@ -2069,7 +2080,7 @@ static int amjdp_out(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
                      const qp_field2d *psit, double dex, const DepOut<R> &out,
                      const qp_field2d *psi = nullptr)
 {
-    int rc;
+    int rc, bands = 1;
     switch (sp->ctx->tune[QP_TUNE_AMJDP]) {
     case 1: rc = amjdp_v<R, 1>(sp, ef, bf, psit, dex, out, psi); break;
     case 2: rc = amjdp_v<R, 2>(sp, ef, bf, psit, dex, out, psi); break;
@@ -2085,10 +2096,14 @@ static int amjdp_out(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
     case 12: rc = amjdp_v<R, 12>(sp, ef, bf, psit, dex, out, psi); break;
     case 13: rc = amjdp_v<R, 13>(sp, ef, bf, psit, dex, out, psi); break;
     case 14: rc = amjdp_v<R, 14>(sp, ef, bf, psit, dex, out, psi); break;
-    default: rc = amjdp_v<R, 0>(sp, ef, bf, psit, dex, out, psi); break;
+    default:
+        bands = deposit_bands(sp->ctx);
+        rc = bands == 4   ? amjdp_v<R, 0, 4>(sp, ef, bf, psit, dex, out, psi)
+             : bands == 2 ? amjdp_v<R, 0, 2>(sp, ef, bf, psit, dex, out, psi)
+                          : amjdp_v<R, 0>(sp, ef, bf, psit, dex, out, psi);
     }
     if (rc) return rc;
-    return deposit_border<R>(sp->ctx, out, 8, 1);
+    return deposit_border<R>(sp->ctx, out, 8, 1, nullptr, bands);
 }
 
 // the species' own cu, dcu, amu (overwritten)

@@ -1016,7 +1016,7 @@ k_amjdp_w(TileGeom g, Soa<R> s, const int *__restrict__ off, const R *fxy, const
 // PPGRBPPUSHF23L_QP (part2d_lib77.f:1066-1408): 3-D Boris push in xi, then the
 // periodic wrap of the reorder (PPPORDER2LB :1936-1977).  One workgroup per
 // source tile walks the tile's particles (a contiguous run of the sorted
-// arrays) 256 at a time, one thread per particle.  A particle leaves for the
+// arrays) NT at a time, one thread per particle.  A particle leaves for the
 // neighbour tile in its direction of motion (dir in {-1,0,1}^2, bin
 // nb = 3 (diry+1) + dirx + 1) and lands in cell cl of it; its rank among the
 // tile's particles bound for the same (nb, cl) follows their order in the
@@ -1044,25 +1044,27 @@ k_amjdp_w(TileGeom g, Soa<R> s, const int *__restrict__ off, const R *fxy, const
 // 1024^2); MODE 2 clears them for the next push.  The two passes read the particle record twice and
 // write it once, where push and scatter read it twice and write it twice.
 constexpr int NBINS = 9 * TCELLS;
+constexpr int PUSH_WIDE = 1024;   // threads of a block where tiles are few (push_t)
 constexpr int BIN_BITS = 12;
 static_assert(NBINS <= 1 << BIN_BITS && TCELLS / 64 == 4, "push: bins and waves");
 constexpr int GROUP = 256;  // tiles per group of the offsets' two-level sum
 
-template <typename R, int MODE>
-__global__ void __launch_bounds__(256)
+template <typename R, int MODE, int NT = 256>
+__global__ void __launch_bounds__(NT)
 k_push(TileGeom g, Soa<R> s, Soa<R> o, const int *__restrict__ off,
        const int *__restrict__ off_new, const R *fxy, const R *bxy, const R *psit, size_t cs,
        R qbm, R dt, R dex, int *bin, int *rank, int *cnt, int *err, int64_t np, int uq, int raw,
        int *tot)
 {
     __shared__ int hist[NBINS];
-    __shared__ unsigned whist[MODE == 1 ? 1 : NBINS];   // byte w: wave w's, in this chunk
+    // byte w of a bin: wave w's particles in this chunk
+    constexpr int NW = NT / 64;
+    __shared__ __attribute__((aligned(16))) unsigned whist[MODE == 1 ? 1 : NBINS * NW / 4];
     __shared__ R fnode[6][289];   // the six fields at the tile's 17 x 17 nodes
     const int S = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int k = tid; k < NBINS; k += TCELLS) {
-        hist[k] = 0;
-        if (MODE != 1) whist[k] = 0;
-    }
+    for (int k = tid; k < NBINS; k += NT) hist[k] = 0;
+    if (MODE != 1)
+        for (int k = tid; k < NBINS * NW / 4; k += NT) whist[k] = 0;
     const int tx0 = S % g.mx1, ty0 = S / g.mx1;
     const int p0 = off[S * TCELLS], p1 = off[(S + 1) * TCELLS];
     // the particle record of chunk c0 is loaded while chunk c0 - 256 is ranked
@@ -1085,11 +1087,11 @@ k_push(TileGeom g, Soa<R> s, Soa<R> o, const int *__restrict__ off,
     // every particle of the tile lies in one of its cells (the sort put it
     // there), so the corners it gathers are tile nodes: read them once
     {
-        constexpr int NF = (6 * 289 + TCELLS - 1) / TCELLS;
+        constexpr int NF = (6 * 289 + NT - 1) / NT;
         R tv[NF];
 #pragma unroll
         for (int k = 0; k < NF; ++k) {
-            const int n = tid + k * TCELLS;
+            const int n = tid + k * NT;
             if (n < 6 * 289) {
                 const int f = n / 289, m = n % 289;
                 const R *pl = f == 0 ? fxy : f == 1 ? fxy + cs : f == 2 ? psit
@@ -1102,7 +1104,7 @@ k_push(TileGeom g, Soa<R> s, Soa<R> o, const int *__restrict__ off,
         }
 #pragma unroll
         for (int k = 0; k < NF; ++k) {
-            const int n = tid + k * TCELLS;
+            const int n = tid + k * NT;
             if (n < 6 * 289) fnode[n / 289][n % 289] = tv[k];
         }
     }
@@ -1112,11 +1114,11 @@ k_push(TileGeom g, Soa<R> s, Soa<R> o, const int *__restrict__ off,
     const R edgelx = (R)(tx0 * TILE), edgely = (R)(ty0 * TILE);
     const R edgerx = edgelx + (R)min(TILE, g.nx - tx0 * TILE);
     const R edgery = edgely + (R)min(TILE, g.ny - ty0 * TILE);
-    for (int c0 = p0; c0 < p1; c0 += TCELLS) {
+    for (int c0 = p0; c0 < p1; c0 += NT) {
         const int i = c0 + tid;
         const bool valid = i < p1;
         const R x = nx_, y = ny_, ppx = npx, ppy = npy, ppz = npz, p6 = np6, p7 = np7, q = nq;
-        if (c0 + TCELLS < p1) fetch(c0 + TCELLS);
+        if (c0 + NT < p1) fetch(c0 + NT);
         int b = 0, dcell = 0;
         R ox_ = R(0), oy_ = R(0), opx = R(0), opy = R(0), opz = R(0);
         if (valid) {
@@ -1270,17 +1272,24 @@ k_push(TileGeom g, Soa<R> s, Soa<R> o, const int *__restrict__ off,
         int rk = __popcll(m & ((1ull << lane) - 1ull));
         const bool lead = valid && rk == 0;
         const int nlead = __popcll(m);   // at most 64
-        if (lead) reinterpret_cast<unsigned char *>(whist)[4 * b + wave] = (unsigned char)nlead;
+        if (lead) reinterpret_cast<unsigned char *>(whist)[NW * b + wave] = (unsigned char)nlead;
         __syncthreads();
         // the tile's earlier chunks, and this chunk's earlier waves
         if (valid) {
-            const unsigned w4 = whist[b] & ((1u << (8 * wave)) - 1u);
-            rk += hist[b] + (int)__builtin_amdgcn_sad_u8(w4, 0u, 0u);
+            unsigned n = (unsigned)hist[b];
+#pragma unroll
+            for (int k = 0; k < NW / 4; ++k) {
+                const int w = wave - 4 * k;   // earlier waves in this word
+                const unsigned v = whist[b * (NW / 4) + k];
+                if (w >= 4) n = __builtin_amdgcn_sad_u8(v, 0u, n);
+                else if (w > 0) n = __builtin_amdgcn_sad_u8(v & ((1u << (8 * w)) - 1u), 0u, n);
+            }
+            rk += (int)n;
         }
         __syncthreads();
         if (lead) {
             atomicAdd(&hist[b], nlead);
-            reinterpret_cast<unsigned char *>(whist)[4 * b + wave] = 0;
+            reinterpret_cast<unsigned char *>(whist)[NW * b + wave] = 0;
         }
         if (MODE == 0 && valid) {
             bin[i] = S * NBINS + b;
@@ -1309,20 +1318,15 @@ k_push(TileGeom g, Soa<R> s, Soa<R> o, const int *__restrict__ off,
     __syncthreads();
     __shared__ int s_tot[9];   // particles bound for each neighbour
     if (MODE == 1 && tid < 9) s_tot[tid] = 0;
-    int h[9];
-#pragma unroll
-    for (int nb = 0; nb < 9; ++nb) {
-        h[nb] = hist[nb * TCELLS + tid];
-        cnt[(size_t)S * NBINS + nb * TCELLS + tid] = h[nb];
-    }
+    for (int n = tid; n < NBINS; n += NT) cnt[(size_t)S * NBINS + n] = hist[n];
     if (MODE != 1) return;
     __syncthreads();
+    for (int n = tid; n < NBINS; n += NT) {   // a wave's bins are one neighbour's
+        int h = hist[n];
+        if (!__any(h)) continue;
 #pragma unroll
-    for (int nb = 0; nb < 9; ++nb) {
-        if (!__any(h[nb])) continue;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) h[nb] += __shfl_xor(h[nb], o);
-        if (lane == 0) atomicAdd(&s_tot[nb], h[nb]);
+        for (int o = 32; o > 0; o >>= 1) h += __shfl_xor(h, o);
+        if (lane == 0) atomicAdd(&s_tot[n / TCELLS], h);
     }
     __syncthreads();
     if (tid < 9 && s_tot[tid])
@@ -2126,14 +2130,20 @@ static int push_t(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
     qp_ctx *c = sp->ctx;
     const TileGeom g = geom(c);
     const bool scatter = c->tune[QP_TUNE_PUSH] == 1;
+    // Blocks of 1024 where every tile has a unit of its own and more particles than
+    // a block of 256 takes at once: four waves a SIMD cover each other's waits.
+    // FP64, 4 a cell, first and second pass: 64 x 32 10.3 + 11.0 -> 7.3 + 8.3 us,
+    // 128^2 10.8 + 12.6 -> 8.2 + 10.3; but 512 tiles (9 a cell) 20 + 36 -> 24 + 38,
+    // and 512^2 FP32 (1024 tiles, 4 a cell) 14.6 + 19.3 -> 17.0 + 27.7.
+    const bool wide = !scatter && c->ntiles <= c->cus && sp->np > (int64_t)256 * c->ntiles;
     const double fields = 6.0 * (c->nx + 1.0) * (c->ny + 1.0) * sizeof(R);
     const Soa<R> a = soa<R>(sp->a), b = soa<R>(sp->b);
     int *off = sp->off.as<int>(), *off_new = sp->off_new.as<int>();
     {
     // in place: 7 arrays read, 5 written; counting: 7 read
     ProfScope _ps(c, QP_PROF_PUSH, (scatter ? 12.0 : 7.0) * sp->np * sizeof(R) + fields);
-    auto kern = scatter ? k_push<R, 0> : k_push<R, 1>;
-    hipLaunchKernelGGL(kern, dim3(c->ntiles), dim3(TCELLS), 0, c->stream, g, a, b, off, off_new,
+    auto kern = scatter ? k_push<R, 0> : wide ? k_push<R, 1, PUSH_WIDE> : k_push<R, 1>;
+    hipLaunchKernelGGL(kern, dim3(c->ntiles), dim3(wide ? PUSH_WIDE : 256), 0, c->stream, g, a, b, off, off_new,
                        ef->rs.as<R>(), bf->rs.as<R>(), psit->rs.as<R>(), c->rplane,
                        (R)sp->qbm, (R)sp->dt, (R)dex, sp->key.as<int>(), sp->slot.as<int>(),
                        sp->bins.as<int>(), sp->err.as<int>(), sp->np, 0, raw ? 1 : 0,
@@ -2172,8 +2182,8 @@ static int push_t(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
         {
         // 8 arrays read, 8 written at their sorted places
         ProfScope _ps(c, QP_PROF_SORT, (sp->q_uniform ? 14.0 : 16.0) * sp->np * sizeof(R) + fields);
-        auto kern = k_push<R, 2>;
-        hipLaunchKernelGGL(kern, dim3(c->ntiles), dim3(TCELLS), 0, c->stream, g, a, b,
+        auto kern = wide ? k_push<R, 2, PUSH_WIDE> : k_push<R, 2>;
+        hipLaunchKernelGGL(kern, dim3(c->ntiles), dim3(wide ? PUSH_WIDE : 256), 0, c->stream, g, a, b,
                            off, off_new, ef->rs.as<R>(), bf->rs.as<R>(), psit->rs.as<R>(),
                            c->rplane, (R)sp->qbm, (R)sp->dt, (R)dex, nullptr, nullptr,
                            sp->bins.as<int>(), sp->err.as<int>(), sp->np, sp->q_uniform ? 1 : 0,

@@ -50,3 +50,32 @@ def test_banded_current_deposit(indx, indy, ppc, precision):
         assert peak > 0.0
         assert np.abs(a - b).max() <= n * n * eps * peak
     assert np.array_equal(got[-1], want[-1])   # the deposit moves no particle
+
+
+def _pushed(indx, indy, ppc, precision, in_place):
+    ctx = qps.Ctx(indx, indy, 4, box=(-10.0, 10.0, -10.0, 10.0, 0.0, 1.0), precision=precision)
+    if in_place:
+        ctx.tune(qps.TUNE_PUSH, 1)
+    sp = qps.Species(ctx, ppc=ppc)
+    f = {n: qps.Field2d(ctx, d) for n, d in (("e", 2), ("b", 3), ("psit", 1))}
+    rng = np.random.default_rng(indx + 7 * indy)
+    for n, d in (("e", 2), ("b", 3), ("psit", 1)):
+        f[n].upload(0.2 * rng.standard_normal((d, ctx.ny + 1, ctx.nx + 1)), space=0)
+    out = []
+    for _ in range(3):
+        sp.push(f["e"], f["b"], f["psit"], ctx.dex)
+        out += [sp.download(), sp.cell_counts()]
+    ctx.close()
+    return out
+
+
+@pytest.mark.parametrize("precision", ["FP64", "FP32"])
+@pytest.mark.parametrize("indx,indy,ppc", [(4, 4, (5, 5)), (6, 5, (2, 2)), (7, 7, (3, 2)),
+                                           (8, 8, (2, 1)), (7, 7, (1, 1)), (9, 8, (2, 2))])
+def test_push_blocks_keep_the_order(indx, indy, ppc, precision):
+    """Blocks of 256 and of 1024 threads put every particle where the push in
+    place and the scatter behind it put it, bit for bit."""
+    print(f"[gpu-test] push blocks {indx} {indy} {ppc} {precision}", flush=True)
+    p = getattr(qps, precision)
+    for a, b in zip(_pushed(indx, indy, ppc, p, False), _pushed(indx, indy, ppc, p, True)):
+        assert np.array_equal(a, b)

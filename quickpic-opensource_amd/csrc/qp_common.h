@@ -264,6 +264,17 @@ __device__ __forceinline__ void run_res_job(const ResJob &j)
     }
 }
 
+// A deposit's border sums left to the field solve (BorderArgs, qp_border.h): the
+// n components' border buffer and destinations.  n = 0: nothing is left.
+struct BorderJob {
+    const void *halo = nullptr;
+    void *p[8] = {};
+    const void *inner[8] = {}, *outer[8] = {};
+    void *p2[8] = {};
+    double scale = 1.0, scale2 = 1.0;
+    int rb = 0, fold = 0, n = 0;
+};
+
 // ---- fused slice-loop kernels (qp_fused.hip) ----
 struct PassFields {
     qp_field2d *cu, *dcu, *amu, *epw, *epwb, *psit, *bxyz;
@@ -293,9 +304,10 @@ struct FrontFields {
     qp_field2d *ehist, *ehist2;   // the corrector seed's history (or null), as fused_pass
 };
 bool fused_fields(const qp_ctx *c);
-int fused_solve_pass(const PassFields &f, double dex, int l, double tol);
+bool fused_border(const qp_ctx *c);
+int fused_solve_pass(const PassFields &f, double dex, int l, double tol, const BorderJob &job);
 int fused_solve_front(const PassFields &f, const FrontFields &fr, double dex, int seed,
-                      const int *seed_hist);
+                      const int *seed_hist, const BorderJob &job);
 // Anderson mixing (depth 1) of the corrector iterate after pass l (f.gprev,
 // f.fprev set; the pass was run by fused_pass with them): unless pass l has
 // converged, epw <- g_l - gamma (g_l - g_{l-1}) and B_perp reassembled; mix =

@@ -19,6 +19,7 @@
 #include <type_traits>
 
 #include "qp_common.h"
+#include "qp_border.h"
 
 struct qp_species {
     qp_ctx *ctx;
@@ -65,10 +66,6 @@ template <typename R> static Soa<R> soa(DevBuf *a)
     return Soa<R>{a[0].as<R>(), a[1].as<R>(), a[2].as<R>(), a[3].as<R>(),
                   a[4].as<R>(), a[5].as<R>(), a[6].as<R>(), a[7].as<R>()};
 }
-
-struct TileGeom {
-    int nx, ny, mx1, my1, ldr;
-};
 
 // Particle positions.  FP64 records hold x and y in grid units, as the
 // reference does.  FP32 records hold them relative to the origin of the
@@ -120,40 +117,6 @@ __device__ __forceinline__ R gather(const Corners<R> &f, R amx, R amy, R dxp, R 
     return d + dyp * (dxp * f.f11 + a);
 }
 
-// (a block of RB rows of cells: 17 x (RB + 1) nodes)
-template <int RB = TILE> __device__ __forceinline__ int halo_index(int i, int j)
-{
-    if (j == 0) return i;
-    if (j == RB) return 17 + i;
-    if (i == 0) return 34 + (j - 1);
-    return 33 + RB + (j - 1);
-}
-
-// Where a deposit's node sums go.  For component c and node value v:
-//   t = v (+ inner[c][node]);  t *= scale;  p[c][node] = (outer[c][node] +) t
-//   p2[c][node] = v * scale2                                (when p2[c] is set)
-// With null inner/outer and unit scales this is a plain overwrite; the other
-// settings restate the field additions and scalings that species2d and the
-// slice loop apply right after a deposit (species2d_class.f03:166-218,
-// simulation_class.f03:682-685), in the same order.
-template <typename R> struct DepOut {
-    R *p[8];
-    const R *inner[8];
-    const R *outer[8];
-    R *p2[8];
-    R scale, scale2;
-};
-
-template <typename R>
-__device__ __forceinline__ void dep_store(const DepOut<R> &o, int c, size_t idx, R v)
-{
-    R t = v;
-    if (o.inner[c]) t = t + o.inner[c][idx];
-    t = t * o.scale;
-    if (o.p2[c]) o.p2[c][idx] = v * o.scale2;
-    o.p[c][idx] = o.outer[c] ? o.outer[c][idx] + t : t;
-}
-
 template <typename R> static DepOut<R> dep_plain(R *const *planes, int n)
 {
     DepOut<R> o{};
@@ -172,7 +135,8 @@ __global__ void k_deposit_border(TileGeom g, const R *__restrict__ halo, size_t 
 {
     if (skip && *skip) return;
     const int comp = blockIdx.y;
-    constexpr int B = TILE / RB;   // blocks of a tile, and their nodes in the buffer
+    constexpr int B = TILE / RB, SH = RB == 16 ? 4 : RB == 8 ? 3 : 2;
+    static_assert(1 << SH == RB, "rows of a block");
     const int myb = g.my1 * B;
     const int rows_n = (myb + 1) * (g.nx + 1);
     const int cols_n = (g.mx1 + 1) * myb * (RB - 1);
@@ -190,27 +154,7 @@ __global__ void k_deposit_border(TileGeom g, const R *__restrict__ halo, size_t 
     } else {
         return;
     }
-    const R *h = halo + comp * halo_cs;
-    auto node_sum = [&](int XX, int YY) -> R {
-        R s = R(0);
-        for (int tyc = YY / RB - 1; tyc <= YY / RB; ++tyc) {
-            if (tyc < 0 || tyc >= myb) continue;
-            int ly = YY - RB * tyc;
-            if (ly < 0 || ly > RB) continue;
-            for (int txc = (XX >> 4) - 1; txc <= (XX >> 4); ++txc) {
-                if (txc < 0 || txc >= g.mx1) continue;
-                int lx = XX - TILE * txc;
-                if (lx < 0 || lx > TILE) continue;
-                s += h[(size_t)(((tyc / B) * g.mx1 + txc) * B + tyc % B) * band_halo(RB) +
-                       halo_index<RB>(lx, ly)];
-            }
-        }
-        return s;
-    };
-    R v;
-    if (fold && Y == g.ny) v = R(0);
-    else if (fold && Y == 0) { v = node_sum(X, 0); v = v + node_sum(X, g.ny); }
-    else v = node_sum(X, Y);
+    const R v = border_node<R>(g, halo + comp * halo_cs, SH, fold, X, Y);
     dep_store(out, comp, (size_t)Y * g.ldr + X, v);
 }
 
@@ -273,7 +217,7 @@ __device__ __forceinline__ void emit_nodes(const R *nacc, const DepOut<R> &out, 
         if (i >= 1 && i < TILE && j >= 1 && j < RB)
             dep_store(out, c, (size_t)(ty * TILE + band * RB + j) * ldr + tx * TILE + i, v);
         else
-            halo[(size_t)(tile * (TILE / RB) + band) * band_halo(RB) + halo_index<RB>(i, j)] = v;
+            halo[(size_t)(tile * (TILE / RB) + band) * band_halo(RB) + halo_index(RB, i, j)] = v;
     }
 }
 
@@ -1008,7 +952,7 @@ k_amjdp_w(TileGeom g, Soa<R> s, const int *__restrict__ off, const R *fxy, const
             if (i >= 1 && i < TILE && j >= 1 && j < TILE)
                 dep_store(out, c, (size_t)(ty * TILE + j) * g.ldr + tx * TILE + i, v);
             else
-                halo[c * halo_cs + (size_t)tile * HALO + halo_index(i, j)] = v;
+                halo[c * halo_cs + (size_t)tile * HALO + halo_index(TILE, i, j)] = v;
         }
     }
 }
@@ -1620,11 +1564,27 @@ static int rebin_unsorted(qp_species *sp, const std::vector<int> *hkeys = nullpt
 
 template <typename R>
 static int deposit_border(qp_ctx *c, const DepOut<R> &out, int ncomp, int fold,
-                          const R *halo = nullptr, int bands = 1)
+                          const R *halo = nullptr, int bands = 1, BorderJob *job = nullptr)
 {
     QP_REQUIRE(ncomp >= 1 && ncomp <= 8, QP_ERR_ARG, "deposit border: %d components", ncomp);
     TileGeom g = geom(c);
     const int rb = TILE / bands, myb = c->my1 * bands;
+    if (job) {
+        *job = BorderJob{};
+        job->halo = halo ? halo : c->halo.as<R>();
+        job->rb = rb;
+        job->fold = fold;
+        job->n = ncomp;
+        for (int k = 0; k < ncomp; ++k) {
+            job->p[k] = out.p[k];
+            job->inner[k] = out.inner[k];
+            job->outer[k] = out.outer[k];
+            job->p2[k] = out.p2[k];
+        }
+        job->scale = (double)out.scale;
+        job->scale2 = (double)out.scale2;
+        return QP_OK;
+    }
     int n = (myb + 1) * (c->nx + 1) + (c->mx1 + 1) * myb * (rb - 1);
     {
     ProfScope _ps(c, QP_PROF_BORDER, 2.0 * ncomp * (double)n * sizeof(R));
@@ -1714,7 +1674,7 @@ static int deposit_q_v(qp_species *sp, const DepOut<R> &out, R *halo, const Beam
 // halo: the tile-border buffer (null: the context's)
 template <typename R>
 static int deposit_q_out(qp_species *sp, const DepOut<R> &out, R *halo = nullptr,
-                         const BeamPlane *bp = nullptr)
+                         const BeamPlane *bp = nullptr, BorderJob *job = nullptr)
 {
     int rc;
     if (!halo) halo = sp->ctx->halo.as<R>();
@@ -1725,7 +1685,7 @@ static int deposit_q_out(qp_species *sp, const DepOut<R> &out, R *halo = nullptr
     default: rc = deposit_q_v<R, 0>(sp, out, halo, bp); break;
     }
     if (rc) return rc;
-    return deposit_border<R>(sp->ctx, out, 1, 1, halo);
+    return deposit_border<R>(sp->ctx, out, 1, 1, halo, 1, job);
 }
 
 template <typename R>
@@ -2082,7 +2042,7 @@ static int amjdp_v(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
 template <typename R>
 static int amjdp_out(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
                      const qp_field2d *psit, double dex, const DepOut<R> &out,
-                     const qp_field2d *psi = nullptr)
+                     const qp_field2d *psi = nullptr, BorderJob *job = nullptr)
 {
     int rc, bands = 1;
     switch (sp->ctx->tune[QP_TUNE_AMJDP]) {
@@ -2107,7 +2067,7 @@ static int amjdp_out(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
                           : amjdp_v<R, 0>(sp, ef, bf, psit, dex, out, psi);
     }
     if (rc) return rc;
-    return deposit_border<R>(sp->ctx, out, 8, 1, nullptr, bands);
+    return deposit_border<R>(sp->ctx, out, 8, 1, nullptr, bands, job);
 }
 
 // the species' own cu, dcu, amu (overwritten)
@@ -2663,7 +2623,8 @@ int species_check_poll(qp_species *sp, bool wait)
 // q = qn + q.  first: q holds nothing yet (the slice loop zeroed it).  bp: the
 // beam plane to convert beside it (or null).
 template <typename R>
-static int qdp_fused_t(qp_species *sp, qp_field2d *q, bool first, const BeamPlane *bp)
+static int qdp_fused_t(qp_species *sp, qp_field2d *q, bool first, const BeamPlane *bp,
+                       BorderJob *job)
 {
     R *qp = q->rs.as<R>();
     DepOut<R> o{};
@@ -2672,16 +2633,17 @@ static int qdp_fused_t(qp_species *sp, qp_field2d *q, bool first, const BeamPlan
     o.outer[0] = sp->qn->rs.as<R>();
     o.p2[0] = sp->q->rs.as<R>();
     o.scale = o.scale2 = R(1);
-    int rc = deposit_q_out<R>(sp, o, nullptr, bp);
+    int rc = deposit_q_out<R>(sp, o, nullptr, bp, job);
     sp->q->state = 0;
     sp->q->gcells = 1;
     q->state = 0;
     return rc;
 }
 
-int species_qdp_fused(qp_species *sp, qp_field2d *q, bool first, const BeamPlane *bp)
+int species_qdp_fused(qp_species *sp, qp_field2d *q, bool first, const BeamPlane *bp,
+                      BorderJob *job)
 {
-    return DISPATCH(sp->ctx, qdp_fused_t, sp, q, first, bp);
+    return DISPATCH(sp->ctx, qdp_fused_t, sp, q, first, bp, job);
 }
 
 // amjdp_species2d plus the slice loop's scaling (species2d_class.f03:187-218,
@@ -2692,7 +2654,7 @@ template <typename R>
 static int amjdp_fused_t(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
                          const qp_field2d *psit, qp_field2d *cu, qp_field2d *dcu,
                          qp_field2d *amu, double dex, bool first, bool last,
-                         const qp_field2d *psi)
+                         const qp_field2d *psi, BorderJob *job)
 {
     const size_t pl = sp->ctx->rplane;
     R *c = cu->rs.as<R>(), *d = dcu->rs.as<R>(), *a = amu->rs.as<R>();
@@ -2705,7 +2667,7 @@ static int amjdp_fused_t(qp_species *sp, const qp_field2d *ef, const qp_field2d 
     o.p2[2] = sp->cu->rs.as<R>() + 2 * pl;
     o.scale = last ? (R)dex : R(1);
     o.scale2 = (R)dex;
-    int rc = amjdp_out<R>(sp, ef, bf, psit, dex, o, psi);
+    int rc = amjdp_out<R>(sp, ef, bf, psit, dex, o, psi, job);
     sp->cu->state = 0;
     cu->state = dcu->state = amu->state = 0;
     return rc;
@@ -2713,9 +2675,9 @@ static int amjdp_fused_t(qp_species *sp, const qp_field2d *ef, const qp_field2d 
 
 int species_amjdp_fused(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
                         const qp_field2d *psit, qp_field2d *cu, qp_field2d *dcu, qp_field2d *amu,
-                        double dex, bool first, bool last, const qp_field2d *psi)
+                        double dex, bool first, bool last, const qp_field2d *psi, BorderJob *job)
 {
     return DISPATCH(sp->ctx, amjdp_fused_t, sp, ef, bf, psit, cu, dcu, amu, dex, first, last,
-                    psi);
+                    psi, job);
 }
 }  // namespace qp

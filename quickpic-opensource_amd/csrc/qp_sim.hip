@@ -22,14 +22,15 @@ int species_check_post(qp_species *sp, int slice);
 void species_err_words(qp_species *sp, const int **err, int **h_err);
 int species_check_mark(qp_species *sp);
 int species_check_poll(qp_species *sp, bool wait);
-int species_qdp_fused(qp_species *sp, qp_field2d *q, bool first, const BeamPlane *bp);
+int species_qdp_fused(qp_species *sp, qp_field2d *q, bool first, const BeamPlane *bp,
+                      BorderJob *job);
 int beam_slice_assign(qp_beam *b, qp_field2d *q, int slice, const int *jdev = nullptr);
 int beam_slice_plane(qp_beam *b, qp_field2d *q, int slice, const int *jdev, BeamPlane *bp);
 int beam_slice_add_dev(qp_beam *b, qp_field2d *q, const int *jdev);
 int species_q3_initial(qp_species *sp, qp_field3d *q3);
 int species_amjdp_fused(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
                         const qp_field2d *psit, qp_field2d *cu, qp_field2d *dcu, qp_field2d *amu,
-                        double dex, bool first, bool last, const qp_field2d *psi);
+                        double dex, bool first, bool last, const qp_field2d *psi, BorderJob *job);
 }  // namespace qp
 
 struct qp_sim {
@@ -233,7 +234,7 @@ int qp_sim_begin_step(qp_sim *s)
 //    species' charge deposit.
 
 // beam charge (:650-655) and plasma charge (:657-661) of slice j
-static int slice_charges(qp_sim *s, int j)
+static int slice_charges(qp_sim *s, int j, BorderJob *job)
 {
     qp_ctx *c = s->ctx;
     QP_REQUIRE(j >= 1 && j <= c->nz, QP_ERR_ARG, "qp_slice_prepare: slice %d outside 1..%d", j,
@@ -251,7 +252,8 @@ static int slice_charges(qp_sim *s, int j)
     else RC(beam_slice_plane(s->bm[0], qb, j + 1, jdev, &bp));
     if (nsp == 0) RC(qp_field2d_as(qe, 0.0));
     for (int i = 0; i < nsp; ++i)
-        RC(species_qdp_fused(s->sp[i], qe, i == 0, i == 0 && bp.q3 ? &bp : nullptr));
+        RC(species_qdp_fused(s->sp[i], qe, i == 0, i == 0 && bp.q3 ? &bp : nullptr,
+                             i == nsp - 1 ? job : nullptr));
     for (size_t i = 1; i < s->bm.size(); ++i)
         RC(jdev ? beam_slice_add_dev(s->bm[i], qb, jdev) : qp_beam_qdpcopy(s->bm[i], qb, j + 1));
     QP_REQUIRE(qb->state == 0 && qe->state == 0, QP_ERR_STATE, "fftrk: data is in ks");
@@ -263,7 +265,7 @@ static int slice_charges(qp_sim *s, int j)
 int qp_slice_prepare(qp_sim *s, int j)
 {
     QP_REQUIRE(s, QP_ERR_ARG, "qp_slice_prepare: null sim");
-    RC(slice_charges(s, j));
+    RC(slice_charges(s, j, nullptr));
     qp_field2d **F = s->f;
     qp_field2d *qb = F[QP_F_QB], *qe = F[QP_F_QE], *psi = F[QP_F_PSI], *fxy = F[QP_F_FXY];
     qp_field2d *epwb = F[QP_F_EPWB];
@@ -302,16 +304,17 @@ struct SliceRun {
     int j, iter_max;
     double tol;
     qp_ctx *c;
-    bool adaptive, mixing, fused;
+    bool adaptive, mixing, fused, bordered;
     int seed = 0, tag0 = 0;
     PassFields pf, pc;
+    BorderJob border;   // the last deposit's, for the solve behind it (fused_border)
 
     SliceRun(qp_sim *sim, int jj, int imax, double t)
         : s(sim), j(jj), iter_max(imax), tol(t), c(sim->ctx), adaptive(t > 0.0),
           // the mixed corrector (QP_TUNE_MIX) applies only to runs to a
           // tolerance outside captured slices
           mixing(t > 0.0 && !sim->graph && sim->ctx->tune[QP_TUNE_MIX] == 1),
-          fused(fused_fields(sim->ctx) && !mixing),
+          fused(fused_fields(sim->ctx) && !mixing), bordered(fused && fused_border(sim->ctx)),
           pf{sim->f[QP_F_CU], sim->f[QP_F_DCU], sim->f[QP_F_AMU], sim->f[QP_F_EPW],
              sim->f[QP_F_EPWB], sim->f[QP_F_PSIT], sim->f[QP_F_BXYZ], nullptr, nullptr},
           pc(pf)
@@ -341,7 +344,7 @@ struct SliceRun {
         if (front) {
             const FrontFields fr{s->f[QP_F_QB], s->f[QP_F_QE], s->f[QP_F_PSI], s->f[QP_F_FXY],
                                  s->epw_hist, hist2};
-            RC(fused_solve_front(pf, fr, c->dex, seed, seed_hist));
+            RC(fused_solve_front(pf, fr, c->dex, seed, seed_hist, border));
         } else {
             RC(fused_pass(pf, c->dex, false, 0, 0.0, seed, s->epw_hist, seed_hist, hist2));
             RC(inverse());
@@ -381,7 +384,8 @@ struct SliceRun {
         for (int i = 0; i < nsp; ++i)
             RC(species_amjdp_fused(s->sp[i], s->f[QP_F_FXY], pf.bxyz, pf.psit, pf.cu, pf.dcu,
                                    pf.amu, c->dex, i == 0, i == nsp - 1,
-                                   l == 1 ? s->f[QP_F_PSI] : nullptr));
+                                   l == 1 ? s->f[QP_F_PSI] : nullptr,
+                                   bordered && i == nsp - 1 ? &border : nullptr));
         c->prof_tag = 0;
         return QP_OK;
     }
@@ -391,7 +395,7 @@ struct SliceRun {
         c->prof_tag = tag0 + l;
         if (c->skip) c->skip = flags() + (l - 1);
         if (fused) {
-            RC(fused_solve_pass(pf, c->dex, l, tol));
+            RC(fused_solve_pass(pf, c->dex, l, tol, border));
         } else {
             qp_field2d *fwd[3] = {pf.cu, pf.dcu, pf.amu};
             const int kinds[3] = {1, 1, 3};
@@ -465,7 +469,7 @@ struct SliceRun {
 int slice_begin(SliceRun &r)
 {
     if (fused_fields(r.c)) {
-        RC(slice_charges(r.s, r.j));
+        RC(slice_charges(r.s, r.j, fused_border(r.c) ? &r.border : nullptr));
         return r.begin(true);
     }
     RC(qp_slice_prepare(r.s, r.j));

@@ -20,6 +20,7 @@
 // components has to fit the 160 KB of LDS for the exchange between the
 // transforms and the modes: 8 (ny + 1) pairs, 66 KB in FP32 and 131 KB in FP64
 // at ny = 1024.
+#include "qp_border.h"
 #include "qp_fft.h"
 #include "qp_pass.h"
 
@@ -29,6 +30,14 @@ template <typename R> struct XtSet {
     const R *src[8];
     R *dst[8];
 };
+
+// A barrier that orders LDS alone: loads and stores of memory stay in flight.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
 
 // 16 bytes of Reals
 template <typename R> struct alignas(16) Quad {
@@ -54,6 +63,13 @@ template <typename R, int L> struct XtShape {
     static_assert((size_t)(S::N + 1) * SW * sizeof(R) <= LDS, "staging fits the FFT's area");
 };
 
+// Up to this nx the forward x transforms form the border sums of the deposit in
+// front of them (a launch less).  With the launches: 128^2 FP64 4.4 + 5.1 us
+// against 8.3 in one, 256 x 512 FP32 5.4 + 6.2 against 10.2; but 512^2 FP32
+// 5.4 + 11.7 against 19.3, and 1024^2 11.7 + 27.4 against 48.9: there the blocks
+// of whole border rows wait longer than a kernel of their own does.
+constexpr int BORDER_MAX = 256;
+
 // x transforms of the rows of every component of the batch (grid.y).  INV =
 // false: rows y of src (pitch ld_src) to columns y of dst ([kx][y], pitch
 // ld_dst).  INV = true: columns y of src to rows y of dst, row 0 also to row
@@ -66,7 +82,8 @@ template <typename R, int L> struct XtShape {
 template <typename R, int L, bool INV>
 __global__ void __launch_bounds__((XtShape<R, L>::BS))
 k_fft_xt(XtSet<R> cs, int nrows, int ld_src, int ld_dst, int types, R scale,
-         const cplx<R> *__restrict__ W, int guard_row, int zero_row, const int *skip, ResJob rj)
+         const cplx<R> *__restrict__ W, int guard_row, int zero_row, const int *skip, ResJob rj,
+         BorderArgs<R> bd)
 {
     using X = XtShape<R, L>;
     using S = typename X::S;
@@ -94,8 +111,14 @@ k_fft_xt(XtSet<R> cs, int nrows, int ld_src, int ld_dst, int types, R scale,
     // evenly over the threads, those of kx = N go to the first CH threads
     constexpr int K = (N * CH + BS - 1) / BS;
     static_assert(N * CH % BS == 0 || N * CH < BS, "whole rounds of pieces");
+    constexpr bool BORDER = !INV && N <= BORDER_MAX;
+    const bool border = BORDER && comp >= bd.first && comp < bd.first + bd.n;
+    const int bc = border ? comp - bd.first : 0;
     if (!INV && y0 == zero_row && nrows == zero_row + 1) {
-        for (int it = tid; it <= N; it += BS) dst[(size_t)it * ld_dst + y0] = R(0);
+        for (int it = tid; it <= N; it += BS) {
+            dst[(size_t)it * ld_dst + y0] = R(0);
+            if (border) dep_store(bd.out, bc, (size_t)y0 * ld_src + it, R(0));
+        }
         return;
     }
     cplx<R> v[8], z[4], zn;
@@ -111,6 +134,45 @@ k_fft_xt(XtSet<R> cs, int nrows, int ld_src, int ld_dst, int types, R scale,
             lb[r] = at(sb, e);
         }
         tw.load(W, t);
+        if (BORDER && border) {
+            // the deposit's border nodes in these rows, all nodes of a row that is
+            // a multiple of 2^sh and every 16th of the others: formed here, stored
+            // to the plane and handed on through LDS
+            constexpr int NC = N / TILE + 1;
+            const R *halo = bd.halo + bc * bd.halo_cs;
+            const int nr = min(X::ROWS, nrows - y0), sh = bd.sh, low = (1 << sh) - 1;
+            const int top = -y0 & low;                       // first whole row
+            const int nw = top < nr ? ((nr - 1 - top) >> sh) + 1 : 0;
+            const int items = nw * (N + 1) + X::ROWS * NC;
+            for (int it = tid; it < items; it += BS) {
+                int i, x;
+                if (it < nw * (N + 1)) {
+                    const int w = it / (N + 1);
+                    i = top + (w << sh);
+                    x = it - w * (N + 1);
+                } else {
+                    // rows fastest: a tile's side is contiguous in the buffer
+                    const int k = it - nw * (N + 1);
+                    i = k % X::ROWS;
+                    x = k / X::ROWS * TILE;
+                    if (i >= nr) continue;
+                    if (((y0 + i) & low) == 0) continue;
+                }
+                const R val = border_node<R>(bd.g, halo, sh, bd.fold, x, y0 + i);
+                stg[i * (N + 1) + x] =
+                    dep_store(bd.out, bc, (size_t)(y0 + i) * ld_src + x, val);
+            }
+            lds_barrier();
+            const bool wa = (ra & low) == 0, wb = ((ra + 1) & low) == 0;
+#pragma unroll
+            for (int r = 0; r < 8; ++r) {
+                const int e = ext_pos<L>(t + r * TF);
+                const bool col = e % TILE == 0;
+                if (live && (wa || col)) la[r] = stg[2 * f * (N + 1) + e];
+                if (hb && (wb || col)) lb[r] = stg[(2 * f + 1) * (N + 1) + e];
+            }
+            lds_barrier();   // buf overwrites the staging area
+        }
 #pragma unroll
         for (int r = 0; r < 8; ++r)
             v[r] = ext_value<R, L>(type, t + r * TF, live ? la[r] : R(0),
@@ -627,7 +689,8 @@ template <typename K> static int grant_lds(qp_ctx *c, K kern, size_t lds)
 }
 
 template <typename R, int L, bool INV>
-static int xt_launch(qp_ctx *c, const XtSet<R> &s, int nc, int types, int zero_row)
+static int xt_launch(qp_ctx *c, const XtSet<R> &s, int nc, int types, int zero_row,
+                     const BorderArgs<R> &bd)
 {
     using X = XtShape<R, L>;
     auto kern = k_fft_xt<R, L, INV>;
@@ -646,7 +709,7 @@ static int xt_launch(qp_ctx *c, const XtSet<R> &s, int nc, int types, int zero_r
     hipLaunchKernelGGL(kern, dim3((groups + 7) & ~7, nc), dim3(X::BS), X::LDS, c->stream, s, nrows,
                        INV ? c->ldk : c->ldr, INV ? c->ldr : c->ldk, types,
                        (R)(INV ? 2.0 : ani), c->twx.as<cplx<R>>(), INV ? c->ny : -1, zero_row,
-                       c->skip, rj);
+                       c->skip, rj, bd);
     }
     QP_LAUNCH_CHECK();
     return QP_OK;
@@ -685,9 +748,10 @@ static int mid_launch(qp_ctx *c, const MidArgs<R> &a)
     return QP_ERR_UNSUPPORTED
 
 template <typename R, bool INV>
-static int xt(qp_ctx *c, const XtSet<R> &s, int nc, int types, int zero_row)
+static int xt(qp_ctx *c, const XtSet<R> &s, int nc, int types, int zero_row,
+              const BorderArgs<R> &bd = BorderArgs<R>{})
 {
-#define QP_CALL(L) xt_launch<R, L, INV>(c, s, nc, types, zero_row)
+#define QP_CALL(L) xt_launch<R, L, INV>(c, s, nc, types, zero_row, bd)
     QP_BY_LENGTH(c->nx, QP_CALL);
 #undef QP_CALL
 }
@@ -708,6 +772,9 @@ bool fused_fields(const qp_ctx *c)
            c->tune[QP_TUNE_FFT] == tune_default_of(c->prec, QP_TUNE_FFT);
 }
 
+// whether they form the border sums of the deposits in front of them
+bool fused_border(const qp_ctx *c) { return fused_fields(c) && c->nx <= BORDER_MAX; }
+
 // x types of the components that k_mid takes and gives: the pair (x, y) of
 // kind_types for cu (kind 1), dcu (1), amu (3); qb, qe (1); fxy (1), psi (1),
 // psit (1), bxyz (2)
@@ -715,7 +782,7 @@ static constexpr int XF_PASS = 0x89, XI_PASS = 0xc, XF_FRONT = 0, XI_FRONT = 0x6
 
 template <typename R>
 static int solve_t(const PassFields &f, const FrontFields *fr, double dex, int l, double tol,
-                   int seed, const int *seed_hist)
+                   int seed, const int *seed_hist, const BorderJob &job)
 {
     qp_ctx *c = f.cu->ctx;
     const size_t rp = c->rplane, kp = c->kplane;
@@ -735,7 +802,26 @@ static int solve_t(const PassFields &f, const FrontFields *fr, double dex, int l
     }
     for (int i = 0; i < nf; ++i) x.dst[i] = sk + i * kp;
     // the plasma deposits leave the guard row ny folded into row 0, so zero
-    int rc = xt<R, false>(c, x, nf, fr ? XF_FRONT : XF_PASS, fr ? -1 : c->ny);
+    // (the front's second component is the plasma's charge)
+    BorderArgs<R> bd{};
+    if (job.n) {
+        bd.g = TileGeom{c->nx, c->ny, c->mx1, c->my1, c->ldr};
+        bd.halo = static_cast<const R *>(job.halo);
+        bd.halo_cs = (size_t)c->ntiles * (TILE / job.rb) * band_halo(job.rb);
+        while ((1 << bd.sh) < job.rb) ++bd.sh;
+        bd.fold = job.fold;
+        bd.first = fr ? 1 : 0;
+        bd.n = job.n;
+        for (int k = 0; k < job.n; ++k) {
+            bd.out.p[k] = static_cast<R *>(job.p[k]);
+            bd.out.inner[k] = static_cast<const R *>(job.inner[k]);
+            bd.out.outer[k] = static_cast<const R *>(job.outer[k]);
+            bd.out.p2[k] = static_cast<R *>(job.p2[k]);
+        }
+        bd.out.scale = (R)job.scale;
+        bd.out.scale2 = (R)job.scale2;
+    }
+    int rc = xt<R, false>(c, x, nf, fr ? XF_FRONT : XF_PASS, fr ? -1 : c->ny, bd);
     if (rc) return rc;
     MidArgs<R> a{};
     a.nx = c->nx; a.ldk = c->ldk; a.cs = kp;
@@ -782,10 +868,10 @@ static int solve_t(const PassFields &f, const FrontFields *fr, double dex, int l
 }
 
 // a corrector pass's field solve, from the deposited cu, dcu, amu
-int fused_solve_pass(const PassFields &f, double dex, int l, double tol)
+int fused_solve_pass(const PassFields &f, double dex, int l, double tol, const BorderJob &job)
 {
-    int rc = f.cu->ctx->prec == QP_FP64 ? solve_t<double>(f, nullptr, dex, l, tol, 0, nullptr)
-                                        : solve_t<float>(f, nullptr, dex, l, tol, 0, nullptr);
+    int rc = f.cu->ctx->prec == QP_FP64 ? solve_t<double>(f, nullptr, dex, l, tol, 0, nullptr, job)
+                                        : solve_t<float>(f, nullptr, dex, l, tol, 0, nullptr, job);
     f.cu->state = f.dcu->state = f.amu->state = f.epw->state = 1;
     f.psit->state = f.bxyz->state = 0;
     return rc;
@@ -793,11 +879,11 @@ int fused_solve_pass(const PassFields &f, double dex, int l, double tol)
 
 // the start of a slice, from its beam and plasma charge; seed as fused_pass
 int fused_solve_front(const PassFields &f, const FrontFields &fr, double dex, int seed,
-                      const int *seed_hist)
+                      const int *seed_hist, const BorderJob &job)
 {
     QP_REQUIRE(!seed || fr.ehist, QP_ERR_ARG, "fused_solve_front: seed without history");
-    int rc = f.cu->ctx->prec == QP_FP64 ? solve_t<double>(f, &fr, dex, 0, 0.0, seed, seed_hist)
-                                        : solve_t<float>(f, &fr, dex, 0, 0.0, seed, seed_hist);
+    int rc = f.cu->ctx->prec == QP_FP64 ? solve_t<double>(f, &fr, dex, 0, 0.0, seed, seed_hist, job)
+                                        : solve_t<float>(f, &fr, dex, 0, 0.0, seed, seed_hist, job);
     fr.qb->state = fr.qe->state = f.epwb->state = 1;
     fr.fxy->state = fr.psi->state = f.psit->state = f.bxyz->state = 0;
     return rc;

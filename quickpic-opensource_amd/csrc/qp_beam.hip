@@ -23,9 +23,9 @@ struct qp_beam {
     double qbm, dt;
     int64_t np, npmax;
     qp::DevBuf a[7], b[7];       // x, y, z, px, py, pz, q (double)
-    qp::DevBuf alive, pos, scan_tmp, moments;
+    qp::DevBuf live, sort_tmp, moments;
     qp::DevBuf key[2], perm[2];  // push: cell keys and particle indices, before and after the sort
-    size_t scan_bytes;           // temporary bytes of the scan and the sort
+    size_t sort_bytes;           // temporary bytes of the sort
     int key_shift, key_bits;     // cell key = linear cell index >> key_shift, below 2^key_bits
     unsigned key_drop;           // key of a dropped particle (sorts last)
     qp::DevBuf q3;               // int64 [nz+1][ny+1][ldr]
@@ -288,43 +288,87 @@ static int64_t load_beam_twiss(qp_ctx *c, const qp_beam_twiss_params &bp, uint64
 }
 
 // PGPOST32L (part3d_lib77.f:554-628), int64 fixed-point accumulation.
-// Particles of one wavefront that sit in the same cell on neighbouring lanes
-// (the push leaves the beam sorted by cell) are summed first, in int64 across
-// the wavefront, and the first lane of each such run adds the sums with one
-// atomic per node. Integer sums make the charge the same, bit for bit, as one
-// atomic per particle and node, whatever the particle order.
+// The push leaves the beam sorted by cell.  A thread takes DEP_RUN particles in
+// order and adds them up while they stay in one cell; the last cells of a
+// wavefront's threads, where they are the same on neighbouring lanes, are summed
+// across the wavefront, and the first lane of each such run adds the sums with
+// one atomic per node.  Integer sums make the charge the same, bit for bit, as
+// one atomic per particle and node, whatever the particle order.  (One particle
+// a thread summed each of them across the wavefront, 102 lane exchanges: 96 us
+// for 4 M sorted particles against 46 us, whose positions and charges are read
+// in 27 us at the rate of a copy.)
+constexpr int DEP_RUN = 8;
+
 __global__ __launch_bounds__(256) void k_beam_deposit(
     int64_t np, const double *__restrict__ x, const double *__restrict__ y,
     const double *__restrict__ z, const double *__restrict__ q, unsigned long long *q3, int ld,
     size_t pl, int nx, int ny, int nz)
 {
-    const int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const int64_t j0 = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) * DEP_RUN;
     const int lane = threadIdx.x & 63;
     constexpr unsigned long long NONE = ~0ull;
     unsigned long long cell = NONE;
     long long w[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (j < np) {
-        const double px = x[j], py = y[j], pz = z[j], qm = q[j];
-        // a particle outside the grid has no nodes to deposit to
-        if (px >= 0.0 && px < (double)nx && py >= 0.0 && py < (double)ny && pz >= 0.0 &&
-            pz < (double)nz) {
-            int nn = (int)px, mm = (int)py, ll = (int)pz;
-            double dxp = qm * (px - (double)nn);
-            double dyp = py - (double)mm;
-            double dzp = pz - (double)ll;
-            double amx = qm - dxp;
-            double amy = 1. - dyp;
-            double dx1 = dxp * dyp;
-            dyp = amx * dyp;
-            amx = amx * amy;
-            double amz = 1. - dzp;
-            amy = dxp * amy;
-            cell = (size_t)ll * pl + (size_t)mm * ld + nn;
-            const double f[8] = {amx * amz, amy * amz, dyp * amz, dx1 * amz,
-                                 amx * dzp, amy * dzp, dyp * dzp, dx1 * dzp};
+    const size_t o[8] = {0, 1, (size_t)ld, (size_t)ld + 1, pl, pl + 1, pl + ld, pl + ld + 1};
+    auto flush = [&](unsigned long long to) {
+        unsigned long long *b = q3 + to;
 #pragma unroll
-            for (int k = 0; k < 8; ++k) w[k] = __double2ll_rn(f[k] * BEAM_FIX);
+        for (int k = 0; k < 8; ++k) atomicAdd(b + o[k], (unsigned long long)w[k]);
+    };
+    double px[DEP_RUN], py[DEP_RUN], pz[DEP_RUN], pq[DEP_RUN];
+    if (j0 + DEP_RUN <= np) {
+        // 16 bytes at a time: the arrays are allocations, j0 a multiple of 8
+#pragma unroll
+        for (int r = 0; r < DEP_RUN; r += 2) {
+            const double2 a = *reinterpret_cast<const double2 *>(x + j0 + r);
+            const double2 b = *reinterpret_cast<const double2 *>(y + j0 + r);
+            const double2 c = *reinterpret_cast<const double2 *>(z + j0 + r);
+            const double2 d = *reinterpret_cast<const double2 *>(q + j0 + r);
+            px[r] = a.x; px[r + 1] = a.y;
+            py[r] = b.x; py[r + 1] = b.y;
+            pz[r] = c.x; pz[r + 1] = c.y;
+            pq[r] = d.x; pq[r + 1] = d.y;
         }
+    } else {
+#pragma unroll
+        for (int r = 0; r < DEP_RUN; ++r) {
+            const int64_t j = j0 + r;
+            // a place behind the last particle is outside the grid
+            px[r] = j < np ? x[j] : -1.0;
+            py[r] = j < np ? y[j] : -1.0;
+            pz[r] = j < np ? z[j] : -1.0;
+            pq[r] = j < np ? q[j] : 0.0;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < DEP_RUN; ++r) {
+        // a particle outside the grid has no nodes to deposit to
+        if (!(px[r] >= 0.0 && px[r] < (double)nx && py[r] >= 0.0 && py[r] < (double)ny &&
+              pz[r] >= 0.0 && pz[r] < (double)nz))
+            continue;
+        const double qm = pq[r];
+        const int nn = (int)px[r], mm = (int)py[r], ll = (int)pz[r];
+        double dxp = qm * (px[r] - (double)nn);
+        double dyp = py[r] - (double)mm;
+        double dzp = pz[r] - (double)ll;
+        double amx = qm - dxp;
+        double amy = 1. - dyp;
+        double dx1 = dxp * dyp;
+        dyp = amx * dyp;
+        amx = amx * amy;
+        double amz = 1. - dzp;
+        amy = dxp * amy;
+        const unsigned long long c = (size_t)ll * pl + (size_t)mm * ld + nn;
+        if (c != cell) {
+            if (cell != NONE) flush(cell);
+            cell = c;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) w[k] = 0;
+        }
+        const double f[8] = {amx * amz, amy * amz, dyp * amz, dx1 * amz,
+                             amx * dzp, amy * dzp, dyp * dzp, dx1 * dzp};
+#pragma unroll
+        for (int k = 0; k < 8; ++k) w[k] += __double2ll_rn(f[k] * BEAM_FIX);
     }
     // a run of equal cells starts where the lane before holds another cell
     const unsigned long long prev = __shfl_up(cell, 1, 64);
@@ -340,16 +384,13 @@ __global__ __launch_bounds__(256) void k_beam_deposit(
             const bool take = lane + d < 64 && orun == run;
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
-                const long long o = __shfl_down(w[k], d, 64);
-                if (take) w[k] += o;
+                const long long v = __shfl_down(w[k], d, 64);
+                if (take) w[k] += v;
             }
         }
     }
     if (!head || cell == NONE) return;
-    unsigned long long *b = q3 + cell;
-    const size_t o[8] = {0, 1, (size_t)ld, (size_t)ld + 1, pl, pl + 1, pl + ld, pl + ld + 1};
-#pragma unroll
-    for (int k = 0; k < 8; ++k) atomicAdd(b + o[k], (unsigned long long)w[k]);
+    flush(cell);
 }
 
 // qdpcopy / copyadd of one xi plane (ufield3d_class.f03:460-490) from the
@@ -388,25 +429,29 @@ struct CellKey {
     }
 };
 
-// PGBPUSH32L_QP (part3d_lib77.f:630-786) with ipbc = 1 and cofd = 0; flags
-// the particles that leave [1, n-1) in any direction, and writes each
-// particle's sort key (its new cell) with its index beside it.
+struct Ptr7 {
+    double *p[7];
+};
+
+// PGBPUSH32L_QP (part3d_lib77.f:630-786) with ipbc = 1 and cofd = 0; stores
+// each particle's sort key beside it: its new cell, or `drop` for the particles
+// that leave [1, n-1) in any direction.  87 us for 4 M particles, its bytes at
+// the rate of a copy, as k_permute's 93 us.  (Storing only the keys here and
+// pushing again while permuting moves a quarter less memory, but the second
+// kernel's scattered reads have fewer waves: 58 + 117 us, a step no shorter.)
 template <typename R>
-__global__ void k_beam_push(int64_t np, double *x, double *y, double *z, double *px, double *py,
-                            double *pz, const R *__restrict__ e3, const R *__restrict__ b3,
-                            size_t vol, int ld, size_t pl, double qtmh, double dtcx, double dtcz,
-                            double rx, double ry, double rz, int *alive, CellKey ck,
-                            unsigned *key, unsigned *idx)
+__global__ void k_beam_push(int64_t np, Ptr7 a, const R *__restrict__ e3,
+                            const R *__restrict__ b3, size_t vol, int ld, size_t pl, double qtmh,
+                            double dtcx, double dtcz, double rx, double ry, double rz, CellKey ck,
+                            unsigned *key)
 {
-    int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (j >= np) return;
-    idx[j] = (unsigned)j;
-    double X = x[j], Y = y[j], Z = z[j];
+    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (i >= np) return;
+    double X = a.p[0][i], Y = a.p[1][i], Z = a.p[2][i];
     // outside the grid nothing can be gathered: dropped without touching the
     // fields (the loader and the push keep every particle in [1, n-1))
     if (!(X >= 0.0 && X < rx + 1.0 && Y >= 0.0 && Y < ry + 1.0 && Z >= 0.0 && Z < rz + 1.0)) {
-        alive[j] = 0;
-        key[j] = ck.drop;
+        key[i] = ck.drop;
         return;
     }
     int nn = (int)X, mm = (int)Y, ll = (int)Z;
@@ -430,37 +475,49 @@ __global__ void k_beam_push(int64_t np, double *x, double *y, double *z, double 
     dx = dx - oy;
     dy = dy + ox;
     double delx = qtmh * dx, dely = qtmh * dy, delz = qtmh * dz;
-    dx = px[j] + delx;
-    dy = py[j] + dely;
-    dz = pz[j] + delz;
+    dx = a.p[3][i] + delx;
+    dy = a.p[4][i] + dely;
+    dz = a.p[5][i] + delz;
     double p2t = dx * dx + dy * dy;
     double p2 = p2t + dz * dz;
     double ngamma = sqrt(1.0 + p2);
     double dtg = dtcx / ngamma;
     double omvz = (1.0 + p2t) / (dz * (dz + ngamma));
-    px[j] = dx;
-    py[j] = dy;
-    pz[j] = dz;
+    a.p[3][i] = dx;
+    a.p[4][i] = dy;
+    a.p[5][i] = dz;
     double nxp = X + dx * dtg, nyp = Y + dy * dtg, nzp = Z + omvz * dtcz;
     bool live = !((nxp < 1.0) || (nxp >= rx) || (nyp < 1.0) || (nyp >= ry) || (nzp < 1.0) ||
                   (nzp >= rz));
-    if (live) { x[j] = nxp; y[j] = nyp; z[j] = nzp; }
-    alive[j] = live ? 1 : 0;
-    key[j] = live ? ck.of(nxp, nyp, nzp) : ck.drop;
+    if (live) {
+        a.p[0][i] = nxp;
+        a.p[1][i] = nyp;
+        a.p[2][i] = nzp;
+    }
+    key[i] = live ? ck.of(nxp, nyp, nzp) : ck.drop;
 }
 
-struct Ptr7 {
-    double *p[7];
-};
-
-// survivor i of the cell-sorted beam is particle perm[i] (i < *nlive)
-__global__ void k_permute(int64_t np, const int *nlive, const unsigned *perm, Ptr7 src, Ptr7 dst)
+// Survivor i of the cell-sorted beam is particle perm[i].  Thread i also finds
+// the number of survivors, where the sorted keys turn to `drop` (a flag per
+// particle and their scan took 30 us of 4 M particles, and the host waited for
+// it before the sort).
+__global__ void k_permute(int64_t np, const unsigned *__restrict__ key, unsigned drop,
+                          const unsigned *__restrict__ perm, Ptr7 src, Ptr7 dst, int *nlive)
 {
-    int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= np || i >= *nlive) return;
+    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (i >= np) return;
+    const bool gone = key[i] == drop;
+    if (gone ? i == 0 : i + 1 == np || key[i + 1] == drop) *nlive = gone ? 0 : (int)(i + 1);
+    if (gone) return;
     const unsigned s = perm[i];
 #pragma unroll
     for (int k = 0; k < 7; ++k) dst.p[k][i] = src.p[k][s];
+}
+
+__global__ void k_iota(unsigned *p, int64_t n)
+{
+    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (i < n) p[i] = (unsigned)i;
 }
 
 __global__ void k_beam_moments(int64_t np, const double *px, const double *py, const double *pz,
@@ -503,8 +560,7 @@ static int beam_alloc(qp_beam *b, int64_t n)
         if (!rc) rc = b->b[k].alloc((size_t)n * 8);
         if (rc) return rc;
     }
-    int rc = b->alive.alloc((size_t)(n + 1) * 4);
-    if (!rc) rc = b->pos.alloc((size_t)(n + 1) * 4);
+    int rc = b->live.alloc(sizeof(int));
     for (int k = 0; k < 2 && !rc; ++k) {
         rc = b->key[k].alloc((size_t)(n + 1) * 4);
         if (!rc) rc = b->perm[k].alloc((size_t)(n + 1) * 4);
@@ -519,15 +575,16 @@ static int beam_alloc(qp_beam *b, int64_t n)
     b->key_drop = (unsigned)(((ncell - 1) >> b->key_shift) + 1);
     b->key_bits = 1;
     while (b->key_bits < 32 && (b->key_drop >> b->key_bits) != 0) ++b->key_bits;
-    size_t scan = 0, sort = 0;
-    QP_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, scan, b->alive.as<int>(), b->pos.as<int>(),
-                                            (int)(n + 1), c->stream));
-    QP_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, sort, b->key[0].as<unsigned>(),
+    // the places before the sort, which leaves them as they are
+    hipLaunchKernelGGL(k_iota, dim3((unsigned)((n + 256) / 256)), dim3(256), 0, c->stream,
+                       b->perm[0].as<unsigned>(), n + 1);
+    QP_LAUNCH_CHECK();
+    b->sort_bytes = 0;
+    QP_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, b->sort_bytes, b->key[0].as<unsigned>(),
                                               b->key[1].as<unsigned>(), b->perm[0].as<unsigned>(),
                                               b->perm[1].as<unsigned>(), (int)n, 0, b->key_bits,
                                               c->stream));
-    b->scan_bytes = std::max(scan, sort);
-    return b->scan_tmp.alloc(b->scan_bytes + 256);
+    return b->sort_tmp.alloc(b->sort_bytes + 256);
 }
 
 static int beam_set(qp_beam *b, std::vector<double> (&h)[7], int64_t n)
@@ -757,7 +814,7 @@ int qp_beam_destroy(qp_beam *b)
     if (!b) return QP_OK;
     if (b->ctx) (void)hipStreamSynchronize(b->ctx->stream);
     for (int k = 0; k < 7; ++k) { b->a[k].release(); b->b[k].release(); }
-    b->alive.release(); b->pos.release(); b->scan_tmp.release(); b->moments.release();
+    b->live.release(); b->sort_tmp.release(); b->moments.release();
     for (int k = 0; k < 2; ++k) { b->key[k].release(); b->perm[k].release(); }
     b->q3.release();
     delete b;
@@ -774,7 +831,8 @@ int qp_beam_qdp(qp_beam *b)
     if (b->np > 0) {
         {
         ProfScope _ps(c, QP_PROF_BEAM_DEPOSIT, 4.0 * 8.0 * (double)b->np);
-        hipLaunchKernelGGL(k_beam_deposit, dim3((unsigned)((b->np + 255) / 256)), dim3(256), 0,
+        const int64_t per = 256 * DEP_RUN;
+        hipLaunchKernelGGL(k_beam_deposit, dim3((unsigned)((b->np + per - 1) / per)), dim3(256), 0,
                            c->stream, b->np, b->a[0].as<double>(), b->a[1].as<double>(),
                            b->a[2].as<double>(), b->a[6].as<double>(),
                            b->q3.as<unsigned long long>(), c->ldr, c->rplane, c->nx, c->ny,
@@ -855,24 +913,19 @@ int qp_beam_push(qp_beam *b, const qp_field3d *ef, const qp_field3d *bf, double 
     dim3 grid((unsigned)((np + 255) / 256));
     const double qtmh = b->qbm * b->dt, dtcx = b->dt / dex, dtcz = b->dt / dez;
     const CellKey ck{c->nx, c->ny, b->key_shift, b->key_drop};
+    Ptr7 src, dst;
+    for (int k = 0; k < 7; ++k) { src.p[k] = b->a[k].as<double>(); dst.p[k] = b->b[k].as<double>(); }
+    unsigned *key = b->key[0].as<unsigned>(), *sorted = b->key[1].as<unsigned>();
+    auto push = [&](auto kern, auto zero) {
+        using R = decltype(zero);
+        hipLaunchKernelGGL(kern, grid, dim3(256), 0, c->stream, np, src, ef->buf.as<R>(),
+                           bf->buf.as<R>(), vol, c->ldr, c->rplane, qtmh, dtcx, dtcz,
+                           (double)(c->nx - 1), (double)(c->ny - 1), (double)(c->nz - 1), ck, key);
+    };
     {
-    ProfScope _ps(c, QP_PROF_BEAM_PUSH, (12.0 * 8.0 + 12.0) * (double)np);   // 6 read, 6 written, flag, key, index
-    if (c->prec == QP_FP64)
-        hipLaunchKernelGGL(k_beam_push<double>, grid, dim3(256), 0, c->stream, np,
-                           b->a[0].as<double>(), b->a[1].as<double>(), b->a[2].as<double>(),
-                           b->a[3].as<double>(), b->a[4].as<double>(), b->a[5].as<double>(),
-                           ef->buf.as<double>(), bf->buf.as<double>(), vol, c->ldr, c->rplane,
-                           qtmh, dtcx, dtcz, (double)(c->nx - 1), (double)(c->ny - 1),
-                           (double)(c->nz - 1), b->alive.as<int>(), ck, b->key[0].as<unsigned>(),
-                           b->perm[0].as<unsigned>());
-    else
-        hipLaunchKernelGGL(k_beam_push<float>, grid, dim3(256), 0, c->stream, np,
-                           b->a[0].as<double>(), b->a[1].as<double>(), b->a[2].as<double>(),
-                           b->a[3].as<double>(), b->a[4].as<double>(), b->a[5].as<double>(),
-                           ef->buf.as<float>(), bf->buf.as<float>(), vol, c->ldr, c->rplane,
-                           qtmh, dtcx, dtcz, (double)(c->nx - 1), (double)(c->ny - 1),
-                           (double)(c->nz - 1), b->alive.as<int>(), ck, b->key[0].as<unsigned>(),
-                           b->perm[0].as<unsigned>());
+    ProfScope _ps(c, QP_PROF_BEAM_PUSH, (12.0 * 8.0 + 4.0) * (double)np);   // 6 read, 6 written, key
+    if (c->prec == QP_FP64) push(k_beam_push<double>, 0.0);
+    else push(k_beam_push<float>, 0.0f);
     }
     QP_LAUNCH_CHECK();
     // The survivors, sorted by cell (a stable sort: equal cells keep their
@@ -880,35 +933,27 @@ int qp_beam_push(qp_beam *b, const qp_field3d *ef, const qp_field3d *bf, double 
     // instead moves the last particle into each hole (part3d_lib77.f:748-776);
     // the survivor set is the same, and the order is the one the gathers of
     // the next push and the atomics of the next charge deposit want.
-    QP_HIP(hipMemsetAsync(b->alive.as<int>() + np, 0, sizeof(int), c->stream));
-    size_t tb = b->scan_bytes;
-    QP_HIP(hipcub::DeviceScan::ExclusiveSum(b->scan_tmp.p, tb, b->alive.as<int>(),
-                                            b->pos.as<int>(), (int)(np + 1), c->stream));
-    int live = 0;
-    QP_HIP(hipMemcpyAsync(&live, b->pos.as<int>() + np, sizeof(int), hipMemcpyDeviceToHost,
-                          c->stream));
     {
     ProfScope _ps(c, QP_PROF_BEAM_PUSH, 16.0 * (double)np);   // keys and indices read and written once
     size_t need = 0;
-    QP_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, need, b->key[0].as<unsigned>(),
-                                              b->key[1].as<unsigned>(), b->perm[0].as<unsigned>(),
-                                              b->perm[1].as<unsigned>(), (int)np, 0, b->key_bits,
-                                              c->stream));
-    QP_REQUIRE(need <= b->scan_bytes, QP_ERR_ALLOC, "beam push: sort needs %zu bytes, %zu held",
-               need, b->scan_bytes);
-    QP_HIP(hipcub::DeviceRadixSort::SortPairs(b->scan_tmp.p, need, b->key[0].as<unsigned>(),
-                                              b->key[1].as<unsigned>(), b->perm[0].as<unsigned>(),
-                                              b->perm[1].as<unsigned>(), (int)np, 0, b->key_bits,
-                                              c->stream));
+    QP_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, need, key, sorted,
+                                              b->perm[0].as<unsigned>(), b->perm[1].as<unsigned>(),
+                                              (int)np, 0, b->key_bits, c->stream));
+    QP_REQUIRE(need <= b->sort_bytes, QP_ERR_ALLOC, "beam push: sort needs %zu bytes, %zu held",
+               need, b->sort_bytes);
+    QP_HIP(hipcub::DeviceRadixSort::SortPairs(b->sort_tmp.p, need, key, sorted,
+                                              b->perm[0].as<unsigned>(), b->perm[1].as<unsigned>(),
+                                              (int)np, 0, b->key_bits, c->stream));
     }
-    Ptr7 src, dst;
-    for (int k = 0; k < 7; ++k) { src.p[k] = b->a[k].as<double>(); dst.p[k] = b->b[k].as<double>(); }
     {
-    ProfScope _ps(c, QP_PROF_BEAM_PUSH, (7.0 * 8.0 * 2.0 + 4.0) * (double)np);
-    hipLaunchKernelGGL(k_permute, grid, dim3(256), 0, c->stream, np, b->pos.as<int>() + np,
-                       b->perm[1].as<unsigned>(), src, dst);
+    // key and place read, 7 read and written
+    ProfScope _ps(c, QP_PROF_BEAM_PUSH, (7.0 * 8.0 * 2.0 + 8.0) * (double)np);
+    hipLaunchKernelGGL(k_permute, grid, dim3(256), 0, c->stream, np, sorted, b->key_drop,
+                       b->perm[1].as<unsigned>(), src, dst, b->live.as<int>());
     }
     QP_LAUNCH_CHECK();
+    int live = 0;
+    QP_HIP(hipMemcpyAsync(&live, b->live.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     QP_HIP(hipStreamSynchronize(c->stream));
     for (int k = 0; k < 7; ++k) std::swap(b->a[k], b->b[k]);
     b->np = live;

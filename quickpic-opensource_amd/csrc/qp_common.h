@@ -305,6 +305,10 @@ struct FrontFields {
 };
 bool fused_fields(const qp_ctx *c);
 bool fused_border(const qp_ctx *c);
+// x transforms of nc planes, between rows y (pitch ldr) and columns y (planes
+// [kx][y], pitch ldk); types: bit i for a cosine transform of plane i
+int fft_x_to_columns(qp_ctx *c, float *const *src, float *const *dst, int nc, int types);
+int fft_x_from_columns(qp_ctx *c, float *const *src, float *const *dst, int nc, int types);
 int fused_solve_pass(const PassFields &f, double dex, int l, double tol, const BorderJob &job);
 int fused_solve_front(const PassFields &f, const FrontFields &fr, double dex, int seed,
                       const int *seed_hist, const BorderJob &job);

@@ -335,6 +335,17 @@ static int k2r_core(qp_ctx *c, R *const *rs, R *const *ks, int nc, int mx, int m
     return rc;
 }
 
+// Whether the x pass of nc components reads or writes the columns that the y pass
+// works on (k_fft_xt), two launches in place of three.  FP32, up to nx, ny = 1024:
+// both directions 64 x 32 19.5 -> 13.7 us, 256^2 22.5 -> 18.0, 1024^2 37 to 59
+// -> 33 to 54 us (1 to 3 components); one component at nx = 512 gives its blocks
+// of 16 rows too few to hide each other's waits (512 x 256 23.6 -> 24.3).  FP64's
+// column pairs take two launches already (256^2 19 against 22 us so).
+static bool x_columns(const qp_ctx *c, int nc)
+{
+    return c->prec == QP_FP32 && fused_fields(c) && (nc > 1 || c->nx != 512);
+}
+
 template <typename R>
 static int r2k_t(qp_ctx *c, qp_field2d *const *fs, const int *kinds, int nf)
 {
@@ -342,6 +353,16 @@ static int r2k_t(qp_ctx *c, qp_field2d *const *fs, const int *kinds, int nf)
     int mx, my;
     const int nc = gather_comps<R>(fs, kinds, nf, rs, ks, &mx, &my);
     if (nc <= 0) return nc;
+    if constexpr (std::is_same<R, float>::value) {
+        if (x_columns(c, nc)) {
+            CompSet<R> y{};
+            for (int i = 0; i < nc; ++i) y.src[i] = y.dst[i] = ks[i];
+            int rc = fft_x_to_columns(c, rs, ks, nc, mx);
+            return rc ? rc
+                      : rowfft0<R>(c, y, nc, c->nx + 1, c->ny, c->ldk, c->ldk, my, 1.0,
+                                   c->twy.as<cplx<R>>(), -1);
+        }
+    }
     return r2k_core<R>(c, rs, ks, nc, mx, my, c->scr_r.as<R>(), c->ldr, c->ldk,
                        c->twx.as<cplx<R>>(), c->twy.as<cplx<R>>());
 }
@@ -353,6 +374,20 @@ static int k2r_t(qp_ctx *c, qp_field2d *const *fs, const int *kinds, int nf)
     int mx, my;
     const int nc = gather_comps<R>(fs, kinds, nf, rs, ks, &mx, &my);
     if (nc <= 0) return nc;
+    if constexpr (std::is_same<R, float>::value) {
+        if (x_columns(c, nc)) {
+            R *sk[MAX_BATCH];
+            CompSet<R> y{};
+            for (int i = 0; i < nc; ++i) {
+                sk[i] = c->scr_k.as<R>() + i * (size_t)(c->nx + 1) * c->ldk;
+                y.src[i] = ks[i];
+                y.dst[i] = sk[i];
+            }
+            int rc = rowfft0<R>(c, y, nc, c->nx + 1, c->ny, c->ldk, c->ldk, my, 2.0,
+                                c->twy.as<cplx<R>>(), -1);
+            return rc ? rc : fft_x_from_columns(c, sk, rs, nc, mx);
+        }
+    }
     return k2r_core<R>(c, rs, ks, nc, mx, my, c->scr_k.as<R>(), c->ldr, c->ldk,
                        c->twx.as<cplx<R>>(), c->twy.as<cplx<R>>());
 }

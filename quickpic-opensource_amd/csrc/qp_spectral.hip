@@ -889,4 +889,24 @@ int fused_solve_front(const PassFields &f, const FrontFields &fr, double dex, in
     return rc;
 }
 
+// the x passes of the transforms of whole fields (qp_fft.hip)
+template <bool INV>
+static int x_pass(qp_ctx *c, float *const *src, float *const *dst, int nc, int types)
+{
+    XtSet<float> s{};
+    for (int i = 0; i < nc; ++i) {
+        s.src[i] = src[i];
+        s.dst[i] = dst[i];
+    }
+    return xt<float, INV>(c, s, nc, types, -1);
+}
+int fft_x_to_columns(qp_ctx *c, float *const *src, float *const *dst, int nc, int types)
+{
+    return x_pass<false>(c, src, dst, nc, types);
+}
+int fft_x_from_columns(qp_ctx *c, float *const *src, float *const *dst, int nc, int types)
+{
+    return x_pass<true>(c, src, dst, nc, types);
+}
+
 }  // namespace qp

@@ -2071,6 +2071,58 @@ static int amjdp_out(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
 }
 
 // the species' own cu, dcu, amu (overwritten)
+// qdp_species2d with the slice's additions fused into the deposit
+// (species2d_class.f03:166-185): this%q = deposit; q = this%q + q;
+// q = qn + q.  first: q holds nothing yet (the slice loop zeroed it).  bp: the
+// beam plane to convert beside it (or null); halo: the tile-border buffer
+// (null: the context's).
+template <typename R>
+static int qdp_fused_t(qp_species *sp, qp_field2d *q, bool first, const BeamPlane *bp,
+                       BorderJob *job, void *halo)
+{
+    R *qp = q->rs.as<R>();
+    DepOut<R> o{};
+    o.p[0] = qp;
+    o.inner[0] = first ? nullptr : qp;
+    o.outer[0] = sp->qn->rs.as<R>();
+    o.p2[0] = sp->q->rs.as<R>();
+    o.scale = o.scale2 = R(1);
+    int rc = deposit_q_out<R>(sp, o, static_cast<R *>(halo), bp, job);
+    if (rc) return rc;
+    sp->q->state = 0;
+    sp->q->gcells = 1;
+    q->state = 0;
+    return QP_OK;
+}
+
+// amjdp_species2d plus the slice loop's scaling (species2d_class.f03:187-218,
+// simulation_class.f03:682-685): cu = this%cu + cu (likewise dcu, amu),
+// this%cu *= dex, and after the last species cu, amu, dcu *= dex.  Of the
+// species' own planes only this%cu(3) is kept (its one later reader, cbq).
+template <typename R>
+static int amjdp_fused_t(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
+                         const qp_field2d *psit, qp_field2d *cu, qp_field2d *dcu,
+                         qp_field2d *amu, double dex, bool first, bool last,
+                         const qp_field2d *psi, BorderJob *job)
+{
+    const size_t pl = sp->ctx->rplane;
+    R *c = cu->rs.as<R>(), *d = dcu->rs.as<R>(), *a = amu->rs.as<R>();
+    R *planes[8] = {c, c + pl, c + 2 * pl, d, d + pl, a, a + pl, a + 2 * pl};
+    DepOut<R> o{};
+    for (int k = 0; k < 8; ++k) {
+        o.p[k] = planes[k];
+        o.inner[k] = first ? nullptr : planes[k];
+    }
+    o.p2[2] = sp->cu->rs.as<R>() + 2 * pl;
+    o.scale = last ? (R)dex : R(1);
+    o.scale2 = (R)dex;
+    int rc = amjdp_out<R>(sp, ef, bf, psit, dex, o, psi, job);
+    sp->cu->state = 0;
+    cu->state = dcu->state = amu->state = 0;
+    return rc;
+}
+
+// amjdp_species2d's deposit (species2d_class.f03:187-218) into the species' planes
 template <typename R>
 static int amjdp_t(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
                    const qp_field2d *psit, double dex)
@@ -2081,6 +2133,27 @@ static int amjdp_t(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
     int rc = amjdp_out<R>(sp, ef, bf, psit, dex, dep_plain<R>(planes, 8));
     sp->cu->state = sp->dcu->state = sp->amu->state = 0;
     return rc;
+}
+
+// amjdp_species2d's deposit and additions in one: this%cu = deposit * dex, and
+// cu = deposit + cu, dcu and amu likewise (species2d_class.f03:187-218)
+template <typename R>
+static int amjdp_add_t(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
+                       const qp_field2d *psit, qp_field2d *cu, qp_field2d *dcu, qp_field2d *amu,
+                       double dex)
+{
+    const size_t pl = sp->ctx->rplane;
+    R *c = cu->rs.as<R>(), *d = dcu->rs.as<R>(), *a = amu->rs.as<R>();
+    R *planes[8] = {c, c + pl, c + 2 * pl, d, d + pl, a, a + pl, a + 2 * pl};
+    DepOut<R> o = dep_plain<R>(planes, 8);
+    for (int k = 0; k < 8; ++k) o.inner[k] = planes[k];
+    for (int k = 0; k < 3; ++k) o.p2[k] = sp->cu->rs.as<R>() + k * pl;
+    o.scale2 = (R)dex;
+    int rc = amjdp_out<R>(sp, ef, bf, psit, dex, o);
+    if (rc) return rc;
+    sp->cu->state = 0;
+    for (qp_field2d *f : {cu, dcu, amu}) f->gcells = sp->cu->gcells;
+    return QP_OK;
 }
 
 template <typename R>
@@ -2288,14 +2361,8 @@ int qp_species_qdp(qp_species *sp, qp_field2d *q)
 {
     SPCHECK(sp);
     QP_REQUIRE(q && q->dim == 1 && q->state == 0, QP_ERR_STATE, "qdp: q must be real space, dim 1");
-    qp_ctx *c = sp->ctx;
-    int rc = c->prec == QP_FP64 ? deposit_q_t<double>(sp, sp->q->rs.as<double>())
-                                : deposit_q_t<float>(sp, sp->q->rs.as<float>());
-    if (rc) return rc;
-    sp->q->state = 0;
-    sp->q->gcells = 1;
-    rc = qp_field2d_add(q, sp->q, q, 0, nullptr, nullptr, nullptr);
-    if (!rc) rc = qp_field2d_add(q, sp->qn, q, 0, nullptr, nullptr, nullptr);
+    int rc = DISPATCH(sp->ctx, qdp_fused_t, sp, q, false, nullptr, nullptr, nullptr);
+    if (!rc) q->gcells = sp->qn->gcells;
     return rc;
 }
 
@@ -2319,14 +2386,8 @@ int qp_species_qdp_noalloc(qp_species *sp, qp_field2d *q)
     void *halo = qp::noalloc_scratch(c->device);
     QP_REQUIRE(halo, QP_ERR_UNSUPPORTED, "qdp_noalloc: no scratch address for device %d",
                c->device);
-    int rc = c->prec == QP_FP64
-                 ? deposit_q_t<double>(sp, sp->q->rs.as<double>(), static_cast<double *>(halo))
-                 : deposit_q_t<float>(sp, sp->q->rs.as<float>(), static_cast<float *>(halo));
-    if (rc) return rc;
-    sp->q->state = 0;
-    sp->q->gcells = 1;
-    rc = qp_field2d_add(q, sp->q, q, 0, nullptr, nullptr, nullptr);
-    if (!rc) rc = qp_field2d_add(q, sp->qn, q, 0, nullptr, nullptr, nullptr);
+    int rc = DISPATCH(c, qdp_fused_t, sp, q, false, nullptr, nullptr, halo);
+    if (!rc) q->gcells = sp->qn->gcells;
     return rc;
 }
 
@@ -2348,6 +2409,15 @@ int qp_species_amjdp(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
                "amjdp: fields must be real space");
     QP_REQUIRE(ef->dim >= 2 && bf->dim == 3 && cu->dim == 3 && dcu->dim >= 2 && amu->dim == 3,
                QP_ERR_ARG, "amjdp: component counts");
+    QP_REQUIRE(cu->state == 0 && dcu->state == 0 && amu->state == 0, QP_ERR_STATE,
+               "field op: states are different");
+    QP_REQUIRE(dcu->dim == 2, QP_ERR_ARG, "field op: dim mismatch");
+    // The additions go with the deposit's stores (four launches less).  Fields that
+    // are also inputs of the deposit, or given twice, are added to behind it.
+    const qp_field2d *out[3] = {cu, dcu, amu};
+    bool apart = cu != dcu && cu != amu && dcu != amu;
+    for (const qp_field2d *f : out) apart = apart && f != ef && f != bf && f != psit;
+    if (apart) return DISPATCH(sp->ctx, amjdp_add_t, sp, ef, bf, psit, cu, dcu, amu, dex);
     int rc = DISPATCH(sp->ctx, amjdp_t, sp, ef, bf, psit, dex);
     if (!rc) rc = qp_field2d_add(cu, sp->cu, cu, 0, nullptr, nullptr, nullptr);
     if (!rc) rc = qp_field2d_add(dcu, sp->dcu, dcu, 0, nullptr, nullptr, nullptr);
@@ -2618,59 +2688,10 @@ int species_check_poll(qp_species *sp, bool wait)
     return QP_ERR_CHECK;
 }
 
-// qdp_species2d with the slice's additions fused into the deposit
-// (species2d_class.f03:166-185): this%q = deposit; q = this%q + q;
-// q = qn + q.  first: q holds nothing yet (the slice loop zeroed it).  bp: the
-// beam plane to convert beside it (or null).
-template <typename R>
-static int qdp_fused_t(qp_species *sp, qp_field2d *q, bool first, const BeamPlane *bp,
-                       BorderJob *job)
-{
-    R *qp = q->rs.as<R>();
-    DepOut<R> o{};
-    o.p[0] = qp;
-    o.inner[0] = first ? nullptr : qp;
-    o.outer[0] = sp->qn->rs.as<R>();
-    o.p2[0] = sp->q->rs.as<R>();
-    o.scale = o.scale2 = R(1);
-    int rc = deposit_q_out<R>(sp, o, nullptr, bp, job);
-    sp->q->state = 0;
-    sp->q->gcells = 1;
-    q->state = 0;
-    return rc;
-}
-
 int species_qdp_fused(qp_species *sp, qp_field2d *q, bool first, const BeamPlane *bp,
                       BorderJob *job)
 {
-    return DISPATCH(sp->ctx, qdp_fused_t, sp, q, first, bp, job);
-}
-
-// amjdp_species2d plus the slice loop's scaling (species2d_class.f03:187-218,
-// simulation_class.f03:682-685): cu = this%cu + cu (likewise dcu, amu),
-// this%cu *= dex, and after the last species cu, amu, dcu *= dex.  Of the
-// species' own planes only this%cu(3) is kept (its one later reader, cbq).
-template <typename R>
-static int amjdp_fused_t(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
-                         const qp_field2d *psit, qp_field2d *cu, qp_field2d *dcu,
-                         qp_field2d *amu, double dex, bool first, bool last,
-                         const qp_field2d *psi, BorderJob *job)
-{
-    const size_t pl = sp->ctx->rplane;
-    R *c = cu->rs.as<R>(), *d = dcu->rs.as<R>(), *a = amu->rs.as<R>();
-    R *planes[8] = {c, c + pl, c + 2 * pl, d, d + pl, a, a + pl, a + 2 * pl};
-    DepOut<R> o{};
-    for (int k = 0; k < 8; ++k) {
-        o.p[k] = planes[k];
-        o.inner[k] = first ? nullptr : planes[k];
-    }
-    o.p2[2] = sp->cu->rs.as<R>() + 2 * pl;
-    o.scale = last ? (R)dex : R(1);
-    o.scale2 = (R)dex;
-    int rc = amjdp_out<R>(sp, ef, bf, psit, dex, o, psi, job);
-    sp->cu->state = 0;
-    cu->state = dcu->state = amu->state = 0;
-    return rc;
+    return DISPATCH(sp->ctx, qdp_fused_t, sp, q, first, bp, job, nullptr);
 }
 
 int species_amjdp_fused(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,

@@ -45,15 +45,18 @@ template <typename R> struct alignas(16) Quad {
 };
 
 // Shape of k_fft_xt: FB row pairs per workgroup, so that the transposed side
-// moves 2 FB Reals (32 to 64 bytes) of a column at a time, within 80 KB of LDS
-// (two workgroups per CU) and 1024 threads.
+// moves 2 FB Reals (16 to 64 bytes) of a column at a time; workgroups next to
+// each other complete its cache lines in one L2.  Small ones: their waits at
+// barriers cover each other.  512^2 FP32, forward and inverse: 16 rows (1024
+// threads) 11.8 and 8.9 us, 8 rows 10.1 and 7.2; 1024^2 8 rows 27.4 and 17.4,
+// 4 rows 26.9 and 17.1; 128^2 FP64 16 rows 8.4 and 5.2, 8 rows 7.6 and 5.0.
 template <typename R, int L> struct XtShape {
     static constexpr int PS = pad_shift<R>();
     using S = FftShape<L, PS>;
-    static constexpr int FB = S::TF == 4 ? 16   // one whole wave
-                              : S::TF * 8 <= 1024 && 8 * S::LDSM * 2 * sizeof(R) <= 81920 ? 8
-                              : S::TF * 4 <= 1024 && 4 * S::LDSM * 2 * sizeof(R) <= 81920 ? 4
-                                                                                          : 2;
+    static constexpr int FB = S::TF == 4         ? 16   // one whole wave
+                              : S::TF * 8 <= 128 ? 8
+                              : S::TF * 4 <= 512 ? 4
+                                                 : 2;
     static constexpr int BS = FB * S::TF;
     static constexpr int ROWS = 2 * FB;        // rows per workgroup
     static constexpr int SW = ROWS + 2;        // row pitch of the staging area
@@ -61,14 +64,15 @@ template <typename R, int L> struct XtShape {
     static constexpr int CH = ROWS / V;        // accesses per column piece
     static constexpr size_t LDS = (size_t)FB * S::LDSM * sizeof(cplx<R>);
     static_assert((size_t)(S::N + 1) * SW * sizeof(R) <= LDS, "staging fits the FFT's area");
+    static_assert(LDS <= 81920, "two workgroups on a CU");
 };
 
 // Up to this nx the forward x transforms form the border sums of the deposit in
-// front of them (a launch less).  With the launches: 128^2 FP64 4.4 + 5.1 us
-// against 8.3 in one, 256 x 512 FP32 5.4 + 6.2 against 10.2; but 512^2 FP32
-// 5.4 + 11.7 against 19.3, and 1024^2 11.7 + 27.4 against 48.9: there the blocks
+// front of them (a launch less).  The two launches against the one: 128^2 FP64
+// 4.4 + 4.9 us, 7.6; 256 x 512 FP32 5.4 + 6.0, 8.9; 512^2 FP32 5.4 + 10.1, 14.0;
+// but 1024^2 11.7 + 26.9, 39.6, and in FP64 14.2 + 39.8, 58.3: there the blocks
 // of whole border rows wait longer than a kernel of their own does.
-constexpr int BORDER_MAX = 256;
+constexpr int BORDER_MAX = 512;
 
 // x transforms of the rows of every component of the batch (grid.y).  INV =
 // false: rows y of src (pitch ld_src) to columns y of dst ([kx][y], pitch

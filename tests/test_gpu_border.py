@@ -1,4 +1,4 @@
-"""Border sums formed by the x transforms (nx <= 256) against the deposit's own
+"""Border sums formed by the x transforms (nx <= 512) against the deposit's own
 border kernel (the separate transforms), which the other tests hold to the
 oracle: the deposited planes themselves, with one and two species, tiles in
 four, two and one band, in grids whose last x-transform block holds only the

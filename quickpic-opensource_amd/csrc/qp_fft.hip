@@ -335,15 +335,17 @@ static int k2r_core(qp_ctx *c, R *const *rs, R *const *ks, int nc, int mx, int m
     return rc;
 }
 
-// Whether the x pass of nc components reads or writes the columns that the y pass
-// works on (k_fft_xt), two launches in place of three.  FP32, up to nx, ny = 1024:
-// both directions 64 x 32 19.5 -> 13.7 us, 256^2 22.5 -> 18.0, 1024^2 37 to 59
-// -> 33 to 54 us (1 to 3 components); one component at nx = 512 gives its blocks
-// of 16 rows too few to hide each other's waits (512 x 256 23.6 -> 24.3).  FP64's
-// column pairs take two launches already (256^2 19 against 22 us so).
-static bool x_columns(const qp_ctx *c, int nc)
+// Whether the x pass reads or writes the columns that the y pass works on
+// (k_fft_xt), two launches in place of three.  FP32, both directions, one and
+// three components: 64 x 32 19.5 -> 13.5 us; 512^2 25.3 and 33.4 -> 21.0 and
+// 25.3; 1024^2 37 and 59 -> 29 and 53; 2048^2 70.6 and 157 -> 69.6 and 151; longer
+// x transforms do not fit the workgroup's LDS.  FP64's column pairs take two
+// launches already (512^2 23.2 and 35.9 against 26.4 and 35.3 us so).  The
+// knob's other values keep the transpose or the column pairs.
+static bool x_columns(const qp_ctx *c)
 {
-    return c->prec == QP_FP32 && fused_fields(c) && (nc > 1 || c->nx != 512);
+    return c->prec == QP_FP32 && c->nx <= 2048 && c->max_lds >= 81920 &&
+           c->tune[QP_TUNE_FFT] == tune_default_of(c->prec, QP_TUNE_FFT);
 }
 
 template <typename R>
@@ -354,7 +356,7 @@ static int r2k_t(qp_ctx *c, qp_field2d *const *fs, const int *kinds, int nf)
     const int nc = gather_comps<R>(fs, kinds, nf, rs, ks, &mx, &my);
     if (nc <= 0) return nc;
     if constexpr (std::is_same<R, float>::value) {
-        if (x_columns(c, nc)) {
+        if (x_columns(c)) {
             CompSet<R> y{};
             for (int i = 0; i < nc; ++i) y.src[i] = y.dst[i] = ks[i];
             int rc = fft_x_to_columns(c, rs, ks, nc, mx);
@@ -375,7 +377,7 @@ static int k2r_t(qp_ctx *c, qp_field2d *const *fs, const int *kinds, int nf)
     const int nc = gather_comps<R>(fs, kinds, nf, rs, ks, &mx, &my);
     if (nc <= 0) return nc;
     if constexpr (std::is_same<R, float>::value) {
-        if (x_columns(c, nc)) {
+        if (x_columns(c)) {
             R *sk[MAX_BATCH];
             CompSet<R> y{};
             for (int i = 0; i < nc; ++i) {

@@ -756,6 +756,8 @@ static int xt(qp_ctx *c, const XtSet<R> &s, int nc, int types, int zero_row,
               const BorderArgs<R> &bd = BorderArgs<R>{})
 {
 #define QP_CALL(L) xt_launch<R, L, INV>(c, s, nc, types, zero_row, bd)
+    if constexpr (sizeof(R) == 4)
+        if (c->nx == 2048) return QP_CALL(12);
     QP_BY_LENGTH(c->nx, QP_CALL);
 #undef QP_CALL
 }

@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("indx,indy", [(4, 4), (4, 10), (5, 6), (6, 5), (7, 4), (8, 8), (9, 8),
-                                       (9, 9), (10, 7), (10, 10), (11, 6), (6, 11)])
+                                       (9, 9), (10, 7), (10, 10), (11, 6), (6, 11), (11, 11)])
 def test_transform_routes_agree(indx, indy):
     print(f"[gpu-test] transform routes {indx} {indy}", flush=True)
     ctx = qps.Ctx(indx, indy, 4, box=(-10.0, 10.0, -10.0, 10.0, 0.0, 1.0), precision=qps.FP32)

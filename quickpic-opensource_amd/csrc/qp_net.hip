@@ -58,16 +58,18 @@ __device__ __forceinline__ v4s load4(const uint16_t *p)
 // wrote them; the seed network's layers hold 0.1 to 2 MB), so there is a wave
 // for every tile, 16 to 768 blocks a convolution of a training step at 128^2,
 // and two ways of not waiting for each step:
-//  k_conv3x3: up to CONV_CIN input channels.  A block's waves are TX x TY pixel
+//  k_conv3x3: the channel counts it is compiled for, up to 192 (3 x 66 pixels and
+//    9 x 16 weight rows of 400 bytes, 137 KB of LDS).  A block's waves are TX x TY pixel
 //    groups, and the pixels around them (zero outside the plane, masked) and the
 //    weights go to LDS first, in loads of 16 bytes that are in flight together.
 //    A row of LDS is a pixel or a (tap, co), padded by 16 bytes: the 16 rows of
 //    an operand then lie in different banks.
-//  k_conv3x3_deep: more channels than LDS holds.  The chain is cut in groups of
+//  k_conv3x3_deep: the others, and operands not aligned to 16 bytes.  The chain is cut in groups of
 //    9 steps, whose loads are issued before the group in front is multiplied.
 // One wave with all output channels of its pixels, loading step by step, took
 // 33.7 us a convolution (27 of a training step); all by k_conv3x3_deep 11.8 us,
-// by k_conv3x3 8.5 us.
+// by k_conv3x3 5.7 us (8.2 us with the channel count as an argument: a wave alone
+// on its SIMD then waited for the scalar address arithmetic of each step).
 // ---------------------------------------------------------------------------
 // D[pixel 4q+i][co]: pixels xp.. of row y
 __device__ __forceinline__ void conv_store(v4f acc, const float *bias, int co, int y, int xp, int W,
@@ -85,7 +87,7 @@ __device__ __forceinline__ void conv_store(v4f acc, const float *bias, int co, i
     }
 }
 
-constexpr int CONV_CIN = 192;   // (3 x 66 pixels and 9 x 16 weight rows) x 400 B: 137 KB of LDS
+constexpr int CONV_CUS = 256;   // compute units of an MI355X
 
 // quotient of small numbers, 0 <= a < 2^20, 1 <= b: ib = 1 / b
 __device__ __forceinline__ int small_div(int a, float ib) { return (int)(((float)a + 0.5f) * ib); }
@@ -96,29 +98,30 @@ __device__ __forceinline__ uint32_t positive2(uint32_t v, uint32_t k)
     return (lo ? v & 0xffffu : 0u) | (hi ? v & 0xffff0000u : 0u);
 }
 
-template <bool MASK>
+template <int KT, bool MASK>   // 16 KT input channels
 __global__ void __launch_bounds__(256)
 k_conv3x3(const uint16_t *__restrict__ x, const uint16_t *__restrict__ mask, int H, int W, int nbx,
-          int tx, int cs_in, int Cin, const uint16_t *__restrict__ w,
+          int tx, int ty, int cs_in, const uint16_t *__restrict__ w,
           const float *__restrict__ bias, uint16_t *out, int cs_out, int Cout, int relu, int accum)
 {
     extern __shared__ uint4 lds4[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int ty = 4 / tx, by = blockIdx.x / nbx, bx = blockIdx.x - by * nbx;
+    const int by = blockIdx.x / nbx, bx = blockIdx.x - by * nbx;
     const int x0 = bx * 16 * tx, y0 = by * ty;        // the block's first pixel
     const int rw = 16 * tx + 2, npx = rw * (ty + 2);  // the pixels around it
-    const int kc = Cin >> 3, ld = kc + 1;             // 16-byte words of a row, pitch
+    constexpr int Cin = 16 * KT, kc = Cin >> 3, ld = kc + 1;   // 16-byte words of a row, pitch
     const float irw = 1.f / (float)rw;
     // thread: word c of the rows r, r + rs, ...; a few threads are left over
-    const int rs = 256 / kc, r = small_div(tid, 1.f / (float)kc), c = tid - r * kc;
+    constexpr int rs = 256 / kc;
+    const int r = tid / kc, c = tid - r * kc;
     const int cot = blockIdx.y;
     const uint16_t *wc = w + ((size_t)16 * cot * Cin + 8 * c);
     // rows y0 - 1 ..: offsets from here are small; outside the plane the block's
     // first pixel is read, and its value is dropped
     const size_t orow = (size_t)y0 * W * cs_in + 8 * c;
     const uint16_t *xc = x + orow, *kc0 = mask + (MASK ? orow : 0);
-    constexpr int UW = 8, UP = 10;
+    constexpr int UW = 9, UP = 10;
     for (int w0 = r, p0 = r; r < rs && (w0 < 144 || p0 < npx); w0 += UW * rs, p0 += UP * rs) {
         uint4 vw[UW], vp[UP], vk[MASK ? UP : 1];
         uint32_t in = 0;   // bit u: inside the plane
@@ -154,36 +157,31 @@ k_conv3x3(const uint16_t *__restrict__ x, const uint16_t *__restrict__ mask, int
     }
     __syncthreads();
     const int wy = wave / tx, y = y0 + wy, px0 = x0 + 16 * (wave - wy * tx);
-    if (y >= H || px0 >= W) return;
+    if (wy >= ty || y >= H || px0 >= W) return;
     const int m = lane & 15, q = lane >> 4;           // A row (pixel) and k quad
     const uint2 *l2 = reinterpret_cast<const uint2 *>(lds4);
-    const int KT = Cin >> 4, ld2 = 2 * ld;
+    constexpr int ld2 = 2 * ld;
     const uint2 *pa = l2 + (wy * rw + 16 * (wave - wy * tx) + m) * ld2 + q;
     const uint2 *pb = l2 + (npx + m) * ld2 + q;
-    int tap = 0, kk = 0;                              // of the next step to load
-    auto load = [&](uint2 *a, uint2 *b) {
+    // a tap's operands are read while the tap before is multiplied
+    uint2 fa[2][KT], fb[2][KT];
+    auto load = [&](int tap, uint2 *a, uint2 *b) {
+        const uint2 *ta = pa + (tap / 3 * rw + tap % 3) * ld2, *tb = pb + 16 * tap * ld2;
 #pragma unroll
-        for (int i = 0; i < 9; ++i) {
-            const int dy = (tap * 11) >> 5;           // tap / 3
-            a[i] = pa[(dy * rw + tap - 3 * dy) * ld2 + 4 * kk];
-            b[i] = pb[16 * tap * ld2 + 4 * kk];
-            if (++kk == KT) { kk = 0; ++tap; }
+        for (int k = 0; k < KT; ++k) {
+            a[k] = ta[4 * k];
+            b[k] = tb[4 * k];
         }
     };
     v4f acc = {0.f, 0.f, 0.f, 0.f};
-    auto multiply = [&](const uint2 *a, const uint2 *b) {
+    load(0, fa[0], fb[0]);
 #pragma unroll
-        for (int i = 0; i < 9; ++i)
-            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(frag(a[i]), frag(b[i]), acc, 0, 0, 0);
-    };
-    uint2 a0[9], b0[9], a1[9], b1[9];
-    load(a0, b0);
-    for (int k = 0; k < KT; k += 2) {
-        if (k + 1 < KT) load(a1, b1);
-        multiply(a0, b0);
-        if (k + 1 >= KT) break;
-        if (k + 2 < KT) load(a0, b0);
-        multiply(a1, b1);
+    for (int tap = 0; tap < 9; ++tap) {
+        if (tap < 8) load(tap + 1, fa[(tap + 1) & 1], fb[(tap + 1) & 1]);
+#pragma unroll
+        for (int k = 0; k < KT; ++k)
+            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(frag(fa[tap & 1][k]),
+                                                            frag(fb[tap & 1][k]), acc, 0, 0, 0);
     }
     conv_store(acc, bias, 16 * cot + m, y, px0 + 4 * q, W, out, cs_out, relu, accum);
 }
@@ -285,7 +283,7 @@ __device__ __forceinline__ int table_entry(const int *first, int n)
 // block, and k_sum_parts adds the partial sums from memory.  All layers of a
 // network go in one launch: at 128^2 a block per (tile, tap, chunk), a serial
 // sum for db and two sums over the chunks, layer by layer, took 68 us a layer;
-// the 14 layers together take 47 us and the sum 4 us.
+// the 14 layers together take 41 us and the sum 4 us.
 // ---------------------------------------------------------------------------
 constexpr int WG_WHOLE = 64;   // one step of the four runs
 constexpr int WG_SLOTS = 16;
@@ -321,6 +319,8 @@ __device__ __forceinline__ void wgrad_runs(const WgradLayer &L, int co, int ci, 
     }
     const int H = L.H, W = L.W, npix = H * W;
     const v4s one = {(short)0x3f80, (short)0x3f80, (short)0x3f80, (short)0x3f80};
+    const bool small = npix < (1 << 20);
+    const float iw = 1.f / (float)W;
     for (int g = 0; g < (NC > 1 ? min(npix, 64) : p1[0] - p0[0]); g += 64) {
         uint16_t d[4][4], yo[4][4], xv[4][6];
 #pragma unroll
@@ -349,7 +349,7 @@ __device__ __forceinline__ void wgrad_runs(const WgradLayer &L, int co, int ci, 
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const int p = p0[v / NV] + g + 16 * (v % NV) + 4 * q;
-            int py = p / W, px = p - py * W;
+            int py = small ? small_div(p, iw) : p / W, px = p - py * W;
             v4s a, b[3];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -408,7 +408,7 @@ __device__ __forceinline__ void wgrad_slots(const WgradLayer &L, int co, int ci,
     }
 }
 
-__global__ void __launch_bounds__(256) k_wgrad(const WgradArgs A)
+__global__ void __launch_bounds__(256, 3) k_wgrad(const WgradArgs A)
 {
     __shared__ v4f red[WG_SLOTS][3][64];
     __shared__ float redb[WG_SLOTS][16];
@@ -860,19 +860,44 @@ int qp_net_conv3x3(void *stream_, const uint16_t *x, const uint16_t *mask, int H
     const int gw = (W + 15) / 16;
     // 16-byte loads of the pixels and weights where they are aligned for it
     const bool al = cs_in % 8 == 0 && !(((uintptr_t)x | (uintptr_t)mask | (uintptr_t)w) & 15);
-    if (cin > 0 && cin <= CONV_CIN && al) {
-        const int tx = gw >= 3 ? 4 : gw, ty = 4 / tx, nbx = (gw + tx - 1) / tx;
+    const int kt = cin / 16;
+    const bool have = kt == 1 || kt == 2 || kt == 3 || kt == 4 || kt == 6 || kt == 8 || kt == 12;
+    if (have && al) {
+        // four pixel groups a block, or fewer where that leaves compute units without
+        // one: a block waits for what it brings to LDS
+        int tx = gw >= 3 ? 4 : gw, ty = 4 / tx;
+        auto blocks = [&](int x, int y) {
+            return (size_t)((H + y - 1) / y) * ((gw + x - 1) / x) * (cout / 16);
+        };
+        while (tx * ty > 1 && 2 * blocks(tx, ty) <= CONV_CUS) {
+            if (ty > 1) ty /= 2;
+            else tx /= 2;
+        }
+        const int nbx = (gw + tx - 1) / tx;
         const size_t lds = (size_t)((16 * tx + 2) * (ty + 2) + 144) * (cin / 8 + 1) * 16;
         const dim3 grid((unsigned)((size_t)((H + ty - 1) / ty) * nbx), cout / 16);
-        const void *k = mask ? (const void *)k_conv3x3<true> : (const void *)k_conv3x3<false>;
-        if (lds > 65536)
-            QP_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        if (mask)
-            hipLaunchKernelGGL(k_conv3x3<true>, grid, dim3(256), lds, st, x, mask, H, W, nbx, tx,
-                               cs_in, cin, w, bias, out, cs_out, cout, relu, accum);
-        else
-            hipLaunchKernelGGL(k_conv3x3<false>, grid, dim3(256), lds, st, x, mask, H, W, nbx, tx,
-                               cs_in, cin, w, bias, out, cs_out, cout, relu, accum);
+        auto launch = [&](auto kern) -> int {
+            if (lds > 65536)
+                QP_HIP(hipFuncSetAttribute((const void *)kern,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, x, mask, H, W, nbx, tx, ty, cs_in, w,
+                               bias, out, cs_out, cout, relu, accum);
+            return QP_OK;
+        };
+        int rc = QP_OK;
+#define CONV_CASE(KT) \
+    case KT: rc = mask ? launch(k_conv3x3<KT, true>) : launch(k_conv3x3<KT, false>); break
+        switch (kt) {
+            CONV_CASE(1);
+            CONV_CASE(2);
+            CONV_CASE(3);
+            CONV_CASE(4);
+            CONV_CASE(6);
+            CONV_CASE(8);
+            CONV_CASE(12);
+        }
+#undef CONV_CASE
+        RC(rc);
         QP_LAUNCH_CHECK();
         return QP_OK;
     }

@@ -127,13 +127,15 @@ int qp_ctx_profile_get(qp_ctx *ctx, int kind, double *total_ms, int64_t *count,
  * B(xi-3) (linearly while only two slices are recorded).  The
  * seed changes only how many passes reach the tolerance; fixed-pass runs
  * (tol <= 0) use the reference's seed whatever the knob.
- * QP_TUNE_FFT = 1 folds the transpose between the x and y passes of every
- * transform into the y pass (column-pair reads / writes) instead of a
- * separate LDS-tiled transpose (the FP64 default).  0 (the FP32 default),
- * 2, 3 and 4 keep the transpose and pad the transforms' LDS by one point per
- * 16 points in FP32 or 8 in FP64 (0), or per 8, 32 or 4 points (2, 3, 4);
- * 5 and 6 fold the transpose only in the k -> real or only in the real -> k
- * direction.  Results are identical.
+ * QP_TUNE_FFT at its default (0 in FP32, 1 in FP64) lets the slice loop run its
+ * field solves with the y transforms and the modes in one kernel (both sides up
+ * to 1024), and the FP32 transforms of whole fields without a transpose (nx up
+ * to 2048).  Otherwise 1 folds the transpose between the x and y passes of
+ * every transform into the y pass (column-pair reads / writes) instead of a
+ * separate LDS-tiled transpose; 0, 2, 3 and 4 keep the transpose and pad the
+ * transforms' LDS by one point per 16 points in FP32 or 8 in FP64 (0), or per
+ * 8, 32 or 4 points (2, 3, 4); 5 and 6 fold the transpose only in the k -> real
+ * or only in the real -> k direction.  Results agree to rounding.
  * QP_TUNE_PUSH selects how the plasma push re-sorts the particles: 0 (default)
  * counts the destination bins in a first pass that stores nothing per
  * particle, then pushes again and stores every particle at its sorted place;

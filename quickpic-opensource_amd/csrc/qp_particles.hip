@@ -247,7 +247,7 @@ k_deposit_q(TileGeom g, Soa<R> s, const int *__restrict__ off, DepOut<R> out, R 
     }
     constexpr int T = TILE / RG, NP = Stage<CH>::N;
     extern __shared__ unsigned char smem_raw[];
-    R *sx = reinterpret_cast<R *>(smem_raw), *sy = sx + NP, *sq = sy + NP, *nacc = sq + NP;
+    R *sx = reinterpret_cast<R *>(smem_raw), *sy = sx + NP, *sq = sy + NP, *nacc = UQ ? sq : sq + NP;
     const int tid = threadIdx.x, tile = blockIdx.x;
     const int tx = tile % g.mx1, ty = tile / g.mx1, kb = tile * TCELLS;
     for (int n = tid; n < 289; n += TCELLS) nacc[n] = R(0);
@@ -1654,7 +1654,7 @@ static int deposit_q_v(qp_species *sp, const DepOut<R> &out, R *halo, const Beam
 {
     qp_ctx *c = sp->ctx;
     constexpr DepShape d = DepTab<R>::q[V];
-    const size_t lds = (3 * (size_t)Stage<d.ch>::N + 289) * sizeof(R);
+    const size_t lds = ((sp->q_uniform ? 2 : 3) * (size_t)Stage<d.ch>::N + 289) * sizeof(R);
     auto kern = sp->q_uniform ? k_deposit_q<R, d.rg, d.ch, d.wpe, true>
                               : k_deposit_q<R, d.rg, d.ch, d.wpe, false>;
     int rc = allow_lds(kern, lds, c);

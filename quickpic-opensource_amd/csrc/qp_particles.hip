@@ -180,8 +180,8 @@ template <int CH> struct Stage {
 // Stages particles [c0, c0 + n) of NA arrays into LDS (padded index lpad):
 // thread tid takes p = tid + k*step, k < K.  Every load of the thread is
 // issued before the first LDS store, so the chunk costs one memory latency.
-template <typename R, int NA, int K>
-__device__ __forceinline__ void stage_in(const R *const (&src)[NA], R *const (&dst)[NA], int c0,
+template <typename R, int NA, int K, int M>
+__device__ __forceinline__ void stage_in(const R *const (&src)[M], R *const (&dst)[M], int c0,
                                          int n, int tid, int step)
 {
     R t[K][NA];
@@ -555,14 +555,17 @@ k_amjdp(TileGeom g, Soa<R> s, const int *__restrict__ off, const R *fxy, const R
         for (int c0 = G0; c0 < G1; c0 += CH) {
             const int n = min(CH, G1 - c0);
             __syncthreads();
+            // the psi gather makes p6 and p7 anew: they are not read (1024^2, 16 a
+            // cell: FP32 178 -> 163 us, FP64 372 -> 350)
+            constexpr int NS = PSI ? 4 : 6;
             if (UQ) {
                 const R *src[6] = {s.x, s.y, s.px, s.py, s.p6, s.p7};
                 R *dst[6] = {sx, sy, spx, spy, sp6, sp7};
-                stage_in<R, 6, CH / TCELLS>(src, dst, c0, n, tid, TCELLS);
+                stage_in<R, NS, CH / TCELLS>(src, dst, c0, n, tid, TCELLS);
             } else {
-                const R *src[7] = {s.x, s.y, s.px, s.py, s.p6, s.p7, s.q};
-                R *dst[7] = {sx, sy, spx, spy, sp6, sp7, sq};
-                stage_in<R, 7, CH / TCELLS>(src, dst, c0, n, tid, TCELLS);
+                const R *src[7] = {s.x, s.y, s.px, s.py, PSI ? s.q : s.p6, s.p7, s.q};
+                R *dst[7] = {sx, sy, spx, spy, PSI ? sq : sp6, sp7, sq};
+                stage_in<R, NS + 1, CH / TCELLS>(src, dst, c0, n, tid, TCELLS);
             }
             __syncthreads();
             int a = i0 + sub;
@@ -570,7 +573,7 @@ k_amjdp(TileGeom g, Soa<R> s, const int *__restrict__ off, const R *fxy, const R
             const int b = min(i1, c0 + n);
             for (int i = a; i < b; i += T) {
                 const int l = lpad(i - c0);
-                R p6 = sp6[l], p7 = sp7[l];
+                R p6 = PSI ? R(0) : sp6[l], p7 = PSI ? R(0) : sp7[l];
                 if (psi) {
                     extpsi_one(FP, fx, fy, sx[l], sy[l], spx[l], spy[l], qbm, dex, p6, p7);
                     sp7[l] = p7;
@@ -2025,9 +2028,9 @@ static int amjdp_v(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
     int rc = allow_lds(kern, lds, c);
     if (rc) return rc;
     {
-    // with psi: one more word per particle (p7 written) and one more plane;
-    // a uniform q is not read (by the kernels with a uniform-charge form)
-    const double words = (psi ? 9.0 : 8.0) - (sp->q_uniform && d.wave == 0 ? 1.0 : 0.0);
+    // with psi: p6 and p7 written but, by the default form, not read, and one more
+    // plane; a uniform q is not read (by the kernels with a uniform-charge form)
+    const double words = (psi ? (d.wave == 0 ? 7.0 : 9.0) : 8.0) - (sp->q_uniform && d.wave == 0 ? 1.0 : 0.0);
     const double planes = psi ? 15.0 : 14.0;
     ProfScope _ps(c, QP_PROF_AMJDP, (words * sp->np + planes * (c->nx + 1.0) * (c->ny + 1.0)) * sizeof(R));
     hipLaunchKernelGGL(kern, dim3(c->ntiles * B), dim3(256), lds, c->stream, geom(c),

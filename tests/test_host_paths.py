@@ -1,0 +1,81 @@
+"""Host paths of the library without a GPU: libqpslice.so on a HIP runtime that
+records kernels instead of running them (hip_stub.cpp).  Each test is a program of
+its own, so that the stub is the only runtime of its process."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+PKG = os.path.join(os.path.dirname(HERE), "quickpic-opensource_amd")
+ROCM = "/opt/rocm/include"
+
+pytestmark = pytest.mark.skipif(
+    not (os.path.isdir(ROCM) and os.path.exists(os.path.join(PKG, "libqpslice.so"))),
+    reason="needs the ROCm headers and the built library")
+
+HEAD = """
+import ctypes as C, os, sys, traceback
+stub = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+sys.path.insert(0, sys.argv[2])
+import qpslice as qps
+
+def sims(n, ind=4):
+    out = []
+    for _ in range(n):
+        ctx = qps.Ctx(ind, ind, 4)
+        sim = qps.Sim(ctx, [qps.Species(ctx, ppc=(1, 1))], [])
+        sim.begin_step()
+        out.append(sim)
+    return out
+
+def refused(fn, *args):
+    try:
+        fn(*args)
+    except qps.QPError as e:
+        return e
+    raise AssertionError("not refused")
+
+def test():
+"""
+
+TAIL = """
+try:
+    test()
+except BaseException:
+    traceback.print_exc()
+    os._exit(1)
+os._exit(0)   # the stub's process ends without the runtime's tear-down
+"""
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("stub") / "libhipstub.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-w", "-I" + ROCM,
+                    os.path.join(HERE, "hip_stub.cpp"), "-o", so], check=True)
+    return so
+
+
+def run(stub, body):
+    p = subprocess.run([sys.executable, "-c", HEAD + textwrap.indent(body, "    ") + TAIL, stub, PKG],
+                       capture_output=True, text=True, timeout=120)
+    assert p.returncode == 0, p.stdout + p.stderr
+
+
+@pytest.mark.parametrize("tol,residual", [(0.0, 0.0), (1e-3, 0.0), (1e-3, 1.0)])
+def test_scan_runs_whatever_device_is_current(stub, tol, residual):
+    """A run by a thread that has another device current: the graphs that are made
+    executable in it are the scan's device's, and the thread keeps its own."""
+    run(stub, f"""
+stub.stub_residual(C.c_size_t(8 * 64), C.c_double({residual}))
+scan = qps.Scan(sims(2), iter_max=6, tol={tol})
+stub.hipSetDevice(1)
+scan.run(2)
+assert stub.stub_graph_launches() >= 4
+d = C.c_int(-1)
+stub.hipGetDevice(C.byref(d))
+assert d.value == 1
+""")

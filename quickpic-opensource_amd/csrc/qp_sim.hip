@@ -658,6 +658,7 @@ struct qp_scan {
     std::vector<ScanInstance> inst;
     int iter_max = 0;
     double tol = 0.0;
+    bool failed = false;               // a run ended with the instances at different slices
 };
 
 }  // extern "C"
@@ -731,31 +732,33 @@ static int slice_capture(ScanSlice &sl, const qp_scan *sc, qp_sim *s)
     return part_capture(sl.end, sc, s, [&](SliceRun &r) -> int { return r.end(); });
 }
 
+// The graph that ends a slice has been enqueued: the host's side of its push, at
+// once, so that the pointers are right whatever fails next.
+static void scan_pushed(ScanInstance &in)
+{
+    for (qp_species *sp : in.s->sp) species_flip(sp, in.offsets);
+    in.parity ^= 1;
+    --in.left;
+}
+
 // enqueues the start of an instance's next slice and as many passes as its last
-// one needed.  None of its passes is in flight: the ones of the slice before
-// that ran have written their residuals.
+// one needed (fixed passes: the slice).  None of its passes is in flight: the
+// ones of the slice before that ran have written their residuals.
 static int scan_start(qp_scan *sc, ScanInstance &in)
 {
     ScanSlice &sl = in.slice[in.parity];
     if (sc->tol <= 0.0) {
         RC(part_launch(sl.start, in.s));
-    } else {
-        volatile double *h = in.s->ctx->h_res;
-        for (int l = 1; l <= sc->iter_max; ++l) h[l % RES_SLOTS] = -1.0;
-        RC(part_launch(sl.start, in.s));
-        const int first = sc->iter_max - (int)sl.pass.size();
-        for (in.done = first; in.done < in.pred; ++in.done)
-            RC(part_launch(sl.pass[in.done - first], in.s));
+        scan_pushed(in);
+        return QP_OK;
     }
+    volatile double *h = in.s->ctx->h_res;
+    for (int l = 1; l <= sc->iter_max; ++l) h[l % RES_SLOTS] = -1.0;
+    RC(part_launch(sl.start, in.s));
+    const int first = sc->iter_max - (int)sl.pass.size();
+    for (in.done = first; in.done < in.pred; ++in.done)
+        RC(part_launch(sl.pass[in.done - first], in.s));
     return QP_OK;
-}
-
-// the slice is enqueued to its end: the next one
-static int scan_next(qp_scan *sc, ScanInstance &in)
-{
-    for (qp_species *sp : in.s->sp) species_flip(sp, in.offsets);
-    in.parity ^= 1;
-    return --in.left ? scan_start(sc, in) : QP_OK;
 }
 
 // One look at an instance that runs to the tolerance: news is set when its
@@ -780,7 +783,49 @@ static int scan_step(qp_scan *sc, ScanInstance &in, bool *news)
     }
     in.pred = conv ? conv : in.done;
     RC(part_launch(sl.end, in.s));
-    return scan_next(sc, in);
+    scan_pushed(in);
+    return in.left ? scan_start(sc, in) : QP_OK;
+}
+
+// nslices slices of every instance, from the parity of each
+static int scan_slices(qp_scan *sc, int nslices)
+{
+    if (sc->tol <= 0.0) {
+        for (int k = 0; k < nslices; ++k)
+            for (ScanInstance &in : sc->inst) RC(scan_start(sc, in));
+        return QP_OK;
+    }
+    size_t busy = nslices ? sc->inst.size() : 0;
+    if (busy)
+        for (ScanInstance &in : sc->inst) RC(scan_start(sc, in));
+    for (int idle = 0; busy;) {
+        bool news = false;
+        for (ScanInstance &in : sc->inst) {
+            if (!in.left) continue;
+            RC(scan_step(sc, in, &news));
+            if (!in.left) --busy;
+        }
+        if (news) {
+            idle = 0;
+        } else if (++idle == SCAN_POLLS) {
+            // a stream that failed, or ended without its residual, ends the wait
+            idle = 0;
+            for (ScanInstance &in : sc->inst) {
+                if (!in.left) continue;
+                const hipError_t e = hipStreamQuery(in.s->ctx->stream);
+                if (e == hipErrorNotReady) {
+                    (void)hipGetLastError();
+                    continue;
+                }
+                QP_HIP(e);
+                bool now = false;
+                RC(scan_step(sc, in, &now));
+                QP_REQUIRE(now, QP_ERR_STATE, "qp_scan_run: a slice ended without a residual");
+                if (!in.left) --busy;
+            }
+        }
+    }
+    return QP_OK;
 }
 
 extern "C" {
@@ -848,6 +893,9 @@ int qp_scan_create(qp_sim *const *sims, int n, int iter_max, double tol, qp_scan
 int qp_scan_run(qp_scan *sc, int nslices)
 {
     QP_REQUIRE(sc && !sc->inst.empty() && nslices >= 0, QP_ERR_ARG, "qp_scan_run: bad argument");
+    QP_REQUIRE(!sc->failed, QP_ERR_STATE,
+               "qp_scan_run: a run before ended in an error, with the simulations at different "
+               "slices; begin a step of each and create the scan again");
     // the buffer parity of every instance (they must agree: an instance
     // advanced by eager slices in between would not match the graphs)
     int parity = -1;
@@ -872,48 +920,18 @@ int qp_scan_run(qp_scan *sc, int nslices)
     }
     // the instances' streams are independent, and the library's eager calls
     // before and after order with the slices on them
-    size_t busy = 0;
     for (ScanInstance &in : sc->inst) {
         in.parity = parity;
         in.left = nslices;
-        if (nslices) {
-            RC(scan_start(sc, in));
-            ++busy;
-        }
     }
-    if (sc->tol <= 0.0) {
-        for (int k = 0; k < nslices; ++k)
-            for (ScanInstance &in : sc->inst) RC(scan_next(sc, in));
-        busy = 0;
+    int rc = scan_slices(sc, nslices);
+    // nothing is left running, also after an error
+    for (ScanInstance &in : sc->inst) {
+        const hipError_t e = hipStreamSynchronize(in.s->ctx->stream);
+        if (!rc && e != hipSuccess) rc = hip_fail(e, "hipStreamSynchronize", __FILE__, __LINE__);
     }
-    for (int idle = 0; busy;) {
-        bool news = false;
-        for (ScanInstance &in : sc->inst) {
-            if (!in.left) continue;
-            RC(scan_step(sc, in, &news));
-            if (!in.left) --busy;
-        }
-        if (news) {
-            idle = 0;
-        } else if (++idle == SCAN_POLLS) {
-            // a stream that failed, or ended without its residual, ends the wait
-            idle = 0;
-            for (ScanInstance &in : sc->inst) {
-                if (!in.left) continue;
-                const hipError_t e = hipStreamQuery(in.s->ctx->stream);
-                if (e == hipErrorNotReady) {
-                    (void)hipGetLastError();
-                    continue;
-                }
-                QP_HIP(e);
-                bool now = false;
-                RC(scan_step(sc, in, &now));
-                QP_REQUIRE(now, QP_ERR_STATE, "qp_scan_run: a slice ended without a residual");
-                if (!in.left) --busy;
-            }
-        }
-    }
-    for (ScanInstance &in : sc->inst) QP_HIP(hipStreamSynchronize(in.s->ctx->stream));
+    sc->failed = rc != QP_OK;
+    RC(rc);
     // the particle move checks of the replayed slices (PPPCHECK2L)
     for (size_t i = 0; i < sc->inst.size(); ++i)
         for (qp_species *sp : sc->inst[i].s->sp) {

@@ -79,3 +79,35 @@ d = C.c_int(-1)
 stub.hipGetDevice(C.byref(d))
 assert d.value == 1
 """)
+
+
+@pytest.mark.parametrize("tol,at", [(0.0, 1), (0.0, 2), (0.0, 3), (1e-3, 3), (1e-3, 4)])
+def test_scan_run_ended_by_an_error(stub, tol, at):
+    """Graph launch `at` of a run fails.  The streams are waited for; every
+    species's pointers are those of the slices that were launched; and the scan,
+    whose simulations are at different slices, runs no further.  Launches in
+    order, for two simulations: fixed passes 0 1 0 1 (slices); to a tolerance,
+    converged in the first graph, starts 0 1, end and next start of 0, of 1."""
+    run(stub, f"""
+stub.stub_residual(C.c_size_t(8 * 64), C.c_double(0.0))
+stub.stub_word.restype = C.c_ulonglong
+s = sims(2)
+
+def buffer(x):
+    x.species[0].push(x.field(qps.F_FXY), x.field(qps.F_BXYZ), x.field(qps.F_PSIT), x.ctx.dex)
+    return stub.stub_word(b"k_push")
+
+at0 = [buffer(x) for x in s]
+at1 = [buffer(x) for x in s]
+assert at0 != at1
+scan = qps.Scan(s, iter_max=3, tol={tol})   # the particles are at at0
+syncs = [stub.stub_syncs(i) for i in range(2)]
+stub.stub_fail_launch({at})
+refused(scan.run, 2)
+# one wait reads the slice word, one follows the error
+assert all(stub.stub_syncs(i) >= n + 2 for i, n in enumerate(syncs))
+e = refused(scan.run, 1)
+assert e.code == -3, e.code   # QP_ERR_STATE
+done = {{0.0: {{1: (0, 0), 2: (1, 0), 3: (1, 1)}}, 1e-3: {{3: (0, 0), 4: (1, 0)}}}}[{tol}][{at}]
+assert [buffer(x) for x in s] == [(at0, at1)[n][i] for i, n in enumerate(done)]
+""")

@@ -138,8 +138,8 @@ struct qp_ctx {
     double prof_bytes[QP_PROF_COUNT];
     // corrector-loop control.  flags (device ints): word l is set once pass l
     // (or an earlier one) has converged; the kernels of pass l+1 test it and
-    // return at once.  h_res (pinned host): residual of pass l in slot
-    // l % RES_SLOTS.
+    // return at once.  h_res (pinned host, coherent): residual of pass l in
+    // slot l % RES_SLOTS.
     qp::DevBuf flags;
     double *h_res;
     qp::ResJob res_job;   // residual sum carried by the next transform launch
@@ -258,7 +258,8 @@ __device__ __forceinline__ void run_res_job(const ResJob &j)
         if (j.flag_out)
             *j.flag_out = ((j.flag_in && *j.flag_in) || (j.tol > 0.0 && res < j.tol)) ? 1 : 0;
         if (j.h_slot) {
-            *j.h_slot = res;
+            // the host may be polling it (qp_scan_run)
+            __hip_atomic_store(j.h_slot, res, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             __threadfence_system();
         }
     }

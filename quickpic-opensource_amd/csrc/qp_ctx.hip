@@ -286,7 +286,9 @@ int qp_ctx_create(int indx, int indy, int indz, const double box[6], int precisi
     if (!rc) rc = c->red.alloc(sizeof(double) * 8192);
     if (!rc) rc = c->flags.alloc(sizeof(int) * 64);
     if (rc) { qp_ctx_destroy(c); return rc; }
-    e = hipHostMalloc((void **)&c->h_res, sizeof(double) * RES_SLOTS, hipHostMallocDefault);
+    // the host reads it while kernels run
+    e = hipHostMalloc((void **)&c->h_res, sizeof(double) * RES_SLOTS,
+                      hipHostMallocCoherent | hipHostMallocMapped);
     if (e != hipSuccess) { c->h_res = nullptr; qp_ctx_destroy(c); return hip_fail(e, "hipHostMalloc", __FILE__, __LINE__); }
     for (int i = 0; i < RES_SLOTS; ++i) c->h_res[i] = -1.0;
     for (int i = 0; i < 2; ++i) {

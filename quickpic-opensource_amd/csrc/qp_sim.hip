@@ -8,6 +8,7 @@
 #include <algorithm>
 #include <cmath>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "qp_common.h"
@@ -663,8 +664,9 @@ struct qp_scan {
 
 }  // extern "C"
 
-// The host polls for the slowest kernels in between: after this many looks
-// without news it asks the stream whether it still runs.
+// The host polls for the slowest kernels in between, giving its core to other
+// threads after a look without news; after this many it asks the stream whether
+// it still runs.
 static constexpr int SCAN_POLLS = 1 << 14;
 
 // Passes in the first graph.  24 slices of 12 instances on 256^2 and 512^2, 4.8
@@ -752,8 +754,9 @@ static int scan_start(qp_scan *sc, ScanInstance &in)
         scan_pushed(in);
         return QP_OK;
     }
-    volatile double *h = in.s->ctx->h_res;
-    for (int l = 1; l <= sc->iter_max; ++l) h[l % RES_SLOTS] = -1.0;
+    double none = -1.0;
+    for (int l = 1; l <= sc->iter_max; ++l)
+        __atomic_store(in.s->ctx->h_res + l % RES_SLOTS, &none, __ATOMIC_RELAXED);
     RC(part_launch(sl.start, in.s));
     const int first = sc->iter_max - (int)sl.pass.size();
     for (in.done = first; in.done < in.pred; ++in.done)
@@ -766,10 +769,10 @@ static int scan_start(qp_scan *sc, ScanInstance &in)
 // the next slice, have been enqueued.
 static int scan_step(qp_scan *sc, ScanInstance &in, bool *news)
 {
-    const volatile double *h = in.s->ctx->h_res;
     int conv = 0;
     for (int l = 1; l <= in.done && !conv; ++l) {
-        const double r = h[l % RES_SLOTS];
+        double r;
+        __atomic_load(in.s->ctx->h_res + l % RES_SLOTS, &r, __ATOMIC_RELAXED);
         if (r == -1.0) return QP_OK;
         if (r >= 0.0 && r < sc->tol) conv = l;
     }
@@ -807,7 +810,10 @@ static int scan_slices(qp_scan *sc, int nslices)
         }
         if (news) {
             idle = 0;
-        } else if (++idle == SCAN_POLLS) {
+            continue;
+        }
+        std::this_thread::yield();
+        if (++idle == SCAN_POLLS) {
             // a stream that failed, or ended without its residual, ends the wait
             idle = 0;
             for (ScanInstance &in : sc->inst) {

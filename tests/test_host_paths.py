@@ -111,3 +111,13 @@ assert e.code == -3, e.code   # QP_ERR_STATE
 done = {{0.0: {{1: (0, 0), 2: (1, 0), 3: (1, 1)}}, 1e-3: {{3: (0, 0), 4: (1, 0)}}}}[{tol}][{at}]
 assert [buffer(x) for x in s] == [(at0, at1)[n][i] for i, n in enumerate(done)]
 """)
+
+
+def test_polled_residuals_are_coherent(stub):
+    """qp_scan_run reads the residuals while kernels run: the memory they are
+    written to is asked for as coherent."""
+    run(stub, """
+ctx = qps.Ctx(4, 4, 4)
+flags = C.c_uint(stub.stub_host_flags(C.c_size_t(8 * 64))).value
+assert flags != 0xffffffff and flags & 0x40000000, hex(flags)   # hipHostMallocCoherent
+""")

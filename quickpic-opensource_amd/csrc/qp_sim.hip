@@ -466,10 +466,11 @@ struct SliceRun {
     }
 };
 
-// what comes before SliceRun::begin, and begin
+// what comes before SliceRun::begin, and begin (which refuses an iter_max below 1:
+// the slice is left prepared then, for qp_slice_finish)
 int slice_begin(SliceRun &r)
 {
-    if (fused_fields(r.c)) {
+    if (fused_fields(r.c) && r.iter_max >= 1) {
         RC(slice_charges(r.s, r.j, fused_border(r.c) ? &r.border : nullptr));
         return r.begin(true);
     }

@@ -121,3 +121,15 @@ ctx = qps.Ctx(4, 4, 4)
 flags = C.c_uint(stub.stub_host_flags(C.c_size_t(8 * 64))).value
 assert flags != 0xffffffff and flags & 0x40000000, hex(flags)   # hipHostMallocCoherent
 """)
+
+
+@pytest.mark.parametrize("ind", [4, 11])
+def test_refused_pass_count_leaves_the_slice_prepared(stub, ind):
+    """qp_slice_run refuses iter_max 0 after the slice's first part, on which
+    qp_slice_finish goes on, with the fused field solves (16^2) as without (2048^2)."""
+    run(stub, f"""
+x = sims(1, {ind})[0]
+e = refused(lambda: x.slice(1, iter_max=0, tol=1e-3))
+assert "iter_max" in str(e)
+assert x.finish(1, iter_max=2)[0] == 2
+""")

@@ -820,8 +820,8 @@ static void add_sum(SumArgs &a, const float *part, int len, float *out)
 
 static int launch_sums(const SumArgs &a, hipStream_t st)
 {
-    if (!a.n) return QP_OK;
-    const int blocks = a.first[a.n - 1] + (a.len[a.n - 1] + 255) / 256;
+    const int blocks = a.n ? a.first[a.n - 1] + (a.len[a.n - 1] + 255) / 256 : 0;
+    if (!blocks) return QP_OK;
     hipLaunchKernelGGL(k_sum_parts, dim3(blocks), dim3(256), 0, st, a);
     QP_LAUNCH_CHECK();
     return QP_OK;

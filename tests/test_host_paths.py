@@ -133,3 +133,17 @@ e = refused(lambda: x.slice(1, iter_max=0, tol=1e-3))
 assert "iter_max" in str(e)
 assert x.finish(1, iter_max=2)[0] == 2
 """)
+
+
+NET = """
+L = qps.lib()
+P = [C.c_void_p(1 << 12 + i) for i in range(8)]   # addresses that only kernels would use
+"""
+
+
+def test_head_gradient_without_outputs(stub):
+    """No output planes: no gradient to add up, and no error."""
+    run(stub, NET + """
+rc = L.qp_net_head_bwd(None, P[0], 32, 32, P[1], 0, C.c_size_t(64), P[2], P[3], 4, P[4], P[5])
+assert rc == 0, L.qp_last_error()
+""")

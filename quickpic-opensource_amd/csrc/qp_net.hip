@@ -64,7 +64,8 @@ __device__ __forceinline__ v4s load4(const uint16_t *p)
 //    weights go to LDS first, in loads of 16 bytes that are in flight together.
 //    A row of LDS is a pixel or a (tap, co), padded by 16 bytes: the 16 rows of
 //    an operand then lie in different banks.
-//  k_conv3x3_deep: the others, and operands not aligned to 16 bytes.  The chain is cut in groups of
+//  k_conv3x3_deep: the others, operands not aligned to 16 bytes, and devices whose
+//    workgroups have less LDS than a layer asks for.  The chain is cut in groups of
 //    9 steps, whose loads are issued before the group in front is multiplied.
 // One wave with all output channels of its pixels, loading step by step, took
 // 33.7 us a convolution (27 of a training step); all by k_conv3x3_deep 11.8 us,
@@ -86,8 +87,6 @@ __device__ __forceinline__ void conv_store(v4f acc, const float *bias, int co, i
         *o = f2bf(v);
     }
 }
-
-constexpr int CONV_CUS = 256;   // compute units of an MI355X
 
 // quotient of small numbers, 0 <= a < 2^20, 1 <= b: ib = 1 / b
 __device__ __forceinline__ int small_div(int a, float ib) { return (int)(((float)a + 0.5f) * ib); }
@@ -845,36 +844,54 @@ using namespace qp;
         if (rc_) return rc_;  \
     } while (0)
 
-extern "C" {
-
-int qp_net_conv3x3(void *stream_, const uint16_t *x, const uint16_t *mask, int H, int W,
-                   int cs_in, int cin, const uint16_t *w, const float *bias, uint16_t *out,
-                   int cs_out, int cout, int relu, int accum)
+// what the convolutions ask of the current device
+struct NetDevice {
+    size_t lds;   // bytes of a workgroup
+    int cus;      // compute units
+};
+static int net_device(NetDevice *d)
 {
-    hipStream_t st = (hipStream_t)stream_;
+    int dev = 0, lds = 0;
+    QP_HIP(hipGetDevice(&dev));
+    QP_HIP(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+    QP_HIP(hipDeviceGetAttribute(&d->cus, hipDeviceAttributeMultiprocessorCount, dev));
+    d->lds = (size_t)lds;
+    return QP_OK;
+}
+
+// dev: the current device, if the caller has asked for it already
+static int conv3x3(const NetDevice *dev, hipStream_t st, const uint16_t *x, const uint16_t *mask,
+                   int H, int W, int cs_in, int cin, const uint16_t *w, const float *bias,
+                   uint16_t *out, int cs_out, int cout, int relu, int accum)
+{
     NET_CHECK(x && w && out && H > 0 && W > 0, "qp_net_conv3x3: bad argument");
     NET_CHECK(cin % 16 == 0 && cout % 16 == 0 && cout <= 192 && cin <= cs_in &&
                   cout <= cs_out && cs_in % 4 == 0,
               "qp_net_conv3x3: channels cin %d cout %d (multiples of 16, cout <= 192)", cin, cout);
     if (cout <= 0) return QP_OK;
+    NetDevice own;
+    if (!dev) {
+        RC(net_device(&own));
+        dev = &own;
+    }
     const int gw = (W + 15) / 16;
     // 16-byte loads of the pixels and weights where they are aligned for it
     const bool al = cs_in % 8 == 0 && !(((uintptr_t)x | (uintptr_t)mask | (uintptr_t)w) & 15);
     const int kt = cin / 16;
     const bool have = kt == 1 || kt == 2 || kt == 3 || kt == 4 || kt == 6 || kt == 8 || kt == 12;
-    if (have && al) {
-        // four pixel groups a block, or fewer where that leaves compute units without
-        // one: a block waits for what it brings to LDS
-        int tx = gw >= 3 ? 4 : gw, ty = 4 / tx;
-        auto blocks = [&](int x, int y) {
-            return (size_t)((H + y - 1) / y) * ((gw + x - 1) / x) * (cout / 16);
-        };
-        while (tx * ty > 1 && 2 * blocks(tx, ty) <= CONV_CUS) {
-            if (ty > 1) ty /= 2;
-            else tx /= 2;
-        }
+    // four pixel groups a block, or fewer where that leaves compute units without
+    // one: a block waits for what it brings to LDS
+    int tx = gw >= 3 ? 4 : gw, ty = 4 / tx;
+    auto blocks = [&](int x, int y) {
+        return (size_t)((H + y - 1) / y) * ((gw + x - 1) / x) * (cout / 16);
+    };
+    while (tx * ty > 1 && 2 * blocks(tx, ty) <= (size_t)dev->cus) {
+        if (ty > 1) ty /= 2;
+        else tx /= 2;
+    }
+    const size_t lds = (size_t)((16 * tx + 2) * (ty + 2) + 144) * (cin / 8 + 1) * 16;
+    if (have && al && lds <= dev->lds) {
         const int nbx = (gw + tx - 1) / tx;
-        const size_t lds = (size_t)((16 * tx + 2) * (ty + 2) + 144) * (cin / 8 + 1) * 16;
         const dim3 grid((unsigned)((size_t)((H + ty - 1) / ty) * nbx), cout / 16);
         auto launch = [&](auto kern) -> int {
             if (lds > 65536)
@@ -911,8 +928,6 @@ int qp_net_conv3x3(void *stream_, const uint16_t *x, const uint16_t *mask, int H
     QP_LAUNCH_CHECK();
     return QP_OK;
 }
-
-}  // extern "C"
 
 // partb: the partial sums of the bias of a single layer, if not in part
 static int wgrad_layers(hipStream_t st, const qp_net_layer *layers, int n, int nchunk, float *part,
@@ -953,6 +968,14 @@ static int wgrad_layers(hipStream_t st, const qp_net_layer *layers, int n, int n
 }
 
 extern "C" {
+
+int qp_net_conv3x3(void *stream_, const uint16_t *x, const uint16_t *mask, int H, int W,
+                   int cs_in, int cin, const uint16_t *w, const float *bias, uint16_t *out,
+                   int cs_out, int cout, int relu, int accum)
+{
+    return conv3x3(nullptr, (hipStream_t)stream_, x, mask, H, W, cs_in, cin, w, bias, out, cs_out,
+                   cout, relu, accum);
+}
 
 int qp_net_wgrad_layers(void *stream_, const qp_net_layer *layers, int n, int nchunk, float *part,
                         size_t npart)
@@ -1250,10 +1273,12 @@ int qp_net_unet_forward(void *st, const qp_net_unet *u, const float *planes, siz
     const qp_net_conv *e = u->enc, *d = u->dec;
     const qp_net_maps &a = u->a;
     const int *c = u->c;
+    NetDevice dev;
+    RC(net_device(&dev));
     auto conv = [&](const uint16_t *x, int l, int cs, const qp_net_conv &v, uint16_t *out,
                     int cs_out) {
-        return qp_net_conv3x3(st, x, nullptr, u->H >> l, u->W >> l, cs, v.cin, v.w, v.b, out, cs_out,
-                              v.cout, 1, 0);
+        return conv3x3(&dev, (hipStream_t)st, x, nullptr, u->H >> l, u->W >> l, cs, v.cin, v.w, v.b,
+                       out, cs_out, v.cout, 1, 0);
     };
     RC(qp_net_pack_input(st, planes, u->nin, plane, ld, u->in_scale, u->H, u->W, a.x0, 16));
     const uint16_t *in = a.x0;
@@ -1287,6 +1312,8 @@ int qp_net_unet_backward(void *st, const qp_net_unet *u, const float *target)
     const qp_net_maps &a = u->a, &g = u->g;
     const int *c = u->c;
     const size_t npix = (size_t)u->H * u->W;
+    NetDevice dev;
+    RC(net_device(&dev));
     RC(qp_net_mse(st, u->out, target, u->nout * npix, u->gout, u->mse_part, u->nmse));
     RC(qp_net_head_bwd(st, a.db[0], c[0], c[0], u->hw, u->nout, npix, u->gout, g.db[0], u->nhead,
                        u->part, u->ghwb));
@@ -1305,8 +1332,8 @@ int qp_net_unet_backward(void *st, const qp_net_unet *u, const float *target)
                     const uint16_t *gy, int cs_y, uint16_t *gx) -> int {
         wg[nwg++] = qp_net_layer{x, gy, y, v.gw, v.gb, cs, v.cin, cs_y, v.cout, u->H >> l, u->W >> l};
         if (!gx) return QP_OK;
-        return qp_net_conv3x3(st, gy, y, u->H >> l, u->W >> l, cs_y, v.cout, v.wt, nullptr, gx, cs,
-                              v.cin, 0, 0);
+        return conv3x3(&dev, (hipStream_t)st, gy, y, u->H >> l, u->W >> l, cs_y, v.cout, v.wt,
+                       nullptr, gx, cs, v.cin, 0, 0);
     };
     for (int l = 0; l < 3; ++l) {
         const qp_net_conv *v = d + 2 * (2 - l);

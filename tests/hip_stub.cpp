@@ -53,6 +53,14 @@ int stub_launched(const char *part)
     for (const Launch &l : launches) n += l.name.find(part) != std::string::npos;
     return n;
 }
+// LDS bytes of the last such launch
+long stub_lds(const char *part)
+{
+    long v = -1;
+    for (const Launch &l : launches)
+        if (l.name.find(part) != std::string::npos) v = (long)l.lds;
+    return v;
+}
 unsigned long long stub_word(const char *part)
 {
     for (const auto &w : words)

@@ -147,3 +147,41 @@ def test_head_gradient_without_outputs(stub):
 rc = L.qp_net_head_bwd(None, P[0], 32, 32, P[1], 0, C.c_size_t(64), P[2], P[3], 4, P[4], P[5])
 assert rc == 0, L.qp_last_error()
 """)
+
+
+CONV = NET + """
+def conv(H, W, cin, cout):
+    stub.stub_clear_launches()
+    rc = L.qp_net_conv3x3(None, P[0], None, H, W, cin, cin, P[1], None, P[2], cout, cout, 1, 0)
+    assert rc == 0, L.qp_last_error()
+    return stub.stub_launched(b"k_conv3x3_deep")
+
+"""
+
+
+@pytest.mark.parametrize("cin", [16, 32, 48, 64, 96, 128, 192])
+def test_convolution_within_the_devices_lds(stub, cin):
+    """A layer whose pixels and weights do not fit a workgroup's LDS is computed
+    from memory; one that does keeps the kernel that stages them."""
+    run(stub, CONV + f"""
+stub.stub_limits(163840, 256)
+assert conv(128, 128, {cin}, 32) == 0
+need = stub.stub_lds(b"k_conv3x3")
+stub.stub_limits(need, 256)
+assert conv(128, 128, {cin}, 32) == 0
+stub.stub_limits(need - 1, 256)
+assert conv(128, 128, {cin}, 32) == 1
+""")
+
+
+def test_convolution_blocks_follow_the_compute_units(stub):
+    """Blocks of four pixel groups (18 x 6 pixels) where four blocks fill the
+    device, of one (18 x 3) where they leave most of it idle."""
+    run(stub, CONV + """
+stub.stub_limits(163840, 4)
+conv(16, 16, 16, 16)
+assert stub.stub_lds(b"k_conv3x3") == (18 * 6 + 144) * 48
+stub.stub_limits(163840, 256)
+conv(16, 16, 16, 16)
+assert stub.stub_lds(b"k_conv3x3") == (18 * 3 + 144) * 48
+""")

@@ -187,6 +187,11 @@ __device__ __forceinline__ bool kmode(const KGrid &g, int &kx, int &ky)
     return kx <= g.nx;
 }
 
+// a b + c, fused.  Written out where several kernels have to give the same bits:
+// left to the compiler, it depends on the kernel which product of a sum is fused.
+__device__ __forceinline__ float fmadd(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fmadd(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
 // dnx = 6.28318530717959/real(nx+nx); dkx = dnx*real(j) (fpois2d_lib77.f:1512)
 template <typename R>
 __device__ __forceinline__ R dk(int n, int k)

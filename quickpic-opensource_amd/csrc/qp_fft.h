@@ -17,10 +17,14 @@ template <typename T> __device__ __forceinline__ T &at(T *base, unsigned i)
     return *reinterpret_cast<T *>(reinterpret_cast<C *>(base) + (unsigned)(i * sizeof(T)));
 }
 
+// Every kernel that runs these transforms gives the same bits.  Which product of a
+// sum the compiler fuses depends on the kernel around the transform (what becomes
+// of an output, and in which block), so the fused ones are written out here, in
+// dft8 and in the order of the twiddles' factors; nothing else can be fused.
 template <typename R>
 __device__ __forceinline__ cplx<R> cmul(cplx<R> a, cplx<R> b)
 {
-    return {a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x};
+    return {fmadd(a.x, b.x, -(a.y * b.y)), fmadd(a.x, b.y, a.y * b.x)};
 }
 template <typename R>
 __device__ __forceinline__ cplx<R> cadd(cplx<R> a, cplx<R> b) { return {a.x + b.x, a.y + b.y}; }
@@ -42,22 +46,29 @@ __device__ __forceinline__ void dft4(cplx<R> &a0, cplx<R> &a1, cplx<R> &a2, cplx
 }
 
 // forward DFT of 8 points in place (natural order): decimation in frequency,
-// X[2m] = DFT4(v[n] + v[n+4]), X[2m+1] = DFT4((v[n] - v[n+4]) w^n), w = e^{-i pi/4}
-template <typename R>
+// X[2m] = DFT4(v[n] + v[n+4]), X[2m+1] = DFT4((v[n] - v[n+4]) w^n), w = e^{-i pi/4}.
+// Of the odd outputs' products with 1/sqrt 2 the ones fused are those that the
+// row transforms (k_fft_rows) have always fused: in the last pass, which stores
+// its outputs one by one (LAST), not those of t3.
+template <bool LAST = false, typename R>
 __device__ __forceinline__ void dft8(cplx<R> *v)
 {
+#pragma clang fp contract(off)
     const R h = (R)0.70710678118654752440;
     cplx<R> a0 = cadd(v[0], v[4]), a1 = cadd(v[1], v[5]), a2 = cadd(v[2], v[6]),
             a3 = cadd(v[3], v[7]);
-    cplx<R> c0 = csub(v[0], v[4]), c1 = csub(v[1], v[5]), c2 = csub(v[2], v[6]),
-            c3 = csub(v[3], v[7]);
-    c1 = {(c1.x + c1.y) * h, (c1.y - c1.x) * h};     // * e^{-i pi/4}
-    c2 = cmi(c2);                                      // * e^{-i pi/2}
-    c3 = {(c3.y - c3.x) * h, -(c3.x + c3.y) * h};    // * e^{-3i pi/4}
+    const cplx<R> c0 = csub(v[0], v[4]), c1 = csub(v[1], v[5]), c2 = cmi(csub(v[2], v[6])),
+                  c3 = csub(v[3], v[7]);
     dft4(a0, a1, a2, a3);
-    dft4(c0, c1, c2, c3);
+    const cplx<R> s1 = {c1.x + c1.y, c1.y - c1.x};                     // c1 e^{-i pi/4} = s1 h
+    const cplx<R> p3 = {(c3.y - c3.x) * h, -(c3.x + c3.y) * h};        // c3 e^{-3i pi/4}
+    const cplx<R> t0 = cadd(c0, c2), t1 = csub(c0, c2);
+    const cplx<R> t2 = {fmadd(s1.x, h, p3.x), fmadd(s1.y, h, p3.y)};
+    const cplx<R> d = LAST ? cplx<R>{s1.x * h - p3.x, s1.y * h - p3.y}
+                           : cplx<R>{fmadd(s1.x, h, -p3.x), fmadd(s1.y, h, -p3.y)};
+    const cplx<R> t3 = cmi(d);
     v[0] = a0; v[2] = a1; v[4] = a2; v[6] = a3;
-    v[1] = c0; v[3] = c1; v[5] = c2; v[7] = c3;
+    v[1] = cadd(t0, t2); v[3] = cadd(t1, t3); v[5] = csub(t0, t2); v[7] = csub(t1, t3);
 }
 
 // LDS index of FFT point i: one pad point after every 2^PS points
@@ -140,22 +151,25 @@ __device__ __forceinline__ void fft_core(cplx<R> (&v)[8], cplx<R> *buf, int t,
         {
             const cplx<R> w1 = tw.w8[3 * (p - 1)], w2 = tw.w8[3 * (p - 1) + 1],
                           w4 = tw.w8[3 * (p - 1) + 2];
-            const cplx<R> w3 = cmul(w1, w2);
-            const cplx<R> w[8] = {w1, w1, w2, w3, w4, cmul(w1, w4), cmul(w2, w4), cmul(w3, w4)};
+            const cplx<R> w3 = cmul(w2, w1);
+            // (the fused product of w7 has always been the other one in FP64)
+            const cplx<R> w7 = sizeof(R) == 4 ? cmul(w3, w4) : cmul(w4, w3);
+            const cplx<R> w[8] = {w1, w1, w2, w3, w4, cmul(w4, w1), cmul(w4, w2), w7};
 #pragma unroll
             for (int r = 0; r < 8; ++r) {
                 v[r] = buf[padk<PS>(t + r * TF)];
                 if (r) v[r] = cmul(v[r], w[r]);
             }
         }
-        dft8(v);
         if (p == S::NR8 - 1 && S::REM == 0) {
             // last pass (Ns = M/8): output index t + r M/8
+            dft8<true>(v);
 #pragma unroll
             for (int i = 0; i < 4; ++i) z[i] = v[i];
             zn = v[4];
             return;
         }
+        dft8(v);
         __syncthreads();
         const int base = (t / Ns) * Ns * 8 + (t & (Ns - 1));
 #pragma unroll
@@ -171,7 +185,7 @@ __device__ __forceinline__ void fft_core(cplx<R> (&v)[8], cplx<R> *buf, int t,
             cplx<R> a0 = buf[padk<PS>(j)];
             cplx<R> a1 = cmul(buf[padk<PS>(j + M / 4)], w1);
             cplx<R> a2 = cmul(buf[padk<PS>(j + M / 2)], w2);
-            cplx<R> a3 = cmul(buf[padk<PS>(j + 3 * M / 4)], cmul(w1, w2));
+            cplx<R> a3 = cmul(buf[padk<PS>(j + 3 * M / 4)], cmul(w2, w1));
             dft4(a0, a1, a2, a3);
             z[s] = a0;
             z[s + 2] = a1;

@@ -120,8 +120,8 @@ k_pass(KGrid g, const R *__restrict__ ffg, const R *__restrict__ ffs, const R *_
         const bool inner = kx > 0 && kx < g.nx && ky > 0 && ky < g.ny;
         psit[o] = psit_mode(inner, fg, dkx, dky, c1, c2, dex);
         const R b3 = bz_mode(tab, kx, ky, fg, fs, dkx, dky, c1, c2);
-        bxyz[o] = e2 * (-dex) - epwb[cs + o];
-        bxyz[cs + o] = e1 * dex + epwb[o];
+        bxyz[o] = bx_mode(e2, epwb[cs + o], dex);
+        bxyz[cs + o] = by_mode(e1, epwb[o], dex);
         bxyz[2 * cs + o] = b3 * dex;
     }
     if (!QP) return;
@@ -248,8 +248,8 @@ __global__ void __launch_bounds__(256) k_slice_end_fields(EndArgs<R> a)
                     const R w1 = a.epwb[m], w2 = a.epwb[cs + m];
                     const R dkx = dk<R>(a.g.nx, kx), dky = dk<R>(a.g.ny, ky);
                     a.kpsit[m] = psit_mode(tab && kx > 0 && ky > 0, fg, dkx, dky, c1, c2, a.dex);
-                    a.kbxyz[m] = e2 * (-a.dex) - w2;
-                    a.kbxyz[cs + m] = e1 * a.dex + w1;
+                    a.kbxyz[m] = bx_mode(e2, w2, a.dex);
+                    a.kbxyz[cs + m] = by_mode(e1, w1, a.dex);
                     a.kbxyz[2 * cs + m] =
                         bz_mode(tab, kx, ky, fg, fs, dkx, dky, c1, c2) * a.dex;
                 }

@@ -1,5 +1,6 @@
 // The slice loop's k-space arithmetic of one mode, shared by the kernels that
-// run it on its own (qp_fused.hip) and between transforms (qp_spectral.hip).
+// run it on its own (qp_fused.hip) and between transforms (qp_spectral.hip).  The
+// fused products are written out (fmadd), so that all of them give the same bits.
 #pragma once
 
 #include "qp_common.h"
@@ -16,23 +17,24 @@ __device__ __forceinline__ bool corrector_mode(bool tab, int kx, int ky, R fg, R
 {
     n1 = n2 = R(0);
     if (!tab || (kx == 0 && ky == 0)) return false;
-    const R at2 = R(1) * fg / (R(1) + aa * fg);
+    const R at2 = R(1) * fg / fmadd(aa, fg, R(1));
     const R at1 = at2 * fs;
+    const R at3 = aa * at2;
     if (kx > 0 && ky > 0) {
-        d1 = -d1 + dkx * a1 - dky * a3;
-        const R aat1 = d1 - dkx * c3 * idex;
-        d2 = -d2 - dkx * a3 + dky * a2;
-        const R aat2 = d2 - dky * c3 * idex;
-        n1 = at1 * aat1 + aa * at2 * old1;
-        n2 = at1 * aat2 + aa * at2 * old2;
+        d1 = fmadd(-dky, a3, fmadd(dkx, a1, -d1));
+        const R aat1 = fmadd(-(dkx * c3), idex, d1);
+        d2 = fmadd(dky, a2, fmadd(-dkx, a3, -d2));
+        const R aat2 = fmadd(-(dky * c3), idex, d2);
+        n1 = fmadd(at3, old1, at1 * aat1);
+        n2 = fmadd(at3, old2, at1 * aat2);
     } else if (kx > 0) {
-        d1 = -d1 + dkx * a1;
-        d2 = -d2 - dkx * a3;
-        n2 = at1 * d2 + aa * at2 * old2;
+        d1 = fmadd(dkx, a1, -d1);
+        d2 = fmadd(-dkx, a3, -d2);
+        n2 = fmadd(at3, old2, at1 * d2);
     } else {
-        d1 = -d1 - dky * a3;
-        d2 = -d2 + dky * a2;
-        n1 = at1 * d1 + aa * at2 * old1;
+        d1 = fmadd(-dky, a3, -d1);
+        d2 = fmadd(dky, a2, -d2);
+        n1 = fmadd(at3, old1, at1 * d1);
     }
     return true;
 }
@@ -41,7 +43,7 @@ __device__ __forceinline__ bool corrector_mode(bool tab, int kx, int ky, R fg, R
 template <typename R>
 __device__ __forceinline__ R psit_mode(bool inner, R fg, R dkx, R dky, R c1, R c2, R dex)
 {
-    const R ps = inner ? fg * (-(dkx * c1 + dky * c2)) : R(0);
+    const R ps = inner ? fg * (-fmadd(dkx, c1, dky * c2)) : R(0);
     return ps * (-dex);
 }
 
@@ -51,18 +53,23 @@ __device__ __forceinline__ R bz_mode(bool tab, int kx, int ky, R fg, R fs, R dkx
 {
     if (!tab) return R(0);
     const R at1 = R(1) * fg * fs;
-    if (kx > 0 && ky > 0) return (dkx * at1) * c2 - (dky * at1) * c1;
+    if (kx > 0 && ky > 0) return fmadd(dkx * at1, c2, -(dky * at1 * c1));
     if (kx > 0) return dkx * at1 * c2;
     if (ky > 0) return -(dky * at1) * c1;
     return R(0);
 }
+
+// The B assembly (simulation_class.f03:677-680): B_x and B_y from the corrector's
+// (e1, e2) and the beam's (b1, b2)
+template <typename R> __device__ __forceinline__ R bx_mode(R e2, R b2, R dex) { return fmadd(e2, -dex, -b2); }
+template <typename R> __device__ __forceinline__ R by_mode(R e1, R b1, R dex) { return fmadd(e1, dex, b1); }
 
 // The seed by extrapolation in xi of one component: e = B(j-1) becomes 2 e - h
 // (seed 2) or 3 e - 3 h + g (seed 3), h = B(j-2), g = B(j-3)
 template <typename R> __device__ __forceinline__ R seed_mode(int seed, R e, R h, R g)
 {
     if (seed == 2) return R(2) * e - h;
-    if (seed == 3) return (R(3) * e - R(3) * h) + g;
+    if (seed == 3) return fmadd(R(3), e, -(R(3) * h)) + g;
     return e;
 }
 

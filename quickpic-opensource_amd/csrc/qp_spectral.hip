@@ -348,8 +348,8 @@ __device__ __forceinline__ void do_mode(const MidArgs<R> &a, int kx, int ky, int
     }
     constexpr int P = FRONT ? 3 : 0;
     out[P] = psit_mode(inner, fg, dkx, dky, c1, c2, a.dex);
-    out[P + 1] = e2 * (-a.dex) - b2;
-    out[P + 2] = e1 * a.dex + b1;
+    out[P + 1] = bx_mode(e2, b2, a.dex);
+    out[P + 2] = by_mode(e1, b1, a.dex);
     out[P + 3] = bz_mode(tab, kx, ky, fg, fs, dkx, dky, c1, c2) * a.dex;
 }
 

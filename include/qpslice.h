@@ -135,7 +135,8 @@ int qp_ctx_profile_get(qp_ctx *ctx, int kind, double *total_ms, int64_t *count,
  * separate LDS-tiled transpose; 0, 2, 3 and 4 keep the transpose and pad the
  * transforms' LDS by one point per 16 points in FP32 or 8 in FP64 (0), or per
  * 8, 32 or 4 points (2, 3, 4); 5 and 6 fold the transpose only in the k -> real
- * or only in the real -> k direction.  Results are identical.
+ * or only in the real -> k direction; 7 is the default's form of the separate
+ * transforms (0's in FP32, 1's in FP64).  Results are identical.
  * QP_TUNE_PUSH selects how the plasma push re-sorts the particles: 0 (default)
  * counts the destination bins in a first pass that stores nothing per
  * particle, then pushes again and stores every particle at its sorted place;

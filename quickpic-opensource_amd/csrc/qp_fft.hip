@@ -232,6 +232,13 @@ static int transpose(qp_ctx *c, const CompSet<R> &cs, int ncomp, int ld_src, int
     return QP_OK;
 }
 
+// the form of the separate transforms (QP_TUNE_FFT; 7: the default's)
+static int fft_form(const qp_ctx *c)
+{
+    const int v = c->tune[QP_TUNE_FFT];
+    return v == 7 ? tune_default_of(c->prec, QP_TUNE_FFT) : v;
+}
+
 // the row transforms of the transpose path; QP_TUNE_FFT values 2-4 select
 // another LDS padding (one pad point per 8, 32 or 4 points)
 template <typename R>
@@ -239,7 +246,7 @@ static int rowfft0(qp_ctx *c, const CompSet<R> &cs, int ncomp, int nrows, int n,
                    int ld_dst, int types, double scale, const cplx<R> *W, int guard_row)
 {
     constexpr int PD = pad_shift<R>();
-    switch (c->tune[QP_TUNE_FFT]) {
+    switch (fft_form(c)) {
     case 2: return rowfft<R, 0, 3>(c, cs, ncomp, nrows, n, ld_src, ld_dst, types, scale, W, guard_row);
     case 3: return rowfft<R, 0, 5>(c, cs, ncomp, nrows, n, ld_src, ld_dst, types, scale, W, guard_row);
     case 4: return rowfft<R, 0, 2>(c, cs, ncomp, nrows, n, ld_src, ld_dst, types, scale, W, guard_row);
@@ -294,7 +301,7 @@ static int r2k_core(qp_ctx *c, R *const *rs, R *const *ks, int nc, int mx, int m
     if (rc) return rc;
     // y pass straight from the column pairs of the x pass (QP_TUNE_FFT 1, or 6:
     // this direction only)
-    if (c->tune[QP_TUNE_FFT] == 1 || c->tune[QP_TUNE_FFT] == 6)
+    if (fft_form(c) == 1 || fft_form(c) == 6)
         return rowfft<R, 1, pad_shift<R>()>(c, b, nc, c->nx + 1, c->ny, ldr, ldk, my, 1.0,
                                             twy, -1);
     rc = transpose<R>(c, b, nc, ldr, ldk, c->ny + 1, c->nx + 1);
@@ -323,7 +330,7 @@ static int k2r_core(qp_ctx *c, R *const *rs, R *const *ks, int nc, int mx, int m
     int rc;
     // y pass written as column pairs of rs (QP_TUNE_FFT 1, or 5: this
     // direction only)
-    if (c->tune[QP_TUNE_FFT] == 1 || c->tune[QP_TUNE_FFT] == 5) {
+    if (fft_form(c) == 1 || fft_form(c) == 5) {
         rc = rowfft<R, 2, pad_shift<R>()>(c, yc, nc, c->nx + 1, c->ny, ldk, ldr, my, 2.0, twy,
                                           -1);
     } else {

@@ -185,3 +185,28 @@ stub.stub_limits(163840, 256)
 conv(16, 16, 16, 16)
 assert stub.stub_lds(b"k_conv3x3") == (18 * 3 + 144) * 48
 """)
+
+
+@pytest.mark.parametrize("precision", ["FP32", "FP64"])
+def test_default_form_of_the_separate_transforms(stub, precision):
+    """QP_TUNE_FFT 7: what the default's number names, a transpose between row
+    passes (FP32) or column pairs (FP64), without the default's fused routes."""
+    run(stub, f"""
+ctx = qps.Ctx(5, 5, 4, precision=qps.{precision})
+sim = qps.Sim(ctx, [qps.Species(ctx, ppc=(1, 1))], [])
+
+def kernels(value):
+    ctx.tune(qps.TUNE_FFT, value)
+    stub.stub_clear_launches()
+    f = qps.Field2d(ctx, 1)
+    f.fftrk(1)
+    f.fftkr(1)
+    sim.begin_step()
+    sim.slice(1)
+    return [stub.stub_launched(k) > 0 for k in (b"k_mid", b"k_fft_xt", b"k_transpose")]
+
+fp32 = {precision == "FP32"}
+assert kernels(-1) == [True, True, False]
+assert kernels(7) == [False, False, fp32]
+assert kernels(1) == [not fp32, not fp32, False]
+""")

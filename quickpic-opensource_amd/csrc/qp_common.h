@@ -24,6 +24,7 @@
 namespace qp {
 
 constexpr int TILE = 16;                 // cells per tile edge (part2d_class.f03:99)
+constexpr int PITCH = 64;                // row pitches of planes are multiples of it
 constexpr int TCELLS = TILE * TILE;      // cells per tile = threads per particle block
 constexpr int HALO = 4 * TILE;           // border nodes of a 17x17 tile block
 // border nodes of a band of rb of a tile's rows, 17 x (rb + 1) nodes

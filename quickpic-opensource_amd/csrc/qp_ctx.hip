@@ -262,8 +262,8 @@ int qp_ctx_create(int indx, int indy, int indz, const double box[6], int precisi
     c->dex = (box[1] - box[0]) / (double)(1 << indx);
     c->dey = (box[3] - box[2]) / (double)(1 << indy);
     c->dxi = (box[5] - box[4]) / (double)(1 << indz);
-    c->ldr = (int)round_up((size_t)c->nx + 1, 64);
-    c->ldk = (int)round_up((size_t)c->ny + 1, 64);
+    c->ldr = (int)round_up((size_t)c->nx + 1, PITCH);
+    c->ldk = (int)round_up((size_t)c->ny + 1, PITCH);
     c->rplane = (size_t)(c->ny + 1) * c->ldr;
     c->kplane = (size_t)(c->nx + 1) * c->ldk;
     c->mx1 = c->nx / TILE;

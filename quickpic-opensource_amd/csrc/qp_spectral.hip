@@ -45,7 +45,7 @@ template <typename R> struct alignas(16) Quad {
 };
 
 // Shape of k_fft_xt: FB row pairs per workgroup, so that the transposed side
-// moves 2 FB Reals (16 to 64 bytes) of a column at a time; workgroups next to
+// moves 2 FB Reals (16 to 256 bytes) of a column at a time; workgroups next to
 // each other complete its cache lines in one L2.  Small ones: their waits at
 // barriers cover each other.  512^2 FP32, forward and inverse: 16 rows (1024
 // threads) 11.8 and 8.9 us, 8 rows 10.1 and 7.2; 1024^2 8 rows 27.4 and 17.4,
@@ -65,6 +65,9 @@ template <typename R, int L> struct XtShape {
     static constexpr size_t LDS = (size_t)FB * S::LDSM * sizeof(cplx<R>);
     static_assert((size_t)(S::N + 1) * SW * sizeof(R) <= LDS, "staging fits the FFT's area");
     static_assert(LDS <= 81920, "two workgroups on a CU");
+    // the last workgroup's rows go on past ny; its columns stay in the pitch,
+    // which is the next multiple of PITCH above ny
+    static_assert(PITCH % ROWS == 0, "whole workgroups of rows in the pitch");
 };
 
 // Up to this nx the forward x transforms form the border sums of the deposit in
@@ -236,7 +239,7 @@ k_fft_xt(XtSet<R> cs, int nrows, int ld_src, int ld_dst, int types, R scale,
     for (int i = 0; i < 4; ++i) stage(t + i * TF, z[i]);
     if (t == 0) stage(N, zn);
     __syncthreads();
-    // columns y0 .. y0 + ROWS - 1 lie within the pitch (ld_dst > ny + 15)
+    // columns y0 .. y0 + ROWS - 1 lie within the pitch (XtShape)
     auto put = [&](int kx, int c) {
         Quad<R> q;
 #pragma unroll

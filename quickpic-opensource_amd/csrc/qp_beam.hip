@@ -26,6 +26,8 @@ struct qp_beam {
     qp::DevBuf live, sort_tmp, moments;
     qp::DevBuf key[2], perm[2];  // push: cell keys and particle indices, before and after the sort
     size_t sort_bytes;           // temporary bytes of the sort
+    double run_len = 0.0;        // mean run of particles of one cell, as the last push sorted
+                                 // them (0: not known); only selects the deposit's kernel
     int key_shift, key_bits;     // cell key = linear cell index >> key_shift, below 2^key_bits
     unsigned key_drop;           // key of a dropped particle (sorts last)
     qp::DevBuf q3;               // int64 [nz+1][ny+1][ldr]
@@ -288,23 +290,35 @@ static int64_t load_beam_twiss(qp_ctx *c, const qp_beam_twiss_params &bp, uint64
 }
 
 // PGPOST32L (part3d_lib77.f:554-628), int64 fixed-point accumulation.
-// The push leaves the beam sorted by cell.  A thread takes DEP_RUN particles in
-// order and adds them up while they stay in one cell; the last cells of a
-// wavefront's threads, where they are the same on neighbouring lanes, are summed
-// across the wavefront, and the first lane of each such run adds the sums with
-// one atomic per node.  Integer sums make the charge the same, bit for bit, as
-// one atomic per particle and node, whatever the particle order.  (One particle
-// a thread summed each of them across the wavefront, 102 lane exchanges: 96 us
-// for 4 M sorted particles against 46 us, whose positions and charges are read
-// in 27 us at the rate of a copy.)
+// The push leaves the beam sorted by cell, so particles next to each other share
+// their nodes.  A thread takes RUN particles in order and adds them up while they
+// stay in one cell; the last cells of a wavefront's threads, where they are the
+// same on neighbouring lanes, are summed across the wavefront, and the first lane
+// of each such run adds the sums with one atomic per node.  Integer sums make the
+// charge the same, bit for bit, as one atomic per particle and node, whatever the
+// particle order and RUN.
+//  RUN = 8: the 102 lane exchanges of the sum are paid once for 512 particles, but a
+//    cell that ends inside a thread is added by that thread alone, cache lines away
+//    from its neighbours' cells.
+//  RUN = 1: 102 exchanges for 64 particles; neighbouring lanes hold neighbouring
+//    cells, whose atomics meet in one line.
+// 4 M sorted particles, RUN 1 and 8, by their mean run in a cell: 1400 308 and 49 us
+// (whose positions and charges are read in 27 us at the rate of a copy), 200 141
+// and 36, 37 90 and 71, 22 131 and 146, 10 97 and 160, 2.6 186 and 543, 1.6 329
+// and 905; in random order 1570 either way.  Fewer particles than fill the chip's
+// waves by eights: 32768 of runs of 162 11.0 and 10.2 us, of 61 9.4 and 10.7, of 1.7
+// 11 and 34.
 constexpr int DEP_RUN = 8;
+constexpr double DEP_LONG = 26.0, DEP_LONG_FEW = 128.0;   // runs from which on RUN = 8 is taken
+constexpr int64_t DEP_FEW = 1 << 17;                      // beams below it: DEP_LONG_FEW
 
+template <int RUN>
 __global__ __launch_bounds__(256) void k_beam_deposit(
     int64_t np, const double *__restrict__ x, const double *__restrict__ y,
     const double *__restrict__ z, const double *__restrict__ q, unsigned long long *q3, int ld,
     size_t pl, int nx, int ny, int nz)
 {
-    const int64_t j0 = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) * DEP_RUN;
+    const int64_t j0 = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) * RUN;
     const int lane = threadIdx.x & 63;
     constexpr unsigned long long NONE = ~0ull;
     unsigned long long cell = NONE;
@@ -315,11 +329,11 @@ __global__ __launch_bounds__(256) void k_beam_deposit(
 #pragma unroll
         for (int k = 0; k < 8; ++k) atomicAdd(b + o[k], (unsigned long long)w[k]);
     };
-    double px[DEP_RUN], py[DEP_RUN], pz[DEP_RUN], pq[DEP_RUN];
-    if (j0 + DEP_RUN <= np) {
+    double px[RUN], py[RUN], pz[RUN], pq[RUN];
+    if (RUN % 2 == 0 && j0 + RUN <= np) {
         // 16 bytes at a time: the arrays are allocations, j0 a multiple of 8
 #pragma unroll
-        for (int r = 0; r < DEP_RUN; r += 2) {
+        for (int r = 0; r + 1 < RUN; r += 2) {
             const double2 a = *reinterpret_cast<const double2 *>(x + j0 + r);
             const double2 b = *reinterpret_cast<const double2 *>(y + j0 + r);
             const double2 c = *reinterpret_cast<const double2 *>(z + j0 + r);
@@ -331,7 +345,7 @@ __global__ __launch_bounds__(256) void k_beam_deposit(
         }
     } else {
 #pragma unroll
-        for (int r = 0; r < DEP_RUN; ++r) {
+        for (int r = 0; r < RUN; ++r) {
             const int64_t j = j0 + r;
             // a place behind the last particle is outside the grid
             px[r] = j < np ? x[j] : -1.0;
@@ -341,7 +355,7 @@ __global__ __launch_bounds__(256) void k_beam_deposit(
         }
     }
 #pragma unroll
-    for (int r = 0; r < DEP_RUN; ++r) {
+    for (int r = 0; r < RUN; ++r) {
         // a particle outside the grid has no nodes to deposit to
         if (!(px[r] >= 0.0 && px[r] < (double)nx && py[r] >= 0.0 && py[r] < (double)ny &&
               pz[r] >= 0.0 && pz[r] < (double)nz))
@@ -443,10 +457,11 @@ template <typename R>
 __global__ void k_beam_push(int64_t np, Ptr7 a, const R *__restrict__ e3,
                             const R *__restrict__ b3, size_t vol, int ld, size_t pl, double qtmh,
                             double dtcx, double dtcz, double rx, double ry, double rz, CellKey ck,
-                            unsigned *key)
+                            unsigned *key, int *changes)
 {
     const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (i >= np) return;
+    if (i == 0) *changes = 0;   // k_permute counts
     double X = a.p[0][i], Y = a.p[1][i], Z = a.p[2][i];
     // outside the grid nothing can be gathered: dropped without touching the
     // fields (the loader and the push keep every particle in [1, n-1))
@@ -500,14 +515,21 @@ __global__ void k_beam_push(int64_t np, Ptr7 a, const R *__restrict__ e3,
 // Survivor i of the cell-sorted beam is particle perm[i].  Thread i also finds
 // the number of survivors, where the sorted keys turn to `drop` (a flag per
 // particle and their scan took 30 us of 4 M particles, and the host waited for
-// it before the sort).
+// it before the sort).  Every `every`-th block counts the places where the key
+// changes, *changes in all, for the deposit's choice of a kernel.
 __global__ void k_permute(int64_t np, const unsigned *__restrict__ key, unsigned drop,
-                          const unsigned *__restrict__ perm, Ptr7 src, Ptr7 dst, int *nlive)
+                          const unsigned *__restrict__ perm, Ptr7 src, Ptr7 dst, int *nlive,
+                          int *changes, unsigned every)
 {
     const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const unsigned k0 = i < np ? key[i] : drop, k1 = i + 1 < np ? key[i + 1] : drop;
+    if (blockIdx.x % every == 0) {
+        const unsigned long long m = __ballot(k0 != k1);
+        if ((threadIdx.x & 63) == 0 && m) atomicAdd(changes, __popcll(m));
+    }
     if (i >= np) return;
-    const bool gone = key[i] == drop;
-    if (gone ? i == 0 : i + 1 == np || key[i + 1] == drop) *nlive = gone ? 0 : (int)(i + 1);
+    const bool gone = k0 == drop;
+    if (gone ? i == 0 : k1 == drop) *nlive = gone ? 0 : (int)(i + 1);
     if (gone) return;
     const unsigned s = perm[i];
 #pragma unroll
@@ -560,7 +582,7 @@ static int beam_alloc(qp_beam *b, int64_t n)
         if (!rc) rc = b->b[k].alloc((size_t)n * 8);
         if (rc) return rc;
     }
-    int rc = b->live.alloc(sizeof(int));
+    int rc = b->live.alloc(2 * sizeof(int));
     for (int k = 0; k < 2 && !rc; ++k) {
         rc = b->key[k].alloc((size_t)(n + 1) * 4);
         if (!rc) rc = b->perm[k].alloc((size_t)(n + 1) * 4);
@@ -595,6 +617,7 @@ static int beam_set(qp_beam *b, std::vector<double> (&h)[7], int64_t n)
                               c->stream));
     QP_HIP(hipStreamSynchronize(c->stream));
     b->np = n;
+    b->run_len = 0.0;
     return QP_OK;
 }
 
@@ -831,9 +854,11 @@ int qp_beam_qdp(qp_beam *b)
     if (b->np > 0) {
         {
         ProfScope _ps(c, QP_PROF_BEAM_DEPOSIT, 4.0 * 8.0 * (double)b->np);
-        const int64_t per = 256 * DEP_RUN;
-        hipLaunchKernelGGL(k_beam_deposit, dim3((unsigned)((b->np + per - 1) / per)), dim3(256), 0,
-                           c->stream, b->np, b->a[0].as<double>(), b->a[1].as<double>(),
+        const bool runs = b->run_len >= (b->np < DEP_FEW ? DEP_LONG_FEW : DEP_LONG);
+        const int64_t per = 256 * (runs ? DEP_RUN : 1);
+        auto kern = runs ? k_beam_deposit<DEP_RUN> : k_beam_deposit<1>;
+        hipLaunchKernelGGL(kern, dim3((unsigned)((b->np + per - 1) / per)), dim3(256), 0, c->stream,
+                           b->np, b->a[0].as<double>(), b->a[1].as<double>(),
                            b->a[2].as<double>(), b->a[6].as<double>(),
                            b->q3.as<unsigned long long>(), c->ldr, c->rplane, c->nx, c->ny,
                            c->nz);
@@ -916,11 +941,14 @@ int qp_beam_push(qp_beam *b, const qp_field3d *ef, const qp_field3d *bf, double 
     Ptr7 src, dst;
     for (int k = 0; k < 7; ++k) { src.p[k] = b->a[k].as<double>(); dst.p[k] = b->b[k].as<double>(); }
     unsigned *key = b->key[0].as<unsigned>(), *sorted = b->key[1].as<unsigned>();
+    int *counts = b->live.as<int>();   // survivors, changes of key in the blocks that count
+    const unsigned every = std::max(1u, grid.x / 256);
     auto push = [&](auto kern, auto zero) {
         using R = decltype(zero);
         hipLaunchKernelGGL(kern, grid, dim3(256), 0, c->stream, np, src, ef->buf.as<R>(),
                            bf->buf.as<R>(), vol, c->ldr, c->rplane, qtmh, dtcx, dtcz,
-                           (double)(c->nx - 1), (double)(c->ny - 1), (double)(c->nz - 1), ck, key);
+                           (double)(c->nx - 1), (double)(c->ny - 1), (double)(c->nz - 1), ck, key,
+                           counts + 1);
     };
     {
     ProfScope _ps(c, QP_PROF_BEAM_PUSH, (12.0 * 8.0 + 4.0) * (double)np);   // 6 read, 6 written, key
@@ -949,14 +977,17 @@ int qp_beam_push(qp_beam *b, const qp_field3d *ef, const qp_field3d *bf, double 
     // key and place read, 7 read and written
     ProfScope _ps(c, QP_PROF_BEAM_PUSH, (7.0 * 8.0 * 2.0 + 8.0) * (double)np);
     hipLaunchKernelGGL(k_permute, grid, dim3(256), 0, c->stream, np, sorted, b->key_drop,
-                       b->perm[1].as<unsigned>(), src, dst, b->live.as<int>());
+                       b->perm[1].as<unsigned>(), src, dst, counts, counts + 1, every);
     }
     QP_LAUNCH_CHECK();
-    int live = 0;
-    QP_HIP(hipMemcpyAsync(&live, b->live.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    int h[2] = {0, 0};
+    QP_HIP(hipMemcpyAsync(h, counts, sizeof(h), hipMemcpyDeviceToHost, c->stream));
     QP_HIP(hipStreamSynchronize(c->stream));
     for (int k = 0; k < 7; ++k) std::swap(b->a[k], b->b[k]);
-    b->np = live;
+    b->np = h[0];
+    // a key of several cells says nothing about runs of one
+    const double counted = (double)((grid.x + every - 1) / every) / (double)grid.x;
+    b->run_len = b->key_shift ? 0.0 : (double)b->np * counted / std::max(1.0, (double)h[1]);
     return QP_OK;
 }
 

@@ -35,6 +35,7 @@ int fail_launch = 0;       // the graph launch (counted from now) that fails
 int graph_launches = 0, instantiations = 0;
 size_t residual_bytes = 0; // a graph launch fills the host allocations of this size
 double residual = 0.0;     // with this value
+int key_changes = 0;       // what a beam push counts
 }  // namespace
 
 extern "C" {
@@ -42,6 +43,7 @@ extern "C" {
 void stub_limits(int lds, int units) { max_lds = lds; cus = units; }
 void stub_fail_launch(int n) { fail_launch = n; }
 void stub_residual(size_t n, double v) { residual_bytes = n; residual = v; }
+void stub_key_changes(int n) { key_changes = n; }
 int stub_graph_launches() { return graph_launches; }
 int stub_instantiations() { return instantiations; }
 int stub_syncs(int stream) { return streams[stream]->syncs; }
@@ -110,6 +112,11 @@ hipError_t hipLaunchKernel(const void *fn, dim3 g, dim3 b, void **args, size_t l
         int *ctl = *static_cast<int **>(args[0]);
         ctl[0] = 1;
         ctl[1] = 0;
+    }
+    if (names[fn].find("k_permute") != std::string::npos && names[fn].find("PiS3_j") != std::string::npos) {
+        // a beam push: every particle lives, and this many places change cell
+        **static_cast<int **>(args[6]) = (int)*static_cast<long long *>(args[0]);
+        **static_cast<int **>(args[7]) = key_changes;
     }
     return hipSuccess;
 }

@@ -515,17 +515,23 @@ __global__ void k_beam_push(int64_t np, Ptr7 a, const R *__restrict__ e3,
 // Survivor i of the cell-sorted beam is particle perm[i].  Thread i also finds
 // the number of survivors, where the sorted keys turn to `drop` (a flag per
 // particle and their scan took 30 us of 4 M particles, and the host waited for
-// it before the sort).  Every `every`-th block counts the places where the key
-// changes, *changes in all, for the deposit's choice of a kernel.
+// it before the sort).  The first wavefront of every `every`-th block counts the
+// places where the key changes, *changes in all, for the deposit's choice of a
+// kernel: up to 127 wavefronts, as their atomics meet in one word (1024 took 11
+// us), each in `samples` stretches of 64 particles from its block to the next.
 __global__ void k_permute(int64_t np, const unsigned *__restrict__ key, unsigned drop,
                           const unsigned *__restrict__ perm, Ptr7 src, Ptr7 dst, int *nlive,
-                          int *changes, unsigned every)
+                          int *changes, unsigned every, int samples)
 {
     const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     const unsigned k0 = i < np ? key[i] : drop, k1 = i + 1 < np ? key[i + 1] : drop;
-    if (blockIdx.x % every == 0) {
-        const unsigned long long m = __ballot(k0 != k1);
-        if ((threadIdx.x & 63) == 0 && m) atomicAdd(changes, __popcll(m));
+    if (blockIdx.x % every == 0 && threadIdx.x < 64) {
+        int n = 0;
+        for (int m = 0; m < samples; ++m) {
+            const int64_t j = i + m * (int64_t)(every * 256 / samples);
+            n += __popcll(__ballot(j < np && key[j] != (j + 1 < np ? key[j + 1] : drop)));
+        }
+        if (threadIdx.x == 0 && n) atomicAdd(changes, n);
     }
     if (i >= np) return;
     const bool gone = k0 == drop;
@@ -941,8 +947,9 @@ int qp_beam_push(qp_beam *b, const qp_field3d *ef, const qp_field3d *bf, double 
     Ptr7 src, dst;
     for (int k = 0; k < 7; ++k) { src.p[k] = b->a[k].as<double>(); dst.p[k] = b->b[k].as<double>(); }
     unsigned *key = b->key[0].as<unsigned>(), *sorted = b->key[1].as<unsigned>();
-    int *counts = b->live.as<int>();   // survivors, changes of key in the blocks that count
-    const unsigned every = std::max(1u, grid.x / 256);
+    int *counts = b->live.as<int>();   // survivors, changes of key where they are counted
+    const unsigned every = std::max(1u, grid.x / 64);
+    const int samples = every > 1 ? 8 : 1;
     auto push = [&](auto kern, auto zero) {
         using R = decltype(zero);
         hipLaunchKernelGGL(kern, grid, dim3(256), 0, c->stream, np, src, ef->buf.as<R>(),
@@ -977,7 +984,8 @@ int qp_beam_push(qp_beam *b, const qp_field3d *ef, const qp_field3d *bf, double 
     // key and place read, 7 read and written
     ProfScope _ps(c, QP_PROF_BEAM_PUSH, (7.0 * 8.0 * 2.0 + 8.0) * (double)np);
     hipLaunchKernelGGL(k_permute, grid, dim3(256), 0, c->stream, np, sorted, b->key_drop,
-                       b->perm[1].as<unsigned>(), src, dst, counts, counts + 1, every);
+                       b->perm[1].as<unsigned>(), src, dst, counts, counts + 1, every,
+                       samples);
     }
     QP_LAUNCH_CHECK();
     int h[2] = {0, 0};
@@ -986,8 +994,12 @@ int qp_beam_push(qp_beam *b, const qp_field3d *ef, const qp_field3d *bf, double 
     for (int k = 0; k < 7; ++k) std::swap(b->a[k], b->b[k]);
     b->np = h[0];
     // a key of several cells says nothing about runs of one
-    const double counted = (double)((grid.x + every - 1) / every) / (double)grid.x;
-    b->run_len = b->key_shift ? 0.0 : (double)b->np * counted / std::max(1.0, (double)h[1]);
+    double counted = 0.0;
+    for (int64_t j = 0; j < np; j += (int64_t)every * 256)
+        for (int m = 0; m < samples; ++m)
+            counted += std::max<int64_t>(
+                0, std::min<int64_t>(64, np - j - m * (int64_t)(every * 256 / samples)));
+    b->run_len = b->key_shift ? 0.0 : counted / std::max(1, h[1]);
     return QP_OK;
 }
 

@@ -113,7 +113,7 @@ hipError_t hipLaunchKernel(const void *fn, dim3 g, dim3 b, void **args, size_t l
         ctl[0] = 1;
         ctl[1] = 0;
     }
-    if (names[fn].find("k_permute") != std::string::npos && names[fn].find("PiS3_j") != std::string::npos) {
+    if (names[fn].find("k_permute") != std::string::npos && names[fn].find("PiS3_ji") != std::string::npos) {
         // a beam push: every particle lives, and this many places change cell
         **static_cast<int **>(args[6]) = (int)*static_cast<long long *>(args[0]);
         **static_cast<int **>(args[7]) = key_changes;

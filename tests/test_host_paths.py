@@ -213,9 +213,9 @@ assert kernels(1) == [not fp32, not fp32, False]
 
 
 @pytest.mark.parametrize("np_,runs,dense", [
-    ((64, 64, 32), 1, True), ((64, 64, 32), 131072 // 27, True), ((64, 64, 32), 131072 // 25, False),
-    ((64, 64, 32), 131072, False), ((16, 16, 16), 4096 // 129, True),
-    ((16, 16, 16), 4096 // 127 + 1, False), ((16, 16, 16), 4096, False)])
+    ((64, 64, 32), 1, True), ((64, 64, 32), 131072 // 28, True), ((64, 64, 32), 131072 // 24, False),
+    ((64, 64, 32), 131072, False), ((16, 16, 16), 4096 // 200, True), ((16, 16, 16), 4096 // 100, False),
+    ((16, 16, 16), 4096, False)])
 def test_beam_deposit_by_the_runs_of_the_last_push(stub, np_, runs, dense):
     """Eight particles a thread where the push found long runs of one cell, one a
     thread where it found short ones, and where the order is not known: before the
@@ -225,8 +225,11 @@ ctx = qps.Ctx(4, 4, 4)
 bm = qps.Beam(ctx, np_={np_}, sigma=(1.0, 1.0, 1.0), center=(0.0, 0.0, 5.0), peak=1.0)
 n = bm.np
 blocks = (n + 255) // 256
-every = max(1, blocks // 256)
-stub.stub_key_changes(max(1, {runs} * ((blocks + every - 1) // every) // blocks))
+every = max(1, blocks // 64)
+samples = 8 if every > 1 else 1
+counted = sum(max(0, min(64, n - j - m * every * 256 // samples))
+              for j in range(0, n, every * 256) for m in range(samples))
+stub.stub_key_changes(max(1, round({runs} * counted / n)))
 e, b = qps.Field3d(ctx, 3), qps.Field3d(ctx, 3)
 
 def eights():

@@ -67,10 +67,13 @@ __device__ __forceinline__ v4s load4(const uint16_t *p)
 //  k_conv3x3_deep: the others, operands not aligned to 16 bytes, and devices whose
 //    workgroups have less LDS than a layer asks for.  The chain is cut in groups of
 //    9 steps, whose loads are issued before the group in front is multiplied.
-// One wave with all output channels of its pixels, loading step by step, took
-// 33.7 us a convolution (27 of a training step); all by k_conv3x3_deep 11.8 us,
-// by k_conv3x3 5.7 us (8.2 us with the channel count as an argument: a wave alone
-// on its SIMD then waited for the scalar address arithmetic of each step).
+//  k_conv3x3_wide: those where the plane alone fills the device with waves.  A wave
+//    computes all output channels of its pixels, step by step, and reads them once
+//    in place of once for every 16 output channels.
+// All by k_conv3x3_wide took 33.7 us a convolution (27 of a training step), by
+// k_conv3x3_deep 11.8 us, by k_conv3x3 5.7 us (8.2 us with the channel count as an
+// argument: a wave alone on its SIMD then waited for the scalar address arithmetic
+// of each step).
 // ---------------------------------------------------------------------------
 // D[pixel 4q+i][co]: pixels xp.. of row y
 __device__ __forceinline__ void conv_store(v4f acc, const float *bias, int co, int y, int xp, int W,
@@ -247,6 +250,66 @@ k_conv3x3_deep(const uint16_t *__restrict__ x, const uint16_t *__restrict__ mask
         multiply(f1);
     }
     conv_store(acc, bias, co, y, px0 + 4 * q, W, out, cs_out, relu, accum);
+}
+
+constexpr int MAXNT = 12;   // 192 output channels
+
+__global__ void __launch_bounds__(256)
+k_conv3x3_wide(const uint16_t *__restrict__ x, const uint16_t *__restrict__ mask, int H, int W,
+               int gw, int cs_in, int Cin, const uint16_t *__restrict__ w,
+               const float *__restrict__ bias, uint16_t *out, int cs_out, int Cout, int relu,
+               int accum)
+{
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = blockIdx.x * 4 + wave;              // this wave's pixel group
+    if (g >= H * gw) return;
+    const int y = g / gw, px0 = (g - y * gw) * 16;
+    const int m = lane & 15, q = lane >> 4;           // A row (pixel) and k quad
+    const int NT = Cout >> 4;
+    v4f acc[MAXNT];
+#pragma unroll
+    for (int t = 0; t < MAXNT; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
+    for (int tap = 0; tap < 9; ++tap) {
+        const int yy = y + tap / 3 - 1, xx = px0 + m + tap % 3 - 1;
+        const bool in = yy >= 0 && yy < H && xx >= 0 && xx < W;
+        const size_t pix = in ? ((size_t)yy * W + xx) * cs_in : 0;
+        for (int c0 = 0; c0 < Cin; c0 += 16) {
+            v4s a = {0, 0, 0, 0};
+            if (in) {
+                a = load4(x + pix + c0 + 4 * q);
+                if (mask) {
+                    const v4s mk = load4(mask + pix + c0 + 4 * q);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (!(bf2f((uint16_t)mk[i]) > 0.f)) a[i] = 0;
+                }
+            }
+            const uint16_t *wt = w + ((size_t)tap * Cout + m) * Cin + c0 + 4 * q;
+#pragma unroll
+            for (int t = 0; t < MAXNT; ++t)
+                if (t < NT)
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+                        a, load4(wt + (size_t)t * 16 * Cin), acc[t], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < MAXNT; ++t)
+        if (t < NT)
+            conv_store(acc[t], bias, 16 * t + m, y, px0 + 4 * q, W, out, cs_out, relu, accum);
+}
+
+// Whether k_conv3x3_wide takes a layer that k_conv3x3 does not: from this many
+// pixel groups a compute unit on.  Ratio of k_conv3x3_wide's time to
+// k_conv3x3_deep's on 128^2 (4 groups a unit), 160^2 (6), 192^2 (9), 224^2 (12) and
+// 256^2 (16): 80 -> 192 channels 1.43, 0.96, 0.83, 0.75, 0.65; 80 -> 48 1.49, 1.13,
+// 1.03, 0.87, 0.74; 256 -> 96 0.72 .. 0.59; 256 -> 32 1.07, 0.80, 0.90, 0.86, 0.75;
+// 64 -> 96, not aligned, 1.13, 1.08, 1.10, 1.08, 0.86; 16 output channels 1.0 at most.
+static bool conv_wide(int cus, long long groups, int cin, int cout)
+{
+    if (cout < 32) return false;
+    const int need = cin < 80 ? 14 : cin <= 208 ? (cout >= 96 ? 6 : 10) : (cout >= 48 ? 4 : 6);
+    return groups >= (long long)need * cus;
 }
 
 // ---------------------------------------------------------------------------
@@ -915,6 +978,13 @@ static int conv3x3(const NetDevice *dev, hipStream_t st, const uint16_t *x, cons
         }
 #undef CONV_CASE
         RC(rc);
+        QP_LAUNCH_CHECK();
+        return QP_OK;
+    }
+    if (conv_wide(dev->cus, (long long)H * gw, cin, cout)) {
+        hipLaunchKernelGGL(k_conv3x3_wide, dim3((unsigned)(((size_t)H * gw + 3) / 4)), dim3(256), 0,
+                           st, x, mask, H, W, gw, cs_in, cin, w, bias, out, cs_out, cout, relu,
+                           accum);
         QP_LAUNCH_CHECK();
         return QP_OK;
     }

@@ -245,3 +245,15 @@ assert eights() == {dense}
 bm.upload(bm.download())
 assert not eights()
 """)
+
+
+@pytest.mark.parametrize("H,W,cin,cout,wide", [
+    (256, 256, 80, 48, True), (128, 128, 80, 48, False), (160, 160, 160, 96, True),
+    (128, 128, 256, 48, True), (256, 256, 80, 16, False), (256, 256, 64, 64, False)])
+def test_convolution_of_a_large_plane(stub, H, W, cin, cout, wide):
+    """Channel counts without a kernel of their own: all output channels in a wave
+    where the plane has waves enough, 16 in a wave elsewhere."""
+    run(stub, CONV + f"""
+conv({H}, {W}, {cin}, {cout})
+assert stub.stub_launched(b"k_conv3x3_wide") == {int(wide)}
+""")

@@ -130,7 +130,7 @@ int qp_ctx_profile_get(qp_ctx *ctx, int kind, double *total_ms, int64_t *count,
  * QP_TUNE_FFT at its default (0 in FP32, 1 in FP64) lets the slice loop run its
  * field solves with the y transforms and the modes in one kernel (both sides up
  * to 1024), and the FP32 transforms of whole fields without a transpose (nx up
- * to 2048).  Otherwise 1 folds the transpose between the x and y passes of
+ * to 1024, at 2048 from 512 rows on).  Otherwise 1 folds the transpose between the x and y passes of
  * every transform into the y pass (column-pair reads / writes) instead of a
  * separate LDS-tiled transpose; 0, 2, 3 and 4 keep the transpose and pad the
  * transforms' LDS by one point per 16 points in FP32 or 8 in FP64 (0), or per

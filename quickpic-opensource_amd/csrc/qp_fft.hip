@@ -345,13 +345,18 @@ static int k2r_core(qp_ctx *c, R *const *rs, R *const *ks, int nc, int mx, int m
 // Whether the x pass reads or writes the columns that the y pass works on
 // (k_fft_xt), two launches in place of three.  FP32, both directions, one and
 // three components: 64 x 32 19.5 -> 13.5 us; 512^2 25.3 and 33.4 -> 21.0 and
-// 25.3; 1024^2 37 and 59 -> 29 and 53; 2048^2 70.6 and 157 -> 69.6 and 151; longer
-// x transforms do not fit the workgroup's LDS.  FP64's column pairs take two
+// 25.3; 1024^2 37 and 59 -> 29 and 53; 2048^2 70.6 and 157 -> 69.6 and 151.  At nx =
+// 2048 a workgroup holds 4 rows, and few rows in all wait for each other longer
+// than a launch takes: 2048 x 32 23.1 and 23.9 against 26.8 and 28.0 us, x 128 26.3
+// and 32.7 against 28.9 and 33.6, x 256 28.7 and 42.9 against 30.1 and 38.4.
+// Longer x transforms do not fit the workgroup's LDS.  FP64's column pairs take two
 // launches already (512^2 23.2 and 35.9 against 26.4 and 35.3 us so).  The
-// knob's other values keep the transpose or the column pairs.
-static bool x_columns(const qp_ctx *c)
+// knob's other values keep the transpose or the column pairs.  nc: components of
+// the batch.
+static bool x_columns(const qp_ctx *c, int nc)
 {
-    return c->prec == QP_FP32 && c->nx <= 2048 && c->max_lds >= 81920 &&
+    return c->prec == QP_FP32 && (c->nx <= 1024 || (c->nx == 2048 && nc * c->ny >= 512)) &&
+           c->max_lds >= 81920 &&
            c->tune[QP_TUNE_FFT] == tune_default_of(c->prec, QP_TUNE_FFT);
 }
 
@@ -363,7 +368,7 @@ static int r2k_t(qp_ctx *c, qp_field2d *const *fs, const int *kinds, int nf)
     const int nc = gather_comps<R>(fs, kinds, nf, rs, ks, &mx, &my);
     if (nc <= 0) return nc;
     if constexpr (std::is_same<R, float>::value) {
-        if (x_columns(c)) {
+        if (x_columns(c, nc)) {
             CompSet<R> y{};
             for (int i = 0; i < nc; ++i) y.src[i] = y.dst[i] = ks[i];
             int rc = fft_x_to_columns(c, rs, ks, nc, mx);
@@ -384,7 +389,7 @@ static int k2r_t(qp_ctx *c, qp_field2d *const *fs, const int *kinds, int nf)
     const int nc = gather_comps<R>(fs, kinds, nf, rs, ks, &mx, &my);
     if (nc <= 0) return nc;
     if constexpr (std::is_same<R, float>::value) {
-        if (x_columns(c)) {
+        if (x_columns(c, nc)) {
             R *sk[MAX_BATCH];
             CompSet<R> y{};
             for (int i = 0; i < nc; ++i) {

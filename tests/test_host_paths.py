@@ -257,3 +257,17 @@ def test_convolution_of_a_large_plane(stub, H, W, cin, cout, wide):
 conv({H}, {W}, {cin}, {cout})
 assert stub.stub_launched(b"k_conv3x3_wide") == {int(wide)}
 """)
+
+
+@pytest.mark.parametrize("indy,dim,columns", [(5, 1, False), (7, 3, False), (8, 1, False),
+                                              (8, 2, True), (9, 1, True)])
+def test_transforms_of_long_rows(stub, indy, dim, columns):
+    """FP32 transforms at nx = 2048: through transposed planes with rows enough."""
+    run(stub, f"""
+ctx = qps.Ctx(11, {indy}, 4, precision=qps.FP32)
+f = qps.Field2d(ctx, {dim})
+f.fftrk(1)
+f.fftkr(1)
+assert stub.stub_launched(b"k_fft_xt") == {2 * columns}
+assert stub.stub_launched(b"k_transpose") == {2 * (not columns)}
+""")

@@ -221,6 +221,35 @@ __device__ __forceinline__ void emit_nodes(const R *nacc, const DepOut<R> &out, 
     }
 }
 
+// The same for the eight components of the current deposit, 289 nodes apart in LDS,
+// all added to planes (DepOut::inner, no outer).  The planes that are added to are read for all of a node's components before the first
+// store: the compiler does not know that the stores leave them alone, and read them
+// one after the other.
+template <typename R, int RB>
+__device__ __forceinline__ void emit_nodes8(const R *nacc, const DepOut<R> &out, int ldr, R *halo,
+                                            size_t halo_cs, int tile, int tx, int ty, int band)
+{
+    for (int n = threadIdx.x; n < 17 * (RB + 1); n += TCELLS) {
+        const int i = n % 17, j = n / 17;
+        if (i >= 1 && i < TILE && j >= 1 && j < RB) {
+            const size_t idx = (size_t)(ty * TILE + band * RB + j) * ldr + tx * TILE + i;
+            R in[8];
+#pragma unroll
+            for (int c = 0; c < 8; ++c) in[c] = out.inner[c][idx];
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {   // dep_store, with no outer plane
+                const R v = nacc[c * 289 + n];
+                if (out.p2[c]) out.p2[c][idx] = v * out.scale2;
+                out.p[c][idx] = (v + in[c]) * out.scale;
+            }
+        } else {
+            R *h = halo + (size_t)(tile * (TILE / RB) + band) * band_halo(RB) + halo_index(RB, i, j);
+#pragma unroll
+            for (int c = 0; c < 8; ++c) h[c * halo_cs] = nacc[c * 289 + n];
+        }
+    }
+}
+
 // Deposit skeleton.  The tile's cells are taken RG rows at a time; inside a
 // group every cell owns T = 16/RG consecutive lanes (lane cl*T + sub), lane
 // sub taking particles sub, sub+T, ... of its cell.  The group's particles
@@ -513,7 +542,13 @@ __device__ __forceinline__ R amjdp_one(const Fields6<R> &F, R fx, R fy, R x, R y
 // and a sparse tile takes fewer, larger groups.  (Compiling each T as its
 // own path was measured slower: 443-444 against 454.6 slices/s at THR = 4.)
 // B: a tile is cut in B bands of rows, one block each (deposit_bands).
-template <typename R, int RG, int CH, int WPE, bool PSI, bool UQ, int THR = 4, int B = 1>
+// ADD: the sums are added to planes (DepOut::inner), which are read together
+// (emit_nodes8).  2048^2, one particle a cell, the deposit and its additions by
+// launches of their own, with the stores but a plane at a time, and so: FP32 329,
+// 355 and 285 us, FP64 603, 655 and 455.  A kernel of its own: the loads would cost
+// the deposits without additions registers (a step at 1024^2 in FP32 4 %).
+template <typename R, int RG, int CH, int WPE, bool PSI, bool UQ, int THR = 4, int B = 1,
+          bool ADD = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, 8)))
 k_amjdp(TileGeom g, Soa<R> s, const int *__restrict__ off, const R *fxy, const R *bxy,
         const R *psit, size_t cs, DepOut<R> out, R *halo, size_t halo_cs, R qbm, R dt, R dex,
@@ -602,6 +637,10 @@ k_amjdp(TileGeom g, Soa<R> s, const int *__restrict__ off, const R *fxy, const R
         }
     }
     __syncthreads();
+    if (ADD) {
+        emit_nodes8<R, RB>(nacc, out, g.ldr, halo, halo_cs, tile, tx, ty, row0 / RB);
+        return;
+    }
 #pragma unroll
     for (int c = 0; c < 8; ++c)
         emit_nodes<R, RB>(nacc + c * 289, out, c, g.ldr, halo + c * halo_cs, tile, tx, ty,
@@ -1994,7 +2033,7 @@ static int extpsi_t(qp_species *sp, const qp_field2d *psi, double dex)
     return QP_OK;
 }
 
-template <typename R, int V, int B = 1>
+template <typename R, int V, int B = 1, bool ADD = false>
 static int amjdp_v(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
                    const qp_field2d *psit, double dex, const DepOut<R> &out,
                    const qp_field2d *psi)
@@ -2019,11 +2058,11 @@ static int amjdp_v(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
     } else {
         lds = (7 * (size_t)Stage<d.ch>::N + 8 * 289) * sizeof(R);
         if (sp->q_uniform)
-            kern = psi ? k_amjdp<R, d.rg, d.ch, d.wpe, true, true, d.thr, B>
-                       : k_amjdp<R, d.rg, d.ch, d.wpe, false, true, d.thr, B>;
+            kern = psi ? k_amjdp<R, d.rg, d.ch, d.wpe, true, true, d.thr, B, ADD>
+                       : k_amjdp<R, d.rg, d.ch, d.wpe, false, true, d.thr, B, ADD>;
         else
-            kern = psi ? k_amjdp<R, d.rg, d.ch, d.wpe, true, false, d.thr, B>
-                       : k_amjdp<R, d.rg, d.ch, d.wpe, false, false, d.thr, B>;
+            kern = psi ? k_amjdp<R, d.rg, d.ch, d.wpe, true, false, d.thr, B, ADD>
+                       : k_amjdp<R, d.rg, d.ch, d.wpe, false, false, d.thr, B, ADD>;
     }
     int rc = allow_lds(kern, lds, c);
     if (rc) return rc;
@@ -2040,6 +2079,17 @@ static int amjdp_v(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
     }
     QP_LAUNCH_CHECK();
     return QP_OK;
+}
+
+// the default shape, by the bands of a tile
+template <typename R, bool ADD>
+static int amjdp_banded(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
+                        const qp_field2d *psit, double dex, const DepOut<R> &out,
+                        const qp_field2d *psi, int bands)
+{
+    return bands == 4   ? amjdp_v<R, 0, 4, ADD>(sp, ef, bf, psit, dex, out, psi)
+           : bands == 2 ? amjdp_v<R, 0, 2, ADD>(sp, ef, bf, psit, dex, out, psi)
+                        : amjdp_v<R, 0, 1, ADD>(sp, ef, bf, psit, dex, out, psi);
 }
 
 template <typename R>
@@ -2065,9 +2115,9 @@ static int amjdp_out(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
     case 14: rc = amjdp_v<R, 14>(sp, ef, bf, psit, dex, out, psi); break;
     default:
         bands = deposit_bands(sp->ctx);
-        rc = bands == 4   ? amjdp_v<R, 0, 4>(sp, ef, bf, psit, dex, out, psi)
-             : bands == 2 ? amjdp_v<R, 0, 2>(sp, ef, bf, psit, dex, out, psi)
-                          : amjdp_v<R, 0>(sp, ef, bf, psit, dex, out, psi);
+        rc = out.inner[0] ? amjdp_banded<R, true>(sp, ef, bf, psit, dex, out, psi, bands)
+                          : amjdp_banded<R, false>(sp, ef, bf, psit, dex, out, psi, bands);
+        break;
     }
     if (rc) return rc;
     return deposit_border<R>(sp->ctx, out, 8, 1, nullptr, bands, job);

@@ -342,20 +342,33 @@ __device__ __forceinline__ int table_entry(const int *first, int n)
 // its four runs are four independent steps, so 56 loads are in flight.  A block
 // has four waves.  Chunks of at most WG_WHOLE pixels: a block goes through all
 // chunks, 16 at a time, and adds them up in LDS.  Larger ones: four chunks a
-// block, and k_sum_parts adds the partial sums from memory.  All layers of a
+// block, or one where waves are few (WG_FEW), and k_sum_parts adds the partial
+// sums from memory.  All layers of a
 // network go in one launch: at 128^2 a block per (tile, tap, chunk), a serial
 // sum for db and two sums over the chunks, layer by layer, took 68 us a layer;
 // the 14 layers together take 41 us and the sum 4 us.
 // ---------------------------------------------------------------------------
 constexpr int WG_WHOLE = 64;   // one step of the four runs
 constexpr int WG_SLOTS = 16;
+// Up to this many waves a compute unit (of a launch's layers together) the four
+// runs of a chunk go to four waves, four steps of one run at once, with the same
+// sums in the same order: a wave's loads wait for each other's, and with few waves
+// nothing else runs.  us, a chunk a wave against four: 1024^2 16 -> 16, 1 chunk
+// 38570 and 10500, 32 chunks (0.4 waves) 1264 and 339; 300^2 64 -> 192, 8 chunks
+// (4.5) 502 and 292; 512^2 96 -> 96, 32 chunks (13.5) 654 and 530; 300^2 64 -> 192,
+// 32 chunks (18) 276 and 276; 256^2 192 -> 192, 32 chunks (54) 499 and 502.
+constexpr int WG_FEW = 16;
 
 struct WgradLayer {
     const uint16_t *x, *dy, *yout;
     float *dw, *db;        // db may be null
-    float *part, *partb;   // partial sums per chunk; null: the block adds up all chunks
+    float *part, *partb;   // partial sums per chunk, of a block that doesn't take all
     int cs_in, cin, cs_out, cout, H, W;
+    int mode;              // WG_*
 };
+// a block takes: all chunks, and adds them up; four chunks, one a wave; one chunk,
+// a run of it a wave
+constexpr int WG_ALL = 0, WG_FOUR = 1, WG_ONE = 2;
 struct WgradArgs {
     WgradLayer l[MAXL];
     int first[MAXL];
@@ -368,11 +381,14 @@ struct WgradTile {
 
 // NC chunks at once, each in its first 4 / NC runs (the others have no pixels: a
 // chunk of at most 16 pixels has one run).  A chunk's tile is r[4 / NC * chunk].
+// NC = 0: run `run` of one chunk alone, four of its steps at once; its tile is r[0].
 template <int NC>
 __device__ __forceinline__ void wgrad_runs(const WgradLayer &L, int co, int ci, int dyo, bool bias,
-                                           const int *p0, const int *p1, int q, WgradTile *r)
+                                           const int *p0, const int *p1, int q, WgradTile *r,
+                                           int run = 0)
 {
-    constexpr int NV = 4 / NC;
+    constexpr int NV = NC ? 4 / (NC ? NC : 1) : 4;
+    constexpr int STEP = NC ? 64 : 256;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
 #pragma unroll
@@ -383,19 +399,19 @@ __device__ __forceinline__ void wgrad_runs(const WgradLayer &L, int co, int ci, 
     const v4s one = {(short)0x3f80, (short)0x3f80, (short)0x3f80, (short)0x3f80};
     const bool small = npix < (1 << 20);
     const float iw = 1.f / (float)W;
-    for (int g = 0; g < (NC > 1 ? min(npix, 64) : p1[0] - p0[0]); g += 64) {
+    for (int g = 0; g < (NC > 1 ? min(npix, 64) : p1[0] - p0[0]); g += STEP) {
         uint16_t d[4][4], yo[4][4], xv[4][6];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             // pixel p of the plane is p - g0 elements of cs on from the bases; a
             // pixel's neighbour (dyo, dx) is dyo W + dx pixels on; past the plane's
             // ends the last or first pixel stands in, and is dropped below
-            const int g0 = min(p0[v / NV] + g, npix - 1);
+            const int g0 = min(p0[v / NV] + g + (NC ? 0 : 64 * v), npix - 1);
             const uint16_t *dyp = L.dy + (size_t)g0 * L.cs_out, *yp = L.yout + (size_t)g0 * L.cs_out;
             const uint16_t *xp = L.x + ((ptrdiff_t)g0 - W - 1) * L.cs_in;
             const int dmax = min(npix - 1 - g0, 63);
             const int xlo = max(0, W + 1 - g0), xhi = min(npix - 1 - g0, 64 + 2 * W) + W + 1;
-            const int p = 16 * (v % NV) + 4 * q;
+            const int p = 16 * (NC ? v % NV : run) + 4 * q;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const uint32_t o = (uint32_t)__mul24(min(p + i, dmax), L.cs_out) + co;
@@ -410,7 +426,8 @@ __device__ __forceinline__ void wgrad_runs(const WgradLayer &L, int co, int ci, 
         }
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const int p = p0[v / NV] + g + 16 * (v % NV) + 4 * q;
+            const int p = p0[v / NV] + g + (NC ? 16 * (v % NV) : 64 * v + 16 * run) + 4 * q;
+            WgradTile &s = r[NC ? v : 0];
             int py = small ? small_div(p, iw) : p / W, px = p - py * W;
             v4s a, b[3];
 #pragma unroll
@@ -425,13 +442,13 @@ __device__ __forceinline__ void wgrad_runs(const WgradLayer &L, int co, int ci, 
             }
 #pragma unroll
             for (int t = 0; t < 3; ++t)
-                r[v].w[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b[t], r[v].w[t], 0, 0, 0);
-            if (bias) r[v].b = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, one, r[v].b, 0, 0, 0);
+                s.w[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b[t], s.w[t], 0, 0, 0);
+            if (bias) s.b = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, one, s.b, 0, 0, 0);
         }
     }
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-        if (v % NV == 0) continue;
+        if (v % NV == 0 || !NC) continue;
 #pragma unroll
         for (int t = 0; t < 3; ++t) r[v - v % NV].w[t] += r[v].w[t];
         r[v - v % NV].b += r[v].b;
@@ -480,14 +497,15 @@ __global__ void __launch_bounds__(256, 3) k_wgrad(const WgradArgs A)
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int m = lane & 15, q = lane >> 4;
-    const int nb = L.part ? (nchunk + 3) / 4 : 1;
+    const int nb = L.mode == WG_ALL ? 1 : L.mode == WG_FOUR ? (nchunk + 3) / 4 : nchunk;
     const int unit = ((int)blockIdx.x - A.first[e]) / nb;
     const int cb = ((int)blockIdx.x - A.first[e]) - unit * nb;
     const int ntc = L.cin >> 4;
     const int ty = unit % 3, cit = (unit / 3) % ntc, cot = unit / 3 / ntc;
     const bool bias = L.db && cit == 0 && ty == 1;
     const int npix = L.H * L.W, per = (npix + nchunk - 1) / nchunk;
-    if (L.part) {
+    const int tid = threadIdx.x;
+    if (L.mode == WG_FOUR) {
         const int chunk = cb * 4 + wave;
         if (chunk >= nchunk) return;
         const int p0 = min(chunk * per, npix), p1 = min(npix, p0 + per);
@@ -505,9 +523,32 @@ __global__ void __launch_bounds__(256, 3) k_wgrad(const WgradArgs A)
         }
         return;
     }
+    // where element tid of a tile belongs
+    const int tl = tid >> 2, tco = cot * 16 + 4 * (tl >> 4) + (tid & 3), tci = cit * 16 + (tl & 15);
+    if (L.mode == WG_ONE) {
+        const int p0 = min(cb * per, npix), p1 = min(npix, p0 + per);
+        WgradTile r[4];
+        wgrad_runs<0>(L, cot * 16 + m, cit * 16 + m, ty - 1, bias, &p0, &p1, q, r, wave);
+#pragma unroll
+        for (int t = 0; t < 3; ++t) red[wave][t][lane] = r[0].w[t];
+        if (m == 0)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) redb[wave][4 * q + i] = r[0].b[i];
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            float v = reinterpret_cast<const float *>(red[0][t])[tid];
+#pragma unroll
+            for (int k = 1; k < 4; ++k) v += reinterpret_cast<const float *>(red[k][t])[tid];
+            L.part[(((size_t)cb * 9 + 3 * ty + t) * L.cout + tco) * L.cin + tci] = v;
+        }
+        if (bias && tid < 16)
+            L.partb[(size_t)cb * L.cout + cot * 16 + tid] =
+                ((redb[0][tid] + redb[1][tid]) + redb[2][tid]) + redb[3][tid];
+        return;
+    }
     // thread t sums element t of the tiles, in the order of the chunks
     float tot[3] = {0.f, 0.f, 0.f}, totb = 0.f;
-    const int tid = threadIdx.x;
     for (int base = 0; base < nchunk; base += WG_SLOTS) {
         const int ns = min(WG_SLOTS, nchunk - base);
         const int co = cot * 16 + m, ci = cit * 16 + m;
@@ -525,10 +566,9 @@ __global__ void __launch_bounds__(256, 3) k_wgrad(const WgradArgs A)
         }
         __syncthreads();
     }
-    const int l = tid >> 2, co = cot * 16 + 4 * (l >> 4) + (tid & 3), ci = cit * 16 + (l & 15);
 #pragma unroll
     for (int t = 0; t < 3; ++t)
-        L.dw[((size_t)(3 * ty + t) * L.cout + co) * L.cin + ci] = tot[t];
+        L.dw[((size_t)(3 * ty + t) * L.cout + tco) * L.cin + tci] = tot[t];
     if (bias && tid < 16) L.db[cot * 16 + tid] = totb;
 }
 
@@ -1000,26 +1040,23 @@ static int conv3x3(const NetDevice *dev, hipStream_t st, const uint16_t *x, cons
 }
 
 // partb: the partial sums of the bias of a single layer, if not in part
-static int wgrad_layers(hipStream_t st, const qp_net_layer *layers, int n, int nchunk, float *part,
-                        size_t npart, float *partb)
+static int wgrad_layers(const NetDevice &dev, hipStream_t st, const qp_net_layer *layers, int n,
+                        int nchunk, float *part, size_t npart, float *partb)
 {
     for (int i0 = 0; i0 < n; i0 += MAXL) {
         WgradArgs a{};
         SumArgs sums{}, sumb{};
         a.n = std::min(MAXL, n - i0);
         a.nchunk = sums.nchunk = sumb.nchunk = nchunk;
-        int blocks = 0;
-        size_t used = 0;
+        size_t used = 0, waves = 0;
         for (int e = 0; e < a.n; ++e) {
             const qp_net_layer &l = layers[i0 + e];
-            const int units = (l.cout / 16) * (l.cin / 16) * 3;
             const int per = (int)(((size_t)l.H * l.W + nchunk - 1) / nchunk);
             const size_t nw = (size_t)9 * l.cout * l.cin, nb = l.db && !partb ? l.cout : 0;
             // a layer whose partial sums find no room: its blocks take all chunks
             const bool parts = per > WG_WHOLE && part && used + (nw + nb) * nchunk <= npart;
             a.l[e] = WgradLayer{l.x, l.dy, l.yout, l.dw, l.db, nullptr, nullptr,
-                                l.cs_x, l.cin, l.cs_y, l.cout, l.H, l.W};
-            a.first[e] = blocks;
+                                l.cs_x, l.cin, l.cs_y, l.cout, l.H, l.W, parts ? WG_FOUR : WG_ALL};
             if (parts) {
                 a.l[e].part = part + used;
                 a.l[e].partb = partb ? partb : part + used + nw * nchunk;
@@ -1027,7 +1064,15 @@ static int wgrad_layers(hipStream_t st, const qp_net_layer *layers, int n, int n
                 if (l.db) add_sum(partb ? sumb : sums, a.l[e].partb, l.cout, l.db);
                 add_sum(sums, a.l[e].part, (int)nw, l.dw);
             }
-            blocks += units * (parts ? (nchunk + 3) / 4 : 1);
+            waves += (size_t)(l.cout / 16) * (l.cin / 16) * 3 * (parts ? nchunk : 4);
+        }
+        int blocks = 0;
+        for (int e = 0; e < a.n; ++e) {
+            WgradLayer &l = a.l[e];
+            if (l.mode == WG_FOUR && waves <= (size_t)WG_FEW * dev.cus) l.mode = WG_ONE;
+            a.first[e] = blocks;
+            blocks += (l.cout / 16) * (l.cin / 16) * 3 *
+                      (l.mode == WG_ALL ? 1 : l.mode == WG_FOUR ? (nchunk + 3) / 4 : nchunk);
         }
         hipLaunchKernelGGL(k_wgrad, dim3(blocks), dim3(256), 0, st, a);
         QP_LAUNCH_CHECK();
@@ -1057,7 +1102,9 @@ int qp_net_wgrad_layers(void *stream_, const qp_net_layer *layers, int n, int nc
                       l.cin % 16 == 0 && l.cout % 16 == 0,
                   "qp_net_wgrad_layers: layer %d", i);
     }
-    return wgrad_layers((hipStream_t)stream_, layers, n, nchunk, part, npart, nullptr);
+    NetDevice dev;
+    RC(net_device(&dev));
+    return wgrad_layers(dev, (hipStream_t)stream_, layers, n, nchunk, part, npart, nullptr);
 }
 
 int qp_net_conv3x3_wgrad(void *stream_, const uint16_t *x, int cs_in, int cin,
@@ -1067,11 +1114,13 @@ int qp_net_conv3x3_wgrad(void *stream_, const uint16_t *x, int cs_in, int cin,
     NET_CHECK(x && dy && yout && part && dw && nchunk > 0, "qp_net_conv3x3_wgrad: bad argument");
     NET_CHECK(cin % 16 == 0 && cout % 16 == 0, "qp_net_conv3x3_wgrad: channels");
     const qp_net_layer l = {x, dy, yout, dw, db, cs_in, cin, cs_out, cout, H, W};
+    NetDevice dev;
+    RC(net_device(&dev));
     // the scratch holds the weights' partial sums; the bias's wait in dw, which is
-    // written behind them, if they fit there
-    const bool room = !db || nchunk <= 9 * cin;
-    return wgrad_layers((hipStream_t)stream_, &l, 1, nchunk, room ? part : nullptr,
-                        (size_t)nchunk * 9 * cout * cin, db ? dw : nullptr);
+    // written behind them
+    const bool room = db && nchunk <= 9 * cin;
+    return wgrad_layers(dev, (hipStream_t)stream_, &l, 1, nchunk, part,
+                        (size_t)nchunk * 9 * cout * cin, room ? dw : nullptr);
 }
 
 int qp_net_flip_layers(void *stream_, const qp_net_flip *layers, int n)

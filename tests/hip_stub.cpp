@@ -16,7 +16,7 @@
 namespace {
 struct Stream { int device; bool capture; int syncs; };
 struct Graph { int device; };
-struct Launch { std::string name; size_t lds; };
+struct Launch { std::string name; size_t lds; long blocks; };
 struct Config { dim3 grid, block; size_t lds; hipStream_t st; };
 
 thread_local int cur = 0;
@@ -54,6 +54,14 @@ int stub_launched(const char *part)
     int n = 0;
     for (const Launch &l : launches) n += l.name.find(part) != std::string::npos;
     return n;
+}
+// workgroups of the last such launch
+long stub_blocks(const char *part)
+{
+    long v = -1;
+    for (const Launch &l : launches)
+        if (l.name.find(part) != std::string::npos) v = l.blocks;
+    return v;
 }
 // LDS bytes of the last such launch
 long stub_lds(const char *part)
@@ -105,7 +113,7 @@ hipError_t hipLaunchKernel(const void *fn, dim3 g, dim3 b, void **args, size_t l
     const size_t limit = granted.count(fn) ? granted[fn] : 65536;
     if (!g.x || !g.y || !g.z || !b.x || lds > limit || lds > (size_t)max_lds)
         return last = hipErrorInvalidConfiguration;
-    launches.push_back({names[fn], lds});
+    launches.push_back({names[fn], lds, (long)g.x * g.y * g.z});
     if (names[fn].find("k_push") != std::string::npos)
         std::memcpy(&words[names[fn]], args[1], 8);
     if (names[fn].find("k_ctl_reset") != std::string::npos) {   // the host reads it back

@@ -271,3 +271,23 @@ f.fftkr(1)
 assert stub.stub_launched(b"k_fft_xt") == {2 * columns}
 assert stub.stub_launched(b"k_transpose") == {2 * (not columns)}
 """)
+
+
+WGRAD = NET + """
+def wgrad(H, W, cin, cout, nchunk, db):
+    stub.stub_clear_launches()
+    rc = L.qp_net_conv3x3_wgrad(None, P[0], cin, cin, P[1], P[2], cout, cout, H, W, nchunk, P[3],
+                                P[4], P[5] if db else None)
+    assert rc == 0, L.qp_last_error()
+    return stub.stub_blocks(b"k_wgrad")
+"""
+
+
+@pytest.mark.parametrize("H,W,cin,cout,nchunk,per_chunk", [
+    (64, 64, 16, 16, 8, 1), (1024, 1024, 16, 16, 32, 1), (1024, 1024, 16, 16, 1, 1),
+    (512, 512, 192, 192, 32, 0.25), (512, 512, 64, 48, 200, 0.25)])
+def test_weight_gradient_of_few_chunks(stub, H, W, cin, cout, nchunk, per_chunk):
+    """A chunk takes four waves where the launch has few, one where it has many."""
+    run(stub, WGRAD + f"""
+assert wgrad({H}, {W}, {cin}, {cout}, {nchunk}, False) == {int(cout // 16 * cin // 16 * 3 * nchunk * per_chunk)}
+""")

@@ -57,3 +57,10 @@ def test_few_chunks(H, W, nchunk, cin, cout, bias):
 @pytest.mark.parametrize("bias", [False, True])
 def test_many_tiles(bias):
     _check(47, 51, 192, 192, 29, bias)
+
+
+@pytest.mark.parametrize("H,W,nchunk", [(130, 100, 144), (130, 100, 145), (131, 100, 200),
+                                        (100, 651, 600)])
+def test_bias_of_more_chunks_than_taps_and_channels(H, W, nchunk):
+    """Its partial sums do not fit where those of the weights leave room."""
+    _check(H, W, 16, 32, nchunk, True)

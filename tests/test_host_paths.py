@@ -291,3 +291,15 @@ def test_weight_gradient_of_few_chunks(stub, H, W, cin, cout, nchunk, per_chunk)
     run(stub, WGRAD + f"""
 assert wgrad({H}, {W}, {cin}, {cout}, {nchunk}, False) == {int(cout // 16 * cin // 16 * 3 * nchunk * per_chunk)}
 """)
+
+
+@pytest.mark.parametrize("nchunk,launches", [(144, 1), (145, 2), (400, 2), (1000, 1)])
+def test_bias_gradient_of_many_chunks(stub, nchunk, launches):
+    """More chunks than 9 cin: the bias's partial sums come in a launch of their
+    own, and the weights' stay spread over the chunks.  Chunks small enough for a
+    block stay there."""
+    run(stub, WGRAD + f"""
+blocks = wgrad(250, 200, 16, 16, {nchunk}, True)
+assert stub.stub_launched(b"k_wgrad") == {launches}
+assert blocks == {3 * nchunk if nchunk < 1000 else 3}
+""")

@@ -67,7 +67,8 @@ __device__ __forceinline__ v4s load4(const uint16_t *p)
 //  k_conv3x3_deep: the others, operands not aligned to 16 bytes, and devices whose
 //    workgroups have less LDS than a layer asks for.  The chain is cut in groups of
 //    9 steps, whose loads are issued before the group in front is multiplied.
-//  k_conv3x3_wide: those where the plane alone fills the device with waves.  A wave
+//  k_conv3x3_wide: those where the plane alone fills the device with waves, and
+//    masked layers of few input and many output channels there.  A wave
 //    computes all output channels of its pixels, step by step, and reads them once
 //    in place of once for every 16 output channels.
 // All by k_conv3x3_wide took 33.7 us a convolution (27 of a training step), by
@@ -309,6 +310,21 @@ static bool conv_wide(int cus, long long groups, int cin, int cout)
 {
     if (cout < 32) return false;
     const int need = cin < 80 ? 14 : cin <= 208 ? (cout >= 96 ? 6 : 10) : (cout >= 48 ? 4 : 6);
+    return groups >= (long long)need * cus;
+}
+
+// And whether a masked one that k_conv3x3 has: it reads pixels and mask once for
+// every 16 output channels, which with up to 48 input channels is what its time goes
+// to.  Ratio of k_conv3x3_wide's time to k_conv3x3's at 160^2, 192^2, 224^2, 256^2 and
+// 1024^2: 16 -> 32 channels 1.11, 1.04, 0.92, 0.86, 0.83; 16 -> 64 0.91, 0.85, 0.69,
+// 0.63, 0.57; 16 -> 192 0.74, 0.67, 0.48, 0.51, 0.41 (1150 -> 477 us); 48 -> 64 1.37
+// .. 1.01, 1.08; 48 -> 96 1.26, 1.22, 1.02, 0.90, 0.95; 48 -> 192 1.35, 1.19, 0.91,
+// 0.87, 0.84; 32 -> 192 1.06, 1.16, 0.98, 0.90, 0.84; 64 -> 192 2.5 at least; 16 -> 192 without a mask 1.44 .. 1.07, 0.94.
+static bool conv_wide_masked(int cus, long long groups, int cin, int cout)
+{
+    if (cin > 48 || cout < (cin == 16 ? 32 : 96)) return false;
+    const int need = cin == 16 ? (cout >= 64 ? 6 : cout >= 48 ? 9 : 12)
+                     : cin == 48 && cout >= 128 ? 12 : 16;
     return groups >= (long long)need * cus;
 }
 
@@ -996,7 +1012,10 @@ static int conv3x3(const NetDevice *dev, hipStream_t st, const uint16_t *x, cons
         else tx /= 2;
     }
     const size_t lds = (size_t)((16 * tx + 2) * (ty + 2) + 144) * (cin / 8 + 1) * 16;
-    if (have && al && lds <= dev->lds) {
+    const bool staged = have && al && lds <= dev->lds;
+    const bool wide = staged ? mask && conv_wide_masked(dev->cus, (long long)H * gw, cin, cout)
+                             : conv_wide(dev->cus, (long long)H * gw, cin, cout);
+    if (staged && !wide) {
         const int nbx = (gw + tx - 1) / tx;
         const dim3 grid((unsigned)((size_t)((H + ty - 1) / ty) * nbx), cout / 16);
         auto launch = [&](auto kern) -> int {
@@ -1024,7 +1043,7 @@ static int conv3x3(const NetDevice *dev, hipStream_t st, const uint16_t *x, cons
         QP_LAUNCH_CHECK();
         return QP_OK;
     }
-    if (conv_wide(dev->cus, (long long)H * gw, cin, cout)) {
+    if (wide) {
         hipLaunchKernelGGL(k_conv3x3_wide, dim3((unsigned)(((size_t)H * gw + 3) / 4)), dim3(256), 0,
                            st, x, mask, H, W, gw, cs_in, cin, w, bias, out, cs_out, cout, relu,
                            accum);

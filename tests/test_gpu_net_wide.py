@@ -25,13 +25,15 @@ def _conv(x, w):
     return torch.nn.functional.conv2d(x.permute(2, 0, 1)[None], k, padding=1)[0].permute(1, 2, 0)
 
 
-@pytest.mark.parametrize("H,W,cin,cout,off", [(97, 258, 80, 96, 0), (50, 500, 256, 32, 0),
-                                              (113, 500, 32, 32, 4)])
+@pytest.mark.parametrize("H,W,cin,cout,pad,off", [
+    (97, 258, 80, 96, 4, 0), (50, 500, 256, 32, 4, 0), (113, 500, 32, 32, 4, 4),
+    (193, 256, 16, 32, 8, 0), (100, 250, 16, 96, 8, 0), (260, 250, 48, 112, 8, 0),
+    (241, 275, 32, 192, 8, 0)])
 @pytest.mark.parametrize("masked", [False, True])
-def test_wide_convolution(H, W, cin, cout, off, masked):
+def test_wide_convolution(H, W, cin, cout, pad, off, masked):
     print(f"[gpu-test] wide conv {H}x{W} {cin}->{cout} off {off} mask {masked}", flush=True)
     g = torch.Generator().manual_seed(H + W + cin)
-    cs = cin + 4
+    cs = cin + pad
     x, m, w = _rand((H, W, cs), g), _rand((H, W, cs), g), _rand((9, cout, cin), g)
     b = torch.randn(cout, generator=g).cuda()
     was = _rand((H, W, cout), g)

@@ -150,9 +150,9 @@ assert rc == 0, L.qp_last_error()
 
 
 CONV = NET + """
-def conv(H, W, cin, cout):
+def conv(H, W, cin, cout, mask=None):
     stub.stub_clear_launches()
-    rc = L.qp_net_conv3x3(None, P[0], None, H, W, cin, cin, P[1], None, P[2], cout, cout, 1, 0)
+    rc = L.qp_net_conv3x3(None, P[0], mask, H, W, cin, cin, P[1], None, P[2], cout, cout, 1, 0)
     assert rc == 0, L.qp_last_error()
     return stub.stub_launched(b"k_conv3x3_deep")
 
@@ -255,6 +255,20 @@ def test_convolution_of_a_large_plane(stub, H, W, cin, cout, wide):
     where the plane has waves enough, 16 in a wave elsewhere."""
     run(stub, CONV + f"""
 conv({H}, {W}, {cin}, {cout})
+assert stub.stub_launched(b"k_conv3x3_wide") == {int(wide)}
+""")
+
+
+@pytest.mark.parametrize("H,W,cin,cout,mask,wide", [
+    (224, 224, 16, 32, True, True), (192, 192, 16, 32, True, False), (192, 192, 16, 48, True, True),
+    (160, 160, 16, 64, True, True), (128, 128, 16, 96, True, False),
+    (224, 224, 48, 128, True, True), (256, 256, 48, 96, True, True),
+    (224, 224, 32, 192, True, False), (256, 256, 48, 64, True, False),
+    (256, 256, 64, 192, True, False), (1024, 1024, 16, 192, False, False)])
+def test_masked_convolution_of_a_large_plane(stub, H, W, cin, cout, mask, wide):
+    """Few input and many output channels: pixels and mask are read once."""
+    run(stub, CONV + f"""
+conv({H}, {W}, {cin}, {cout}, P[3] if {mask} else None)
 assert stub.stub_launched(b"k_conv3x3_wide") == {int(wide)}
 """)
 

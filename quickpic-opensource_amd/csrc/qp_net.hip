@@ -64,7 +64,7 @@ __device__ __forceinline__ v4s load4(const uint16_t *p)
 //    weights go to LDS first, in loads of 16 bytes that are in flight together.
 //    A row of LDS is a pixel or a (tap, co), padded by 16 bytes: the 16 rows of
 //    an operand then lie in different banks.
-//  k_conv3x3_deep: the others, operands not aligned to 16 bytes, and devices whose
+//  k_conv3x3_deep: others, operands not aligned to 16 bytes, and devices whose
 //    workgroups have less LDS than a layer asks for.  The chain is cut in groups of
 //    9 steps, whose loads are issued before the group in front is multiplied.
 //  k_conv3x3_wide: those where the plane alone fills the device with waves, and
@@ -319,7 +319,8 @@ static bool conv_wide(int cus, long long groups, int cin, int cout)
 // 1024^2: 16 -> 32 channels 1.11, 1.04, 0.92, 0.86, 0.83; 16 -> 64 0.91, 0.85, 0.69,
 // 0.63, 0.57; 16 -> 192 0.74, 0.67, 0.48, 0.51, 0.41 (1150 -> 477 us); 48 -> 64 1.37
 // .. 1.01, 1.08; 48 -> 96 1.26, 1.22, 1.02, 0.90, 0.95; 48 -> 192 1.35, 1.19, 0.91,
-// 0.87, 0.84; 32 -> 192 1.06, 1.16, 0.98, 0.90, 0.84; 64 -> 192 2.5 at least; 16 -> 192 without a mask 1.44 .. 1.07, 0.94.
+// 0.87, 0.84; 32 -> 192 1.06, 1.16, 0.98, 0.90, 0.84; 64 -> 192 2.5 at least;
+// 16 -> 192 without a mask 1.44 .. 1.07, 0.94.
 static bool conv_wide_masked(int cus, long long groups, int cin, int cout)
 {
     if (cin > 48 || cout < (cin == 16 ? 32 : 96)) return false;
@@ -358,7 +359,7 @@ __device__ __forceinline__ int table_entry(const int *first, int n)
 // its four runs are four independent steps, so 56 loads are in flight.  A block
 // has four waves.  Chunks of at most WG_WHOLE pixels: a block goes through all
 // chunks, 16 at a time, and adds them up in LDS.  Larger ones: four chunks a
-// block, or one where waves are few (WG_FEW), and k_sum_parts adds the partial
+// block, or one where waves are few (wgrad_few), and k_sum_parts adds the partial
 // sums from memory.  All layers of a
 // network go in one launch: at 128^2 a block per (tile, tap, chunk), a serial
 // sum for db and two sums over the chunks, layer by layer, took 68 us a layer;
@@ -367,13 +368,17 @@ __device__ __forceinline__ int table_entry(const int *first, int n)
 constexpr int WG_WHOLE = 64;   // one step of the four runs
 constexpr int WG_SLOTS = 16;
 // Up to this many waves a compute unit (of a launch's layers together) the four
-// runs of a chunk go to four waves, four steps of one run at once, with the same
-// sums in the same order: a wave's loads wait for each other's, and with few waves
-// nothing else runs.  us, a chunk a wave against four: 1024^2 16 -> 16, 1 chunk
-// 38570 and 10500, 32 chunks (0.4 waves) 1264 and 339; 300^2 64 -> 192, 8 chunks
-// (4.5) 502 and 292; 512^2 96 -> 96, 32 chunks (13.5) 654 and 530; 300^2 64 -> 192,
-// 32 chunks (18) 276 and 276; 256^2 192 -> 192, 32 chunks (54) 499 and 502.
-constexpr int WG_FEW = 16;
+// runs of a chunk of `per` pixels go to four waves, four steps of one run at once,
+// with the same sums in the same order: a wave's loads wait for each other's, and
+// with few waves nothing else runs.  A chunk of few steps leaves such waves without
+// pixels.  us, a chunk a wave against four, 32 chunks of 128, 192, 256, 512, 1024 and
+// 4096 pixels: 16 -> 16 channels (0.4 waves) 12.5 and 12.2, 14.0 and 12.0, 16.1 and
+// 12.1, 25.4 and 12.1, 43 and 17, 151 and 46; 48 -> 48 (3.4) 13.1 and 14.3, 15.0 and
+// 14.0, 17.6 and 14.5, 26 and 19, 44 and 30, 153 and 91; 128 -> 64 (12) 19 and 27,
+// 22 and 28, 26 and 28, 39 and 41, 66 and 66, 227 and 224; 512^2 96 -> 96 (13.5, 8192
+// pixels) 654 and 530; 300^2 64 -> 192 (18, 2813) 276 and 276; 1024^2 16 -> 16, one
+// chunk: 38.6 and 10.5 ms.
+static int wgrad_few(int per) { return per >= 768 ? 16 : per >= 192 ? 4 : 0; }
 
 struct WgradLayer {
     const uint16_t *x, *dy, *yout;
@@ -1107,7 +1112,8 @@ static int wgrad_layers(const NetDevice &dev, hipStream_t st, const qp_net_layer
         int blocks = 0;
         for (int e = 0; e < a.n; ++e) {
             WgradLayer &l = a.l[e];
-            if (l.mode == WG_FOUR && waves <= (size_t)WG_FEW * dev.cus) l.mode = WG_ONE;
+            const int per = (l.H * l.W + nchunk - 1) / nchunk;
+            if (l.mode == WG_FOUR && waves <= (size_t)wgrad_few(per) * dev.cus) l.mode = WG_ONE;
             a.first[e] = blocks;
             blocks += (l.cout / 16) * (l.cin / 16) * 3 *
                       (l.mode == WG_ALL ? 1 : l.mode == WG_FOUR ? (nchunk + 3) / 4 : nchunk);

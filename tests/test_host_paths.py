@@ -299,9 +299,11 @@ def wgrad(H, W, cin, cout, nchunk, db):
 
 @pytest.mark.parametrize("H,W,cin,cout,nchunk,per_chunk", [
     (64, 64, 16, 16, 8, 1), (1024, 1024, 16, 16, 32, 1), (1024, 1024, 16, 16, 1, 1),
-    (512, 512, 192, 192, 32, 0.25), (512, 512, 64, 48, 200, 0.25)])
+    (32, 190, 16, 16, 32, 0.25), (96, 64, 48, 48, 32, 1), (160, 160, 64, 96, 32, 1),
+    (128, 128, 64, 96, 32, 0.25), (512, 512, 192, 192, 32, 0.25), (512, 512, 64, 48, 200, 0.25)])
 def test_weight_gradient_of_few_chunks(stub, H, W, cin, cout, nchunk, per_chunk):
-    """A chunk takes four waves where the launch has few, one where it has many."""
+    """A chunk of many pixels takes four waves where the launch has few, one where it
+    has many."""
     run(stub, WGRAD + f"""
 assert wgrad({H}, {W}, {cin}, {cout}, {nchunk}, False) == {int(cout // 16 * cin // 16 * 3 * nchunk * per_chunk)}
 """)
@@ -315,5 +317,5 @@ def test_bias_gradient_of_many_chunks(stub, nchunk, launches):
     run(stub, WGRAD + f"""
 blocks = wgrad(250, 200, 16, 16, {nchunk}, True)
 assert stub.stub_launched(b"k_wgrad") == {launches}
-assert blocks == {3 * nchunk if nchunk < 1000 else 3}
+assert blocks == {3 * nchunk if nchunk < 200 else 3 * nchunk // 4 if nchunk < 1000 else 3}
 """)

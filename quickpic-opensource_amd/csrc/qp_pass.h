@@ -20,22 +20,29 @@ __device__ __forceinline__ bool corrector_mode(bool tab, int kx, int ky, R fg, R
     const R at2 = R(1) * fg / fmadd(aa, fg, R(1));
     const R at1 = at2 * fs;
     const R at3 = aa * at2;
+    // through values of its own: branches that store to different arguments end up
+    // as one store by a selected address, and what lies there in scratch
+    R s1, s2, m1 = R(0), m2 = R(0);
     if (kx > 0 && ky > 0) {
-        d1 = fmadd(-dky, a3, fmadd(dkx, a1, -d1));
-        const R aat1 = fmadd(-(dkx * c3), idex, d1);
-        d2 = fmadd(dky, a2, fmadd(-dkx, a3, -d2));
-        const R aat2 = fmadd(-(dky * c3), idex, d2);
-        n1 = fmadd(at3, old1, at1 * aat1);
-        n2 = fmadd(at3, old2, at1 * aat2);
+        s1 = fmadd(-dky, a3, fmadd(dkx, a1, -d1));
+        const R aat1 = fmadd(-(dkx * c3), idex, s1);
+        s2 = fmadd(dky, a2, fmadd(-dkx, a3, -d2));
+        const R aat2 = fmadd(-(dky * c3), idex, s2);
+        m1 = fmadd(at3, old1, at1 * aat1);
+        m2 = fmadd(at3, old2, at1 * aat2);
     } else if (kx > 0) {
-        d1 = fmadd(dkx, a1, -d1);
-        d2 = fmadd(-dkx, a3, -d2);
-        n2 = fmadd(at3, old2, at1 * d2);
+        s1 = fmadd(dkx, a1, -d1);
+        s2 = fmadd(-dkx, a3, -d2);
+        m2 = fmadd(at3, old2, at1 * s2);
     } else {
-        d1 = fmadd(-dky, a3, -d1);
-        d2 = fmadd(dky, a2, -d2);
-        n1 = fmadd(at3, old1, at1 * d1);
+        s1 = fmadd(-dky, a3, -d1);
+        s2 = fmadd(dky, a2, -d2);
+        m1 = fmadd(at3, old1, at1 * s1);
     }
+    d1 = s1;
+    d2 = s2;
+    n1 = m1;
+    n2 = m2;
     return true;
 }
 

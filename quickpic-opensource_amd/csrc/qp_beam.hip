@@ -24,6 +24,7 @@ struct qp_beam {
     int64_t np, npmax;
     qp::DevBuf a[7], b[7];       // x, y, z, px, py, pz, q (double)
     qp::DevBuf live, sort_tmp, moments;
+    int *h_live = nullptr;   // pinned copy of live
     qp::DevBuf key[2], perm[2];  // push: cell keys and particle indices, before and after the sort
     size_t sort_bytes;           // temporary bytes of the sort
     double run_len = 0.0;        // mean run of particles of one cell, as the last push sorted
@@ -519,6 +520,7 @@ __global__ void k_beam_push(int64_t np, Ptr7 a, const R *__restrict__ e3,
 // places where the key changes, *changes in all, for the deposit's choice of a
 // kernel: up to 127 wavefronts, as their atomics meet in one word (1024 took 11
 // us), each in `samples` stretches of 64 particles from its block to the next.
+constexpr int SAMPLES = 8;
 __global__ void k_permute(int64_t np, const unsigned *__restrict__ key, unsigned drop,
                           const unsigned *__restrict__ perm, Ptr7 src, Ptr7 dst, int *nlive,
                           int *changes, unsigned every, int samples)
@@ -526,11 +528,18 @@ __global__ void k_permute(int64_t np, const unsigned *__restrict__ key, unsigned
     const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     const unsigned k0 = i < np ? key[i] : drop, k1 = i + 1 < np ? key[i + 1] : drop;
     if (blockIdx.x % every == 0 && threadIdx.x < 64) {
-        int n = 0;
-        for (int m = 0; m < samples; ++m) {
-            const int64_t j = i + m * (int64_t)(every * 256 / samples);
-            n += __popcll(__ballot(j < np && key[j] != (j + 1 < np ? key[j + 1] : drop)));
+        const int64_t step = every * 256 / samples;
+        unsigned a[SAMPLES], b[SAMPLES];   // all in flight: one after the other 1.8 us more
+#pragma unroll
+        for (int m = 0; m < SAMPLES; ++m) {
+            const int64_t j = i + m * step;
+            const bool in = m < samples && j < np;
+            a[m] = in ? key[j] : drop;
+            b[m] = in && j + 1 < np ? key[j + 1] : drop;
         }
+        int n = 0;
+#pragma unroll
+        for (int m = 0; m < SAMPLES; ++m) n += __popcll(__ballot(a[m] != b[m]));
         if (threadIdx.x == 0 && n) atomicAdd(changes, n);
     }
     if (i >= np) return;
@@ -589,6 +598,7 @@ static int beam_alloc(qp_beam *b, int64_t n)
         if (rc) return rc;
     }
     int rc = b->live.alloc(2 * sizeof(int));
+    if (!rc) QP_HIP(hipHostMalloc((void **)&b->h_live, 2 * sizeof(int), hipHostMallocDefault));
     for (int k = 0; k < 2 && !rc; ++k) {
         rc = b->key[k].alloc((size_t)(n + 1) * 4);
         if (!rc) rc = b->perm[k].alloc((size_t)(n + 1) * 4);
@@ -844,6 +854,7 @@ int qp_beam_destroy(qp_beam *b)
     if (b->ctx) (void)hipStreamSynchronize(b->ctx->stream);
     for (int k = 0; k < 7; ++k) { b->a[k].release(); b->b[k].release(); }
     b->live.release(); b->sort_tmp.release(); b->moments.release();
+    if (b->h_live) (void)hipHostFree(b->h_live);
     for (int k = 0; k < 2; ++k) { b->key[k].release(); b->perm[k].release(); }
     b->q3.release();
     delete b;
@@ -949,7 +960,7 @@ int qp_beam_push(qp_beam *b, const qp_field3d *ef, const qp_field3d *bf, double 
     unsigned *key = b->key[0].as<unsigned>(), *sorted = b->key[1].as<unsigned>();
     int *counts = b->live.as<int>();   // survivors, changes of key where they are counted
     const unsigned every = std::max(1u, grid.x / 64);
-    const int samples = every > 1 ? 8 : 1;
+    const int samples = every > 1 ? SAMPLES : 1;
     auto push = [&](auto kern, auto zero) {
         using R = decltype(zero);
         hipLaunchKernelGGL(kern, grid, dim3(256), 0, c->stream, np, src, ef->buf.as<R>(),
@@ -988,8 +999,8 @@ int qp_beam_push(qp_beam *b, const qp_field3d *ef, const qp_field3d *bf, double 
                        samples);
     }
     QP_LAUNCH_CHECK();
-    int h[2] = {0, 0};
-    QP_HIP(hipMemcpyAsync(h, counts, sizeof(h), hipMemcpyDeviceToHost, c->stream));
+    int *h = b->h_live;
+    QP_HIP(hipMemcpyAsync(h, counts, 2 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
     QP_HIP(hipStreamSynchronize(c->stream));
     for (int k = 0; k < 7; ++k) std::swap(b->a[k], b->b[k]);
     b->np = h[0];

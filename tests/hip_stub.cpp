@@ -32,6 +32,7 @@ auto &words = *new std::map<std::string, unsigned long long>;   // k_push: its a
 thread_local std::vector<Config> configs;
 int max_lds = 163840, cus = 256;
 int fail_launch = 0;       // the graph launch (counted from now) that fails
+int pageable = 0;          // copies to host memory that is not pinned
 int graph_launches = 0, instantiations = 0;
 size_t residual_bytes = 0; // a graph launch fills the host allocations of this size
 double residual = 0.0;     // with this value
@@ -44,6 +45,7 @@ void stub_limits(int lds, int units) { max_lds = lds; cus = units; }
 void stub_fail_launch(int n) { fail_launch = n; }
 void stub_residual(size_t n, double v) { residual_bytes = n; residual = v; }
 void stub_key_changes(int n) { key_changes = n; }
+int stub_pageable() { return pageable; }
 int stub_graph_launches() { return graph_launches; }
 int stub_instantiations() { return instantiations; }
 int stub_syncs(int stream) { return streams[stream]->syncs; }
@@ -169,8 +171,9 @@ hipError_t hipHostMalloc(void **p, size_t n, unsigned flags)
 hipError_t hipHostFree(void *p) { host_flags.erase(p); host_bytes.erase(p); std::free(p); return hipSuccess; }
 static bool capturing(hipStream_t st) { return st && reinterpret_cast<Stream *>(st)->capture; }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { std::memcpy(d, s, n); return hipSuccess; }
-hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t st)
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind kind, hipStream_t st)
 {
+    if (kind == hipMemcpyDeviceToHost && !host_bytes.count(d)) ++pageable;
     if (!capturing(st)) std::memcpy(d, s, n);
     return hipSuccess;
 }

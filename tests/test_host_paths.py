@@ -319,3 +319,15 @@ blocks = wgrad(250, 200, 16, 16, {nchunk}, True)
 assert stub.stub_launched(b"k_wgrad") == {launches}
 assert blocks == {3 * nchunk if nchunk < 200 else 3 * nchunk // 4 if nchunk < 1000 else 3}
 """)
+
+
+def test_beam_push_reads_its_counts_into_pinned_memory(stub):
+    """A copy to pageable memory goes through a staging buffer, with a wait of its own."""
+    run(stub, """
+ctx = qps.Ctx(4, 4, 4)
+bm = qps.Beam(ctx, np_=(8, 8, 8), sigma=(1.0, 1.0, 1.0), center=(0.0, 0.0, 5.0), peak=1.0)
+e, b = qps.Field3d(ctx, 3), qps.Field3d(ctx, 3)
+was = stub.stub_pageable()
+bm.push(e, b, ctx.dex, ctx.dxi)
+assert stub.stub_pageable() == was
+""")

@@ -138,7 +138,7 @@ hipError_t hipFuncSetAttribute(const void *fn, hipFuncAttribute, int v)
 }
 hipError_t hipGetLastError() { const hipError_t e = last; last = hipSuccess; return e; }
 const char *hipGetErrorString(hipError_t) { return "stub error"; }
-hipError_t hipSetDevice(int d) { cur = d; return d == 0 || d == 1 ? hipSuccess : hipErrorInvalidDevice; }
+hipError_t hipSetDevice(int d) { cur = d; return d >= 0 && d < 4 ? hipSuccess : hipErrorInvalidDevice; }
 hipError_t hipGetDevice(int *d) { *d = cur; return hipSuccess; }
 hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t a, int)
 {

@@ -167,8 +167,10 @@ def test_convolution_within_the_devices_lds(stub, cin):
 stub.stub_limits(163840, 256)
 assert conv(128, 128, {cin}, 32) == 0
 need = stub.stub_lds(b"k_conv3x3")
+stub.hipSetDevice(1)
 stub.stub_limits(need, 256)
 assert conv(128, 128, {cin}, 32) == 0
+stub.hipSetDevice(2)
 stub.stub_limits(need - 1, 256)
 assert conv(128, 128, {cin}, 32) == 1
 """)
@@ -181,6 +183,7 @@ def test_convolution_blocks_follow_the_compute_units(stub):
 stub.stub_limits(163840, 4)
 conv(16, 16, 16, 16)
 assert stub.stub_lds(b"k_conv3x3") == (18 * 6 + 144) * 48
+stub.hipSetDevice(1)
 stub.stub_limits(163840, 256)
 conv(16, 16, 16, 16)
 assert stub.stub_lds(b"k_conv3x3") == (18 * 3 + 144) * 48

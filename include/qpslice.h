@@ -130,13 +130,14 @@ int qp_ctx_profile_get(qp_ctx *ctx, int kind, double *total_ms, int64_t *count,
  * QP_TUNE_FFT at its default (0 in FP32, 1 in FP64) lets the slice loop run its
  * field solves with the y transforms and the modes in one kernel (both sides up
  * to 1024), and the FP32 transforms of whole fields without a transpose (nx up
- * to 1024, at 2048 from 512 rows on).  Otherwise 1 folds the transpose between the x and y passes of
- * every transform into the y pass (column-pair reads / writes) instead of a
- * separate LDS-tiled transpose; 0, 2, 3 and 4 keep the transpose and pad the
- * transforms' LDS by one point per 16 points in FP32 or 8 in FP64 (0), or per
- * 8, 32 or 4 points (2, 3, 4); 5 and 6 fold the transpose only in the k -> real
- * or only in the real -> k direction; 7 is the default's form of the separate
- * transforms (0's in FP32, 1's in FP64).  Results are identical.
+ * to 1024, at 2048 from 512 rows of all components on).  Otherwise 1 folds
+ * the transpose between the x and y passes of every transform into the y pass
+ * (column-pair reads / writes) instead of a separate LDS-tiled transpose; 0,
+ * 2, 3 and 4 keep the transpose and pad the transforms' LDS by one point per
+ * 16 points in FP32 or 8 in FP64 (0), or per 8, 32 or 4 points (2, 3, 4); 5
+ * and 6 fold the transpose only in the k -> real or only in the real -> k
+ * direction; 7 is the default's form of the separate transforms (0's in FP32,
+ * 1's in FP64).  Results are identical.
  * QP_TUNE_PUSH selects how the plasma push re-sorts the particles: 0 (default)
  * counts the destination bins in a first pass that stores nothing per
  * particle, then pushes again and stores every particle at its sorted place;
@@ -459,15 +460,18 @@ int qp_sim_renew(qp_sim *sim, double s);
  * same graphs serve every slice; with tol > 0 a slice is cut into graphs
  * between its passes, of which qp_scan_run launches as many as each
  * simulation's residuals ask for (the kernels of a pass behind the converged
- * one return at once; the stopping test and the result are qp_slice_run's); the particle
- * move check is read once per qp_scan_run; the mixed corrector and the 3-D
- * diagnostics (cbq, psi, current) are not available (QP_ERR_UNSUPPORTED).
+ * one return at once; the stopping test and the result are qp_slice_run's);
+ * the particle move check is read once per qp_scan_run; the mixed corrector
+ * and the 3-D diagnostics (cbq, psi, current) are not available
+ * (QP_ERR_UNSUPPORTED).
  * Create after qp_sim_begin_step; the simulations must have profiling off. */
 typedef struct qp_scan qp_scan;
 int qp_scan_create(qp_sim *const *sims, int n, int iter_max, double tol, qp_scan **out);
 /* nslices slices of every simulation (each continues from its last slice),
  * ordered after the work already enqueued on the simulations' streams and
- * before later work; waits for them, then checks the particle moves */
+ * before later work; waits for them, then checks the particle moves.  After an
+ * error the simulations stand at different slices: the scan refuses further
+ * runs (QP_ERR_STATE) */
 int qp_scan_run(qp_scan *scan, int nslices);
 /* passes[j - 1] = corrector passes of slice j (j = 1..nslices) of one
  * simulation, as the captured slices recorded them */

@@ -545,7 +545,7 @@ __device__ __forceinline__ R amjdp_one(const Fields6<R> &F, R fx, R fy, R x, R y
 // ADD: the sums are added to planes (DepOut::inner), which are read together
 // (emit_nodes8).  2048^2, one particle a cell, the deposit and its additions by
 // launches of their own, with the stores but a plane at a time, and so: FP32 329,
-// 355 and 285 us, FP64 603, 655 and 455.  A kernel of its own: the loads would cost
+// 355 and 260 us, FP64 603, 655 and 447.  A kernel of its own: the loads would cost
 // the deposits without additions registers (a step at 1024^2 in FP32 4 %).
 template <typename R, int RG, int CH, int WPE, bool PSI, bool UQ, int THR = 4, int B = 1,
           bool ADD = false>
@@ -1019,16 +1019,16 @@ k_amjdp_w(TileGeom g, Soa<R> s, const int *__restrict__ off, const R *fxy, const
 // MODE 0 stores the pushed particle in place with its bin and rank (k_scatter
 // then moves it).  MODE 1 stores nothing per particle: only the histogram,
 // counted with LDS integer atomics (the same counts in any order; no ranks).
-// MODE 2 runs after MODE 1 and k_bin_starts (cnt then holds each bin's start
-// within its cell) and the scan of the new cell counts into off_new: it
-// repeats the push on the unchanged input, so bins and ranks are those of
-// MODE 1, and stores each particle at off_new[cell] + start + rank of the
-// alternate arrays o.  raw: fxy holds grad(psi) still, and the gathered E_perp
-// is formed from it and B_perp (efield_x, efield_y).  tot (MODE 1): the
-// particles bound for every tile, summed for k_bin_offsets (one atomic per
-// neighbour that gets any: one per wave and group of tiles took 80 us more at
-// 1024^2); MODE 2 clears them for the next push.  The two passes read the particle record twice and
-// write it once, where push and scatter read it twice and write it twice.
+// MODE 2 runs after MODE 1 and k_bin_offsets, which turns cnt into each bin's
+// start within its cell and fills off_new: it repeats the push on the unchanged
+// input, so bins and ranks are those of MODE 1, and stores each particle at
+// off_new[cell] + start + rank of the alternate arrays o.  raw: fxy holds
+// grad(psi) still, and the gathered E_perp is formed from it and B_perp
+// (efield_x, efield_y).  tot (MODE 1): the particles bound for every tile, summed
+// for k_bin_offsets (one atomic per neighbour that gets any: one per wave and
+// group of tiles took 80 us more at 1024^2); MODE 2 clears them for the next push.
+// The two passes read the particle record twice and write it once, where push and
+// scatter read it twice and write it twice.
 constexpr int NBINS = 9 * TCELLS;
 constexpr int PUSH_WIDE = 1024;   // threads of a block where tiles are few (push_t)
 constexpr int BIN_BITS = 12;
@@ -1053,7 +1053,7 @@ k_push(TileGeom g, Soa<R> s, Soa<R> o, const int *__restrict__ off,
         for (int k = tid; k < NBINS * NW / 4; k += NT) whist[k] = 0;
     const int tx0 = S % g.mx1, ty0 = S / g.mx1;
     const int p0 = off[S * TCELLS], p1 = off[(S + 1) * TCELLS];
-    // the particle record of chunk c0 is loaded while chunk c0 - 256 is ranked
+    // the particle record of chunk c0 is loaded while chunk c0 - NT is ranked
     R nx_ = R(0), ny_ = R(0), npx = R(0), npy = R(0), npz = R(0), np6 = R(1), np7 = R(1);
     R nq = R(0);
     auto fetch = [&](int c) {
@@ -1640,7 +1640,6 @@ static int deposit_border(qp_ctx *c, const DepOut<R> &out, int ncomp, int fold,
     return QP_OK;
 }
 
-// species charge into a real-space plane (overwritten), guard-folded
 // Deposit launch shapes: rows per group RG (16/RG lanes per cell; 0: chosen
 // per tile), staging chunk CH and a waves-per-SIMD floor WPE (4 caps the
 // kernel at 128 VGPRs).  Variant 0 of each table is the default; qp_ctx_tune
@@ -1730,10 +1729,10 @@ static int deposit_q_out(qp_species *sp, const DepOut<R> &out, R *halo = nullptr
     return deposit_border<R>(sp->ctx, out, 1, 1, halo, 1, job);
 }
 
-template <typename R>
-static int deposit_q_t(qp_species *sp, R *plane, R *halo = nullptr)
+// species charge into a real-space plane (overwritten), guard-folded
+template <typename R> static int deposit_q_t(qp_species *sp, R *plane)
 {
-    return deposit_q_out<R>(sp, dep_plain<R>(&plane, 1), halo);
+    return deposit_q_out<R>(sp, dep_plain<R>(&plane, 1));
 }
 
 // Marks the species' charge uniform (or not); a uniform q is written into
@@ -2123,7 +2122,6 @@ static int amjdp_out(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
     return deposit_border<R>(sp->ctx, out, 8, 1, nullptr, bands, job);
 }
 
-// the species' own cu, dcu, amu (overwritten)
 // qdp_species2d with the slice's additions fused into the deposit
 // (species2d_class.f03:166-185): this%q = deposit; q = this%q + q;
 // q = qn + q.  first: q holds nothing yet (the slice loop zeroed it).  bp: the
@@ -2175,7 +2173,8 @@ static int amjdp_fused_t(qp_species *sp, const qp_field2d *ef, const qp_field2d 
     return rc;
 }
 
-// amjdp_species2d's deposit (species2d_class.f03:187-218) into the species' planes
+// amjdp_species2d's deposit (species2d_class.f03:187-218) into the species' own
+// cu, dcu, amu (overwritten)
 template <typename R>
 static int amjdp_t(qp_species *sp, const qp_field2d *ef, const qp_field2d *bf,
                    const qp_field2d *psit, double dex)

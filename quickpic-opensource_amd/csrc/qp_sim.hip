@@ -674,7 +674,9 @@ static constexpr int SCAN_POLLS = 1 << 14;
 // to 5.8 passes of at most 20: one graph holding a slice of all instances with
 // all 20 passes 87 ms (a pass after convergence still costs its launches), cut
 // with a wait for the slowest instance in each slice 80 ms and 33 ms for freeing
-// its graphs, the instances apart from each other 76 ms and 1 ms.
+// its graphs, the instances apart from each other 76 ms and 1 ms.  The number
+// rests on that scan: a slice that converges sooner launches four all the same
+// (they return at once).
 static constexpr int SCAN_FIRST = 4;
 
 static void part_free(ScanPart &p)

@@ -9,12 +9,14 @@
 //   inverse x  scratch planes [kx][y] -> rows y of the real planes
 //
 // The arithmetic is that of the separate transforms and k-space kernels, value
-// by value, so the fields are theirs.  Only rows of one kx meet in a mode, so
-// no planes cross memory between the two y transforms.  The field solves of a
+// by value and with the same fused multiply-adds, so the fields are theirs bit
+// for bit.  Only rows of one kx meet in a mode, so no planes cross memory
+// between the two y transforms.  The field solves of a
 // slice (4.2 to 5.25 passes) took, with the separate kernels and with these:
 //   512^2 FP32   334 -> 243 us      1024^2 FP32  724 -> 601 us
 //   1024^2 FP64  511 -> 451 us (two passes)
-//   128^2 FP64   a whole slice 198 -> 158 us (35 -> 25 launches)
+//   128^2 FP64   a whole slice of one species, two passes, 29 -> 16 launches
+//                (with what they let the other kernels take over)
 //
 // Which grids: both sides up to 1024 (fused_fields).  A row pair of all eight
 // components has to fit the 160 KB of LDS for the exchange between the

@@ -192,8 +192,10 @@ def run_sequential(insts, nslices):
 
 def run_graph(insts, nslices, chunk=None):
     """All instances from their captured slices, replayed nslices times
-    (in runs of `chunk` slices); returns the wall time of the replays.  Each
-    instance's passes per slice go to x.passes."""
+    (in runs of `chunk` slices); returns the wall time of the runs, which holds
+    making the graphs of further passes executable where a slice first needs
+    them (beside running kernels: measured, it does not show).  Each instance's
+    passes per slice go to x.passes."""
     for x in insts:
         x.begin()
     scan = qps.Scan([x.sim for x in insts], iter_max=insts[0].iter, tol=insts[0].tol)
